@@ -98,6 +98,21 @@ struct alignas(128) WideNode {
 };
 static_assert(sizeof(WideNode) == 128, "wide node layout");
 
+// Box of a wave-tree group and the tree itself (wave_tree.hpp).
+struct alignas(16) GroupBox {
+  float lo[3], pad0, hi[3], pad1;
+};
+static_assert(sizeof(GroupBox) == 32, "group box layout");
+
+struct WaveTree {
+  const GroupBox *l0, *l1, *l2;
+  uint32_t c0, c1, c2;  // groups per level
+  uint32_t n;           // leaves
+  double centre[3];
+  const double *LX, *LY, *LZ;
+  const uint32_t *leaf_id;
+};
+
 __host__ __device__ inline uint64_t order_key(uint64_t b) {
   if (b == 0x8000000000000000ull) b = 0;  // -0 -> +0
   return (b >> 63) ? ~b : (b ^ 0x8000000000000000ull);

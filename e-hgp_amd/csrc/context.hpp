@@ -67,6 +67,8 @@ struct Context {
   DevBuf<uint32_t> parent_int, parent_leaf;
   DevBuf<uint32_t> wit;       // 6 witnesses per internal node (lo xyz, hi xyz)
   DevBuf<WideNode> wide;      // FP32 two-level copy of the internal nodes (ball and k-NN queries)
+  DevBuf<GroupBox> groups;    // wave tree: level 0, 1 and 2 boxes (wave_tree.hpp), relative to centre
+  double centre[3] = {0, 0, 0};
   DevBuf<uint32_t> counter;
   RadixSorter sorter;
   Scanner scanner;
@@ -102,6 +104,7 @@ struct Context {
 
 // lbvh.hip
 void canonicalize_and_build(Context &c);
+WaveTree wave_tree(const Context &c);
 void export_snapshot(Context &c, uint64_t *leaves, uint64_t *nodes, uint64_t *counters);
 
 }  // namespace mhgp

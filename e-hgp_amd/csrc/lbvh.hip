@@ -371,6 +371,75 @@ __global__ void k_wide_nodes(int64_t m, const Node *__restrict__ nodes, const do
   out[i] = w;
 }
 
+// Wave-tree boxes (wave_tree.hpp): one workgroup per level-1 group, its 16
+// waves reducing four level-0 groups each; the level-1 box follows from them
+// in LDS.  Bound by the read of the leaves (24 B each).
+constexpr int kGroupBlock = 1024;
+__global__ void __launch_bounds__(kGroupBlock) k_group_boxes(int64_t n, double cx, double cy, double cz,
+                                                             const double *__restrict__ LX,
+                                                             const double *__restrict__ LY,
+                                                             const double *__restrict__ LZ, GroupBox *l0,
+                                                             GroupBox *l1) {
+  __shared__ float box[64][6];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c0 = (n + 63) / 64;
+  for (int j = wave; j < 64; j += kGroupBlock / 64) {
+    const int64_t g = (int64_t)blockIdx.x * 64 + j;
+    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    const int64_t p = g * 64 + lane;
+    if (p < n) {
+      const double d[3] = {LX[p] - cx, LY[p] - cy, LZ[p] - cz};
+      for (int a = 0; a < 3; ++a) {
+        v[a] = __double2float_rd(d[a]);
+        v[3 + a] = __double2float_ru(d[a]);
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        v[a] = fminf(v[a], __shfl_xor(v[a], o));
+        v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
+      }
+    if (lane == 0) {
+      for (int a = 0; a < 6; ++a) box[j][a] = v[a];
+      if (g < c0) l0[g] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float v[6];
+    for (int a = 0; a < 6; ++a) v[a] = box[lane][a];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        v[a] = fminf(v[a], __shfl_xor(v[a], o));
+        v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
+      }
+    if (lane == 0) l1[blockIdx.x] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
+  }
+}
+
+// Level-2 boxes, one wave per group (clouds of more than 262 144 points).
+__global__ void __launch_bounds__(64) k_group_top(uint32_t c1, const GroupBox *__restrict__ l1, GroupBox *l2) {
+  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+  float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  if (i < c1)
+    for (int a = 0; a < 3; ++a) {
+      v[a] = l1[i].lo[a];
+      v[3 + a] = l1[i].hi[a];
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      v[a] = fminf(v[a], __shfl_xor(v[a], o));
+      v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
+    }
+  if (threadIdx.x == 0) l2[blockIdx.x] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
+}
+
 // Power-of-two change of unit (context.hpp, scale_exp): possible only when
 // every scaled coordinate stays a normal (or zero) finite binary64.
 __global__ void k_scale_check(const double *__restrict__ X, const double *__restrict__ Y,
@@ -500,8 +569,21 @@ void canonicalize_and_build(Context &c) {
   if (internal)
     hipLaunchKernelGGL(k_wide_nodes, dim3(blocks_for(internal, 256)), dim3(256), 0, s, internal, c.nodes.p, c.LX.p,
                        c.LY.p, c.LZ.p, c.wide.p);
+  const int64_t c0 = (n + 63) / 64, c1 = (c0 + 63) / 64, c2 = (c1 + 63) / 64;
+  c.groups.ensure(c0 + c1 + c2);
+  for (int a = 0; a < 3; ++a) c.centre[a] = std::ldexp(0.5 * bounds[a] + 0.5 * bounds[3 + a], c.scale_exp);
+  hipLaunchKernelGGL(k_group_boxes, dim3(c1), dim3(kGroupBlock), 0, s, n, c.centre[0], c.centre[1], c.centre[2],
+                     c.LX.p, c.LY.p, c.LZ.p, c.groups.p, c.groups.p + c0);
+  if (c2 > 1)
+    hipLaunchKernelGGL(k_group_top, dim3(c2), dim3(64), 0, s, (uint32_t)c1, c.groups.p + c0, c.groups.p + c0 + c1);
   MHGP_LAUNCH_CHECK();
   c.lbvh_ready = true;
+}
+
+WaveTree wave_tree(const Context &c) {
+  const uint32_t n = (uint32_t)c.n, c0 = (n + 63) / 64, c1 = (c0 + 63) / 64, c2 = (c1 + 63) / 64;
+  return {c.groups.p, c.groups.p + c0, c.groups.p + c0 + c1, c0, c1, c2, n,
+          {c.centre[0], c.centre[1], c.centre[2]}, c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p};
 }
 
 void export_snapshot(Context &c, uint64_t *leaves, uint64_t *nodes_out, uint64_t *counters) {

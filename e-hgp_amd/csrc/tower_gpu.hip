@@ -875,14 +875,12 @@ __global__ void k_raw_of_dense(int64_t M, const uint32_t *__restrict__ dense, ui
 }
 
 // FP64 squared distance from every point to the last of its listed neighbours;
-// 0 (the list is never used) when the traversal that made the list dropped a
-// subtree (flag 4) or left a slot empty.
-__global__ void k_nn_last_d2(int64_t n, const uint32_t *__restrict__ nn, const uint8_t *__restrict__ flags,
-                             const double *__restrict__ X, const double *__restrict__ Y,
-                             const double *__restrict__ Z, double *d2) {
+// 0 (the list is never used) when a slot is empty.
+__global__ void k_nn_last_d2(int64_t n, const uint32_t *__restrict__ nn, const double *__restrict__ X,
+                             const double *__restrict__ Y, const double *__restrict__ Z, double *d2) {
   int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  bool whole = (flags[p] & 4) == 0;
+  bool whole = true;
   for (int j = 0; j < kNearK; ++j) whole &= nn[p * kNearK + j] < (uint64_t)n;
   const uint32_t q = nn[p * kNearK + kNearK - 1];
   if (!whole) {
@@ -937,8 +935,8 @@ void tower_prefetch_neighbours(Context &c) {
   MHGP_HIP(hipEventRecord(W.nn_start, c.stream));
   MHGP_HIP(hipStreamWaitEvent(W.vm_stream, W.nn_start, 0));
   knn_all(c, kNearK, W.nn.p, W.nn_flags.p, W.vm_stream);
-  hipLaunchKernelGGL(k_nn_last_d2, dim3(blocks_for(c.n, 256)), dim3(256), 0, W.vm_stream, c.n, W.nn.p, W.nn_flags.p,
-                     c.X.p, c.Y.p, c.Z.p, W.nn_d2.p);
+  hipLaunchKernelGGL(k_nn_last_d2, dim3(blocks_for(c.n, 256)), dim3(256), 0, W.vm_stream, c.n, W.nn.p, c.X.p,
+                     c.Y.p, c.Z.p, W.nn_d2.p);
   MHGP_LAUNCH_CHECK();
   MHGP_HIP(hipEventRecord(W.nn_done, W.vm_stream));
   W.nn_pending = true;
