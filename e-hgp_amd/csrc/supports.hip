@@ -37,7 +37,6 @@
 #include <cstdio>
 #include <cstring>
 #include <condition_variable>
-#include <map>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -48,14 +47,14 @@
 #include "predicates.hpp"
 #include "supports.hpp"
 #include "timing.hpp"
-#include "traverse.hpp"
+#include "wave_tree.hpp"
 
 namespace mhgp {
 
 int64_t catalog_device_bytes(const CatalogBuffers &b) {
   return b.radius.bytes() + b.gcount.bytes() + b.goff.bytes() + b.glist.bytes() + b.need.bytes() +
          b.status.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
-         b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.scratch.bytes() + b.anchors.bytes() + b.overflow.bytes() +
+         b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.scratch.bytes() + b.anchors.bytes() +
          b.total.bytes() + b.run_count.bytes() + b.run_pos.bytes() + b.run_gidx.bytes() + b.run_new.bytes() +
          b.run_link.bytes() + b.run_rec.bytes();
 }
@@ -1608,257 +1607,94 @@ __global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anch
   anchor_faces<false, true>(P, w, u, M, &sK, &sregion);
 }
 
-// Ball count / emit around every anchor of the list.
-// Pruning runs in FP32 on the two-level LBVH copy (boxes rounded outward, the
-// radius inflated by the rounding of the query and of the FP32 arithmetic; a
-// non-finite bound prunes nothing); the leaf test is the FP64 one.
-template <bool EMIT, int B>
-__global__ void __launch_bounds__(B) k_gather(int64_t n, const WideNode *__restrict__ wide,
-                                                const double *__restrict__ LX,
-                                                const double *__restrict__ LY,
-                                                const double *__restrict__ LZ,
-                                                const uint32_t *__restrict__ leaf_id,
-                                                const uint32_t *__restrict__ leaf_pos,
-                                                const uint32_t *__restrict__ anchors, uint32_t count,
-                                                const double *__restrict__ radius, uint32_t *gcount,
-                                                const uint64_t *__restrict__ goff, uint32_t *glist,
-                                                uint32_t *overflow) {
-  // depth-first over 4-way nodes: at most 3 pending siblings per level
-  constexpr int kStack = 96;
-  __shared__ uint32_t stk[kStack * B];
-  const int lane = threadIdx.x;
-  uint32_t a = blockIdx.x * blockDim.x + lane;
-  if (a >= count) return;
-  const uint32_t u = anchors[a];
-  const uint32_t p = leaf_pos[u];
-  const double q[3] = {LX[p], LY[p], LZ[p]};
-  const double R = radius[u];
-  const double R2 = R * R * (1.0 + 1e-9);
-  const float qf[3] = {(float)q[0], (float)q[1], (float)q[2]};
-  const double qmax = fmax(fmax(fabs(q[0]), fabs(q[1])), fabs(q[2]));
-  const double rb = sqrt(R2) * (1.0 + 1e-6) + qmax * 1e-6 + 1e-30;
-  float Tf = (float)(rb * rb * (1.0 + 1e-5));
-  if (!(Tf < 3.0e38f)) Tf = INFINITY;
-  uint32_t cnt = 0;
-  uint64_t base = EMIT ? goff[u] : 0;
-  int sp = 0;
-  if (n > 1) stk[(sp++) * B + lane] = 0;
-  while (sp) {
-    const WideNode &N = wide[stk[(--sp) * B + lane]];
-    for (int c = 0; c < 4; ++c) {
-      const uint32_t x = N.child[c];
-      if (x == kInvalid) continue;
-      float d2 = 0.f;
-      for (int ax = 0; ax < 3; ++ax) {
-        const float d = fmaxf(fmaxf(N.lo[c][ax] - qf[ax], qf[ax] - N.hi[c][ax]), 0.f);
-        d2 += d * d;
-      }
-      if (d2 > Tf) continue;
-      if (x & kLeafBit) {
-        const uint32_t lp = x & ~kLeafBit;
-        if (lp == p) continue;
-        const double dx = LX[lp] - q[0], dy = LY[lp] - q[1], dz = LZ[lp] - q[2];
-        if (dx * dx + dy * dy + dz * dz <= R2) {
-          if (EMIT) glist[base + cnt] = leaf_id[lp];
-          cnt++;
-        }
-      } else if (sp < kStack) {
-        stk[(sp++) * B + lane] = x;
-      } else {
-        atomicOr(overflow, 1u);
-      }
-    }
-  }
-  if (!EMIT) gcount[u] = cnt;
-}
-
-// The same gather with one wave per anchor, for the widened passes, whose
-// radii hold hundreds to thousands of points: the wave pops up to 64 pending
-// nodes at once (one per lane), tests their four children, and appends hits
-// and pending children with ballot prefix counts, so one anchor's traversal
-// is spread over 64 lanes instead of walked by one.  The traversal order is
-// fixed, so the count and emit passes visit the same points.
-constexpr int kWaveGatherStack = 4096;
-constexpr int kWaveGatherBlock = 128;  // two waves, two anchors per workgroup
+// Ball count / emit around every anchor of the list: one wave per anchor over
+// the wave tree, hits appended with ballot prefix counts.  The traversal
+// order is fixed, so the count and emit passes visit the same points.  Bound
+// by VALU issue of the group tests and distances.  With one thread per anchor
+// walking the binary tree a pass took 230 us at 256 points and 0.7-0.9 ms at
+// 17 117; the catalogue of 256 points went from 2.92 to 2.27 ms with this and
+// the radius kernel below, the 17 117-point pipeline from 23.5 to 22.1 ms.
+constexpr int kGatherBlock = 256;  // four waves, four anchors
 template <bool EMIT>
-__global__ void __launch_bounds__(kWaveGatherBlock) k_gather_wave(int64_t n, const WideNode *__restrict__ wide,
-                                                                  const double *__restrict__ LX,
-                                                                  const double *__restrict__ LY,
-                                                                  const double *__restrict__ LZ,
-                                                                  const uint32_t *__restrict__ leaf_id,
-                                                                  const uint32_t *__restrict__ leaf_pos,
-                                                                  const uint32_t *__restrict__ anchors, uint32_t count,
-                                                                  const double *__restrict__ radius, uint32_t *gcount,
-                                                                  const uint64_t *__restrict__ goff, uint32_t *glist,
-                                                                  uint32_t *overflow) {
-  __shared__ uint32_t stk[kWaveGatherBlock / 64][kWaveGatherStack];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t a = blockIdx.x * (kWaveGatherBlock / 64) + wave;
+__global__ void __launch_bounds__(kGatherBlock) k_gather(WaveTree T, const uint32_t *__restrict__ leaf_pos,
+                                                         const uint32_t *__restrict__ anchors, uint32_t count,
+                                                         const double *__restrict__ radius, uint32_t *gcount,
+                                                         const uint64_t *__restrict__ goff, uint32_t *glist) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t a = blockIdx.x * (kGatherBlock / 64) + (threadIdx.x >> 6);
   if (a >= count) return;  // uniform over the wave
-  uint32_t *S = stk[wave];
   const uint64_t below = (1ull << lane) - 1ull;
   const uint32_t u = anchors[a];
   const uint32_t p = leaf_pos[u];
-  const double q[3] = {LX[p], LY[p], LZ[p]};
+  const double q[3] = {T.LX[p], T.LY[p], T.LZ[p]};
   const double R = radius[u];
   const double R2 = R * R * (1.0 + 1e-9);
-  const float qf[3] = {(float)q[0], (float)q[1], (float)q[2]};
-  const double qmax = fmax(fmax(fabs(q[0]), fabs(q[1])), fabs(q[2]));
-  const double rb = sqrt(R2) * (1.0 + 1e-6) + qmax * 1e-6 + 1e-30;
-  float Tf = (float)(rb * rb * (1.0 + 1e-5));
-  if (!(Tf < 3.0e38f)) Tf = INFINITY;
-  uint32_t cnt = 0, sp = 0;
+  const WaveQuery Q(T, q[0], q[1], q[2]);
+  float Tf = Q.bound(R2);
   const uint64_t base = EMIT ? goff[u] : 0;
-  if (n > 1) {
-    if (lane == 0) S[0] = 0;
-    sp = 1;
-  }
-  bool lost = false;
-  wave_sync();
-  while (sp > 0) {
-    const uint32_t take = min(sp, 64u);
-    sp -= take;
-    const uint32_t node = (uint32_t)lane < take ? S[sp + lane] : kInvalid;
-    wave_sync();  // every pop is read before a push overwrites it
-    const WideNode *N = node != kInvalid ? &wide[node] : nullptr;
-    for (int c = 0; c < 4; ++c) {
-      bool hit = false, push = false;
-      uint32_t x = kInvalid;
-      if (N) {
-        x = N->child[c];
-        if (x != kInvalid) {
-          float d2 = 0.f;
-          for (int ax = 0; ax < 3; ++ax) {
-            const float d = fmaxf(fmaxf(N->lo[c][ax] - qf[ax], qf[ax] - N->hi[c][ax]), 0.f);
-            d2 += d * d;
-          }
-          if (d2 <= Tf) {
-            if (x & kLeafBit) {
-              const uint32_t lp = x & ~kLeafBit;
-              if (lp != p) {
-                const double dx = LX[lp] - q[0], dy = LY[lp] - q[1], dz = LZ[lp] - q[2];
-                hit = dx * dx + dy * dy + dz * dz <= R2;
-                if (hit) x = lp;
-              }
-            } else {
-              push = true;
-            }
-          }
-        }
-      }
-      const uint64_t mh = __ballot(hit);
-      if (EMIT && hit) glist[base + cnt + (uint32_t)__popcll(mh & below)] = leaf_id[x];
-      cnt += (uint32_t)__popcll(mh);
-      const uint64_t mp = __ballot(push);
-      const uint32_t slot = sp + (uint32_t)__popcll(mp & below);
-      if (push) {
-        if (slot < (uint32_t)kWaveGatherStack) S[slot] = x;
-        else lost = true;
-      }
-      sp = min(sp + (uint32_t)__popcll(mp), (uint32_t)kWaveGatherStack);
-    }
-    wave_sync();
-  }
-  if (lost) atomicOr(overflow, 1u);
+  uint32_t cnt = 0;
+  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+    const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
+    const double dx = T.LX[at] - q[0], dy = T.LY[at] - q[1], dz = T.LZ[at] - q[2];
+    const bool hit = lp < T.n && lp != p && dx * dx + dy * dy + dz * dz <= R2;
+    const uint64_t m = __ballot(hit);
+    if (EMIT && hit) glist[base + cnt + (uint32_t)__popcll(m & below)] = T.leaf_id[at];
+    cnt += (uint32_t)__popcll(m);
+  });
   if (!EMIT && lane == 0) gcount[u] = cnt;
 }
 
 // Initial gather radius of every point: factor x the distance to its kq-th
-// nearest neighbour (kq <= 32), found in FP32 over the two-level LBVH copy
-// with a register-resident sorted list.  The radius only sizes the first
-// gather; the certificate widens any anchor it does not cover.
-constexpr int kRadiusK = 32;
-constexpr int kRadiusStack = 64;
-template <int B>
-__global__ void __launch_bounds__(B) k_knn_radius(int64_t n, int kq, float factor, const WideNode *__restrict__ wide,
-                                                    const double *__restrict__ LX, const double *__restrict__ LY,
-                                                    const double *__restrict__ LZ,
-                                                    const uint32_t *__restrict__ leaf_id, double *radius) {
-  __shared__ uint32_t stk[kRadiusStack * B];
-  const int lane = threadIdx.x;
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + lane;
-  if (p >= n) return;
-  const float q[3] = {(float)LX[p], (float)LY[p], (float)LZ[p]};
-  float best[kRadiusK];
+// nearest neighbour (kq <= 32), from outward-rounded FP32 differences.  The
+// radius only sizes the first gather; the certificate widens any anchor it
+// does not cover.  One wave per point over the wave tree, lane l holding the
+// l-th smallest squared distance so far; bound by VALU issue (182 us at 256
+// points with one thread per point).
+constexpr int kRadiusBlock = 256;  // four waves, four points
+__global__ void __launch_bounds__(kRadiusBlock) k_knn_radius(WaveTree T, int kq, float factor, double *radius) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t p = blockIdx.x * (kRadiusBlock / 64) + (threadIdx.x >> 6);
+  if (p >= T.n) return;
+  const double x = T.LX[p], y = T.LY[p], z = T.LZ[p];
+  const float q[3] = {(float)x, (float)y, (float)z};
+  const WaveQuery Q(T, x, y, z);
+  // the differences are taken in the input's frame, whose FP32 rounding
+  // (query half an ulp, box one ulp per axis) can bring a point nearer by up
+  // to this much
+  const float off = 3.5e-7f * fmaxf(fmaxf(fabsf(q[0]), fabsf(q[1])), fabsf(q[2]));
+  float best = INFINITY, cut = INFINITY, Tf = INFINITY;
+  auto group = [&](uint32_t g) {
+    const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
+    const double v[3] = {T.LX[at], T.LY[at], T.LZ[at]};
+    float d2 = 0.f;
 #pragma unroll
-  for (int j = 0; j < kRadiusK; ++j) best[j] = INFINITY;
-  // starting bound: the farthest of kq Morton-order neighbours, a set of kq
-  // other points, so the kq-th nearest distance cannot exceed it (inflated
-  // past the rounding of the outward FP32 leaf boxes, so the traversal still
-  // meets those kq points below the bound)
-  float bound = INFINITY;
-  if (n > kq) {
-    int64_t lo = p - kq / 2;
-    if (lo < 0) lo = 0;
-    if (lo + kq >= n) lo = n - 1 - kq;
-    float m = 0.f;
-    for (int64_t j = lo; j <= lo + kq; ++j) {
-      if (j == p) continue;
-      const float dx = (float)LX[j] - q[0], dy = (float)LY[j] - q[1], dz = (float)LZ[j] - q[2];
-      m = fmaxf(m, dx * dx + dy * dy + dz * dz);
+    for (int a = 0; a < 3; ++a) {
+      const float d = fmaxf(fmaxf(__double2float_rd(v[a]) - q[a], q[a] - __double2float_ru(v[a])), 0.f);
+      d2 += d * d;
     }
-    bound = m * (1.0f + 1e-4f) + 1e-30f;
-  }
-  float cut = bound;  // min(bound, the kq-th smallest so far)
-  int sp = 0;
-  if (n > 1) stk[(sp++) * B + lane] = 0;
-  while (sp) {
-    const WideNode &N = wide[stk[(--sp) * B + lane]];
-    // leaves are taken at once; inner children are pushed far to near, so
-    // the nearest is expanded first and the bound shrinks early
-    float cd[4];
-    uint32_t cx[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const uint32_t x = N.child[c];
-      cd[c] = -1.f;
-      cx[c] = x;
-      if (x == kInvalid) continue;
-      float d2 = 0.f;
-      for (int a = 0; a < 3; ++a) {
-        const float d = fmaxf(fmaxf(N.lo[c][a] - q[a], q[a] - N.hi[c][a]), 0.f);
-        d2 += d * d;
-      }
-      if (!(d2 < cut)) continue;
-      if (x & kLeafBit) {
-        if ((x & ~kLeafBit) == (uint32_t)p) continue;
-        // sorted insertion over static indices (the list stays in registers)
-#pragma unroll
-        for (int j = kRadiusK - 1; j > 0; --j) best[j] = d2 < best[j - 1] ? best[j - 1] : (d2 < best[j] ? d2 : best[j]);
-        best[0] = fminf(best[0], d2);
-        float c2 = INFINITY;
-#pragma unroll
-        for (int j = 0; j < kRadiusK; ++j) c2 = j == kq - 1 ? best[j] : c2;
-        cut = fminf(bound, c2);
-      } else {
-        cd[c] = d2;
-      }
+    const bool valid = lp < T.n && lp != p;
+    uint64_t cand = __ballot(valid && d2 < cut);
+    if (!cand) return;
+    while (cand) {
+      const int i = __builtin_amdgcn_readfirstlane(__ffsll((long long)cand) - 1);
+      cand &= cand - 1;
+      const float cd = __uint_as_float(lane_u32(__float_as_uint(d2), i));
+      const uint32_t pos = (uint32_t)__popcll(__ballot(best <= cd));
+      const float up = __shfl_up(best, 1u);
+      best = lane < pos ? best : (lane == pos ? cd : up);
+      cut = __uint_as_float(lane_u32(__float_as_uint(best), kq - 1));
+      cand &= __ballot(d2 < cut);
     }
-    // descending distance (a five-comparator network), then push
-#pragma unroll
-    for (int e = 0; e < 5; ++e) {
-      const int i = e == 0 ? 0 : e == 1 ? 2 : e == 2 ? 0 : e == 3 ? 1 : 1;
-      const int j = e == 0 ? 1 : e == 1 ? 3 : e == 2 ? 2 : e == 3 ? 3 : 2;
-      if (cd[i] < cd[j]) {
-        const float td = cd[i];
-        cd[i] = cd[j];
-        cd[j] = td;
-        const uint32_t tx = cx[i];
-        cx[i] = cx[j];
-        cx[j] = tx;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if (!(cd[c] >= 0.f) || !(cd[c] < cut)) continue;
-      if (sp < kRadiusStack) stk[(sp++) * B + lane] = cx[c];
-    }
-  }
-  // a subtree dropped by a full stack can only raise the kq-th distance found
-  const double d = sqrt((double)cut) * (1.0 + 1e-6);
-  radius[leaf_id[p]] = (double)factor * d;
+    const double r = sqrt((double)cut) * (1.0 + 1e-6) + (double)off;
+    Tf = cut > 0.f ? Q.bound(r * r) : -1.f;  // nothing enters below a zero distance
+  };
+  const uint32_t own = p >> 6;
+  group(own);
+  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+    if (g != own) group(g);
+  });
+  if (lane == 0) radius[T.leaf_id[p]] = (double)factor * (sqrt((double)cut) * (1.0 + 1e-6));
 }
-
 
 // exclusive scan of gcount over the anchor list into goff (single workgroup)
 __global__ void k_scan_offsets(const uint32_t *__restrict__ anchors, uint32_t count,
@@ -1948,90 +1784,15 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
                      std::vector<FallbackRec> &fbs, std::vector<uint32_t> &fb_region,
                      mhgp_catalog_info *info);
 
-// Workgroup tile (queries per workgroup, one query per lane) of the two
-// LBVH traversal kernels of the catalogue, the 32nd-neighbour radius and the
-// gather.  The tile is picked per device and cloud-size class (powers of two
-// of n) by timing every candidate on the first cloud of the class, once per
-// process; both kernels are idempotent, so the timing runs are real work.
-constexpr int kTiles[3] = {64, 128, 256};
-struct TileChoice {
-  int radius = 128, gather = 128;
-};
-std::mutex g_tile_mu;
-std::map<std::pair<int, int>, TileChoice> g_tiles;
-
-template <int B>
 void launch_radius(hipStream_t s, Context &c, int kq, CatalogBuffers &Bf) {
-  hipLaunchKernelGGL(k_knn_radius<B>, dim3(blocks_for(c.n, B)), dim3(B), 0, s, c.n, kq, 2.2f, c.wide.p, c.LX.p,
-                     c.LY.p, c.LZ.p, c.leaf_id.p, Bf.radius.p);
-}
-void launch_radius(int B, hipStream_t s, Context &c, int kq, CatalogBuffers &Bf) {
-  if (B == 64) launch_radius<64>(s, c, kq, Bf);
-  else if (B == 256) launch_radius<256>(s, c, kq, Bf);
-  else launch_radius<128>(s, c, kq, Bf);
-}
-
-template <bool EMIT, int B>
-void launch_gather(hipStream_t s, Context &c, CatalogBuffers &Bf, uint32_t cnt, uint32_t *overflow) {
-  hipLaunchKernelGGL((k_gather<EMIT, B>), dim3(blocks_for(cnt, B)), dim3(B), 0, s, c.n, c.wide.p, c.LX.p, c.LY.p,
-                     c.LZ.p, c.leaf_id.p, c.leaf_pos.p, Bf.anchors.p, cnt, Bf.radius.p, Bf.gcount.p, Bf.goff.p,
-                     Bf.glist.p, overflow);
-}
-template <bool EMIT>
-void launch_gather(int B, hipStream_t s, Context &c, CatalogBuffers &Bf, uint32_t cnt, uint32_t *overflow) {
-  if (B == 64) launch_gather<EMIT, 64>(s, c, Bf, cnt, overflow);
-  else if (B == 256) launch_gather<EMIT, 256>(s, c, Bf, cnt, overflow);
-  else launch_gather<EMIT, 128>(s, c, Bf, cnt, overflow);
+  hipLaunchKernelGGL(k_knn_radius, dim3(blocks_for(c.n, kRadiusBlock / 64)), dim3(kRadiusBlock), 0, s, wave_tree(c),
+                     kq, 2.2f, Bf.radius.p);
 }
 
 template <bool EMIT>
-void launch_gather_wave(hipStream_t s, Context &c, CatalogBuffers &Bf, uint32_t cnt, uint32_t *overflow) {
-  const uint32_t per = kWaveGatherBlock / 64;
-  hipLaunchKernelGGL((k_gather_wave<EMIT>), dim3((cnt + per - 1) / per), dim3(kWaveGatherBlock), 0, s, c.n, c.wide.p,
-                     c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p, c.leaf_pos.p, Bf.anchors.p, cnt, Bf.radius.p, Bf.gcount.p,
-                     Bf.goff.p, Bf.glist.p, overflow);
-}
-
-// Times `run(tile)` for every candidate tile; returns the fastest.
-template <class F>
-int fastest_tile(hipStream_t s, F &&run) {
-  hipEvent_t a, b;
-  MHGP_HIP(hipEventCreate(&a));
-  MHGP_HIP(hipEventCreate(&b));
-  int best = 128;
-  float best_ms = INFINITY;
-  for (int B : kTiles) {
-    run(B);  // warm (code objects, caches)
-    MHGP_HIP(hipEventRecord(a, s));
-    run(B);
-    MHGP_HIP(hipEventRecord(b, s));
-    MHGP_HIP(hipEventSynchronize(b));
-    float ms = 0;
-    MHGP_HIP(hipEventElapsedTime(&ms, a, b));
-    if (ms < best_ms) { best_ms = ms; best = B; }
-  }
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
-  return best;
-}
-
-TileChoice tiles_for(Context &c, CatalogBuffers &Bf, int kq, uint32_t *overflow) {
-  const std::pair<int, int> key{c.device, (int)std::ilogb((double)std::max<int64_t>(c.n, 1))};
-  {
-    std::lock_guard<std::mutex> g(g_tile_mu);
-    auto it = g_tiles.find(key);
-    if (it != g_tiles.end()) return it->second;
-  }
-  hipStream_t s = c.stream;
-  TileChoice t;
-  t.radius = fastest_tile(s, [&](int B) { launch_radius(B, s, c, kq, Bf); });
-  // the gather's count pass over every point in Morton order, as the first
-  // anchor pass takes them
-  const uint32_t cnt = (uint32_t)c.n;
-  MHGP_HIP(hipMemcpyAsync(Bf.anchors.p, c.leaf_id.p, cnt * 4, hipMemcpyDeviceToDevice, s));
-  t.gather = fastest_tile(s, [&](int B) { launch_gather<false>(B, s, c, Bf, cnt, overflow); });
-  std::lock_guard<std::mutex> g(g_tile_mu);
-  return g_tiles.emplace(key, t).first->second;
+void launch_gather(hipStream_t s, Context &c, CatalogBuffers &Bf, uint32_t cnt) {
+  hipLaunchKernelGGL((k_gather<EMIT>), dim3(blocks_for(cnt, kGatherBlock / 64)), dim3(kGatherBlock), 0, s,
+                     wave_tree(c), c.leaf_pos.p, Bf.anchors.p, cnt, Bf.radius.p, Bf.gcount.p, Bf.goff.p, Bf.glist.p);
 }
 
 // Rendezvous of the clouds of one batch: each cloud's thread reaches its
@@ -2192,14 +1953,10 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   // initial gather radius: twice the distance to the min(32, n-1)-th neighbour
   const int kq = (int)std::min<int64_t>(32, n - 1);
   StageTimer tm(s);
-  DevBuf<uint32_t> &overflow = B.overflow;
   DevBuf<uint64_t> &total = B.total;
-  overflow.ensure(1);
   total.ensure(1);
-  MHGP_HIP(hipMemsetAsync(overflow.p, 0, 4, s));
   B.glist.ensure(1);
-  const TileChoice tile = tiles_for(c, B, kq, overflow.p);
-  launch_radius(tile.radius, s, c, kq, B);
+  launch_radius(s, c, kq, B);
   MHGP_LAUNCH_CHECK();
   std::vector<uint32_t> anchors(n);
   std::iota(anchors.begin(), anchors.end(), 0u);
@@ -2236,7 +1993,6 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   B.fb_region.ensure(reg_cap);
   MHGP_HIP(hipMemsetAsync(B.counters.p, 0, 8 * 8, s));
   MHGP_HIP(hipMemsetAsync(B.status.p, 0, n * 4, s));
-  MHGP_HIP(hipMemsetAsync(overflow.p, 0, 4, s));
   open_anchors = 0;
   largest_open = 0;
   std::vector<uint32_t> pending = anchors;
@@ -2245,18 +2001,14 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     if (iter > 12) throw CapacityError("anchor gather radii did not converge");
     const uint32_t cnt = (uint32_t)pending.size();
     MHGP_HIP(hipMemcpyAsync(B.anchors.p, pending.data(), cnt * 4, hipMemcpyHostToDevice, s));
-    // the first pass takes one thread per anchor (small radii); the widened
-    // passes one wave per anchor
-    if (iter == 0) launch_gather<false>(tile.gather, s, c, B, cnt, overflow.p);
-    else launch_gather_wave<false>(s, c, B, cnt, overflow.p);
+    launch_gather<false>(s, c, B, cnt);
     hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, s, B.anchors.p, cnt, B.gcount.p,
                        B.goff.p, total.p);
     uint64_t tot = 0;
     MHGP_HIP(hipMemcpyAsync(&tot, total.p, 8, hipMemcpyDeviceToHost, s));
     MHGP_HIP(hipStreamSynchronize(s));
     B.glist.ensure(tot + 1);
-    if (iter == 0) launch_gather<true>(tile.gather, s, c, B, cnt, overflow.p);
-    else launch_gather_wave<true>(s, c, B, cnt, overflow.p);
+    launch_gather<true>(s, c, B, cnt);
     Params P{};
     P.X = c.X.p; P.Y = c.Y.p; P.Z = c.Z.p;
     P.gcount = B.gcount.p; P.goff = B.goff.p; P.glist = B.glist.p; P.radius = B.radius.p;
@@ -2445,13 +2197,13 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
         const uint32_t ac = (uint32_t)again.size();
         copy_wait(B.radius.p, rad.data(), n * 8, hipMemcpyHostToDevice, s);
         MHGP_HIP(hipMemcpyAsync(B.anchors.p, again.data(), ac * 4, hipMemcpyHostToDevice, s));
-        launch_gather_wave<false>(s, c, B, ac, overflow.p);
+        launch_gather<false>(s, c, B, ac);
         hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, s, B.anchors.p, ac, B.gcount.p,
                            B.goff.p, total.p);
         MHGP_HIP(hipMemcpyAsync(&tot, total.p, 8, hipMemcpyDeviceToHost, s));
         MHGP_HIP(hipStreamSynchronize(s));
         B.glist.ensure(tot + 1);
-        launch_gather_wave<true>(s, c, B, ac, overflow.p);
+        launch_gather<true>(s, c, B, ac);
         MHGP_HIP(hipMemcpyAsync(gc.data(), B.gcount.p, n * 4, hipMemcpyDeviceToHost, s));
         MHGP_HIP(hipStreamSynchronize(s));
         tm.mark("catalogue big regather");
@@ -2463,10 +2215,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     pending = next;
   }
   tm.mark("catalogue big anchors");
-  uint32_t ovf = 0;
-  copy_wait(&ovf, overflow.p, 4, hipMemcpyDeviceToHost, s);
   copy_wait(ctr, B.counters.p, sizeof(ctr), hipMemcpyDeviceToHost, s);
-  if (ovf) throw std::runtime_error("LBVH traversal stack overflow in the gather");
   if (ctr[4]) throw std::runtime_error("face side queue overflow");
   if (ctr[0] <= event_cap && ctr[1] <= fb_cap && ctr[2] <= reg_cap) break;
   if (attempt >= 2) throw CapacityError("catalogue record queues did not settle after regrowth");

@@ -65,7 +65,6 @@ struct CatalogBuffers {
   DevBuf<uint32_t> ambiguous;     // open-run starts, and the runs left to the host (start, length)
   // small per-call device scratch, kept so that no call frees device memory
   // (a free waits for the whole device, side streams included)
-  DevBuf<uint32_t> overflow;      // gather traversal overflow flag
   DevBuf<uint64_t> total;         // gathered entries of a pass
   DevBuf<uint64_t> run_count;     // open runs, runs left to the host
   DevBuf<uint32_t> run_pos, run_gidx, run_new, run_link;
