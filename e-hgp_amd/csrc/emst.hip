@@ -7,16 +7,23 @@
 // is unique, so the output equals the complete-graph Kruskal anchor
 // (emst.cpp:326).
 //
-// Device rounds: node tags -> per-point search -> per-component atomic minima
-// -> hooking with 2-cycle breaking -> pointer jumping.  FP64 distances that
-// are not provably ordered (near ties that are not both exact) are flagged and
-// settled on the host with exact integer arithmetic.
+// Points and components are numbered by Morton position (a component by one
+// of its points).  A round: labels of the wave tree's groups -> per-point
+// search, one wave per point -> per-component minima -> hooking with 2-cycle
+// breaking -> roots.  A point's nearest external point stays its nearest
+// while it is external (the external set only shrinks), so a search is run
+// again only for points whose last result was absorbed, and not at all when
+// that result's distance, a lower bound ever after, exceeds what another point
+// of the component already offers.  FP64 distances that are not provably
+// ordered (near ties that are not both exact) are flagged and settled on the
+// host with exact integer arithmetic.
 #include <algorithm>
 
 #include "pipeline.hpp"
 #include "stages.hpp"
 #include "timing.hpp"
 #include "traverse.hpp"
+#include "wave_tree.hpp"
 
 namespace mhgp {
 
@@ -27,221 +34,246 @@ __device__ inline uint64_t edge_key(uint32_t a, uint32_t b) {
   return ((uint64_t)lo << 32) | hi;
 }
 
-__global__ void k_init_labels(int64_t n, uint32_t *label) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) label[i] = (uint32_t)i;
+// counters: [0] edges, [1] components, [2] ambiguous components
+struct Rounds {
+  uint32_t *label;                  // component of each position
+  uint32_t *glabel;                 // uniform component of each wave-tree group (levels 0, 1, 2), or kInvalid
+  uint32_t *best_p;                 // nearest external position, kInvalid: none that counts
+  double *best_d;                   // its squared distance; without one, a lower bound of it
+  uint8_t *best_flag;               // 1: near tie, 4: the distance is not exact
+  uint64_t *comp_d, *comp_e;        // per component: least distance (bits), least edge key at it
+  uint32_t *comp_amb, *comp_cw, *comp_ce;  // tie flag; entries in the rounding window, exact equal ones
+  uint32_t *hook, *root;
+  uint32_t *edges, *counters;
+};
+
+__device__ inline double as_double(uint64_t b) { return __longlong_as_double((long long)b); }
+
+__device__ inline void reset_component(const Rounds &R, int64_t p) {
+  R.comp_d[p] = 0x7ff0000000000000ull;  // +infinity
+  R.comp_e[p] = ~0ull;
+  R.comp_amb[p] = 0;
+  R.comp_cw[p] = 0;
+  R.comp_ce[p] = 0;
 }
 
-__global__ void k_zero(uint32_t *a, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = 0;
-}
-
-// Bottom-up: node_label = common label of all leaves below, or kInvalid.
-__global__ void k_node_labels(int64_t n, const Node *__restrict__ nodes,
-                              const uint32_t *__restrict__ parent_int,
-                              const uint32_t *__restrict__ parent_leaf,
-                              const uint32_t *__restrict__ leaf_id,
-                              const uint32_t *__restrict__ label, uint32_t *node_label,
-                              uint32_t *counter) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_start(int64_t n, Rounds R) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < 3) R.counters[p] = 0;
   if (p >= n) return;
-  uint32_t node = parent_leaf[p];
-  while (node != kInvalid) {
-    __threadfence();
-    if (atomicAdd(&counter[node], 1u) == 0) return;
-    __threadfence();
-    const Node nd = nodes[node];
-    uint32_t l[2];
-    uint32_t ch[2] = {nd.left, nd.right};
-    for (int c = 0; c < 2; ++c) {
-      uint32_t x = ch[c];
-      l[c] = (x & kLeafBit) ? label[leaf_id[x & ~kLeafBit]]
-                            : ((volatile uint32_t *)node_label)[x];
+  R.label[p] = (uint32_t)p;
+  R.best_p[p] = kInvalid;
+  R.best_d[p] = 0.0;
+  R.best_flag[p] = 0;
+  reset_component(R, p);
+}
+
+__device__ inline uint32_t wave_uniform(uint32_t v, bool valid) {
+  const uint64_t m = __ballot(valid);
+  if (!m) return kInvalid;
+  const uint32_t f = lane_u32(v, __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1));
+  return __ballot(valid && v != f) ? kInvalid : f;
+}
+
+// Component shared by all leaves of each wave-tree group, one workgroup per
+// level-1 group (as the boxes are made); thread per position: the results of
+// the last round that still hold offer their distance to their component.
+constexpr int kLabelBlock = 1024;
+__global__ void __launch_bounds__(kLabelBlock) k_group_labels(WaveTree T, Rounds R) {
+  __shared__ uint32_t lab[64];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  for (uint32_t j = wave; j < 64; j += kLabelBlock / 64) {
+    const uint32_t g = blockIdx.x * 64 + j, p = g * 64 + lane;
+    const bool valid = g < T.c0 && p < T.n;
+    const uint32_t l = valid ? R.label[p] : kInvalid;
+    const uint32_t f = wave_uniform(l, valid);
+    if (lane == 0) {
+      lab[j] = f;
+      if (g < T.c0) R.glabel[g] = f;
     }
-    ((volatile uint32_t *)node_label)[node] = (l[0] == l[1]) ? l[0] : kInvalid;
-    node = parent_int[node];
+    if (!valid) continue;
+    const uint32_t b = R.best_p[p];
+    if (b == kInvalid) continue;
+    if (R.label[b] == l) {
+      R.best_p[p] = kInvalid;  // absorbed; its distance stays a lower bound
+    } else {
+      const uint64_t d = dbits(R.best_d[p]);
+      if (d < R.comp_d[l]) atomicMin((unsigned long long *)&R.comp_d[l], (unsigned long long)d);
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const uint32_t f = wave_uniform(lab[lane], blockIdx.x * 64 + lane < T.c0);
+    if (lane == 0) R.glabel[T.c0 + blockIdx.x] = f;
   }
 }
 
-// Lightest external edge of every point under kappa.
-__global__ void __launch_bounds__(128) k_search(int64_t n, const Node *__restrict__ nodes,
-                                                const double *__restrict__ LX,
-                                                const double *__restrict__ LY,
-                                                const double *__restrict__ LZ,
-                                                const uint32_t *__restrict__ leaf_id,
-                                                const uint32_t *__restrict__ label,
-                                                const uint32_t *__restrict__ node_label,
-                                                uint32_t *best_v, double *best_d,
-                                                uint8_t *best_flag) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const uint32_t u = leaf_id[p];
-  const uint32_t lu = label[u];
-  const double q[3] = {LX[p], LY[p], LZ[p]};
+__global__ void __launch_bounds__(64) k_top_labels(WaveTree T, Rounds R) {
+  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+  const uint32_t f = wave_uniform(i < T.c1 ? R.glabel[T.c0 + i] : kInvalid, i < T.c1);
+  if (threadIdx.x == 0) R.glabel[T.c0 + T.c1 + blockIdx.x] = f;
+}
+
+// Lightest external edge under kappa of every point whose last one is gone:
+// each lane keeps its own best over the groups, the wave combines them at the
+// end.  The component's best offer bounds the search from the start.
+constexpr int kSearchBlock = 256;  // four waves, four points
+__global__ void __launch_bounds__(kSearchBlock) k_search(WaveTree T, Rounds R) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t p = blockIdx.x * (kSearchBlock / 64) + (threadIdx.x >> 6);
+  if (p >= T.n || R.best_p[p] != kInvalid) return;
+  const uint32_t lu = R.label[p];
+  const double offer = as_double(R.comp_d[lu]);
+  const double limit = offer * (1.0 + kSlack) + kSlackAbs;
+  if (R.best_d[p] > limit) return;
+  const uint32_t u = T.leaf_id[p];
+  const double q[3] = {T.LX[p], T.LY[p], T.LZ[p]};
+  const WaveQuery Q(T, q[0], q[1], q[2]);
   double bd = INFINITY;
-  uint32_t bv = kInvalid;
-  bool bx = true;
-  uint8_t flag = 0;
-  uint32_t stack[64];
-  int sp = 0;
-  if (node_label[0] != lu) stack[sp++] = 0;
-  while (sp) {
-    const Node &N = nodes[stack[--sp]];
-    uint32_t ch[2] = {N.left, N.right};
-    double cd[2] = {INFINITY, INFINITY};
-    for (int c = 0; c < 2; ++c) {
-      uint32_t x = ch[c];
-      if (x & kLeafBit) {
-        uint32_t lp = x & ~kLeafBit;
-        uint32_t v = leaf_id[lp];
-        if (label[v] == lu) continue;
-        bool ex;
-        double d = d2_flag(q, LX[lp], LY[lp], LZ[lp], ex);
-        if (d > bd * (1.0 + kSlack) + kSlackAbs) continue;
-        bool both = ex && bx;
-        bool better;
-        if (d == bd && both) {
-          better = edge_key(u, v) < edge_key(u, bv);
-        } else {
-          if (!both && bd < INFINITY && fabs(d - bd) <= kSlack * bd + kSlackAbs) flag = 1;  // order not provable
-          better = d < bd || (d == bd && edge_key(u, v) < edge_key(u, bv));
-        }
-        if (better) { bd = d; bv = v; bx = ex; }
-      } else if (node_label[x] != lu) {
-        cd[c] = box_d2(q, nodes[x].lo, nodes[x].hi);
+  uint32_t bp = kInvalid, bv = kInvalid;
+  bool bx = true, near_tie = false;
+  double bound = limit;
+  float Tf = Q.bound(bound);
+  auto group = [&](uint32_t g) {
+    const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
+    const bool valid = lp < T.n && R.label[at] != lu;
+    if (!__ballot(valid)) return;
+    bool ex;
+    const double d = d2_flag(q, T.LX[at], T.LY[at], T.LZ[at], ex);
+    const bool in = valid && d <= bound;
+    if (!__ballot(in)) return;
+    if (in && d <= bd * (1.0 + kSlack) + kSlackAbs) {
+      const uint32_t v = T.leaf_id[at];
+      const bool both = ex && bx;
+      if (!both && bd < INFINITY && fabs(d - bd) <= kSlack * bd + kSlackAbs) near_tie = true;  // order not provable
+      if (d < bd || (d == bd && edge_key(u, v) < edge_key(u, bv))) {
+        if (bd < INFINITY && !(fabs(d - bd) <= kSlack * bd + kSlackAbs)) near_tie = false;
+        bd = d;
+        bp = lp;
+        bv = v;
+        bx = ex;
       }
     }
-    int first = cd[0] <= cd[1] ? 0 : 1;
-    for (int o = 1; o >= 0; --o) {
-      int c = o ? 1 - first : first;
-      if (cd[c] == INFINITY || cd[c] > bd * (1.0 + kSlack) + kSlackAbs) continue;
-      if (sp < 64) stack[sp++] = ch[c]; else flag = 2;
-    }
+    double m = bd;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o));
+    bound = fmin(bound, m * (1.0 + kSlack) + kSlackAbs);
+    Tf = Q.bound(bound);
+  };
+  const uint32_t own = p >> 6;
+  if (R.glabel[own] == kInvalid) group(own);
+  const uint32_t *gl = R.glabel;
+  wave_tree_visit(
+      T, Q, Tf,
+      [&](int level, uint32_t i) { return gl[(level == 0 ? 0u : level == 1 ? T.c0 : T.c0 + T.c1) + i] != lu; },
+      [&](uint32_t g) {
+        if (g != own) group(g);
+      });
+  double m = bd;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o));
+  if (!(m <= limit) || m == INFINITY) {
+    // nothing the component can use: every external point lies beyond the offer
+    if (lane == 0) R.best_d[p] = fmax(R.best_d[p], offer);
+    return;
   }
-  best_v[u] = bv;
-  best_d[u] = bd;
-  best_flag[u] = flag | (bx ? 0 : 4);
-}
-
-__global__ void k_comp_reset(int64_t n, uint64_t *comp_d, uint64_t *comp_e, uint32_t *comp_amb) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  comp_d[i] = ~0ull;
-  comp_e[i] = ~0ull;
-  comp_amb[i] = 0;
-}
-
-__global__ void k_comp_min(int64_t n, const uint32_t *__restrict__ label,
-                           const uint32_t *__restrict__ best_v, const double *__restrict__ best_d,
-                           uint64_t *comp_d) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n || best_v[u] == kInvalid) return;
-  atomicMin((unsigned long long *)&comp_d[label[u]], (unsigned long long)dbits(best_d[u]));
+  // lanes within rounding of the least distance: proven when alone or all exact
+  const bool win = bd <= m * (1.0 + kSlack) + kSlackAbs;
+  const uint64_t w = __ballot(win);
+  const bool exact = !__ballot(win && !bx);
+  const bool tie = __ballot(win && near_tie) != 0 || (!exact && __popcll(w) > 1);
+  uint64_t key = win && bd == m ? edge_key(u, bv) : ~0ull;
+  uint64_t least = key;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) least = min(least, (uint64_t)__shfl_xor((unsigned long long)least, o));
+  if (key == least && key != ~0ull) {  // one lane: edge keys are distinct
+    R.best_p[p] = bp;
+    R.best_d[p] = m;
+    R.best_flag[p] = (tie ? 1 : 0) | (bx ? 0 : 4);
+    const uint64_t b = dbits(m);
+    if (b < R.comp_d[lu]) atomicMin((unsigned long long *)&R.comp_d[lu], (unsigned long long)b);
+  }
 }
 
 // Entries within rounding of a component's FP64 minimum decide whether the
 // winner is proven: a single entry in the window is the exact minimum; several
 // entries are settled on the device only when all are exact and equal (ties
 // then break on the edge key).  Otherwise the component goes to the host.
-__global__ void k_comp_tie(int64_t n, const uint32_t *__restrict__ label,
-                           const uint32_t *__restrict__ best_v, const double *__restrict__ best_d,
-                           const uint8_t *__restrict__ best_flag, const uint64_t *__restrict__ comp_d,
-                           uint64_t *comp_e, uint32_t *comp_amb, uint32_t *comp_cw,
-                           uint32_t *comp_ce) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n || best_v[u] == kInvalid) return;
-  const uint32_t l = label[u];
-  double m;
-  uint64_t mb = comp_d[l];
-  memcpy(&m, &mb, 8);
-  const double d = best_d[u];
-  if (best_flag[u] & 2) atomicOr(&comp_amb[l], 16u);  // truncated search: best is only a bound
+__global__ void k_comp_tie(WaveTree T, Rounds R) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= T.n || R.best_p[p] == kInvalid) return;
+  const uint32_t l = R.label[p];
+  const uint64_t mb = R.comp_d[l];
+  const double m = as_double(mb), d = R.best_d[p];
   if (d - m > kSlack * m + kSlackAbs) return;
-  atomicAdd(&comp_cw[l], 1u);
-  if (best_flag[u] & 3) atomicOr(&comp_amb[l], 1u);
+  atomicAdd(&R.comp_cw[l], 1u);
+  if (R.best_flag[p] & 1) atomicOr(&R.comp_amb[l], 1u);
   if (dbits(d) == mb) {
-    atomicMin((unsigned long long *)&comp_e[l], (unsigned long long)edge_key((uint32_t)u, best_v[u]));
-    if (!(best_flag[u] & 4)) atomicAdd(&comp_ce[l], 1u);
+    atomicMin((unsigned long long *)&R.comp_e[l],
+              (unsigned long long)edge_key(T.leaf_id[p], T.leaf_id[R.best_p[p]]));
+    if (!(R.best_flag[p] & 4)) atomicAdd(&R.comp_ce[l], 1u);
   }
 }
 
-__global__ void k_comp_decide(int64_t n, const uint32_t *__restrict__ label,
-                              const uint32_t *__restrict__ comp_cw,
-                              const uint32_t *__restrict__ comp_ce, uint32_t *comp_amb) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= n || label[l] != (uint32_t)l) return;
-  if (comp_cw[l] >= 2 && comp_cw[l] != comp_ce[l]) comp_amb[l] |= 8u;
+__global__ void k_comp_decide(int64_t n, Rounds R) {
+  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (l == 0) R.counters[1] = 0;
+  if (l >= n || R.label[l] != (uint32_t)l) return;
+  if (R.comp_cw[l] >= 2 && R.comp_cw[l] != R.comp_ce[l]) R.comp_amb[l] |= 8u;
+  if (R.comp_amb[l]) atomicAdd(&R.counters[2], 1u);
 }
 
-// Every component root l hooks to the component across its winning edge.
-__global__ void k_hook(int64_t n, const uint32_t *__restrict__ label,
-                       const uint64_t *__restrict__ comp_e, uint32_t *hook) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= n) return;
-  if (label[l] != (uint32_t)l) { hook[l] = kInvalid; return; }
-  uint64_t e = comp_e[l];
-  if (e == ~0ull) { hook[l] = (uint32_t)l; return; }
-  uint32_t a = (uint32_t)(e >> 32), b = (uint32_t)e;
-  uint32_t other = label[a] == (uint32_t)l ? b : a;
-  hook[l] = label[other];
+// Every component hooks to the one across its winning edge and emits that
+// edge; of two that chose the same edge (keys are unique) the smaller stays a
+// root and emits it.  Nothing happens while ambiguous components wait for
+// the host (counters[2]).
+__global__ void k_hook(int64_t n, const uint32_t *__restrict__ leaf_pos, Rounds R) {
+  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= n || R.counters[2] || R.label[l] != (uint32_t)l) return;
+  const uint64_t e = R.comp_e[l];
+  if (e == ~0ull) {
+    R.hook[l] = (uint32_t)l;
+    return;
+  }
+  const uint32_t a = R.label[leaf_pos[(uint32_t)(e >> 32)]], b = R.label[leaf_pos[(uint32_t)e]];
+  const uint32_t other = a == (uint32_t)l ? b : a;
+  const bool mutual = R.comp_e[other] == e;
+  R.hook[l] = mutual && (uint32_t)l < other ? (uint32_t)l : other;
+  if (mutual && (uint32_t)l > other) return;
+  const uint32_t slot = atomicAdd(&R.counters[0], 1u);
+  if (slot >= (uint32_t)n) return;
+  R.edges[2 * slot] = (uint32_t)(e >> 32);
+  R.edges[2 * slot + 1] = (uint32_t)e;
 }
 
-__global__ void k_emit(int64_t n, const uint32_t *__restrict__ label,
-                       const uint64_t *__restrict__ comp_e, uint32_t *hook, uint32_t *edges,
-                       uint32_t *counters) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= n || label[l] != (uint32_t)l) return;
-  uint32_t h = hook[l];
-  if (h == (uint32_t)l) return;
-  bool mutual = hook[h] == (uint32_t)l;
-  if (mutual && (uint32_t)l > h) return;  // the partner emits the shared edge
-  uint64_t e = comp_e[l];
-  uint32_t slot = atomicAdd(&counters[0], 1u);
-  edges[2 * slot] = (uint32_t)(e >> 32);
-  edges[2 * slot + 1] = (uint32_t)e;
+// Root of every component in the hook forest, by path halving: concurrent
+// threads only ever store an ancestor of a component as its hook.
+__global__ void k_roots(int64_t n, Rounds R) {
+  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= n || R.counters[2] || R.label[l] != (uint32_t)l) return;
+  volatile uint32_t *hook = R.hook;
+  uint32_t x = (uint32_t)l;
+  for (int64_t step = 0; step < n; ++step) {
+    const uint32_t h = hook[x];
+    if (h == x) break;
+    const uint32_t g = hook[h];
+    if (g == h) {
+      x = h;
+      break;
+    }
+    hook[x] = g;
+    x = g;
+  }
+  R.root[l] = x;
+  if (x == (uint32_t)l) atomicAdd(&R.counters[1], 1u);
 }
 
-__global__ void k_break_cycles(int64_t n, const uint32_t *__restrict__ label, uint32_t *hook) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= n || label[l] != (uint32_t)l) return;
-  uint32_t h = hook[l];
-  if (h != (uint32_t)l && hook[h] == (uint32_t)l && (uint32_t)l < h) hook[l] = (uint32_t)l;
-}
-
-__global__ void k_jump(int64_t n, const uint32_t *__restrict__ label, uint32_t *hook) {
-  int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= n || label[l] != (uint32_t)l) return;
-  uint32_t h = hook[l];
-  uint32_t hh = hook[h];
-  if (hh != h) hook[l] = hh;
-}
-
-__global__ void k_relabel(int64_t n, uint32_t *label, const uint32_t *__restrict__ hook,
-                          uint32_t *counters) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n) return;
-  uint32_t r = hook[label[u]];
-  label[u] = r;
-  if (r == (uint32_t)u) atomicAdd(&counters[1], 1u);
-}
-
-// Roots must be component minima so that labels stay "least PointId";
-// k_relabel keeps the hook root, which is the smallest label on a 2-cycle
-// but not the smallest PointId of the merged set.  Recompute minima.
-__global__ void k_min_label(int64_t n, const uint32_t *__restrict__ label, uint32_t *minid) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u < n) atomicMin(&minid[label[u]], (uint32_t)u);
-}
-
-__global__ void k_fill(uint32_t *a, int64_t n, uint32_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
-}
-
-__global__ void k_apply_min(int64_t n, uint32_t *label, const uint32_t *__restrict__ minid) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u < n) label[u] = minid[label[u]];
+// New labels, and the component arrays cleared for the next round.
+__global__ void k_relabel(int64_t n, Rounds R) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n || R.counters[2]) return;
+  R.label[p] = R.root[R.label[p]];
+  reset_component(R, p);
 }
 
 }  // namespace
@@ -292,10 +324,10 @@ void emst_host(Context &c, uint32_t *edges_out) {
   EmstBuffers &B = *c.emst;
   hipStream_t s = c.stream;
   const int T = 256;
-  const int G = blocks_for(n, T);
+  const dim3 G(blocks_for(n, T)), B256(T);
+  const WaveTree W = wave_tree(c);
   B.label.ensure(n);
-  B.next_label.ensure(n);
-  B.node_label.ensure(n);
+  B.node_label.ensure((size_t)W.c0 + W.c1 + W.c2);
   B.best_v.ensure(n);
   B.best_d.ensure(n);
   B.best_flag.ensure(n);
@@ -306,41 +338,40 @@ void emst_host(Context &c, uint32_t *edges_out) {
   B.comp_ce.ensure(n);
   B.edges.ensure(2 * n);
   B.counters.ensure(4);
-  DevBuf<uint32_t> &hook = B.hook;
-  hook.ensure(n);
-  hipLaunchKernelGGL(k_init_labels, dim3(G), dim3(T), 0, s, n, B.label.p);
-  MHGP_HIP(hipMemsetAsync(B.counters.p, 0, 4 * sizeof(uint32_t), s));
+  B.hook.ensure(n);
+  B.next_label.ensure(n);
+  const Rounds R{B.label.p,  B.node_label.p, B.best_v.p,  B.best_d.p,  B.best_flag.p,  B.comp_d.p, B.comp_e.p,
+                 B.comp_amb.p, B.comp_cw.p,    B.comp_ce.p, B.hook.p,    B.next_label.p, B.edges.p,  B.counters.p};
+  hipLaunchKernelGGL(k_start, G, B256, 0, s, n, R);
   int64_t components = n;
   for (int round = 0; components > 1; ++round) {
     if (round > 64) throw std::runtime_error("Borůvka did not converge");
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(n - 1, T)), dim3(T), 0, s, c.counter.p, n - 1);
-    hipLaunchKernelGGL(k_node_labels, dim3(G), dim3(T), 0, s, n, c.nodes.p, c.parent_int.p,
-                       c.parent_leaf.p, c.leaf_id.p, B.label.p, B.node_label.p, c.counter.p);
-    hipLaunchKernelGGL(k_search, dim3(blocks_for(n, 128)), dim3(128), 0, s, n, c.nodes.p, c.LX.p,
-                       c.LY.p, c.LZ.p, c.leaf_id.p, B.label.p, B.node_label.p, B.best_v.p,
-                       B.best_d.p, B.best_flag.p);
-    hipLaunchKernelGGL(k_comp_reset, dim3(G), dim3(T), 0, s, n, B.comp_d.p, B.comp_e.p, B.comp_amb.p);
-    hipLaunchKernelGGL(k_comp_min, dim3(G), dim3(T), 0, s, n, B.label.p, B.best_v.p, B.best_d.p,
-                       B.comp_d.p);
-    hipLaunchKernelGGL(k_zero, dim3(G), dim3(T), 0, s, B.comp_cw.p, n);
-    hipLaunchKernelGGL(k_zero, dim3(G), dim3(T), 0, s, B.comp_ce.p, n);
-    hipLaunchKernelGGL(k_comp_tie, dim3(G), dim3(T), 0, s, n, B.label.p, B.best_v.p, B.best_d.p,
-                       B.best_flag.p, B.comp_d.p, B.comp_e.p, B.comp_amb.p, B.comp_cw.p,
-                       B.comp_ce.p);
-    hipLaunchKernelGGL(k_comp_decide, dim3(G), dim3(T), 0, s, n, B.label.p, B.comp_cw.p,
-                       B.comp_ce.p, B.comp_amb.p);
-    MHGP_LAUNCH_CHECK();
-    // host exact settlement of ambiguous components (rare)
-    std::vector<uint32_t> amb(n);
-    MHGP_HIP(hipMemcpyAsync(amb.data(), B.comp_amb.p, n * 4, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipStreamSynchronize(s));
-    bool any = false;
-    for (int64_t l = 0; l < n && !any; ++l) any = amb[l] != 0;
-    if (any) {
-      std::vector<uint32_t> label(n);
+    hipLaunchKernelGGL(k_group_labels, dim3(W.c1), dim3(kLabelBlock), 0, s, W, R);
+    if (W.c2 > 1) hipLaunchKernelGGL(k_top_labels, dim3(W.c2), dim3(64), 0, s, W, R);
+    hipLaunchKernelGGL(k_search, dim3(blocks_for(n, kSearchBlock / 64)), dim3(kSearchBlock), 0, s, W, R);
+    hipLaunchKernelGGL(k_comp_tie, G, B256, 0, s, W, R);
+    hipLaunchKernelGGL(k_comp_decide, G, B256, 0, s, n, R);
+    for (;;) {
+      hipLaunchKernelGGL(k_hook, G, B256, 0, s, n, c.leaf_pos.p, R);
+      hipLaunchKernelGGL(k_roots, G, B256, 0, s, n, R);
+      hipLaunchKernelGGL(k_relabel, G, B256, 0, s, n, R);
+      MHGP_LAUNCH_CHECK();
+      uint32_t cnt[3];
+      copy_wait(cnt, B.counters.p, sizeof cnt, hipMemcpyDeviceToHost, s);
+      if (cnt[2] == 0) {
+        components = cnt[1];
+        if (cnt[0] + components != (uint64_t)n) throw std::runtime_error("Borůvka edge count mismatch");
+        break;
+      }
+      // host exact settlement of ambiguous components (rare); the kernels
+      // above left the round as it was
+      std::vector<uint32_t> at(n), ids(n), amb(n), label(n);
       std::vector<uint64_t> ce(n);
-      copy_wait(label.data(), B.label.p, n * 4, hipMemcpyDeviceToHost, s);
+      MHGP_HIP(hipMemcpyAsync(at.data(), B.label.p, n * 4, hipMemcpyDeviceToHost, s));
+      MHGP_HIP(hipMemcpyAsync(ids.data(), c.leaf_id.p, n * 4, hipMemcpyDeviceToHost, s));
+      MHGP_HIP(hipMemcpyAsync(amb.data(), B.comp_amb.p, n * 4, hipMemcpyDeviceToHost, s));
       copy_wait(ce.data(), B.comp_e.p, n * 8, hipMemcpyDeviceToHost, s);
+      for (int64_t p = 0; p < n; ++p) label[ids[p]] = at[p];  // component by PointId
       const ExactCloud &ex = exact_cloud(c);
       const std::vector<double> &xyz = c.host->xyz;
       for (int64_t l = 0; l < n; ++l) {
@@ -356,24 +387,8 @@ void emst_host(Context &c, uint32_t *edges_out) {
         ce[l] = best;
       }
       copy_wait(B.comp_e.p, ce.data(), n * 8, hipMemcpyHostToDevice, s);
+      MHGP_HIP(hipMemsetAsync(B.counters.p + 2, 0, sizeof(uint32_t), s));
     }
-    hipLaunchKernelGGL(k_hook, dim3(G), dim3(T), 0, s, n, B.label.p, B.comp_e.p, hook.p);
-    hipLaunchKernelGGL(k_emit, dim3(G), dim3(T), 0, s, n, B.label.p, B.comp_e.p, hook.p,
-                       B.edges.p, B.counters.p);
-    hipLaunchKernelGGL(k_break_cycles, dim3(G), dim3(T), 0, s, n, B.label.p, hook.p);
-    for (int j = 0; j < 24; ++j)
-      hipLaunchKernelGGL(k_jump, dim3(G), dim3(T), 0, s, n, B.label.p, hook.p);
-    MHGP_HIP(hipMemsetAsync(B.counters.p + 1, 0, sizeof(uint32_t), s));
-    hipLaunchKernelGGL(k_relabel, dim3(G), dim3(T), 0, s, n, B.label.p, hook.p, B.counters.p);
-    hipLaunchKernelGGL(k_fill, dim3(G), dim3(T), 0, s, B.next_label.p, n, kInvalid);
-    hipLaunchKernelGGL(k_min_label, dim3(G), dim3(T), 0, s, n, B.label.p, B.next_label.p);
-    hipLaunchKernelGGL(k_apply_min, dim3(G), dim3(T), 0, s, n, B.label.p, B.next_label.p);
-    MHGP_LAUNCH_CHECK();
-    uint32_t cnt[2];
-    MHGP_HIP(hipMemcpyAsync(cnt, B.counters.p, 8, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipStreamSynchronize(s));
-    components = cnt[1];
-    if (cnt[0] + components != (uint64_t)n) throw std::runtime_error("Borůvka edge count mismatch");
   }
   StageTimer tm(s);
   // kappa order: FP64 squared lengths sorted on the device; runs of values

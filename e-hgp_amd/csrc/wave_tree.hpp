@@ -49,27 +49,28 @@ struct WaveQuery {
 
 // Calls leaf(g) for every level-0 group whose box lies within the squared
 // bound Tf, which leaf may shrink as it goes (pending groups are tested
-// against it again).  Uniform over the wave: every lane makes the call with
-// the same query and bound, and leaf(g) runs with all lanes active.
-template <class F>
-__device__ inline void wave_tree_visit(const WaveTree &T, const WaveQuery &Q, float &Tf, F &&leaf) {
+// against it again), and whose ancestors and itself pass keep(level, group).
+// Uniform over the wave: every lane makes the call with the same query and
+// bound, and leaf(g) runs with all lanes active.
+template <class K, class F>
+__device__ inline void wave_tree_visit(const WaveTree &T, const WaveQuery &Q, float &Tf, K &&keep, F &&leaf) {
   const uint32_t lane = threadIdx.x & 63u;
   for (uint32_t b2 = 0; b2 < T.c2; b2 += 64) {
     const uint32_t i2 = b2 + lane;
     // a single top group holds every leaf: nothing to test
-    uint64_t m2 = T.c2 == 1 ? 1ull : __ballot(i2 < T.c2 && !(Q.d2(T.l2[min(i2, T.c2 - 1)]) > Tf));
+    uint64_t m2 = T.c2 == 1 ? 1ull : __ballot(i2 < T.c2 && keep(2, min(i2, T.c2 - 1)) && !(Q.d2(T.l2[min(i2, T.c2 - 1)]) > Tf));
     while (m2) {
       const uint32_t g2 = b2 + (uint32_t)(__ffsll((long long)m2) - 1);
       m2 &= m2 - 1;
       const uint32_t i1 = g2 * 64 + lane;
       const float d1 = Q.d2(T.l1[min(i1, T.c1 - 1)]);
-      uint64_t rem1 = __ballot(i1 < T.c1);
+      uint64_t rem1 = __ballot(i1 < T.c1 && keep(1, min(i1, T.c1 - 1)));
       for (uint64_t m1 = __ballot(!(d1 > Tf)) & rem1; m1; m1 = __ballot(!(d1 > Tf)) & rem1) {
         const int k1 = __ffsll((long long)m1) - 1;
         rem1 &= ~((2ull << k1) - 1ull);  // this one is taken; the ones before it lie outside the bound
         const uint32_t g1 = g2 * 64 + (uint32_t)k1, i0 = g1 * 64 + lane;
         const float d0 = Q.d2(T.l0[min(i0, T.c0 - 1)]);
-        uint64_t rem0 = __ballot(i0 < T.c0);
+        uint64_t rem0 = __ballot(i0 < T.c0 && keep(0, min(i0, T.c0 - 1)));
         for (uint64_t m0 = __ballot(!(d0 > Tf)) & rem0; m0; m0 = __ballot(!(d0 > Tf)) & rem0) {
           const int k0 = __ffsll((long long)m0) - 1;
           rem0 &= ~((2ull << k0) - 1ull);
@@ -78,6 +79,11 @@ __device__ inline void wave_tree_visit(const WaveTree &T, const WaveQuery &Q, fl
       }
     }
   }
+}
+
+template <class F>
+__device__ inline void wave_tree_visit(const WaveTree &T, const WaveQuery &Q, float &Tf, F &&leaf) {
+  wave_tree_visit(T, Q, Tf, [](int, uint32_t) { return true; }, leaf);
 }
 
 // Value of lane `src` (uniform) in every lane, and the value of the lane

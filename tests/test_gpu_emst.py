@@ -31,6 +31,29 @@ def test_emst_matches_kruskal(name):
     assert np.array_equal(e, ref)
 
 
+@pytest.mark.parametrize("name", ["two", "group64", "group65", "level4097", "chain", "near_ties", "far_away"])
+def test_emst_rounds_at_their_edges(name):
+    """Group and level edges of the wave tree, a chain whose components all
+    hook one way (the longest hook path), tied lengths that FP64 cannot prove
+    (settled on the host), and a cloud far from the origin."""
+    print(f"emst edge case {name}", flush=True)
+    if name in ("two", "group64", "group65", "level4097"):
+        n = {"two": 2, "group64": 64, "group65": 65, "level4097": 4097}[name]
+        pts = workloads.uniform_cloud(n, seed=n)
+    elif name == "chain":
+        step = 1.0 + 1e-3 * np.arange(2500)
+        pts = np.stack([np.cumsum(step), np.zeros(2500), np.zeros(2500)], axis=1)
+    elif name == "near_ties":
+        pts = np.stack(np.meshgrid(np.arange(6), np.arange(6), np.arange(6)), -1).reshape(-1, 3) * 0.1
+    else:
+        pts = workloads.uniform_cloud(1500, seed=4) + 1.0e7
+    ref = oracle.emst(oracle.canonicalize(pts))
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        e = ctx.emst().astype(np.int64)
+    assert np.array_equal(e, np.asarray(ref, dtype=np.int64).reshape(e.shape))
+
+
 def test_emst_50k_lattice_weight():
     from scipy.sparse import coo_matrix
     from scipy.sparse.csgraph import minimum_spanning_tree
