@@ -1083,18 +1083,36 @@ __device__ inline bool face_feasible(const Work &w, uint32_t si, uint32_t sj, do
 // points at the front of the point arrays, masks by region slot, cell radii
 // in w.rho); *sK == 0 and *sregion == kInvalid on entry, visible to every
 // lane.  Marks the anchor done.
-template <bool BIG, bool F32>
+//
+// An anchor may be split over several workgroups (SPLIT: blockIdx.y of
+// gridDim.y, each with its own copy of the region): the candidate vertices
+// are listed in region order, so every workgroup sees the same numbering of
+// the faces, and takes its share of them and of the pairs.  The workgroups
+// beyond one per kSplitFaces candidate faces have nothing to do; the status is
+// left to the caller.
+constexpr uint64_t kSplitFaces = 2048;
+template <bool BIG, bool F32, bool SPLIT>
 __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t *sK_,
                              uint32_t *sregion_) {
   uint32_t &sK = *sK_;
   uint32_t &sregion = *sregion_;
   const int t = threadIdx.x;
-  // candidate vertices (ids above the anchor); their order only decides
-  // which lane takes which face (a rank sort by direction cell, to give
-  // neighbouring lanes overlapping pencil capsules, measured slower); the
-  // FP32 copies of the region's coordinates for the face passes
+  // candidate vertices (ids above the anchor) in region order (a rank sort
+  // by direction cell, to give neighbouring lanes overlapping pencil capsules,
+  // measured slower); the FP32 copies of the region's coordinates for the
+  // face passes
+  if (t < 64) {
+    uint32_t k = 0;
+    for (uint32_t s0 = 0; s0 < M; s0 += 64) {
+      const uint32_t s = s0 + t;
+      const bool above = s < M && w.gid[min(s, M - 1)] > u;
+      const uint64_t m = __ballot(above);
+      if (above) w.kidx[k + (uint32_t)__popcll(m & ((1ull << t) - 1ull))] = s;
+      k += (uint32_t)__popcll(m);
+    }
+    if (t == 0) sK = k;
+  }
   for (uint32_t s = t; s < M; s += blockDim.x) {
-    if (w.gid[s] > u) w.kidx[atomicAdd(&sK, 1u)] = s;
     if (F32) {
       w.fx[s] = (float)w.gx[s];
       w.fy[s] = (float)w.gy[s];
@@ -1103,8 +1121,16 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   }
   __syncthreads();
   const uint32_t Kc = sK;
+  const uint64_t F = Kc ? (uint64_t)Kc * (Kc - 1) / 2 : 0;
+  uint32_t part = 0, parts = 1;
+  if (SPLIT) {
+    part = blockIdx.y;
+    parts = (uint32_t)min((uint64_t)gridDim.y, F / kSplitFaces + 1);
+    if (part >= parts) return;
+  }
   // 3. pairs (u, v), v > u
-  for (uint32_t k = t; k < Kc; k += blockDim.x) process_pair(P, w, u, M, w.kidx[k], &sregion);
+  for (uint32_t k = part * blockDim.x + t; k < Kc; k += parts * blockDim.x)
+    process_pair(P, w, u, M, w.kidx[k], &sregion);
   // 4. faces (u, v, w), u < v < w, whose members share a cell.  Each wave
   // takes 64 candidate faces at a time: first passes one per lane, then the
   // queued sides and tetrahedra one per lane (LDS path; the global-memory
@@ -1120,7 +1146,6 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   WaveQueues *q = BIG ? nullptr : &wq;
   if (lane == 0) { q_n[wave][0] = 0; q_n[wave][1] = 0; }
   wave_sync();
-  const uint64_t F = (uint64_t)Kc * (Kc - 1) / 2;
   // candidate face fidx -> region slots of (v, w): the pair (i < j) of the
   // strictly lower triangle
   auto face_of = [&](uint64_t fidx, uint32_t &si, uint32_t &sj) {
@@ -1132,7 +1157,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     sj = w.kidx[j];
   };
   if (BIG) {
-    for (uint64_t base = (uint64_t)wave * 64; base < F; base += (uint64_t)nwaves * 64) {
+    for (uint64_t base = ((uint64_t)part * nwaves + wave) * 64; base < F; base += (uint64_t)parts * nwaves * 64) {
       const uint64_t fidx = base + lane;
       if (fidx >= F) continue;
       uint32_t si, sj;
@@ -1149,8 +1174,8 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     // next round.  The lists keep region slots only; a lane recomputes the
     // face's rmax (same arithmetic, same value).
     uint32_t nf = 0;  // faces in the wave's list (uniform)
-    uint64_t cbase = (uint64_t)wave * 64;
-    const uint64_t cstride = (uint64_t)nwaves * 64;
+    uint64_t cbase = ((uint64_t)part * nwaves + wave) * 64;
+    const uint64_t cstride = (uint64_t)parts * nwaves * 64;
     for (;;) {
       while (nf <= 64 && cbase < F) {
         const uint64_t fidx = cbase + lane;
@@ -1229,7 +1254,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     if (*w.cand) atomicAdd(&P.counters[3], (unsigned long long)*w.cand);
     if (w.flops && *w.flops) atomicAdd(&P.counters[5], *w.flops);
     if (w.flops32 && *w.flops32) atomicAdd(&P.counters[6], *w.flops32);
-    P.status[u] = ST_DONE;
+    if (!SPLIT) P.status[u] = ST_DONE;
   }
 }
 
@@ -1454,7 +1479,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
     }
     return;
   }
-  anchor_faces<BIG, F32>(P, w, u, M, &sK, &sregion);
+  anchor_faces<BIG, F32, false>(P, w, u, M, &sK, &sregion);
 }
 
 // The LDS path in two sizes: most anchors fit the small one, which leaves
@@ -1572,7 +1597,14 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
 // stay below 1 024, as the packed queue items need).  Same parameters and
 // slab layout as k_anchor_big's probe launch; anchors not probed, or with
 // larger regions, are left to it.
+//
+// One workgroup per anchor left the chip idle wherever tens of anchors held
+// such regions (43 anchors: 313 ms, each workgroup alone on its CU): the
+// launch asks for kRegionParts workgroups in all, a few per CU slot so that
+// the longest ones do not end it alone.  A 2 003-point mixture's catalogue:
+// 885 -> 332 ms.
 constexpr int kRegionCapHuge = 1023;
+constexpr uint32_t kRegionParts = 4096;
 template <int RCAP, int RMIN>
 __global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anchor_region(Params P) {
   const uint32_t a = blockIdx.x;
@@ -1604,7 +1636,15 @@ __global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anch
   if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; }
   __syncthreads();
   Work w{gx, gy, gz, gid, rho, kidx, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz};
-  anchor_faces<false, true>(P, w, u, M, &sK, &sregion);
+  anchor_faces<false, true, true>(P, w, u, M, &sK, &sregion);
+}
+
+// Anchors whose region the LDS kernels have enumerated.
+__global__ void k_region_done(Params P, uint32_t rmax) {
+  const uint32_t a = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a >= P.anchor_count) return;
+  const uint32_t u = P.anchors[a];
+  if (P.status[u] == ST_PROBED && P.need[u] <= (double)rmax) P.status[u] = ST_DONE;
 }
 
 // Ball count / emit around every anchor of the list: one wave per anchor over
@@ -2154,8 +2194,12 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
             hipLaunchKernelGGL(k_anchor_big, dim3(bn), dim3(kBlock), 0, s, Q);
             // probed regions that fit LDS: enumerated there, from this chunk's slabs
             if (probe && force_path != 2) {
-              hipLaunchKernelGGL((k_anchor_region<kRegionCapWide, 0>), dim3(bn), dim3(kBlock), 0, s, Q);
-              hipLaunchKernelGGL((k_anchor_region<kRegionCapHuge, kRegionCapWide>), dim3(bn), dim3(kBlock), 0, s, Q);
+              const uint32_t parts = std::clamp<uint32_t>(kRegionParts / bn, 1, 64);
+              hipLaunchKernelGGL((k_anchor_region<kRegionCapHuge, kRegionCapWide>), dim3(bn, parts), dim3(kBlock), 0, s,
+                                 Q);
+              hipLaunchKernelGGL((k_anchor_region<kRegionCapWide, 0>), dim3(bn, parts), dim3(kBlock), 0, s, Q);
+              hipLaunchKernelGGL(k_region_done, dim3(blocks_for(bn, 256)), dim3(256), 0, s, Q,
+                                 (uint32_t)kRegionCapHuge);
             }
             MHGP_LAUNCH_CHECK();
           }
