@@ -1,19 +1,16 @@
 // Batched processing of many clouds: groups of clouds run side by side, one
-// host thread and one context (stream) each, and the first anchor pass of
-// every cloud of a group is one persistent launch over all of them
-// (k_anchor_persist, supports.hip).  A group holds as many clouds as fit the
-// memory cap by their predicted device bytes (at most `group`).  Each cloud
-// then runs what the plain path runs: exact EMST, catalogue (the remaining
-// anchor passes per cloud), and the tower unless the catalogue is
-// conditional.  Results and towers are kept per cloud.
+// host thread and one context (stream) each.  A group holds as many clouds as
+// fit the memory cap by their predicted device bytes (at most `group`).  Each
+// cloud runs what the plain path runs: exact EMST, catalogue, and the tower
+// unless the catalogue is conditional.  Results and towers are kept per cloud.
 #include <algorithm>
 #include <chrono>
 #include <memory>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../../include/mhgp.h"
-#include "batch.hpp"
 #include "pipeline.hpp"
 #include "tower_state.hpp"
 
@@ -72,7 +69,6 @@ void batch_run(int device, int64_t count, const double *const *xyz, const int64_
     }
     const int G = (int)(j - i);
     while ((int)pool.size() < G) pool.push_back(batch_context(device));
-    auto rv = anchor_batch_create(device, G);
     std::vector<std::thread> th;
     for (int t = 0; t < G; ++t)
       th.emplace_back([&, t] {
@@ -85,20 +81,11 @@ void batch_run(int device, int64_t count, const double *const *xyz, const int64_
           if (!cp || cp->poisoned) cp = batch_context(device);
           Context &c = *cp;
           MHGP_HIP(hipSetDevice(device));
-          c.batch = rv.get();
-          c.batch_slot = t;
           upload_host(c, xyz[cloud], n[cloud]);
           std::vector<uint32_t> edges(2 * std::max<int64_t>(c.n - 1, 0));
           emst_host(c, edges.data());
           mhgp_catalog_info ci{};
-          try {
-            supports(c, k_max[cloud], &ci);
-          } catch (...) {
-            anchor_batch_leave(*rv, t);
-            throw;
-          }
-          anchor_batch_leave(*rv, t);  // a cloud that had no anchor pass
-          c.batch = nullptr;
+          supports(c, k_max[cloud], &ci);
           r.event_count = ci.event_count;
           if (ci.status != 0) {
             r.status = 1;  // budget stop: conditional, no tower
@@ -128,17 +115,16 @@ void batch_run(int device, int64_t count, const double *const *xyz, const int64_
           code = MHGP_E_INTERNAL;
           if (cp) cp->poisoned = true;
         }
-        anchor_batch_leave(*rv, t);
-        if (cp) cp->batch = nullptr;
         r.code = code;
         r.service_ms = std::chrono::duration<double, std::milli>(Clock::now() - a).count();
         r.latency_ms = std::chrono::duration<double, std::milli>(Clock::now() - t_start).count();
       });
     for (auto &x : th) x.join();
-    const AnchorBatchStats st = anchor_batch_stats(*rv);
     out.info.groups++;
-    out.info.anchors += st.anchors;
-    out.info.anchor_ms += st.ms;
+    for (int t = 0; t < G; ++t) {
+      out.info.anchors += n[i + t];
+      if (pool[t]) out.info.anchor_ms += std::exchange(pool[t]->stats.anchor_ms, 0.0);
+    }
     i = j;
   }
   for (auto &c : pool)

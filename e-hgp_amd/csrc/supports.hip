@@ -36,12 +36,9 @@
 #include <cfloat>
 #include <cstdio>
 #include <cstring>
-#include <condition_variable>
 #include <memory>
-#include <mutex>
 #include <numeric>
 
-#include "batch.hpp"
 #include "wave.hpp"
 #include "pipeline.hpp"
 #include "predicates.hpp"
@@ -52,8 +49,8 @@
 namespace mhgp {
 
 int64_t catalog_device_bytes(const CatalogBuffers &b) {
-  return b.radius.bytes() + b.gcount.bytes() + b.goff.bytes() + b.glist.bytes() + b.need.bytes() +
-         b.status.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
+  return b.radius.bytes() + b.gcount.bytes() + b.goff.bytes() + b.glist.bytes() + b.region.bytes() +
+         b.lists.bytes() + b.big.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
          b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.scratch.bytes() + b.anchors.bytes() +
          b.total.bytes() + b.run_count.bytes() + b.run_pos.bytes() + b.run_gidx.bytes() + b.run_new.bytes() +
          b.run_link.bytes() + b.run_rec.bytes();
@@ -62,6 +59,7 @@ int64_t catalog_device_bytes(const CatalogBuffers &b) {
 namespace {
 
 constexpr int kBlock = 256;
+constexpr int kRegionCapHuge = 1023;  // the largest region enumerated in LDS
 
 // LDS written by some lanes of a wave, then read by other lanes of it
 __device__ inline void wave_sync() {
@@ -70,7 +68,16 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-enum : uint32_t { ST_PENDING = 0, ST_DONE = 1, ST_WIDEN = 2, ST_BIG = 3, ST_HUGE = 4, ST_PROBED = 5 };
+// Lists the probes append to (B.lists, kLists rows of n entries; their lengths
+// are counters[kListCount ..]).  The first three hold PointIds for a later
+// pass: gathers to widen, gathers beyond the small probe, gathers beyond LDS.
+// The others hold the probed anchors of one launch (their index in it, which
+// is also their slab's) by the size of their region.
+enum { L_WIDEN = 0, L_WIDE = 1, L_BIG = 2, L_SMALL = 3, L_MID = 4, L_LARGE = 5, L_SLAB = 6, kLists = 7 };
+constexpr int kListCount = 8;    // counters: list lengths
+constexpr int kOpenCount = 16;   // counters: open anchors, their largest region
+constexpr int kOpenLargest = 17;
+constexpr int kCounters = 24;
 
 // Regions of the global-memory path are enumerated face by face in
 // O(region^3) work; beyond the context's region limit (at most this) one
@@ -85,30 +92,46 @@ struct Params {
   const uint32_t *gcount;
   const uint64_t *goff;
   const uint32_t *glist;
-  const double *radius;
+  double *radius;
   const double *cells;           // 8 doubles per cell
   const float *cellf;            // 8 floats per cell: the FP32 cell (see cell_f)
   double blo[3], bhi[3];         // cloud AABB
   int s_max;
-  double *need;
-  uint32_t *status;
+  uint32_t *region;              // region size of a probed anchor
+  uint32_t *lists;               // kLists rows of list_cap entries
+  uint32_t list_cap;
   EventRec *events;
   uint64_t event_cap;
   FallbackRec *fallbacks;
   uint64_t fallback_cap;
   uint32_t *fb_region;
   uint64_t fb_region_cap;
-  unsigned long long *counters;  // [0] events [1] fallbacks [2] region words [3] candidates
+  unsigned long long *counters;  // [0] events [1] fallbacks [2] region words [3] candidates [4] queue errors
+                                 // [5] FP64 [6] FP32 operations, then the lists' lengths and the open anchors
   const uint32_t *anchors;
   uint32_t anchor_count;
-  int big;                       // 1: arrays live in global scratch slabs
-  int probe;                     // 1: stop once the region size is known (ST_PROBED)
+  int probe;                     // 1: stop once the region is in the slab
   double *scratch;
   uint64_t slab_doubles;
-  uint32_t gcap, rcap;
+  uint32_t gcap;                 // gathered points a slab holds
   int count_flops;               // 1: count the FP64 (counters[5]) and FP32 (counters[6]) operations
   uint32_t region_limit;         // largest region the global-memory path enumerates
 };
+
+__device__ inline void list_add(const Params &P, int list, uint32_t v) {
+  const unsigned long long at = atomicAdd(&P.counters[kListCount + list], 1ull);
+  if (at < P.list_cap) P.lists[(size_t)list * P.list_cap + at] = v;
+}
+
+// The certificate needs a larger gather than radius Rg (one lane).
+__device__ inline void widen(const Params &P, uint32_t u, double need, double Rg) {
+  P.radius[u] = fmax(need * 1.02, Rg * 1.05);
+  list_add(P, L_WIDEN, u);
+}
+
+// Anchor u's region of M points is in slab a (one lane): queued for the
+// enumeration of its size, or left open beyond the region limit.
+__device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t M);
 
 struct Work {
   double *gx, *gy, *gz;
@@ -1042,6 +1065,28 @@ __device__ bool member_mask(const Params &P, const Work &w, uint32_t i, float rm
 
 constexpr int kCoverCap = 10;  // s_max - 1 <= 10
 
+// Certificate radius of cell c from its (s_max-1)-th cover radius bk: with the
+// FP32 slack, at most the AABB exit distance of the cell, rounded up to a
+// float (a larger radius only enlarges the region).
+__device__ inline float cell_radius(const Params &P, int c, float bk, double ux, double uy, double uz) {
+  const double *cd = P.cells + 8 * c;
+  const double chord = cd[5];
+  const double rc = (double)bk * (1.0 + 1e-4);
+  double dir[3] = {cd[0], cd[1], cd[2]};
+  double uu[3] = {ux, uy, uz};
+  double e = INFINITY;
+  for (int a = 0; a < 3; ++a) {
+    double lo = dir[a] - chord, hi = dir[a] + chord;
+    if (lo > 0) e = fmin(e, (P.bhi[a] - uu[a]) / lo);
+    else if (hi < 0) e = fmin(e, (P.blo[a] - uu[a]) / hi);
+  }
+  e = fmax(e, 0.0) * (1.0 + 1e-9) + 1e-300;
+  const double rd = fmin(rc, e);
+  float rf = (float)rd;
+  if (!((double)rf >= rd)) rf = rd <= (double)FLT_MIN ? FLT_MIN : nextafterf(rf, INFINITY);
+  return rf;
+}
+
 // Face (u, v, w) of region slots si, sj: false when v and w share no cell or
 // when the triangle's circumradius exceeds every shared cell's certificate
 // radius (well-conditioned faces only; FP64 r2 is then accurate to ~1e-10).
@@ -1082,16 +1127,15 @@ __device__ inline bool face_feasible(const Work &w, uint32_t si, uint32_t sj, do
 // Pairs, faces and tetrahedra of anchor u over its compacted region (M
 // points at the front of the point arrays, masks by region slot, cell radii
 // in w.rho); *sK == 0 and *sregion == kInvalid on entry, visible to every
-// lane.  Marks the anchor done.
+// lane.
 //
 // An anchor may be split over several workgroups (SPLIT: blockIdx.y of
 // gridDim.y, each with its own copy of the region): the candidate vertices
 // are listed in region order, so every workgroup sees the same numbering of
 // the faces, and takes its share of them and of the pairs.  The workgroups
-// beyond one per kSplitFaces candidate faces have nothing to do; the status is
-// left to the caller.
+// beyond one per kSplitFaces candidate faces have nothing to do.
 constexpr uint64_t kSplitFaces = 2048;
-template <bool BIG, bool F32, bool SPLIT>
+template <bool BIG, bool F32, bool SPLIT, int WAVES>
 __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t *sK_,
                              uint32_t *sregion_) {
   uint32_t &sK = *sK_;
@@ -1135,12 +1179,12 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   // takes 64 candidate faces at a time: first passes one per lane, then the
   // queued sides and tetrahedra one per lane (LDS path; the global-memory
   // path works in place).
-  __shared__ uint32_t q_side[kBlock / 64][kSideQ];
-  __shared__ float q_side_r[kBlock / 64][kSideQ];
-  __shared__ uint32_t q_face[kBlock / 64][128];
-  __shared__ float q_key[kBlock / 64][128];
-  __shared__ uint32_t q_tet[kBlock / 64][kTetQ];
-  __shared__ uint32_t q_n[kBlock / 64][2];
+  __shared__ uint32_t q_side[WAVES][kSideQ];
+  __shared__ float q_side_r[WAVES][kSideQ];
+  __shared__ uint32_t q_face[WAVES][128];
+  __shared__ float q_key[WAVES][128];
+  __shared__ uint32_t q_tet[WAVES][kTetQ];
+  __shared__ uint32_t q_n[WAVES][2];
   const int wave = t >> 6, lane = t & 63, nwaves = (int)(blockDim.x >> 6);
   WaveQueues wq{q_side[wave], q_side_r[wave], q_tet[wave], &q_n[wave][0], &q_n[wave][1]};
   WaveQueues *q = BIG ? nullptr : &wq;
@@ -1254,14 +1298,12 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     if (*w.cand) atomicAdd(&P.counters[3], (unsigned long long)*w.cand);
     if (w.flops && *w.flops) atomicAdd(&P.counters[5], *w.flops);
     if (w.flops32 && *w.flops32) atomicAdd(&P.counters[6], *w.flops32);
-    if (!SPLIT) P.status[u] = ST_DONE;
   }
 }
 
-// BIG: arrays in global slabs, regions beyond LDS; the face phase works in
-// place instead of through the wave queues.
-template <bool BIG, bool F32>
-__device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
+// The whole work of one anchor on a global slab: certificate, region, and
+// (unless P.probe) the enumeration in place.
+__device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t a) {
   __shared__ uint32_t sM, sK, sflag, sregion;
   const int t = threadIdx.x;
   const uint32_t G = P.gcount[u];
@@ -1328,9 +1370,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
   const bool by_distance = G <= 4 * blockDim.x;
   uint32_t covers = 0;  // point-cell tests (FP32 count)
   for (int c = t; c < kCells; c += blockDim.x) {
-    const double *cd = P.cells + 8 * c;
     const CellF cf = cell_f(P.cellf + 8 * c);
-    const double chord = cd[5];
     float best[kCoverCap];
 #pragma unroll
     for (int j = 0; j < kCoverCap; ++j) best[j] = INFINITY;
@@ -1353,21 +1393,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
     float bk = INFINITY;
 #pragma unroll
     for (int j = 0; j < kCoverCap; ++j) bk = j == need_cover - 1 ? best[j] : bk;
-    const double rc = (double)bk * (1.0 + 1e-4);
-    double dir[3] = {cd[0], cd[1], cd[2]};
-    double uu[3] = {ux, uy, uz};
-    double e = INFINITY;
-    for (int a = 0; a < 3; ++a) {
-      double lo = dir[a] - chord, hi = dir[a] + chord;
-      if (lo > 0) e = fmin(e, (P.bhi[a] - uu[a]) / lo);
-      else if (hi < 0) e = fmin(e, (P.blo[a] - uu[a]) / hi);
-    }
-    e = fmax(e, 0.0) * (1.0 + 1e-9) + 1e-300;
-    // stored in FP32, rounded up (a larger radius only enlarges the region)
-    const double rd = fmin(rc, e);
-    float rf = (float)rd;
-    if (!((double)rf >= rd)) rf = rd <= (double)FLT_MIN ? FLT_MIN : nextafterf(rf, INFINITY);
-    w.rho[c] = rf;
+    w.rho[c] = cell_radius(P, c, bk, ux, uy, uz);
   }
   add_flops32(w, (uint64_t)covers * kF32Cover);
   __syncthreads();
@@ -1383,8 +1409,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
     s_rmax2 = (float)(2.0 * m) * 1.0001f;
     for (int wd = 0; wd < kCells / 64; ++wd) s_wlim[wd] = (float)(2.0 * wm[wd]) * 1.0001f;
     if (2.0 * m > Rg) {
-      P.need[u] = 2.0 * m;
-      P.status[u] = ST_WIDEN;
+      widen(P, u, 2.0 * m, Rg);
       sflag = 1;
     }
   }
@@ -1392,8 +1417,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
   if (sflag) return;
   const float rmax2 = s_rmax2;
   // 2. region membership masks, compacted in gathered order (chunks of four
-  // points per lane; the LDS path has a single chunk, so every FP32 offset is
-  // read before the first mask overwrites the area they share)
+  // points per lane)
   uint32_t members = 0;
   for (uint32_t c0 = 0; c0 < G; c0 += 4 * blockDim.x) {
     const uint32_t g = min(G - c0, 4 * blockDim.x);
@@ -1422,11 +1446,9 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
 #pragma unroll
     for (uint32_t r = 0; r < 4; ++r) {
       if (!mem[r]) continue;
-      if (slot < P.rcap) {
-        w.ridx[slot] = b0 + r;
+      w.ridx[slot] = b0 + r;
 #pragma unroll
-        for (int k = 0; k < 6; ++k) w.rmask[6 * slot + k] = mk[r][k];
-      }
+      for (int k = 0; k < 6; ++k) w.rmask[6 * slot + k] = mk[r][k];
       slot++;
     }
     members += scan_buf[blockDim.x - 1];
@@ -1435,17 +1457,6 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
   if (t == 0) sM = members;
   __syncthreads();
   const uint32_t M = sM;
-  if (M > P.rcap) {
-    if (t == 0) P.status[u] = ST_BIG;
-    return;
-  }
-  if (P.big && M > P.region_limit) {
-    if (t == 0) {
-      P.need[u] = (double)M;  // the region's size, reported with the conditional status
-      P.status[u] = ST_HUGE;
-    }
-    return;
-  }
   // the region's points move to the front of the point arrays, in region
   // order: from here on a region slot indexes them directly.  ridx ascends,
   // so every source lies at or after its destination and after the
@@ -1471,91 +1482,232 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u) {
     __syncthreads();
   }
   if (P.probe) {
-    // the region is known and compacted in the slab: its size is reported,
-    // and a region that fits LDS is enumerated there (k_anchor_region)
-    if (t == 0) {
-      P.need[u] = (double)M;
-      P.status[u] = ST_PROBED;
-    }
+    // the region is known and compacted in the slab; one that fits LDS is
+    // enumerated there (k_anchor_region)
+    if (t == 0) probed(P, u, a, M);
     return;
   }
-  anchor_faces<BIG, F32, false>(P, w, u, M, &sK, &sregion);
+  anchor_faces<true, true, false, kBlock / 64>(P, w, u, M, &sK, &sregion);
 }
 
-// The LDS path in two sizes: most anchors fit the small one, which leaves
-// room for four waves per SIMD; the wide one (one workgroup per CU) takes the
-// anchors whose gather or region outgrow it, before the global-memory path.
-template <int GCAP, int RCAP>
-__device__ void anchor_lds(const Params &P, uint32_t a) {
-  __shared__ double gx[GCAP], gy[GCAP], gz[GCAP];
+// Slab of one probed anchor (in doubles), for G gathered points:
+// [0, 3G) coordinates x, y, z relative to the anchor; [3G, 3G + kCells) cell
+// radii (float); [3G + kCells, 9G + kCells) masks, six words per point; then
+// PointIds.  The global-memory kernel adds its own arrays behind them.
+__host__ __device__ inline uint64_t slab_masks(uint64_t G) { return 3 * G + kCells; }
+__host__ __device__ inline uint64_t slab_ids(uint64_t G) { return 9 * G + kCells; }
+__host__ __device__ inline uint64_t probe_slab_doubles(uint64_t G) { return (slab_ids(G) + (G + 1) / 2 + 1) & ~1ull; }
+
+__device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t M) {
+  if (M > P.region_limit) {
+    // budget stop: the anchor stays open, the catalogue is conditional
+    atomicAdd(&P.counters[kOpenCount], 1ull);
+    atomicMax(&P.counters[kOpenLargest], (unsigned long long)M);
+    return;
+  }
+  P.region[u] = M;
+  if (M) list_add(P, M <= kRegionCap ? L_SMALL : M <= kRegionCapWide ? L_MID : M <= kRegionCapHuge ? L_LARGE : L_SLAB, a);
+}
+
+// Certificate and region of one anchor per workgroup, gathers of up to GCAP
+// points in LDS: six waves, one direction cell per lane.  A cell's radius
+// takes a scan of the points in increasing distance; the membership masks come
+// from the transposed loop, a wave per mask word and a ballot per point, so
+// that the cell stays in registers, the point is a broadcast and a word's scan
+// ends at the first point beyond the word's largest ball.  The region goes to
+// the anchor's slab, and its enumeration is another launch (k_anchor_region):
+// this kernel needs few registers and no enumeration queues, so more waves
+// share a CU than when one kernel did both, and the enumeration is split over
+// as many workgroups as its size asks for.  VALU bound.  Against one kernel per
+// anchor (two LDS sizes): catalogue of a 2 003-point mixture 332 -> 116 ms,
+// pipeline of 17 117 points K 4 19.3 -> 17.0 ms.
+constexpr int kProbeBlock = kCells;
+template <int GCAP>
+__global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
+  constexpr int kPer = (GCAP + kProbeBlock - 1) / kProbeBlock;
+  constexpr int kWaves = kProbeBlock / 64;
+  __shared__ __align__(16) float4 fc[GCAP];   // FP32 offset and distance (rounded up), ascending
   __shared__ uint32_t gid[GCAP];
-  __shared__ float rho[kCells];
-  __shared__ uint32_t ridx[RCAP];
-  // the FP32 offsets (16 B per gathered point) live in the mask area until
-  // the masks are written
-  __shared__ __align__(16) uint64_t rmask[6 * RCAP];
-  static_assert(sizeof(uint64_t) * 6 * RCAP >= sizeof(float4) * GCAP, "fc alias");
-  __shared__ uint32_t kidx[RCAP];
+  __shared__ __align__(16) uint64_t rmask[6 * GCAP];
+  __shared__ float wmax[kWaves];
+  __shared__ uint32_t wcount[kPer][kWaves];
+  __shared__ unsigned long long flops32;
+  const uint32_t a = blockIdx.x;
   if (a >= P.anchor_count) return;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const uint32_t u = P.anchors[a];
-  if (P.gcount[u] > P.gcap) {
-    if (threadIdx.x == 0) P.status[u] = ST_BIG;
+  const uint32_t G = P.gcount[u];
+  if (G > (uint32_t)GCAP) {
+    if (t == 0) list_add(P, GCAP < kGatherCapWide && G <= (uint32_t)kGatherCapWide ? L_WIDE : L_BIG, u);
     return;
   }
-  __shared__ uint32_t cand;
-  __shared__ unsigned long long flops, flops32;
-  if (threadIdx.x == 0) { cand = 0; flops = 0; flops32 = 0; }
-  __syncthreads();
-  // FP32 region coordinates in the tails of the gather arrays, free once the
-  // region is compacted to the front
-  static_assert(2 * (GCAP - RCAP) >= RCAP, "FP32 region copies fit the gather tails");
-  Work w{gx, gy, gz, gid, rho, ridx, rmask, kidx, reinterpret_cast<float4 *>(rmask), &cand,
-         P.count_flops ? &flops : nullptr, reinterpret_cast<float *>(gx + RCAP),
-         reinterpret_cast<float *>(gy + RCAP), reinterpret_cast<float *>(gz + RCAP),
-         P.count_flops ? &flops32 : nullptr};
-  anchor_work<false, true>(P, w, u);
-}
-
-__global__ void __launch_bounds__(kBlock, 3) k_anchor_lds(Params P) {
-  anchor_lds<kGatherCap, kRegionCap>(P, blockIdx.x);
-}
-__global__ void __launch_bounds__(kBlock, 2) k_anchor_lds_wide(Params P) {
-  anchor_lds<kGatherCapWide, kRegionCapWide>(P, blockIdx.x);
-}
-
-// One persistent launch over the first anchor pass of several clouds (a
-// batch): the workgroups take anchors from a shared counter until every
-// cloud's list is done.  Item i belongs to the job j with
-// offsets[j] <= i < offsets[j + 1]; each job carries its cloud's parameters
-// (coordinates, gathers, record queues).  The item index is uniform across
-// the workgroup, so a job's parameters are read with scalar loads.
-__global__ void __launch_bounds__(kBlock, 3) k_anchor_persist(const Params *__restrict__ jobs,
-                                                              const uint32_t *__restrict__ offsets, int njobs,
-                                                              unsigned int *head) {
-  __shared__ uint32_t s_item;
-  const uint32_t total = offsets[njobs];
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(head, 1u);
-    __syncthreads();
-    const uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();
-    if (item >= total) return;
-    int lo = 0, hi = njobs - 1;  // last job whose offset is <= item
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (offsets[mid] <= item) lo = mid;
-      else hi = mid - 1;
+  if (t == 0) flops32 = 0;
+  const uint64_t off = P.goff[u];
+  const double ux = P.X[u], uy = P.Y[u], uz = P.Z[u];
+  const double Rg = P.radius[u];  // before the first barrier: one lane may widen it below
+  // load, ranked by distance (the keys sit in the mask area until the masks come)
+  float *key = reinterpret_cast<float *>(rmask);
+  float4 mine[kPer];
+  uint32_t id[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = t + r * kProbeBlock;
+    mine[r] = make_float4(0.f, 0.f, 0.f, INFINITY);
+    id[r] = 0;
+    if (i < G) {
+      id[r] = P.glist[off + i];
+      const double x = P.X[id[r]] - ux, y = P.Y[id[r]] - uy, z = P.Z[id[r]] - uz;
+      mine[r] = make_float4((float)x, (float)y, (float)z, (float)sqrt(x * x + y * y + z * z) * (1.0f + 1e-6f));
+      key[i] = mine[r].w;
     }
-    const int j = __builtin_amdgcn_readfirstlane(lo);
-    anchor_lds<kGatherCap, kRegionCap>(jobs[j], item - offsets[j]);
-    __syncthreads();
+  }
+  const uint32_t G4 = (G + 3) & ~3u;
+  if (t < 4 && G + t < G4) key[G + t] = INFINITY;
+  __syncthreads();
+  uint32_t rank[kPer] = {};
+  for (uint32_t j = 0; j < G4; j += 4) {
+    const float4 k4 = *reinterpret_cast<const float4 *>(key + j);
+    const float kv[4] = {k4.x, k4.y, k4.z, k4.w};
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const uint32_t i = t + r * kProbeBlock;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) rank[r] += kv[q] < mine[r].w || (kv[q] == mine[r].w && j + q < i);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r)
+    if (t + r * kProbeBlock < G) {
+      fc[rank[r]] = mine[r];
+      gid[rank[r]] = id[r];
+    }
+  __syncthreads();
+  // 1. direction-cell certificate (FP32; every rounding errs towards larger
+  // radii): a point at distance l covers at radius >= l / 2 (up to the FP32
+  // rounding, inside the factor below), so once l / 2 exceeds the list's last
+  // entry no later point can enter it (and dropping points only enlarges the
+  // radius anyway)
+  const int c = t;
+  const CellF cf = cell_f(P.cellf + 8 * c);
+  float rho;
+  {
+    float best[kCoverCap];
+#pragma unroll
+    for (int j = 0; j < kCoverCap; ++j) best[j] = INFINITY;
+    uint32_t covers = 0;
+    for (uint32_t i = 0; i < G; ++i) {
+      const float4 q = fc[i];
+      if (!(q.w > kTinyLen)) continue;  // skipping a point only enlarges the radius
+      if (q.w * 0.49999f > best[kCoverCap - 1]) break;
+      covers++;
+      const float ct = (q.x * cf.dx + q.y * cf.dy + q.z * cf.dz) * __builtin_amdgcn_rcpf(q.w);
+      if (ct <= 0.0f) continue;
+      const float st = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - ct * ct));
+      const float cs = ct * cf.cosd - st * cf.sind;  // cos(theta + delta)
+      if (cs < 0.01f) continue;  // ill-conditioned cover: skipped
+      const float r = q.w * __builtin_amdgcn_rcpf(2.0f * cs);
+      if (!(r < best[kCoverCap - 1])) continue;
+#pragma unroll
+      for (int j = kCoverCap - 1; j > 0; --j) best[j] = __builtin_amdgcn_fmed3f(best[j - 1], r, best[j]);
+      best[0] = fminf(best[0], r);
+    }
+    if (P.count_flops) atomicAdd(&flops32, (unsigned long long)covers * kF32Cover);
+    float bk = INFINITY;
+#pragma unroll
+    for (int j = 0; j < kCoverCap; ++j) bk = j == P.s_max - 2 ? best[j] : bk;
+    rho = cell_radius(P, c, bk, ux, uy, uz);
+  }
+  float m = rho;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+  // 2 max rho over the word's cells in FP32, past the slack of the test
+  const float wlim = (float)(2.0 * (double)m) * 1.0001f;
+  if (lane == 0) wmax[wave] = m;
+  __syncthreads();
+  double need = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) need = fmax(need, 2.0 * (double)wmax[w]);
+  if (need > Rg) {  // uniform
+    if (t == 0) widen(P, u, need, Rg);
+    return;
+  }
+  // 2. region membership masks, word `wave`: FP32 with slack, a point may
+  // only be included too often
+  {
+    uint32_t tests = 0;
+    bool open = true;  // points up to the word's limit
+    for (uint32_t i0 = 0; i0 < G; i0 += 64) {
+      uint64_t word = 0;
+      const uint32_t n = min(64u, G - i0);
+      for (uint32_t j = 0; open && j < n; ++j) {
+        const float4 q = fc[i0 + j];
+        bool in = true;  // distance lost to underflow: member everywhere
+        if (q.w > kTinyLen) {
+          if (q.w > wlim) {
+            open = false;
+            break;
+          }
+          tests++;
+          const float ct = (q.x * cf.dx + q.y * cf.dy + q.z * cf.dz) * __builtin_amdgcn_rcpf(q.w);
+          const float cm = ct >= cf.cosd ? 1.0f  // cos(max(theta - delta, 0))
+                                         : ct * cf.cosd + __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - ct * ct)) * cf.sind;
+          in = q.w <= 2.0f * rho * (cm + 1e-5f) * (1.0f + 1e-5f);
+        }
+        const uint64_t b = __ballot(in);
+        word = (uint32_t)lane == j ? b : word;
+      }
+      if (i0 + lane < G) rmask[6 * (i0 + lane) + wave] = word;
+    }
+    if (P.count_flops && lane == 0) atomicAdd(&flops32, (unsigned long long)tests * 64 * kF32Mask);
+  }
+  __syncthreads();
+  // members, compacted in order of distance into the slab
+  uint64_t bits[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const uint32_t i = t + r * kProbeBlock;
+    uint64_t any = 0;
+    if (i < G)
+      for (int k = 0; k < 6; ++k) any |= rmask[6 * i + k];
+    bits[r] = __ballot(any != 0);
+    if (lane == 0) wcount[r][wave] = (uint32_t)__popcll(bits[r]);
+  }
+  __syncthreads();
+  double *slab = P.scratch + (uint64_t)a * P.slab_doubles;
+  const uint64_t S = P.gcap;
+  float *srho = reinterpret_cast<float *>(slab + 3 * S);
+  uint64_t *smask = reinterpret_cast<uint64_t *>(slab + slab_masks(S));
+  uint32_t *sgid = reinterpret_cast<uint32_t *>(slab + slab_ids(S));
+  srho[c] = rho;
+  uint32_t M = 0;
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    uint32_t slot = M;
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < wave) slot += wcount[r][w];
+      M += wcount[r][w];
+    }
+    if (!((bits[r] >> lane) & 1)) continue;
+    slot += (uint32_t)__popcll(bits[r] & ((1ull << lane) - 1ull));
+    const uint32_t i = t + r * kProbeBlock, v = gid[i];
+    slab[slot] = P.X[v] - ux;
+    slab[S + slot] = P.Y[v] - uy;
+    slab[2 * S + slot] = P.Z[v] - uz;
+    sgid[slot] = v;
+    for (int k = 0; k < 6; ++k) smask[6 * (uint64_t)slot + k] = rmask[6 * i + k];
+  }
+  if (t == 0) {
+    // a region beyond the LDS enumerations is probed again on its own slab
+    if (M > (uint32_t)kRegionCapHuge) list_add(P, L_BIG, u);
+    else probed(P, u, a, M);
+    if (P.count_flops) atomicAdd(&P.counters[6], flops32);
   }
 }
 
 // Offset (in doubles, even) of the FP32 offsets in a global slab of gather
 // capacity G; the slab holds big_fc_offset(G) + 2G doubles.
 __host__ __device__ inline uint64_t big_fc_offset(uint64_t G) {
-  return (3 * G + kCells + 6 * G + (3 * G + 1) / 2 + 1 + 1) & ~1ull;
+  return (slab_ids(G) + (3 * G + 1) / 2 + 1 + 1) & ~1ull;
 }
 
 // Anchors whose gather or region exceeds LDS: the same work on global slabs.
@@ -1570,8 +1722,8 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
   w.gy = slab + G;
   w.gz = slab + 2 * G;
   w.rho = reinterpret_cast<float *>(slab + 3 * G);
-  w.rmask = (uint64_t *)(slab + 3 * G + kCells);
-  w.gid = (uint32_t *)(slab + 3 * G + kCells + 6 * G);
+  w.rmask = (uint64_t *)(slab + slab_masks(G));
+  w.gid = (uint32_t *)(slab + slab_ids(G));
   w.ridx = w.gid + G;
   w.kidx = w.ridx + G;
   w.fc = reinterpret_cast<float4 *>(slab + big_fc_offset(G));
@@ -1586,36 +1738,32 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
   __syncthreads();
   w.cand = &cand;
   w.flops = P.count_flops ? &flops : nullptr;
-  anchor_work<true, true>(P, w, u);
+  anchor_work(P, w, u, a);
 }
 
-// Regions measured by the global-memory path's probe that fit LDS: the
-// anchor's compacted region (coordinates, PointIds, masks) and cell radii are
-// loaded from its slab into LDS, and the face phase runs there with the wave
-// queues.  Two sizes: regions of up to 640 points (two workgroups per CU) and
-// of 641 to 1 023 points (one workgroup per CU, 93 KB of LDS; region slots
-// stay below 1 024, as the packed queue items need).  Same parameters and
-// slab layout as k_anchor_big's probe launch; anchors not probed, or with
-// larger regions, are left to it.
+// Enumeration of probed regions that fit LDS: the region (coordinates,
+// PointIds, masks) and cell radii are loaded from the anchor's slab, and the
+// face phase runs on them with the wave queues.  Three sizes: up to 384 points
+// (three workgroups per CU at 168 VGPRs), up to 640 (two) and up to 1 023 (one;
+// region slots stay below 1 024, as the packed queue items need).  list:
+// the launch's slabs with such a region.
 //
 // One workgroup per anchor left the chip idle wherever tens of anchors held
-// such regions (43 anchors: 313 ms, each workgroup alone on its CU): the
-// launch asks for kRegionParts workgroups in all, a few per CU slot so that
+// large regions (43 anchors: 313 ms, each workgroup alone on its CU): a launch
+// asks for about kRegionParts workgroups in all, a few per CU slot so that
 // the longest ones do not end it alone.  A 2 003-point mixture's catalogue:
 // 885 -> 332 ms.
-constexpr int kRegionCapHuge = 1023;
 constexpr uint32_t kRegionParts = 4096;
-template <int RCAP, int RMIN>
-__global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anchor_region(Params P) {
-  const uint32_t a = blockIdx.x;
-  if (a >= P.anchor_count) return;
+template <int RCAP, int WAVES, int PER_SIMD>
+__global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P, const uint32_t *__restrict__ list) {
+  const uint32_t a = list[blockIdx.x];
   const uint32_t u = P.anchors[a];
-  if (P.status[u] != ST_PROBED || !(P.need[u] <= (double)RCAP) || !(P.need[u] > (double)RMIN)) return;
-  const uint32_t M = (uint32_t)P.need[u];
+  const uint32_t M = P.region[u];
+  if (M > (uint32_t)RCAP) return;
   const uint64_t G = P.gcap;
   const double *slab = P.scratch + (uint64_t)a * P.slab_doubles;
-  const uint64_t *smask = (const uint64_t *)(slab + 3 * G + kCells);
-  const uint32_t *sgid = (const uint32_t *)(slab + 3 * G + kCells + 6 * G);
+  const uint64_t *smask = (const uint64_t *)(slab + slab_masks(G));
+  const uint32_t *sgid = (const uint32_t *)(slab + slab_ids(G));
   __shared__ double gx[RCAP], gy[RCAP], gz[RCAP];
   __shared__ uint32_t gid[RCAP];
   __shared__ float rho[kCells];
@@ -1623,7 +1771,7 @@ __global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anch
   __shared__ uint32_t kidx[RCAP];
   __shared__ float fx[RCAP], fy[RCAP], fz[RCAP];
   __shared__ uint32_t cand, sK, sregion;
-  __shared__ unsigned long long flops;
+  __shared__ unsigned long long flops, flops32;
   const int t = threadIdx.x;
   for (uint32_t i = t; i < M; i += blockDim.x) {
     gx[i] = slab[i];
@@ -1633,18 +1781,11 @@ __global__ void __launch_bounds__(kBlock, RCAP <= kRegionCapWide ? 2 : 1) k_anch
   }
   for (uint32_t i = t; i < 6 * M; i += blockDim.x) rmask[i] = smask[i];
   for (int c = t; c < kCells; c += blockDim.x) rho[c] = reinterpret_cast<const float *>(slab + 3 * G)[c];
-  if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; }
+  if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; flops32 = 0; }
   __syncthreads();
-  Work w{gx, gy, gz, gid, rho, kidx, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz};
-  anchor_faces<false, true, true>(P, w, u, M, &sK, &sregion);
-}
-
-// Anchors whose region the LDS kernels have enumerated.
-__global__ void k_region_done(Params P, uint32_t rmax) {
-  const uint32_t a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= P.anchor_count) return;
-  const uint32_t u = P.anchors[a];
-  if (P.status[u] == ST_PROBED && P.need[u] <= (double)rmax) P.status[u] = ST_DONE;
+  Work w{gx, gy, gz, gid, rho, kidx, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz,
+         P.count_flops ? &flops32 : nullptr};
+  anchor_faces<false, true, true, WAVES>(P, w, u, M, &sK, &sregion);
 }
 
 // Ball count / emit around every anchor of the list: one wave per anchor over
@@ -1835,120 +1976,6 @@ void launch_gather(hipStream_t s, Context &c, CatalogBuffers &Bf, uint32_t cnt) 
                      wave_tree(c), c.leaf_pos.p, Bf.anchors.p, cnt, Bf.radius.p, Bf.gcount.p, Bf.goff.p, Bf.glist.p);
 }
 
-// Rendezvous of the clouds of one batch: each cloud's thread reaches its
-// first anchor pass, registers its parameters and waits; the last of them
-// queues one persistent launch over every registered cloud on the batch's
-// stream (after each cloud's own stream has reached that point), and every
-// cloud's stream then waits for that launch.  A cloud that will not reach
-// the pass (an error, a cloud too small for supports) leaves instead.
-struct AnchorBatch {
-  int device = 0;
-  std::mutex mu;
-  std::condition_variable cv;
-  int expected = 0, arrived = 0;
-  bool launched = false;
-  std::string error;
-  std::vector<char> done;  // per slot: arrived or left
-  std::vector<Params> jobs;
-  std::vector<uint32_t> counts, off;  // host sources of the launch's copies, kept until the batch ends
-  std::vector<hipEvent_t> ready;
-  hipStream_t stream = nullptr;
-  hipEvent_t t0 = nullptr, t1 = nullptr;
-  DevBuf<Params> d_jobs;
-  DevBuf<uint32_t> d_off;
-  DevBuf<unsigned int> d_head;
-  int64_t anchors = 0;
-  ~AnchorBatch() {
-    if (stream) (void)hipStreamSynchronize(stream);
-    for (hipEvent_t e : ready) (void)hipEventDestroy(e);
-    if (t0) (void)hipEventDestroy(t0);
-    if (t1) (void)hipEventDestroy(t1);
-    if (stream) (void)hipStreamDestroy(stream);
-  }
-  void launch_locked() {
-    try {
-      MHGP_HIP(hipSetDevice(device));
-      if (!stream) {
-        MHGP_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        MHGP_HIP(hipEventCreate(&t0));
-        MHGP_HIP(hipEventCreate(&t1));
-      }
-      for (hipEvent_t e : ready) MHGP_HIP(hipStreamWaitEvent(stream, e, 0));
-      const int J = (int)jobs.size();
-      off.assign(J + 1, 0);
-      for (int j = 0; j < J; ++j) off[j + 1] = off[j] + counts[j];
-      anchors = off[J];
-      d_jobs.ensure(J);
-      d_off.ensure(J + 1);
-      d_head.ensure(1);
-      MHGP_HIP(hipMemcpyAsync(d_jobs.p, jobs.data(), J * sizeof(Params), hipMemcpyHostToDevice, stream));
-      MHGP_HIP(hipMemcpyAsync(d_off.p, off.data(), (J + 1) * 4, hipMemcpyHostToDevice, stream));
-      MHGP_HIP(hipMemsetAsync(d_head.p, 0, 4, stream));
-      int cus = 0;
-      MHGP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-      // three workgroups per CU fit the kernel's LDS and registers
-      const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(off[J], (uint32_t)std::max(cus, 1) * 3));
-      MHGP_HIP(hipEventRecord(t0, stream));
-      if (off[J])
-        hipLaunchKernelGGL(k_anchor_persist, dim3(grid), dim3(kBlock), 0, stream, d_jobs.p, d_off.p, J, d_head.p);
-      MHGP_HIP(hipEventRecord(t1, stream));
-      MHGP_LAUNCH_CHECK();
-    } catch (const std::exception &e) {
-      error = e.what();
-    }
-    launched = true;
-    cv.notify_all();
-  }
-  void arrive(int slot, Context &c, const Params &P, uint32_t count) {
-    hipEvent_t ev = nullptr;
-    MHGP_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    MHGP_HIP(hipEventRecord(ev, c.stream));
-    std::unique_lock<std::mutex> g(mu);
-    if (slot < 0 || slot >= (int)done.size() || done[slot]) throw std::logic_error("batch slot reused");
-    done[slot] = 1;
-    jobs.push_back(P);
-    counts.push_back(count);
-    ready.push_back(ev);
-    arrived++;
-    if (arrived == expected) launch_locked();
-    else cv.wait(g, [&] { return launched; });
-    if (!error.empty()) throw HipError("batched anchor launch: " + error);
-    g.unlock();
-    MHGP_HIP(hipStreamWaitEvent(c.stream, t1, 0));
-  }
-  void leave(int slot) {
-    std::lock_guard<std::mutex> g(mu);
-    if (slot < 0 || slot >= (int)done.size() || done[slot]) return;
-    done[slot] = 1;
-    expected--;
-    if (!launched && arrived > 0 && arrived == expected) launch_locked();
-  }
-};
-
-std::shared_ptr<AnchorBatch> anchor_batch_create(int device, int participants) {
-  auto b = std::make_shared<AnchorBatch>();
-  b->device = device;
-  b->expected = participants;
-  b->done.assign(participants, 0);
-  return b;
-}
-
-void anchor_batch_leave(AnchorBatch &b, int slot) { b.leave(slot); }
-
-AnchorBatchStats anchor_batch_stats(AnchorBatch &b) {
-  AnchorBatchStats st{};
-  std::lock_guard<std::mutex> g(b.mu);
-  st.jobs = (int64_t)b.jobs.size();
-  st.anchors = b.anchors;
-  if (b.launched && b.error.empty() && b.t1) {
-    float ms = 0;
-    MHGP_HIP(hipEventSynchronize(b.t1));
-    MHGP_HIP(hipEventElapsedTime(&ms, b.t0, b.t1));
-    st.ms = ms;
-  }
-  return st;
-}
-
 void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
                      std::vector<FallbackRec> &fbs, std::vector<uint32_t> &fb_region,
                      mhgp_catalog_info *info) {
@@ -1969,9 +1996,9 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   B.radius.ensure(n);
   B.gcount.ensure(n);
   B.goff.ensure(n);
-  B.need.ensure(n);
-  B.status.ensure(n);
-  B.counters.ensure(8);
+  B.region.ensure(n);
+  B.lists.ensure((size_t)kLists * n);
+  B.counters.ensure(kCounters);
   B.anchors.ensure(n);
   if (B.cells.cap < 8 * kCells) {
     auto cells = make_cells();
@@ -1998,22 +2025,13 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   B.glist.ensure(1);
   launch_radius(s, c, kq, B);
   MHGP_LAUNCH_CHECK();
-  std::vector<uint32_t> anchors(n);
-  std::iota(anchors.begin(), anchors.end(), 0u);
-  // anchors in Morton order: neighbouring workgroups share cache lines
-  {
-    std::vector<uint32_t> lid(n);
-    copy_wait(lid.data(), c.leaf_id.p, n * 4, hipMemcpyDeviceToHost, s);
-    anchors = lid;
-  }
   double bounds[6];
   copy_wait(bounds, c.bounds.p, sizeof(bounds), hipMemcpyDeviceToHost, s);
   uint64_t event_cap = std::max<uint64_t>(1024, (uint64_t)n * (smax >= 11 ? 640 : 64 * smax));
   uint64_t fb_cap = std::max<uint64_t>(4096, (uint64_t)n / 4);
   uint64_t reg_cap = std::max<uint64_t>(1 << 20, (uint64_t)n * 64);
+  uint64_t ctr[kCounters];
   int64_t widened = 0;
-  int64_t open_anchors = 0, largest_open = 0;
-  uint64_t ctr[8];
   // The record queues have a fixed capacity per launch; records past it are
   // dropped on the device and counted.  A catalogue that outgrows them runs
   // again with queues sized from the counts (the widened gather radii are
@@ -2031,55 +2049,183 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   B.events.ensure(event_cap);
   B.fallbacks.ensure(fb_cap);
   B.fb_region.ensure(reg_cap);
-  MHGP_HIP(hipMemsetAsync(B.counters.p, 0, 8 * 8, s));
-  MHGP_HIP(hipMemsetAsync(B.status.p, 0, n * 4, s));
-  open_anchors = 0;
-  largest_open = 0;
-  std::vector<uint32_t> pending = anchors;
-  std::vector<uint32_t> big;
-  for (int iter = 0; !pending.empty(); ++iter) {
-    if (iter > 12) throw CapacityError("anchor gather radii did not converge");
-    const uint32_t cnt = (uint32_t)pending.size();
-    MHGP_HIP(hipMemcpyAsync(B.anchors.p, pending.data(), cnt * 4, hipMemcpyHostToDevice, s));
+  MHGP_HIP(hipMemsetAsync(B.counters.p, 0, kCounters * 8, s));
+  widened = 0;
+  Params P{};
+  P.X = c.X.p; P.Y = c.Y.p; P.Z = c.Z.p;
+  P.gcount = B.gcount.p; P.goff = B.goff.p; P.radius = B.radius.p;
+  P.cells = B.cells.p;
+  P.cellf = B.cellf.p;
+  for (int a = 0; a < 3; ++a) { P.blo[a] = bounds[a]; P.bhi[a] = bounds[3 + a]; }
+  P.s_max = smax;
+  P.region = B.region.p;
+  P.lists = B.lists.p;
+  P.list_cap = (uint32_t)n;
+  P.events = B.events.p; P.event_cap = event_cap;
+  P.fallbacks = B.fallbacks.p; P.fallback_cap = fb_cap;
+  P.fb_region = B.fb_region.p; P.fb_region_cap = reg_cap;
+  P.counters = (unsigned long long *)B.counters.p;
+  P.count_flops = c.count_flops ? 1 : 0;
+  P.region_limit = std::min<uint32_t>(c.region_limit, kBigRegionMax);
+  auto list = [&](int l) { return B.lists.p + (size_t)l * n; };
+  auto read_counters = [&] { copy_wait(ctr, B.counters.p, sizeof ctr, hipMemcpyDeviceToHost, s); };
+  // clears the lengths of lists [first, last)
+  auto clear_lists = [&](int first, int last) {
+    MHGP_HIP(hipMemsetAsync(B.counters.p + kListCount + first, 0, (last - first) * 8, s));
+  };
+  // enumerates the regions of one probe launch (ctr holds its list lengths),
+  // the largest first
+  auto enumerate = [&](const Params &Q) {
+    for (int l = L_LARGE; l >= L_SMALL; --l) {
+      const uint32_t m = (uint32_t)ctr[kListCount + l];
+      if (!m) continue;
+      const dim3 grid(m, std::clamp<uint32_t>(kRegionParts / m, 1, 64));
+      if (l == L_LARGE)
+        hipLaunchKernelGGL((k_anchor_region<kRegionCapHuge, 8, 2>), grid, dim3(512), 0, s, Q, list(l));
+      else if (l == L_MID)
+        hipLaunchKernelGGL((k_anchor_region<kRegionCapWide, 4, 2>), grid, dim3(256), 0, s, Q, list(l));
+      else
+        hipLaunchKernelGGL((k_anchor_region<kRegionCap, 4, 3>), grid, dim3(256), 0, s, Q, list(l));
+      MHGP_LAUNCH_CHECK();
+    }
+  };
+  // scratch for slabs: 8 GiB, 1 GiB in a context with a device capacity; and
+  // at most a quarter of the device memory still free (other contexts on the
+  // device keep theirs), but never below 1 GiB
+  auto slab_budget = [&]() -> uint64_t {
+    if (c.capacity_bytes > 0) return 1ull << 30;
+    size_t free_b = 0, total_b = 0;
+    MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
+    return std::max<uint64_t>(1ull << 30, std::min<uint64_t>(8ull << 30, free_b / 4));
+  };
+  // Probes `count` anchors of the device list in chunks whose slabs fit the
+  // chunk budget (2 GiB; under a capacity a quarter of what it leaves, at
+  // least 1 MiB), each chunk enumerated before the next one takes its slabs.
+  auto probe_lds = [&](const uint32_t *anchors, uint32_t count, bool wide) {
+    const uint32_t g = wide ? kGatherCapWide : kGatherCap;
+    const uint64_t slab = probe_slab_doubles(g);
+    uint64_t budget = 2ull << 30;
+    if (c.capacity_bytes > 0)
+      budget = std::clamp<int64_t>((c.capacity_bytes - device_bytes(c)) / 4 + (int64_t)B.scratch.bytes(), 1 << 20, 1 << 30);
+    const uint32_t most = (uint32_t)std::max<uint64_t>(1, budget / (slab * 8));
+    const uint32_t chunks = (count + most - 1) / most, per = (count + chunks - 1) / chunks;
+    B.scratch.ensure(slab * per);
+    for (uint32_t a0 = 0; a0 < count; a0 += per) {
+      Params Q = P;
+      Q.anchors = anchors + a0;
+      Q.anchor_count = std::min(per, count - a0);
+      Q.gcap = g;
+      Q.scratch = B.scratch.p;
+      Q.slab_doubles = slab;
+      clear_lists(L_SMALL, kLists);
+      if (wide)
+        hipLaunchKernelGGL(k_anchor_probe<kGatherCapWide>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
+      else
+        hipLaunchKernelGGL(k_anchor_probe<kGatherCap>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
+      MHGP_LAUNCH_CHECK();
+      read_counters();
+      enumerate(Q);
+    }
+  };
+  // anchors in Morton order: neighbouring workgroups share cache lines
+  MHGP_HIP(hipMemcpyAsync(B.anchors.p, c.leaf_id.p, n * 4, hipMemcpyDeviceToDevice, s));
+  uint32_t cnt = (uint32_t)n;
+  for (int iter = 0; cnt > 0; ++iter) {
+    if (iter > 24) throw CapacityError("anchor gather radii did not converge");
     launch_gather<false>(s, c, B, cnt);
     hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, s, B.anchors.p, cnt, B.gcount.p,
                        B.goff.p, total.p);
     uint64_t tot = 0;
-    MHGP_HIP(hipMemcpyAsync(&tot, total.p, 8, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipStreamSynchronize(s));
+    copy_wait(&tot, total.p, 8, hipMemcpyDeviceToHost, s);
     B.glist.ensure(tot + 1);
     launch_gather<true>(s, c, B, cnt);
-    Params P{};
-    P.X = c.X.p; P.Y = c.Y.p; P.Z = c.Z.p;
-    P.gcount = B.gcount.p; P.goff = B.goff.p; P.glist = B.glist.p; P.radius = B.radius.p;
-    P.cells = B.cells.p;
-    P.cellf = B.cellf.p;
-    for (int a = 0; a < 3; ++a) { P.blo[a] = bounds[a]; P.bhi[a] = bounds[3 + a]; }
-    P.s_max = smax;
-    P.need = B.need.p; P.status = B.status.p;
-    P.events = B.events.p; P.event_cap = event_cap;
-    P.fallbacks = B.fallbacks.p; P.fallback_cap = fb_cap;
-    P.fb_region = B.fb_region.p; P.fb_region_cap = reg_cap;
-    P.counters = (unsigned long long *)B.counters.p;
-    P.anchors = B.anchors.p; P.anchor_count = cnt;
-    P.big = 0; P.gcap = kGatherCap; P.rcap = kRegionCap;
-    P.count_flops = c.count_flops ? 1 : 0;
-    P.region_limit = std::min<uint32_t>(c.region_limit, kBigRegionMax);
+    P.glist = B.glist.p;
     tm.mark("catalogue gather");
-    uint64_t ctr_before[8];
-    copy_wait(ctr_before, B.counters.p, sizeof(ctr_before), hipMemcpyDeviceToHost, s);
-    if (c.batch && attempt == 0 && iter == 0) {
-      // first pass of a batched cloud: one persistent launch over the batch
-      c.batch->arrive(c.batch_slot, c, P, cnt);
-    } else if (!force_path) {
+    uint64_t before[kCounters];
+    copy_wait(before, B.counters.p, sizeof before, hipMemcpyDeviceToHost, s);
+    clear_lists(0, kLists);
     c.anchor_clock.start(s);
-    hipLaunchKernelGGL(k_anchor_lds, dim3(cnt), dim3(kBlock), 0, s, P);
+    if (!force_path) {
+      probe_lds(B.anchors.p, cnt, false);
+      if (const uint32_t wc = (uint32_t)ctr[kListCount + L_WIDE]) {
+        probe_lds(list(L_WIDE), wc, true);
+        if (tm.on) std::fprintf(stderr, "[mhgp] wide anchors: %u\n", wc);
+      }
+    }
     c.anchor_clock.stop(s);
-    MHGP_LAUNCH_CHECK();
-    {
-      uint64_t ctr_after[8];
-      copy_wait(ctr_after, B.counters.p, sizeof(ctr_after), hipMemcpyDeviceToHost, s);
-      const uint64_t ev = ctr_after[0] - ctr_before[0];
+    tm.mark("catalogue anchors");
+    // gathers beyond LDS: probed on slabs in chunks of anchors of similar
+    // gather size (ascending), each chunk's slabs sized by its own largest
+    // gather within the scratch budget, so that a few anchors that gather most
+    // of the cloud do not shrink every launch to a handful of workgroups
+    std::vector<uint32_t> big(force_path ? cnt : (uint32_t)ctr[kListCount + L_BIG]);
+    if (!big.empty()) {
+      copy_wait(big.data(), force_path ? B.anchors.p : list(L_BIG), big.size() * 4, hipMemcpyDeviceToHost, s);
+      std::vector<uint32_t> gc(n);
+      copy_wait(gc.data(), B.gcount.p, n * 4, hipMemcpyDeviceToHost, s);
+      const uint64_t kScratchBudget = slab_budget();
+      auto slab_of = [](uint32_t g) { return big_fc_offset(g) + 2ull * g; };
+      // the probed regions beyond LDS come back in `slabs`
+      auto launch_big = [&](std::vector<uint32_t> todo, int probe, std::vector<uint32_t> &slabs) {
+        std::sort(todo.begin(), todo.end(),
+                  [&](uint32_t x, uint32_t y) { return gc[x] < gc[y] || (gc[x] == gc[y] && x < y); });
+        const size_t lc = todo.size();
+        std::vector<std::pair<size_t, uint32_t>> chunks;  // (end, gather cap)
+        uint64_t scratch = 0;
+        for (size_t b0 = 0; b0 < lc;) {
+          size_t b1 = b0;
+          uint32_t g = 64;
+          while (b1 < lc) {
+            const uint32_t gn = std::max<uint32_t>(64, gc[todo[b1]]);
+            if (b1 > b0 && slab_of(gn) * 8 * (b1 - b0 + 1) > kScratchBudget) break;
+            g = gn;
+            ++b1;
+          }
+          chunks.push_back({b1, g});
+          scratch = std::max<uint64_t>(scratch, slab_of(g) * (b1 - b0));
+          b0 = b1;
+        }
+        B.scratch.ensure(scratch);
+        B.big.ensure(lc);
+        MHGP_HIP(hipMemcpyAsync(B.big.p, todo.data(), lc * 4, hipMemcpyHostToDevice, s));
+        size_t b0 = 0;
+        for (const auto &ch : chunks) {
+          const uint32_t bn = (uint32_t)(ch.first - b0), g = ch.second;
+          Params Q = P;
+          Q.anchors = B.big.p + b0; Q.anchor_count = bn; Q.probe = probe;
+          Q.scratch = B.scratch.p; Q.slab_doubles = slab_of(g); Q.gcap = g;
+          if (probe) clear_lists(L_SMALL, kLists);
+          hipLaunchKernelGGL(k_anchor_big, dim3(bn), dim3(kBlock), 0, s, Q);
+          MHGP_LAUNCH_CHECK();
+          if (probe) {
+            read_counters();
+            // test hook: every region through the slab enumeration
+            if (force_path != 2) enumerate(Q);
+            for (int l = force_path == 2 ? L_SMALL : L_SLAB; l <= L_SLAB; ++l) {
+              std::vector<uint32_t> at(ctr[kListCount + l]);
+              if (!at.empty()) copy_wait(at.data(), list(l), at.size() * 4, hipMemcpyDeviceToHost, s);
+              for (uint32_t i : at) {
+                if (i >= bn) throw std::runtime_error("malformed region list from the device");
+                slabs.push_back(todo[b0 + i]);
+              }
+            }
+          }
+          b0 = ch.first;
+        }
+      };
+      // first the regions only, so that one the path cannot take is refused
+      // before any long launch
+      std::vector<uint32_t> slabs, none;
+      launch_big(big, 1, slabs);
+      tm.mark("catalogue big probe (+ LDS regions)");
+      if (!slabs.empty()) launch_big(slabs, 0, none);
+      tm.mark("catalogue big on slabs");
+      if (tm.on)
+        std::fprintf(stderr, "[mhgp] big anchors: %zu, %zu on slabs\n", big.size(), slabs.size());
+    }
+    read_counters();
+    if (!force_path) {
+      const uint64_t ev = ctr[0] - before[0];
       c.stats.anchor_ms += c.anchor_clock.ms();
       c.stats.anchor_launches++;
       c.stats.gathered_points += (int64_t)tot;
@@ -2087,179 +2233,17 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
       // algorithmic bytes: every gathered neighbour read once (id + FP64 xyz),
       // every record written once
       c.stats.anchor_bytes += (int64_t)tot * 28 + (int64_t)ev * (int64_t)sizeof(EventRec);
-      // FP64 operations of the certified predicates the launch evaluated
-      c.stats.anchor_flops += (int64_t)(ctr_after[5] - ctr_before[5]);
-      c.stats.anchor_flops32 += (int64_t)(ctr_after[6] - ctr_before[6]);
+      // FP64 and FP32 operations of the certified predicates the launches evaluated
+      c.stats.anchor_flops += (int64_t)(ctr[5] - before[5]);
+      c.stats.anchor_flops32 += (int64_t)(ctr[6] - before[6]);
     }
-    }
-    tm.mark("catalogue anchors");
-    std::vector<uint32_t> st(n);
-    std::vector<double> need(n), rad(n);
-    std::vector<uint32_t> gc(n);
-    MHGP_HIP(hipMemcpyAsync(st.data(), B.status.p, n * 4, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipMemcpyAsync(need.data(), B.need.p, n * 8, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipMemcpyAsync(rad.data(), B.radius.p, n * 8, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipMemcpyAsync(gc.data(), B.gcount.p, n * 4, hipMemcpyDeviceToHost, s));
-    MHGP_HIP(hipStreamSynchronize(s));
-    if (force_path)
-      for (uint32_t u : pending) st[u] = ST_BIG;
-    std::vector<uint32_t> next, wide_list;
-    for (int tier = 0; tier < 2; ++tier) {
-      std::vector<uint32_t> wide;
-      for (uint32_t u : (tier == 0 ? pending : wide_list)) {
-        if (st[u] == ST_WIDEN) {
-          rad[u] = std::max(need[u] * 1.02, rad[u] * 1.05);
-          next.push_back(u);
-          widened++;
-        } else if (st[u] == ST_BIG) {
-          if (tier == 0 && !force_path && gc[u] <= (uint32_t)kGatherCapWide) wide.push_back(u);
-          else big.push_back(u);
-        }
-      }
-      if (tier == 1 || wide.empty()) break;
-      // anchors that outgrew the small LDS path: the wide one
-      wide_list = wide;
-      const uint32_t wc = (uint32_t)wide.size();
-      MHGP_HIP(hipMemcpyAsync(B.anchors.p, wide.data(), wc * 4, hipMemcpyHostToDevice, s));
-      Params W2 = P;
-      W2.anchor_count = wc;
-      W2.gcap = kGatherCapWide;
-      W2.rcap = kRegionCapWide;
-      hipLaunchKernelGGL(k_anchor_lds_wide, dim3(wc), dim3(kBlock), 0, s, W2);
-      MHGP_LAUNCH_CHECK();
-      MHGP_HIP(hipMemcpyAsync(st.data(), B.status.p, n * 4, hipMemcpyDeviceToHost, s));
-      MHGP_HIP(hipMemcpyAsync(need.data(), B.need.p, n * 8, hipMemcpyDeviceToHost, s));
-      MHGP_HIP(hipStreamSynchronize(s));
-      if (tm.on) std::fprintf(stderr, "[mhgp] wide anchors: %u\n", wc);
-      tm.mark("catalogue wide anchors");
-    }
-    // big anchors: widen inside the big path too
-    if (!big.empty()) {
-      std::vector<uint32_t> redo;
-      for (int biter = 0; !big.empty(); ++biter) {
-        if (biter > 12) throw std::runtime_error("big anchors did not converge");
-        const uint32_t bc = (uint32_t)big.size();
-        uint32_t gmax = 0;
-        for (uint32_t u : big) gmax = std::max(gmax, gc[u]);
-        gmax = std::max<uint32_t>(gmax, 64);
-        // the CSR of the big anchors is still valid from this iteration's gather
-        std::vector<uint32_t> again;
-        // Launches in chunks of anchors of similar gather size (ascending), each
-        // chunk's slabs sized by its own largest gather within one scratch
-        // budget: a few anchors that gather most of the cloud no longer shrink
-        // every launch to a handful of workgroups.  The budget (8 GiB, 1 GiB
-        // in a context with a device capacity) keeps hundreds of workgroups
-        // per launch even for gathers of 100 000 points (~10 MB of slab each).
-        // The slabs are reused from one chunk to the next.
-        uint64_t kScratchBudget = c.capacity_bytes > 0 ? (1ull << 30) : (8ull << 30);  // bytes
-        if (c.capacity_bytes <= 0) {
-          // and at most a quarter of the device memory still free (other
-          // contexts on the device keep theirs), but never below 1 GiB
-          size_t free_b = 0, total_b = 0;
-          MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
-          kScratchBudget = std::max<uint64_t>(1ull << 30, std::min<uint64_t>(kScratchBudget, free_b / 4));
-        }
-        auto slab_of = [](uint32_t g) { return big_fc_offset(g) + 2ull * g; };
-        auto launch_big = [&](const std::vector<uint32_t> &list_in, int probe) {
-          std::vector<uint32_t> list(list_in);
-          std::sort(list.begin(), list.end(),
-                    [&](uint32_t x, uint32_t y) { return gc[x] < gc[y] || (gc[x] == gc[y] && x < y); });
-          const size_t lc = list.size();
-          std::vector<std::pair<size_t, uint32_t>> chunks;  // (end, gather cap)
-          uint64_t scratch = 0;
-          for (size_t b0 = 0; b0 < lc;) {
-            size_t b1 = b0;
-            uint32_t g = 64;
-            while (b1 < lc) {
-              const uint32_t gn = std::max<uint32_t>(64, gc[list[b1]]);
-              if (b1 > b0 && slab_of(gn) * 8 * (b1 - b0 + 1) > kScratchBudget) break;
-              g = gn;
-              ++b1;
-            }
-            chunks.push_back({b1, g});
-            scratch = std::max<uint64_t>(scratch, slab_of(g) * (b1 - b0));
-            b0 = b1;
-          }
-          B.scratch.ensure(scratch);
-          size_t b0 = 0;
-          for (const auto &ch : chunks) {
-            const uint32_t bn = (uint32_t)(ch.first - b0), g = ch.second;
-            MHGP_HIP(hipMemcpyAsync(B.anchors.p, list.data() + b0, bn * 4, hipMemcpyHostToDevice, s));
-            b0 = ch.first;
-            Params Q = P;
-            // the gather CSR may have been reallocated by a regather below
-            Q.gcount = B.gcount.p; Q.goff = B.goff.p; Q.glist = B.glist.p; Q.radius = B.radius.p;
-            Q.anchors = B.anchors.p; Q.anchor_count = bn; Q.big = 1; Q.probe = probe;
-            Q.scratch = B.scratch.p; Q.slab_doubles = slab_of(g); Q.gcap = g; Q.rcap = g;
-            hipLaunchKernelGGL(k_anchor_big, dim3(bn), dim3(kBlock), 0, s, Q);
-            // probed regions that fit LDS: enumerated there, from this chunk's slabs
-            if (probe && force_path != 2) {
-              const uint32_t parts = std::clamp<uint32_t>(kRegionParts / bn, 1, 64);
-              hipLaunchKernelGGL((k_anchor_region<kRegionCapHuge, kRegionCapWide>), dim3(bn, parts), dim3(kBlock), 0, s,
-                                 Q);
-              hipLaunchKernelGGL((k_anchor_region<kRegionCapWide, 0>), dim3(bn, parts), dim3(kBlock), 0, s, Q);
-              hipLaunchKernelGGL(k_region_done, dim3(blocks_for(bn, 256)), dim3(256), 0, s, Q,
-                                 (uint32_t)kRegionCapHuge);
-            }
-            MHGP_LAUNCH_CHECK();
-          }
-          MHGP_HIP(hipMemcpyAsync(st.data(), B.status.p, n * 4, hipMemcpyDeviceToHost, s));
-          MHGP_HIP(hipMemcpyAsync(need.data(), B.need.p, n * 8, hipMemcpyDeviceToHost, s));
-          MHGP_HIP(hipStreamSynchronize(s));
-        };
-        // first the region sizes only (no enumeration), so that a region the
-        // path cannot take is refused before any long launch
-        launch_big(big, 1);
-        tm.mark("catalogue big probe (+ LDS regions)");
-        std::vector<uint32_t> full;
-        for (uint32_t u : big) {
-          if (st[u] == ST_WIDEN) {
-            rad[u] = std::max(need[u] * 1.02, rad[u] * 1.05);
-            again.push_back(u);
-            widened++;
-          } else if (st[u] == ST_HUGE) {
-            // budget stop: the anchor stays open, the catalogue is conditional
-            open_anchors++;
-            largest_open = std::max<int64_t>(largest_open, (int64_t)need[u]);
-          } else if (st[u] == ST_PROBED) {
-            full.push_back(u);
-          } else if (st[u] == ST_DONE) {
-            // region enumerated in LDS after the probe
-          } else {
-            throw std::runtime_error("a big anchor did not complete its probe");
-          }
-        }
-        if (tm.on)
-          std::fprintf(stderr, "[mhgp] big pass %d: %u anchors, gather cap %u: %zu widen, %zu on slabs, %lld open so far\n",
-                       biter, bc, gmax, again.size(), full.size(), (long long)open_anchors);
-        if (!full.empty()) launch_big(full, 0);
-        tm.mark("catalogue big on slabs");
-        for (uint32_t u : full)
-          if (st[u] != ST_DONE) throw std::runtime_error("a big anchor did not complete");
-        if (again.empty()) break;
-        // regather the widened big anchors
-        const uint32_t ac = (uint32_t)again.size();
-        copy_wait(B.radius.p, rad.data(), n * 8, hipMemcpyHostToDevice, s);
-        MHGP_HIP(hipMemcpyAsync(B.anchors.p, again.data(), ac * 4, hipMemcpyHostToDevice, s));
-        launch_gather<false>(s, c, B, ac);
-        hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, s, B.anchors.p, ac, B.gcount.p,
-                           B.goff.p, total.p);
-        MHGP_HIP(hipMemcpyAsync(&tot, total.p, 8, hipMemcpyDeviceToHost, s));
-        MHGP_HIP(hipStreamSynchronize(s));
-        B.glist.ensure(tot + 1);
-        launch_gather<true>(s, c, B, ac);
-        MHGP_HIP(hipMemcpyAsync(gc.data(), B.gcount.p, n * 4, hipMemcpyDeviceToHost, s));
-        MHGP_HIP(hipStreamSynchronize(s));
-        tm.mark("catalogue big regather");
-        big = again;
-      }
-      big.clear();
-    }
-    copy_wait(B.radius.p, rad.data(), n * 8, hipMemcpyHostToDevice, s);
-    pending = next;
+    // the widened gathers are the next pass
+    cnt = (uint32_t)ctr[kListCount + L_WIDEN];
+    widened += cnt;
+    if (cnt) MHGP_HIP(hipMemcpyAsync(B.anchors.p, list(L_WIDEN), cnt * 4, hipMemcpyDeviceToDevice, s));
   }
   tm.mark("catalogue big anchors");
-  copy_wait(ctr, B.counters.p, sizeof(ctr), hipMemcpyDeviceToHost, s);
+  read_counters();
   if (ctr[4]) throw std::runtime_error("face side queue overflow");
   if (ctr[0] <= event_cap && ctr[1] <= fb_cap && ctr[2] <= reg_cap) break;
   if (attempt >= 2) throw CapacityError("catalogue record queues did not settle after regrowth");
@@ -2290,9 +2274,9 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   tm.mark("catalogue download");
   info->candidate_count = (int64_t)ctr[3];
   info->anchors_widened = widened;
-  info->anchors_open = open_anchors;
-  info->largest_open_region = largest_open;
-  info->status = open_anchors ? 1 : 0;
+  info->anchors_open = (int64_t)ctr[kOpenCount];
+  info->largest_open_region = (int64_t)ctr[kOpenLargest];
+  info->status = ctr[kOpenCount] ? 1 : 0;
 }
 
 }  // namespace mhgp

@@ -8,10 +8,10 @@
 namespace mhgp {
 
 constexpr int kCells = 384;      // 6 cube faces x 8 x 8 direction cells
-constexpr int kGatherCap = 600;  // gathered neighbours held in LDS
-constexpr int kRegionCap = 384;  // region members held in LDS
+constexpr int kGatherCap = 600;  // gathered neighbours the probe holds in LDS
+constexpr int kRegionCap = 384;  // region members the smallest enumeration holds in LDS
 constexpr uint32_t kRegionLimitMax = 2048;  // largest candidate region any path enumerates
-constexpr int kGatherCapWide = 1024;  // the same for the wide LDS path
+constexpr int kGatherCapWide = 1024;  // the same for the wide probe and the next enumeration
 constexpr int kRegionCapWide = 640;
 constexpr int kMaxInterior = 10; // s_max - 2 for s_max <= 11 (K_max <= 10)
 
@@ -46,15 +46,16 @@ struct CatalogBuffers {
   DevBuf<uint32_t> gcount;        // gathered count per anchor
   DevBuf<uint64_t> goff;          // CSR offsets
   DevBuf<uint32_t> glist;         // gathered ids
-  DevBuf<double> need;            // radius required by the certificate (0 = satisfied)
-  DevBuf<uint32_t> status;        // per anchor: 0 pending, 1 done, 2 widen, 3 big
+  DevBuf<uint32_t> region;        // region size of a probed anchor
+  DevBuf<uint32_t> lists;         // anchors by what comes next for them (supports.hip)
+  DevBuf<uint32_t> big;           // anchors of a global-memory launch
   DevBuf<EventRec> events;
   DevBuf<FallbackRec> fallbacks;
   DevBuf<uint32_t> fb_region;     // region member ids of anchors with fallbacks
-  DevBuf<uint64_t> counters;      // events, fallbacks, region words, candidates
+  DevBuf<uint64_t> counters;      // events, fallbacks, region words, candidates, operations, list lengths
   DevBuf<double> cells;           // per cell: dir xyz, cos d, sin d, chord
   DevBuf<float> cellf;            // per cell: the FP32 cell of the certificate and the masks
-  DevBuf<double> scratch;         // global slabs for anchors too big for LDS
+  DevBuf<double> scratch;         // slabs: the regions of probed anchors
   DevBuf<uint32_t> anchors;       // anchor list of the current launch
   // canonical order on the device: records (device emitted + host settled),
   // their order by (exact level, rank, support) and dense exact level classes

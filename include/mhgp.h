@@ -330,11 +330,8 @@ int mhgp_server_release(mhgp_server *srv, int64_t ticket);
 void mhgp_server_destroy(mhgp_server *srv);
 
 /* Batched processing of many clouds in one call.  Clouds run in groups, side
- * by side (one host thread and one context per cloud of a group); the first
- * anchor pass of the catalogue of every cloud of a group is ONE persistent
- * launch over all of their anchors (workgroups take anchors from a shared
- * counter across clouds), then each cloud continues as the plain path does:
- * the remaining anchor passes, the tower unless the catalogue is conditional.
+ * by side (one host thread and one context per cloud of a group), each as on
+ * the plain path: catalogue, the tower unless the catalogue is conditional.
  * A group holds at most `group` clouds (<= 0: 32) whose predicted device
  * bytes fit memory_cap_bytes (<= 0: 80% of the device's memory).  Results per
  * cloud as for the server; a failing cloud fails alone.  No reference
@@ -346,9 +343,9 @@ typedef struct mhgp_batch mhgp_batch;
 
 typedef struct {
   int64_t clouds;
-  int64_t groups;     /* persistent launches */
-  int64_t anchors;    /* anchors those launches processed */
-  double anchor_ms;   /* their device time, summed */
+  int64_t groups;
+  int64_t anchors;    /* anchors their catalogues processed */
+  double anchor_ms;   /* device time of their anchor kernels, summed */
   double wall_ms;     /* the whole call */
 } mhgp_batch_info;
 
