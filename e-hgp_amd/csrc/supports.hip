@@ -152,7 +152,6 @@ struct Work {
 // the value, its magnitude bound and the certification test.
 constexpr uint32_t kFlopPairSide = 18;   // PairSphere::side
 constexpr uint32_t kFlopTetSide = 21;    // TetSphere::side
-constexpr uint32_t kFlopCapsule = 8;     // Capsule::outside
 constexpr uint32_t kFlopFacePoint = 33;  // TriSphere::power + height, two certified signs
 constexpr uint32_t kFlopSweepKey = 24;   // sweep_key
 constexpr uint32_t kFlopTriInit = 66;    // TriSphere::init
@@ -164,12 +163,13 @@ __device__ inline void add_flops(const Work &w, uint64_t v) {
   if (w.flops && v) atomicAdd(w.flops, (unsigned long long)v);
 }
 // FP32 operations of the FP32 tests, counted the same way (the certificate
-// and mask tests of a cell, the capsule test, the face, pair and tetrahedron
+// and mask tests of a cell, the pencil tests, the face, pair and tetrahedron
 // polynomials with their bounds, a key interval); reciprocals and square
 // roots count one each.
 constexpr uint32_t kF32Cover = 16;      // one point against one cell (certificate)
 constexpr uint32_t kF32Mask = 16;       // one point against one cell (membership)
-constexpr uint32_t kF32Capsule = 8;     // capsule_chunk_f, per slot
+constexpr uint32_t kF32Pencil = 19;     // Pencil::outside, per slot
+constexpr uint32_t kF32Cell = 28;       // one shared cell of a face (face_interval)
 constexpr uint32_t kF32FacePoint = 31;  // TriSphereF::eval and two certified signs
 constexpr uint32_t kF32Key = 16;        // key_bounds_32
 constexpr uint32_t kF32PairSide = 17;   // PairSphereF::side
@@ -590,54 +590,65 @@ __device__ inline void key_bounds_32(float Pv, float PA, float H, float HA, floa
 // already ahead), each checked against the inside points behind the side.
 // One pass over the region fills the side's sweep list; the candidates are
 // packed into a mask before any tetrahedron is classified.
-// Capsule holding every sphere of a face's pencil that can be critical:
-// centres c3 + t n with |t| <= T, radii <= Rb.  A point farther than T + Rb
-// from c3 is outside all of them (checked with a relative margin).
-struct Capsule {
-  V3 c3;
-  double bound2;  // (T + Rb)^2 with margin; INFINITY disables the test
-  __device__ bool outside(const V3 &p) const {
-    const V3 d = sub(p, c3);
-    return dot(d, d) > bound2;
+// The part of a face's pencil that can be critical: spheres through u, v, w
+// with centres c3 + t n, t in an interval [tl, tu] (face_interval).  A point's
+// power against such a sphere is linear in t, so a point outside both end
+// spheres is outside all of them.  FP32 with the anchor at the origin:
+// outside when p.p > 2 p.c for both end centres c, by a margin of
+// 1e-3 p.p + a, which exceeds the rounding of the products (below
+// 1e-6 |p| |c|) for every |p|: 2 sqrt(1e-3 a) >= 1e-6 |c| for a = 1e-8 |c|^2.
+struct Pencil {
+  float l[3], u[3];  // twice the end centres
+  float a;           // infinite: every point is kept
+  __device__ bool outside(float x, float y, float z) const {
+    const float pp = x * x + y * y + z * z;
+    const float dl = x * l[0] + y * l[1] + z * l[2], du = x * u[0] + y * u[1] + z * u[2];
+    return pp * 0.999f - a > fmaxf(dl, du);
   }
 };
 
-// The face passes scan the region in chunks of 64 slots: first the capsule
+// Ends of the pencil for t in [lo, hi] x r3 (r3: the face's circumradius);
+// lo = -infinity: not restricted.
+__device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi) {
+  Pencil c{};
+  c.a = INFINITY;
+  if (!(lo > -INFINITY)) return c;
+  const double s = 1.0 / f.D;
+  const V3 k = {f.g.x * s, f.g.y * s, f.g.z * s};  // twice the circumcentre
+  const double q = sqrt(dot(k, k) * s);            // 2 r3 / |n|
+  const double l = lo * q, h = hi * q;
+  const double cl[3] = {k.x + l * f.n.x, k.y + l * f.n.y, k.z + l * f.n.z};
+  const double cu[3] = {k.x + h * f.n.x, k.y + h * f.n.y, k.z + h * f.n.z};
+  double ll = 0, uu = 0;
+  for (int i = 0; i < 3; ++i) {
+    c.l[i] = (float)cl[i];
+    c.u[i] = (float)cu[i];
+    ll += cl[i] * cl[i];
+    uu += cu[i] * cu[i];
+  }
+  c.a = (float)(1e-8 * fmax(ll, uu)) + 1e-34f;
+  return c;
+}
+
+// The face passes scan the region in chunks of 64 slots: first the pencil
 // test of every slot of the chunk (a bit mask), then the point work for the
 // set bits only, in ascending slot order, exactly the order of a plain scan.
 // The lanes of a wave run the point work as often as the busiest lane of the
 // chunk needs it, instead of once for every slot that any lane needs.
-// tests counts the slots tested (the face's own vertices excluded).
-__device__ inline uint64_t capsule_chunk(const Work &w, const Capsule &cap, uint32_t s0, uint32_t M, uint32_t vi,
-                                         uint32_t wi, uint32_t &tests) {
+// tests32 counts the slots tested (the face's own vertices excluded).
+__device__ inline uint64_t pencil_chunk(const Work &w, const Pencil &c, uint32_t s0, uint32_t M, uint32_t vi,
+                                        uint32_t wi, uint32_t &tests32) {
   const uint32_t cn = min(64u, M - s0);
   uint64_t in = 0;
 #pragma unroll 4
   for (uint32_t j = 0; j < cn; ++j) {
     const uint32_t gi = s0 + j;
-    const bool keep = gi != vi && gi != wi && !cap.outside(gpt(w, gi));
+    const bool keep = !c.outside(w.fx[gi], w.fy[gi], w.fz[gi]);
     in |= (uint64_t)keep << j;
   }
-  tests += cn - (vi - s0 < cn ? 1u : 0u) - (wi - s0 < cn ? 1u : 0u);
-  return in;
-}
-
-// The same test on the FP32 coordinates: centre rounded to FP32 and the
-// squared bound widened by 1e-5 (rounded up), which covers the FP32
-// rounding of the coordinates, the centre and the distance (about 3e-6 of
-// the bound for a point near it).
-__device__ inline uint64_t capsule_chunk_f(const Work &w, float cx, float cy, float cz, float b2, uint32_t s0,
-                                           uint32_t M, uint32_t vi, uint32_t wi, uint32_t &tests32) {
-  const uint32_t cn = min(64u, M - s0);
-  uint64_t in = 0;
-#pragma unroll 4
-  for (uint32_t j = 0; j < cn; ++j) {
-    const uint32_t gi = s0 + j;
-    const float dx = w.fx[gi] - cx, dy = w.fy[gi] - cy, dz = w.fz[gi] - cz;
-    const bool keep = gi != vi && gi != wi && !(dx * dx + dy * dy + dz * dz > b2);
-    in |= (uint64_t)keep << j;
-  }
-  tests32 += cn - (vi - s0 < cn ? 1u : 0u) - (wi - s0 < cn ? 1u : 0u);
+  if (vi - s0 < cn) in &= ~(1ull << (vi - s0));
+  if (wi - s0 < cn) in &= ~(1ull << (wi - s0));
+  tests32 += cn;
   return in;
 }
 
@@ -646,11 +657,11 @@ __device__ inline uint64_t capsule_chunk_f(const Work &w, float cx, float cy, fl
 // leads to are queued and then taken one per lane, so the lanes of a wave
 // run passes of equal length instead of waiting for the face with the most
 // apexes.  A full queue falls back to doing the work in place.
-constexpr uint32_t kSideQ = 128;  // >= 2 items for each of a wave's 64 faces
+constexpr uint32_t kSideQ = 64;
 constexpr uint32_t kTetQ = 256;
 struct WaveQueues {
   uint32_t *side;    // vi | wi << 10 | side << 20 | cin << 21 (region slots, < 1024)
-  float *side_r;     // the face's rmax (a float, see face_feasible): the side pass rebuilds exactly the face pass's capsule
+  float *side_lo, *side_hi;  // the face's pencil interval: the side pass rebuilds exactly the face pass's pencil
   uint32_t *tet;     // vi | wi << 10 | zi << 20
   uint32_t *nside, *ntet;
 };
@@ -659,7 +670,7 @@ __device__ void process_tet(const Params &P, const Work &w, uint32_t u, uint32_t
                             uint32_t zi, uint32_t *region_slot);
 
 __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uint32_t M, const TriSphere &f,
-                                 const Capsule &cap, uint32_t vi, uint32_t wi, uint32_t wid, int side,
+                                 const Pencil &pen, uint32_t vi, uint32_t wi, uint32_t wid, int side,
                                  int cin_side, int K, uint32_t *region_slot, WaveQueues *q) {
   const int need = K - cin_side;  // slots left for points swept before z
   if (need <= 0) return;
@@ -673,7 +684,7 @@ __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uin
   // apex nor be swept before one (dropping it only loosens the threshold)
 #pragma unroll 1
   for (uint32_t s0 = 0; s0 < M; s0 += 64) {
-    uint64_t in = capsule_chunk(w, cap, s0, M, vi, wi, tests);
+    uint64_t in = pencil_chunk(w, pen, s0, M, vi, wi, tests);
 #pragma unroll 1
     while (in) {
       const uint32_t s = s0 + (uint32_t)(__ffsll((long long)in) - 1);
@@ -697,7 +708,8 @@ __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uin
       }
     }
   }
-  add_flops(w, (uint64_t)tests * kFlopCapsule + (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
+  add_flops(w, (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
+  add_flops32(w, (uint64_t)tests * kF32Pencil);
   // the face pass certified every sign with the same arithmetic
   if (undecided) return;
   const double thr = top.threshold(need);
@@ -712,7 +724,7 @@ __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uin
       if (zi == vi || zi == wi || w.gid[zi] <= wid) continue;
       const V3 p = gpt(w, zi);
       tests++;
-      if (cap.outside(p)) continue;
+      if (pen.outside(w.fx[zi], w.fy[zi], w.fz[zi])) continue;
       evals++;
       double Pw, PA, H, HA;
       f.power(p, Pw, PA);
@@ -726,7 +738,8 @@ __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uin
       if (cin_side + beh.count_above(tau + terr) >= K) continue;
       process_tet(P, w, u, M, vi, wi, zi, region_slot);
     }
-    add_flops(w, (uint64_t)tests * kFlopCapsule + (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
+    add_flops(w, (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
+    add_flops32(w, (uint64_t)tests * kF32Pencil);
     return;
   }
   uint32_t cand = 0;
@@ -756,49 +769,30 @@ __device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uin
   }
 }
 
-// The pencil capsule of face (u, v, w) for critical radii up to rmax.
-__device__ inline Capsule face_capsule(const TriSphere &f, double rmax) {
-  Capsule cap;
-  cap.c3 = {0.0, 0.0, 0.0};
-  cap.bound2 = INFINITY;
-  if (f.D > 1e-6 * f.DA) {
-    const double s2 = 0.5 / f.D;
-    cap.c3 = {f.g.x * s2, f.g.y * s2, f.g.z * s2};
-    const double r3 = sqrt(dot(cap.c3, cap.c3));
-    const double T = sqrt(fmax(0.0, rmax * rmax - r3 * r3));
-    const double Rb = fmax(rmax, r3);
-    cap.bound2 = (T + Rb) * (T + Rb) * (1.0 + 1e-6);
-  }
-  return cap;
-}
-
 // Apexes of one side from the FP32 lists its face's first pass filled (the
 // tail of face_side_apexes).  When a point left or missed the list with a
 // lower bound within the threshold, the side takes its own pass instead
 // (queued, with the full scan that case needs).
 __device__ inline void fused_side(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi, uint32_t wi,
                                   uint32_t wid, int side, int cin_side, int K, const SweepListF &top,
-                                  const BehindListF &beh, double rmax, uint32_t *region_slot, WaveQueues *q) {
+                                  const BehindListF &beh, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
   const int need = K - cin_side;
   const float thr = top.threshold(need);
   if (top.evicted_lo != INFINITY && top.evicted_lo <= thr) {
-    if (!q) {
-      // in place (global-memory path): the face's sphere rebuilt (same
-      // arithmetic, same values), then the side's own pass
-      TriSphere f;
-      f.init(gpt(w, vi), gpt(w, wi));
-      const Capsule cap = face_capsule(f, rmax);
-      face_side_apexes(P, w, u, M, f, cap, vi, wi, wid, side, cin_side, K, region_slot, nullptr);
-      return;
+    if (q) {
+      const uint32_t at = atomicAdd(q->nside, 1u);
+      if (at < kSideQ) {
+        q->side[at] = vi | (wi << 10) | ((uint32_t)side << 20) | ((uint32_t)cin_side << 21);
+        q->side_lo[at] = lo;
+        q->side_hi[at] = hi;
+        return;
+      }
     }
-    // at most 2 items for each of the wave's 64 faces: the queue cannot fill
-    const uint32_t at = atomicAdd(q->nside, 1u);
-    if (at < kSideQ) {
-      q->side[at] = vi | (wi << 10) | ((uint32_t)side << 20) | ((uint32_t)cin_side << 21);
-      q->side_r[at] = (float)rmax;  // exact: rmax is a float value
-    } else {
-      atomicAdd(&P.counters[4], 1ull);  // reported by the host as an internal error
-    }
+    // in place (global-memory path, full queue): the face's sphere rebuilt
+    // (same arithmetic, same values), then the side's own pass
+    TriSphere f;
+    f.init(gpt(w, vi), gpt(w, wi));
+    face_side_apexes(P, w, u, M, f, face_pencil(f, lo, hi), vi, wi, wid, side, cin_side, K, region_slot, q);
     return;
   }
   uint32_t cand = 0;
@@ -832,15 +826,17 @@ __device__ inline void fused_side(const Params &P, const Work &w, uint32_t u, ui
 // pass certifies every side and insideness, builds the triangle's interior,
 // counts the inside points ahead of each side and fills both sides' sweep
 // lists, from which the apexes follow (fused_side).  QUEUED (LDS paths):
-// tetrahedra and rescans go to the wave's queues; otherwise in place.  F32:
-// the pass runs on the region's FP32 copies.
-template <bool QUEUED, bool F32>
+// tetrahedra and rescans go to the wave's queues; otherwise in place.  The
+// pass runs on the region's FP32 copies (FP64 only for the points whose FP32
+// signs are not certified) and sees the points that some sphere of the face's
+// pencil within [lo, hi] (face_interval; n oriented as v x w) can hold.
+template <bool QUEUED>
 __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
-                             uint32_t wi, double rmax, uint32_t *region_slot, WaveQueues *q) {
+                             uint32_t wi, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
   // the sphere is built from its points in PointId order, so its FP64 level
   // (and every later tetrahedron's) does not depend on the enumeration order
   uint32_t ids[2] = {w.gid[vi], w.gid[wi]};
-  if (ids[0] > ids[1]) { uint32_t t = ids[0]; ids[0] = ids[1]; ids[1] = t; uint32_t q = vi; vi = wi; wi = q; }
+  if (ids[0] > ids[1]) { uint32_t t = ids[0]; ids[0] = ids[1]; ids[1] = t; uint32_t q = vi; vi = wi; wi = q; float l = lo; lo = -hi; hi = -l; }
   TriSphere f;
   const int wc = f.init(gpt(w, vi), gpt(w, wi));
   add_flops(w, kFlopTriInit);
@@ -853,18 +849,19 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   const uint32_t wid = ids[1];
   const int smax = P.s_max;
   const int K = smax - 3;  // an apex must be among the first K points swept
-  // pencil capsule: a critical sphere through u, v, w has its direction in a
-  // cell shared by v and w, so its radius is at most rmax; its centre is
-  // c3 + t n with r3^2 + t^2 <= rmax^2.  Only well-conditioned faces use it.
-  const Capsule cap = face_capsule(f, rmax);
+  const Pencil pen = face_pencil(f, lo, hi);
+  // the triangle's own sphere (t = 0) is critical only within the interval;
+  // a side that the interval does not reach has no apexes
+  const bool tri = lo <= 0.0f && hi >= 0.0f;
   // the triangle's level, before the pass (the vertices need not stay live)
   const double tri_level = f.level(), tri_level_err = f.level_err();
-  int cin0 = 0, cin1 = 0;  // inside the triangle's sphere, ahead of side 0 / 1
+  // inside the triangle's sphere, ahead of side 0 / 1
+  int cin0 = hi < 0.0f ? K : 0, cin1 = lo > 0.0f ? K : 0;
   int total_in = 0;
   // region slots of the first 8 inside points, 16 bits each, 2 per word (a
   // triangle event has at most s_max - 3 <= 8 interior points)
   uint32_t tri_pk[4] = {0u, 0u, 0u, 0u};
-  uint32_t tests = 0, evals = 0;
+  uint32_t evals = 0;
   SweepListF top0, top1;  // outside points ahead of side 0 / 1
   BehindListF beh0, beh1;  // inside points behind side 0 / 1
   top0.init();
@@ -872,64 +869,40 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   beh0.init();
   beh1.init();
   constexpr uint32_t kFlopPoint = kFlopFacePoint + kFlopSweepKey;
-  uint32_t tests32 = 0, evals32 = 0, keys32 = 0;  // FP32 work (F32 path)
-  // the FP32 path: capsule and face polynomials in FP32, FP64 only for the
-  // points whose FP32 signs are not certified (no FP64 capsule tests counted)
+  uint32_t tests32 = 0, evals32 = 0, keys32 = 0;  // FP32 work
   TriSphereF f32;
-  float ccx = 0.0f, ccy = 0.0f, ccz = 0.0f, cb2 = INFINITY;
-  if (F32) {
-    f32.init(f);
-    ccx = (float)cap.c3.x;
-    ccy = (float)cap.c3.y;
-    ccz = (float)cap.c3.z;
-    const double b2 = cap.bound2 * (1.0 + 1e-5);
-    cb2 = (float)b2;
-    if (!((double)cb2 >= b2)) cb2 = nextafterf(cb2, INFINITY);
-  }
-  // points outside the capsule are outside the triangle's sphere and every
-  // feasible one
+  f32.init(f);
 #pragma unroll 1
   for (uint32_t s0 = 0; s0 < M; s0 += 64) {
-    uint64_t in = F32 ? capsule_chunk_f(w, ccx, ccy, ccz, cb2, s0, M, vi, wi, tests32)
-                      : capsule_chunk(w, cap, s0, M, vi, wi, tests);
+    uint64_t in = pencil_chunk(w, pen, s0, M, vi, wi, tests32);
 #pragma unroll 1
     while (in) {
       const uint32_t gi = s0 + (uint32_t)(__ffsll((long long)in) - 1);
       in &= in - 1;
-      int sp = 0, sh = 0;
       float hf = 0.0f, lf = 0.0f;
-      if (F32) {
-        float P32, PA32, H32, HA32;
-        f32.eval(w.fx[gi], w.fy[gi], w.fz[gi], P32, PA32, H32, HA32);
-        sp = cert32(P32, PA32);
-        sh = cert32(H32, HA32);
-        evals32++;
-        if (sp != 0 && sh != 0) {
-          key_bounds_32(P32, PA32, H32, HA32, hf, lf);
-          keys32++;
-        }
-      }
-      if (sp == 0 || sh == 0) {
+      float P32, PA32, H32, HA32;
+      f32.eval(w.fx[gi], w.fy[gi], w.fz[gi], P32, PA32, H32, HA32);
+      int sp = cert32(P32, PA32), sh = cert32(H32, HA32);
+      evals32++;
+      if (sp != 0 && sh != 0) {
+        key_bounds_32(P32, PA32, H32, HA32, hf, lf);
+        keys32++;
+      } else {
         const V3 p = gpt(w, gi);
         evals++;
         double Pw, PA, H, HA;
-        if (F32) {
-          // rare: the FP64 sphere is rebuilt (same arithmetic, same values)
-          // rather than kept live through the pass
-          TriSphere f64;
-          f64.init(gpt(w, vi), gpt(w, wi));
-          f64.power(p, Pw, PA);
-          f64.height(p, H, HA);
-        } else {
-          f.power(p, Pw, PA);
-          f.height(p, H, HA);
-        }
+        // rare: the FP64 sphere is rebuilt (same arithmetic, same values)
+        // rather than kept live through the pass
+        TriSphere f64;
+        f64.init(gpt(w, vi), gpt(w, wi));
+        f64.power(p, Pw, PA);
+        f64.height(p, H, HA);
         sp = cert_sign(Pw, PA);
         sh = cert_sign(H, HA);
         // every sign the side passes use is certified here, before anything is emitted
         if (sp == 0 || sh == 0) {
-          add_flops(w, (uint64_t)tests * kFlopCapsule + (uint64_t)evals * kFlopPoint);
-          add_flops32(w, (uint64_t)tests32 * kF32Capsule + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+          add_flops(w, (uint64_t)evals * kFlopPoint);
+          add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
           emit_fallback(P, w, u, 3, ids, 3, M, region_slot);
           return;
         }
@@ -957,17 +930,19 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
       cin0 += sh > 0;
       cin1 += sh < 0;
       // both sides saturated and the triangle out of rank: nothing left here
-      if (cin0 >= K && cin1 >= K && total_in + 3 > smax) {
-        add_flops(w, (uint64_t)tests * kFlopCapsule + (uint64_t)evals * kFlopPoint);
-        add_flops32(w, (uint64_t)tests32 * kF32Capsule + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+      if (cin0 >= K && cin1 >= K && (!tri || total_in + 3 > smax)) {
+        add_flops(w, (uint64_t)evals * kFlopPoint);
+        add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
         return;
       }
     }
   }
-  add_flops(w, (uint64_t)tests * kFlopCapsule + (uint64_t)evals * kFlopPoint);
-  add_flops32(w, (uint64_t)tests32 * kF32Capsule + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+  add_flops(w, (uint64_t)evals * kFlopPoint);
+  add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
   // triangle event
-  if (wc > 0 && total_in + 3 <= smax) {
+  if (!tri) {
+    // not critical by the certificate
+  } else if (wc > 0 && total_in + 3 <= smax) {
     atomicAdd(w.cand, 1u);
     uint32_t tri_int[kMaxInterior];
 #pragma unroll
@@ -982,20 +957,20 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   if (K <= 0) return;
   // queued on the LDS paths, in place on the global-memory path
   WaveQueues *qq = QUEUED ? q : nullptr;
-  if (cin0 < K) fused_side(P, w, u, M, vi, wi, wid, 0, cin0, K, top0, beh0, rmax, region_slot, qq);
-  if (cin1 < K) fused_side(P, w, u, M, vi, wi, wid, 1, cin1, K, top1, beh1, rmax, region_slot, qq);
+  if (cin0 < K) fused_side(P, w, u, M, vi, wi, wid, 0, cin0, K, top0, beh0, lo, hi, region_slot, qq);
+  if (cin1 < K) fused_side(P, w, u, M, vi, wi, wid, 1, cin1, K, top1, beh1, lo, hi, region_slot, qq);
 }
 
 // A queued side of a face: the face's sphere rebuilt (same arithmetic, same
 // values), then the side's pass.
-__device__ void side_item(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t lo, double rmax,
+__device__ void side_item(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t item, float lo, float hi,
                           uint32_t *region_slot, WaveQueues *q) {
-  const uint32_t vi = lo & 1023u, wi = (lo >> 10) & 1023u, side = (lo >> 20) & 1u, cin_side = lo >> 21;
+  const uint32_t vi = item & 1023u, wi = (item >> 10) & 1023u, side = (item >> 20) & 1u, cin_side = item >> 21;
   TriSphere f;
   f.init(gpt(w, vi), gpt(w, wi));
   add_flops(w, kFlopTriInit);
-  const Capsule cap = face_capsule(f, rmax);
-  face_side_apexes(P, w, u, M, f, cap, vi, wi, w.gid[wi], (int)side, (int)cin_side, P.s_max - 3, region_slot, q);
+  face_side_apexes(P, w, u, M, f, face_pencil(f, lo, hi), vi, wi, w.gid[wi], (int)side, (int)cin_side, P.s_max - 3,
+                   region_slot, q);
 }
 
 __device__ void tet_item(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t item,
@@ -1087,41 +1062,87 @@ __device__ inline float cell_radius(const Params &P, int c, float bk, double ux,
   return rf;
 }
 
-// Face (u, v, w) of region slots si, sj: false when v and w share no cell or
-// when the triangle's circumradius exceeds every shared cell's certificate
-// radius (well-conditioned faces only; FP64 r2 is then accurate to ~1e-10).
-// rmax, the largest radius over the shared cells, is rounded up to a float
-// value, so that the queued side passes can keep it in a float and rebuild
-// exactly the first pass's capsule (a larger bound only prunes less).
-__device__ inline bool face_feasible(const Work &w, uint32_t si, uint32_t sj, double &rmax, float *key = nullptr) {
+// Face (u, v, w) of region slots si, sj: the part of its pencil of spheres
+// that the certificate leaves.  A critical sphere through the three points has
+// its centre at c3 + t n (n the unit normal along v x w, t = s r3), its
+// direction in a cell shared by v and w and its radius r3 sqrt(1 + s^2) within
+// that cell's rho.  The directions of the pencil inside a cell of centre g and
+// angular radius delta are an interval of s, the roots of
+// (g.c + s g.n)^2 = cos^2 delta (1 + s^2) (c the unit vector to c3); [lo, hi]
+// spans the intervals of the shared cells.  Returns false when there is none.
+//
+// FP32 on unit vectors normalised in FP64: the products lose below 2e-6, which
+// the cells' cosines lowered by 1e-4 cover (a cell only grows), and the radius
+// bound carries 2e-5.  Where a cell holds (nearly) the normal itself the roots
+// are unbounded and its interval is taken as that whole side.  An
+// ill-conditioned face is not restricted (lo = -infinity).
+// key: the squared radius of the larger end sphere (it only orders the faces
+// into waves of similar work).
+__device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si, uint32_t sj, float &lo, float &hi,
+                                     float &key) {
+  uint64_t sh[6];
   bool share = false;
-  for (int k = 0; k < 6; ++k) share |= (w.rmask[6 * si + k] & w.rmask[6 * sj + k]) != 0;
-  rmax = 0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    sh[k] = w.rmask[6 * si + k] & w.rmask[6 * sj + k];
+    share |= sh[k] != 0;
+  }
   if (!share) return false;
   const V3 a = gpt(w, si), b = gpt(w, sj);
   const double aa = dot(a, a), bb = dot(b, b), ab = dot(a, b);
   const double D = aa * bb - ab * ab;
+  lo = -INFINITY;
+  hi = INFINITY;
+  key = INFINITY;
+  if (!(D > 1e-6 * (aa * bb + fabs(ab) * fabs(ab)))) return true;
   const V3 amb = sub(a, b);
-  const double r2 = D > 0 ? aa * bb * dot(amb, amb) / (4.0 * D) : INFINITY;
+  const double r2 = aa * bb * dot(amb, amb) / (4.0 * D);
+  const double al = bb * (aa - ab), be = aa * (bb - ab);
+  const V3 g = {al * a.x + be * b.x, al * a.y + be * b.y, al * a.z + be * b.z}, n = cross(a, b);
+  const double ig = __builtin_amdgcn_rsq(dot(g, g)), in = __builtin_amdgcn_rsq(D);
+  const float cx = (float)(g.x * ig), cy = (float)(g.y * ig), cz = (float)(g.z * ig);
+  const float nx = (float)(n.x * in), ny = (float)(n.y * in), nz = (float)(n.z * in);
+  const float ir3 = (float)__builtin_amdgcn_rsq(r2);
+  if (!(fabsf(cx) <= 1.001f && fabsf(nx) <= 1.001f && ir3 > 1e-30f && ir3 < 1e30f)) return true;  // out of FP32's range
+  float l = INFINITY, h = -INFINITY;
+  uint32_t cells = 0;
+#pragma unroll
   for (int k = 0; k < 6; ++k) {
-    uint64_t mm = w.rmask[6 * si + k] & w.rmask[6 * sj + k];
+    uint64_t mm = sh[k];
     while (mm) {
-      const int bit = __ffsll((long long)mm) - 1;
+      const int c = 64 * k + __ffsll((long long)mm) - 1;
       mm &= mm - 1;
-      rmax = fmax(rmax, w.rho[64 * k + bit]);
+      cells++;
+      const float ratio = w.rho[c] * ir3;
+      const float sc2 = ratio * ratio * (1.0f + 2e-5f) - (1.0f - 1e-5f);
+      if (sc2 < 0.0f) continue;
+      const CellF cf = cell_f(P.cellf + 8 * c);
+      const float ga = cf.dx * cx + cf.dy * cy + cf.dz * cz, gn = cf.dx * nx + cf.dy * ny + cf.dz * nz;
+      const float cd = cf.cosd - 1e-4f, kk = cd * cd;
+      const float q = ga * ga + gn * gn - kk, den = kk - gn * gn;
+      if (q < 0.0f) continue;
+      const float sc = __builtin_amdgcn_sqrtf(sc2);
+      float s1, s2;
+      if (den > 0.02f) {
+        if (ga <= 0.0f) continue;  // the opposite direction
+        const float root = cd * __builtin_amdgcn_sqrtf(q), inv = __builtin_amdgcn_rcpf(den);
+        s1 = fmaxf((ga * gn - root) * inv, -sc);
+        s2 = fminf((ga * gn + root) * inv, sc);
+      } else {
+        s1 = gn > 0.0f ? 0.0f : -sc;
+        s2 = gn > 0.0f ? sc : 0.0f;
+      }
+      if (s1 > s2) continue;
+      l = fminf(l, s1);
+      h = fmaxf(h, s2);
     }
   }
-  float rf = (float)rmax;
-  if ((double)rf < rmax) rf = nextafterf(rf, INFINITY);
-  rmax = (double)rf;
-  const bool well = D > 1e-6 * (aa * bb + fabs(ab) * fabs(ab));
-  if (key) {
-    // the squared extent of the face's pencil capsule (an estimate, it only
-    // orders the faces into waves of similar work)
-    const double r3 = sqrt(r2), t = sqrt(fmax(rmax * rmax - r2, 0.0)) + fmax(rmax, r3);
-    *key = well ? (float)(t * t) : INFINITY;
-  }
-  return !(well && r2 > rmax * rmax * (1.0 + 1e-6));
+  add_flops32(w, (uint64_t)cells * kF32Cell);
+  lo = l;
+  hi = h;
+  const float e = fmaxf(fabsf(l), fabsf(h));
+  key = (float)r2 * (1.0f + e * e);
+  return l <= h;
 }
 
 // Pairs, faces and tetrahedra of anchor u over its compacted region (M
@@ -1135,7 +1156,7 @@ __device__ inline bool face_feasible(const Work &w, uint32_t si, uint32_t sj, do
 // the faces, and takes its share of them and of the pairs.  The workgroups
 // beyond one per kSplitFaces candidate faces have nothing to do.
 constexpr uint64_t kSplitFaces = 2048;
-template <bool BIG, bool F32, bool SPLIT, int WAVES>
+template <bool BIG, bool SPLIT, int WAVES>
 __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t *sK_,
                              uint32_t *sregion_) {
   uint32_t &sK = *sK_;
@@ -1157,11 +1178,9 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     if (t == 0) sK = k;
   }
   for (uint32_t s = t; s < M; s += blockDim.x) {
-    if (F32) {
-      w.fx[s] = (float)w.gx[s];
-      w.fy[s] = (float)w.gy[s];
-      w.fz[s] = (float)w.gz[s];
-    }
+    w.fx[s] = (float)w.gx[s];
+    w.fy[s] = (float)w.gy[s];
+    w.fz[s] = (float)w.gz[s];
   }
   __syncthreads();
   const uint32_t Kc = sK;
@@ -1180,13 +1199,13 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   // queued sides and tetrahedra one per lane (LDS path; the global-memory
   // path works in place).
   __shared__ uint32_t q_side[WAVES][kSideQ];
-  __shared__ float q_side_r[WAVES][kSideQ];
+  __shared__ float q_side_lo[WAVES][kSideQ], q_side_hi[WAVES][kSideQ];
   __shared__ uint32_t q_face[WAVES][128];
-  __shared__ float q_key[WAVES][128];
+  __shared__ float q_key[WAVES][128], q_lo[WAVES][128], q_hi[WAVES][128];
   __shared__ uint32_t q_tet[WAVES][kTetQ];
   __shared__ uint32_t q_n[WAVES][2];
   const int wave = t >> 6, lane = t & 63, nwaves = (int)(blockDim.x >> 6);
-  WaveQueues wq{q_side[wave], q_side_r[wave], q_tet[wave], &q_n[wave][0], &q_n[wave][1]};
+  WaveQueues wq{q_side[wave], q_side_lo[wave], q_side_hi[wave], q_tet[wave], &q_n[wave][0], &q_n[wave][1]};
   WaveQueues *q = BIG ? nullptr : &wq;
   if (lane == 0) { q_n[wave][0] = 0; q_n[wave][1] = 0; }
   wave_sync();
@@ -1206,17 +1225,15 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if (fidx >= F) continue;
       uint32_t si, sj;
       face_of(fidx, si, sj);
-      double rmax;
-      if (face_feasible(w, si, sj, rmax)) process_face<false, false>(P, w, u, M, si, sj, rmax, &sregion, q);
+      float lo, hi, key;
+      if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false>(P, w, u, M, si, sj, lo, hi, &sregion, q);
     }
   } else {
-    // Each wave first collects up to 128 feasible faces in its LDS list (the
-    // faces that fail the shared-cell or radius test cost only the test),
-    // orders them by the extent of their pencil capsules, then runs the
-    // first passes of the 64 largest one per lane (lanes of similar work),
-    // then the queued sides and tetrahedra; the smaller ones wait for the
-    // next round.  The lists keep region slots only; a lane recomputes the
-    // face's rmax (same arithmetic, same value).
+    // Each wave first collects up to 128 feasible faces in its LDS list with
+    // their pencil intervals (the faces without one cost only the test),
+    // orders them by the extent of their pencils, then runs the first passes
+    // of the 64 largest one per lane (lanes of similar work), then the queued
+    // sides and tetrahedra; the smaller ones wait for the next round.
     uint32_t nf = 0;  // faces in the wave's list (uniform)
     uint64_t cbase = ((uint64_t)part * nwaves + wave) * 64;
     const uint64_t cstride = (uint64_t)parts * nwaves * 64;
@@ -1225,17 +1242,18 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
         const uint64_t fidx = cbase + lane;
         bool ok = false;
         uint32_t si = 0, sj = 0;
-        float key = 0.0f;
+        float key = 0.0f, lo = 0.0f, hi = 0.0f;
         if (fidx < F) {
           face_of(fidx, si, sj);
-          double rmax;
-          ok = face_feasible(w, si, sj, rmax, &key);
+          ok = face_interval(P, w, si, sj, lo, hi, key);
         }
         const uint64_t m = __ballot(ok);
         if (ok) {
           const uint32_t at = nf + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
           q_face[wave][at] = si | (sj << 10);
           q_key[wave][at] = key;
+          q_lo[wave][at] = lo;
+          q_hi[wave][at] = hi;
         }
         nf += (uint32_t)__popcll(m);
         cbase += cstride;
@@ -1245,14 +1263,19 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if (nf > 64) {
         // rank sort of the list by key (ties by position), ascending
         uint32_t fv[2], rk[2];
+        float lv[2], hv[2], kv[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t i = (uint32_t)lane + 64u * h;
           fv[h] = 0;
           rk[h] = 0;
+          lv[h] = hv[h] = kv[h] = 0.0f;
           if (i < nf) {
             const float ki = q_key[wave][i];
+            kv[h] = ki;
             fv[h] = q_face[wave][i];
+            lv[h] = q_lo[wave][i];
+            hv[h] = q_hi[wave][i];
             uint32_t r = 0;
             for (uint32_t j = 0; j < nf; ++j) {
               const float kj = q_key[wave][j];
@@ -1264,7 +1287,12 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
         wave_sync();
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          if ((uint32_t)lane + 64u * h < nf) q_face[wave][rk[h]] = fv[h];
+          if ((uint32_t)lane + 64u * h < nf) {
+            q_face[wave][rk[h]] = fv[h];
+            q_lo[wave][rk[h]] = lv[h];
+            q_hi[wave][rk[h]] = hv[h];
+            q_key[wave][rk[h]] = kv[h];
+          }
         wave_sync();
       }
       const uint32_t take = min(nf, 64u);
@@ -1272,14 +1300,12 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if ((uint32_t)lane < take) {
         const uint32_t fv = q_face[wave][nf + lane];
         const uint32_t si = fv & 1023u, sj = fv >> 10;
-        double rmax;
-        face_feasible(w, si, sj, rmax);
-        process_face<true, F32>(P, w, u, M, si, sj, rmax, &sregion, q);
+        process_face<true>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
       }
       wave_sync();
       const uint32_t ns = min(q_n[wave][0], kSideQ);
       for (uint32_t it = lane; it < ns; it += 64)
-        side_item(P, w, u, M, q_side[wave][it], (double)q_side_r[wave][it], &sregion, q);
+        side_item(P, w, u, M, q_side[wave][it], q_side_lo[wave][it], q_side_hi[wave][it], &sregion, q);
       wave_sync();
       // whole rounds of 64 tetrahedra (the top of the queue); the rest waits
       // for the next round's, so that the lanes stay busy
@@ -1487,7 +1513,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
     if (t == 0) probed(P, u, a, M);
     return;
   }
-  anchor_faces<true, true, false, kBlock / 64>(P, w, u, M, &sK, &sregion);
+  anchor_faces<true, false, kBlock / 64>(P, w, u, M, &sK, &sregion);
 }
 
 // Slab of one probed anchor (in doubles), for G gathered points:
@@ -1785,7 +1811,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   __syncthreads();
   Work w{gx, gy, gz, gid, rho, kidx, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz,
          P.count_flops ? &flops32 : nullptr};
-  anchor_faces<false, true, true, WAVES>(P, w, u, M, &sK, &sregion);
+  anchor_faces<false, true, WAVES>(P, w, u, M, &sK, &sregion);
 }
 
 // Ball count / emit around every anchor of the list: one wave per anchor over
