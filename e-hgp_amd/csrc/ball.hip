@@ -4,7 +4,7 @@
 // pair_support_stream.cpp:1781-1952): how many points lie strictly inside
 // the sphere, how many on it (the support included) and which are inside.
 //
-// One thread per query: the FP64 circumball bounds an LBVH ball traversal
+// One wave per query: the FP64 circumball bounds a traversal of the wave tree
 // (with a relative margin far above its rounding error), every point in range
 // is placed by the certified predicates of predicates.hpp, and what they
 // cannot decide (points exactly or nearly on the sphere, ill-conditioned
@@ -15,13 +15,12 @@
 #include "../host/exact.hpp"
 #include "pipeline.hpp"
 #include "predicates.hpp"
-#include "traverse.hpp"
+#include "wave_tree.hpp"
 
 namespace mhgp {
 
 namespace {
 
-constexpr int kBallStack = 40;  // LBVH depth is 18 at 50k points, 32 at 200k; overflow goes to the host
 constexpr uint32_t kHostQuery = 1u;
 
 struct BallParams {
@@ -30,10 +29,7 @@ struct BallParams {
   int64_t queries;
   uint32_t cap;           // interior ids kept per query
   const double *X, *Y, *Z;
-  const Node *nodes;
-  const double *LX, *LY, *LZ;
-  const uint32_t *leaf_id;
-  int64_t n;
+  WaveTree tree;
   uint32_t *interior;     // cap per query
   uint32_t *nin, *nshell, *flags;
   uint32_t *und;          // (query, point) pairs for the host
@@ -43,15 +39,23 @@ struct BallParams {
 
 __device__ inline V3 pt(const BallParams &B, uint32_t id) { return {B.X[id], B.Y[id], B.Z[id]}; }
 
-__global__ void __launch_bounds__(64) k_closed_ball(BallParams B) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// With one thread per query a call took as long as its largest ball (ill-
+// conditioned supports have spheres holding much of the cloud): 103 ms for
+// 4 099 queries of 50 000 points.  Bound by the predicates of the points in
+// range, 64 at a time.
+constexpr int kBallBlock = 256;  // four waves, four queries
+__global__ void __launch_bounds__(kBallBlock) k_closed_ball(BallParams B) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const int64_t q = (int64_t)blockIdx.x * (kBallBlock / 64) + (threadIdx.x >> 6);
   if (q >= B.queries) return;
   const int m = B.sizes[q];
   uint32_t sid[4];
   for (int i = 0; i < 4; ++i) sid[i] = i < m ? B.ids[4 * q + i] : kInvalid;
-  B.nin[q] = 0;
-  B.nshell[q] = (uint32_t)m;
-  B.flags[q] = 0;
+  if (lane == 0) {
+    B.nin[q] = 0;
+    B.nshell[q] = (uint32_t)m;
+    B.flags[q] = 0;
+  }
   if (m == 1) {  // radius zero: nothing inside, the point alone on it
     return;
   }
@@ -82,63 +86,91 @@ __global__ void __launch_bounds__(64) k_closed_ball(BallParams B) {
     off = {tt.N.x * s2, tt.N.y * s2, tt.N.z * s2};
   }
   if (!good) {  // dependent or ill-conditioned support: the host classifies it
-    B.flags[q] = kHostQuery;
+    if (lane == 0) B.flags[q] = kHostQuery;
     return;
   }
   r2 = dot(off, off);
   const double c[3] = {o.x + off.x, o.y + off.y, o.z + off.z};
   const double R2 = r2 * (1.0 + 1e-6) + 1e-300;  // every point beyond is certainly outside
   uint32_t nin = 0, nsh = (uint32_t)m;
-  // the interior row keeps the cap smallest ids (their largest and its slot
-  // tracked), so a truncated list does not depend on the traversal order
+  // the interior row keeps the cap smallest ids, so a truncated list does not
+  // depend on the traversal order: up to 64 of them sorted across the lanes;
+  // beyond that the row itself, whose largest id (the wave's search) makes way
+  // for a smaller one
   uint32_t *row = B.interior + (size_t)q * B.cap;
-  uint32_t rmax = 0, rmax_at = 0;
-  uint32_t stack[kBallStack];
-  int sp = 0;
-  stack[sp++] = 0;
-  while (sp) {
-    const Node &N = B.nodes[stack[--sp]];
-    const uint32_t ch[2] = {N.left, N.right};
-    for (int cc = 0; cc < 2; ++cc) {
-      const uint32_t x = ch[cc];
-      if (x & kLeafBit) {
-        const uint32_t lp = x & ~kLeafBit;
-        const double dx = B.LX[lp] - c[0], dy = B.LY[lp] - c[1], dz = B.LZ[lp] - c[2];
-        if (dx * dx + dy * dy + dz * dz > R2) continue;
-        const uint32_t id = B.leaf_id[lp];
-        bool on_support = false;
-        for (int i = 0; i < m; ++i) on_support |= sid[i] == id;
-        if (on_support) continue;
-        const V3 p = sub(pt(B, id), o);
-        const int sd = m == 2 ? ps.side(p) : (m == 3 ? ts.side(p) : tt.side(p));
-        if (sd < 0) {
-          if (nin < B.cap) {
-            row[nin] = id;
-            if (id >= rmax) { rmax = id; rmax_at = nin; }
-          } else if (B.cap && id < rmax) {
-            row[rmax_at] = id;
-            rmax = 0;
-            for (uint32_t k = 0; k < B.cap; ++k)
-              if (row[k] >= rmax) { rmax = row[k]; rmax_at = k; }
-          }
-          nin++;
-        } else if (sd == 0) {
-          const unsigned long long at = atomicAdd(B.nund, 1ull);
-          if (at < B.und_cap) {
-            B.und[2 * at] = (uint32_t)q;
-            B.und[2 * at + 1] = id;
-          } else {
-            B.flags[q] = kHostQuery;  // list full: the whole query goes to the host
-          }
-        }
-      } else if (box_d2(c, B.nodes[x].lo, B.nodes[x].hi) <= R2) {
-        if (sp < kBallStack) stack[sp++] = x;
-        else B.flags[q] = kHostQuery;
+  const bool in_lanes = B.cap <= 64;
+  uint32_t list = kInvalid, rmax = kInvalid;
+  const WaveTree &T = B.tree;
+  const WaveQuery Q(T, c[0], c[1], c[2]);
+  float Tf = Q.bound(R2);
+  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+    const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
+    const double dx = T.LX[at] - c[0], dy = T.LY[at] - c[1], dz = T.LZ[at] - c[2];
+    bool near = lp < T.n && !(dx * dx + dy * dy + dz * dz > R2);
+    if (!__ballot(near)) return;
+    const uint32_t id = T.leaf_id[at];
+    for (int i = 0; i < m; ++i) near = near && sid[i] != id;
+    int sd = 1;
+    if (near) {
+      const V3 p = sub({T.LX[at], T.LY[at], T.LZ[at]}, o);
+      sd = m == 2 ? ps.side(p) : (m == 3 ? ts.side(p) : tt.side(p));
+    }
+    if (near && sd == 0) {
+      const unsigned long long slot = atomicAdd(B.nund, 1ull);
+      if (slot < B.und_cap) {
+        B.und[2 * slot] = (uint32_t)q;
+        B.und[2 * slot + 1] = id;
+      } else {
+        B.flags[q] = kHostQuery;  // list full: the whole query goes to the host
       }
     }
+    const bool inside = near && sd < 0;
+    uint64_t in = __ballot(inside);
+    if (in_lanes && B.cap) {
+      for (uint64_t left = __ballot(inside && id < lane_u32(list, (int)B.cap - 1)); left;) {
+        const int i = __builtin_amdgcn_readfirstlane(__ffsll((long long)left) - 1);
+        left &= left - 1;
+        const uint32_t x = lane_u32(id, i);
+        const uint32_t pos = (uint32_t)__popcll(__ballot(list < x)), up = __shfl_up(list, 1u);
+        list = lane < pos ? list : (lane == pos ? x : up);
+        left &= __ballot(id < lane_u32(list, (int)B.cap - 1));
+      }
+    } else if (!in_lanes) {
+      const uint32_t slot = nin + (uint32_t)__popcll(in & ((1ull << lane) - 1ull));
+      if (inside && slot < B.cap) row[slot] = id;
+      for (uint64_t left = __ballot(inside && slot >= B.cap); left;) {
+        const int i = __builtin_amdgcn_readfirstlane(__ffsll((long long)left) - 1);
+        left &= left - 1;
+        const uint32_t x = lane_u32(id, i);
+        if (x >= rmax) continue;  // not below the largest kept
+        __threadfence_block();    // the row's stores by other lanes
+        uint32_t top = 0, where = 0;
+        for (uint32_t k = lane; k < B.cap; k += 64) {
+          const uint32_t v = ((volatile uint32_t *)row)[k];
+          if (v >= top) {
+            top = v;
+            where = k;
+          }
+        }
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) {
+          const uint32_t v = __shfl_xor(top, s), k = __shfl_xor(where, s);
+          if (v > top) {  // ids are distinct
+            top = v;
+            where = k;
+          }
+        }
+        rmax = top;
+        if (x < top && lane == 0) row[where] = x;
+      }
+    }
+    nin += (uint32_t)__popcll(in);
+  });
+  if (in_lanes && lane < min(nin, B.cap)) row[lane] = list;
+  if (lane == 0) {
+    B.nin[q] = nin;
+    B.nshell[q] = nsh;
   }
-  B.nin[q] = nin;
-  B.nshell[q] = nsh;
 }
 
 // Allocation-free variant: the host-query flag of each query is folded into
@@ -273,11 +305,11 @@ void closed_ball(Context &c, const uint32_t *ids, const uint8_t *sizes, int64_t 
   BallParams B{};
   B.ids = d_ids.p; B.sizes = d_sizes.p; B.queries = Q; B.cap = cap;
   B.X = c.X.p; B.Y = c.Y.p; B.Z = c.Z.p;
-  B.nodes = c.nodes.p; B.LX = c.LX.p; B.LY = c.LY.p; B.LZ = c.LZ.p; B.leaf_id = c.leaf_id.p; B.n = c.n;
+  B.tree = wave_tree(c);
   B.interior = d_int.p; B.nin = d_nin.p; B.nshell = d_nsh.p; B.flags = d_flags.p;
   B.und = d_und.p; B.nund = (unsigned long long *)d_nund.p; B.und_cap = und_cap;
   if (c.n > 1) {
-    hipLaunchKernelGGL(k_closed_ball, dim3(blocks_for(Q, 64)), dim3(64), 0, s, B);
+    hipLaunchKernelGGL(k_closed_ball, dim3(blocks_for(Q, kBallBlock / 64)), dim3(kBallBlock), 0, s, B);
     MHGP_LAUNCH_CHECK();
   } else {
     MHGP_HIP(hipMemsetAsync(d_nin.p, 0, Q * 4, s));
@@ -402,10 +434,10 @@ void closed_ball_noalloc(Context &c, const uint32_t *ids, const uint8_t *sizes, 
     BallParams B{};
     B.ids = d_ids; B.sizes = d_sizes; B.queries = Q; B.cap = cap;
     B.X = c.X.p; B.Y = c.Y.p; B.Z = c.Z.p;
-    B.nodes = c.nodes.p; B.LX = c.LX.p; B.LY = c.LY.p; B.LZ = c.LZ.p; B.leaf_id = c.leaf_id.p; B.n = c.n;
+    B.tree = wave_tree(c);
     B.interior = d_int; B.nin = d_nin; B.nshell = d_nsh; B.flags = d_flags;
     B.und = d_und; B.nund = d_nund; B.und_cap = L.und_cap;
-    hipLaunchKernelGGL(k_closed_ball, dim3(blocks_for(Q, 64)), dim3(64), 0, s, B);
+    hipLaunchKernelGGL(k_closed_ball, dim3(blocks_for(Q, kBallBlock / 64)), dim3(kBallBlock), 0, s, B);
     MHGP_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_fold_flags, dim3(blocks_for(Q, 256)), dim3(256), 0, s, d_nin, d_flags, Q);
     MHGP_LAUNCH_CHECK();

@@ -86,6 +86,42 @@ __device__ inline void wave_tree_visit(const WaveTree &T, const WaveQuery &Q, fl
   wave_tree_visit(T, Q, Tf, [](int, uint32_t) { return true; }, leaf);
 }
 
+// A level-0 group near the query (the nearest box under the nearest level-1
+// box), where a search bound starts out tight.  Uniform over the wave.
+__device__ inline uint32_t wave_near_group(const WaveTree &T, const WaveQuery &Q) {
+  const uint32_t lane = threadIdx.x & 63u;
+  float d = INFINITY;
+  uint32_t g = 0;
+  for (uint32_t i = lane; i < T.c1; i += 64) {
+    const float e = Q.d2(T.l1[i]);
+    if (e < d) {
+      d = e;
+      g = i;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float e = __shfl_xor(d, o);
+    const uint32_t h = __shfl_xor(g, o);
+    if (e < d || (e == d && h < g)) {
+      d = e;
+      g = h;
+    }
+  }
+  uint32_t i = min(g * 64 + lane, T.c0 - 1);
+  d = Q.d2(T.l0[i]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float e = __shfl_xor(d, o);
+    const uint32_t h = __shfl_xor(i, o);
+    if (e < d || (e == d && h < i)) {
+      d = e;
+      i = h;
+    }
+  }
+  return __builtin_amdgcn_readfirstlane(i);
+}
+
 // Value of lane `src` (uniform) in every lane, and the value of the lane
 // below (lane 0 keeps its own).
 __device__ inline uint32_t lane_u32(uint32_t v, int src) { return __builtin_amdgcn_readlane(v, src); }

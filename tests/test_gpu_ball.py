@@ -100,3 +100,12 @@ def test_closed_ball_truncated_lists_are_the_smallest_ids():
         sups.append(sup)
     print("closed ball: 7x7x7 grid, 400 supports, cap 5", flush=True)
     _check(pts, sups, cap=5)
+
+
+@pytest.mark.parametrize("cap", [0, 1, 63, 64, 65, 200])
+def test_closed_ball_interior_lists_at_the_lane_capacity(cap):
+    """Interior lists around 64 ids, where they move from the lanes to memory,
+    for balls that hold more points than that."""
+    pts = workloads.uniform_cloud(400, seed=35)
+    print(f"closed ball: uniform n=400, cap {cap}", flush=True)
+    _check(pts, _random_supports(np.random.default_rng(2), 400, 40), cap=cap)
