@@ -49,9 +49,7 @@ struct Context {
   DevBuf<uint32_t> perm;
   DevBuf<uint32_t> status;  // [0] duplicate flag, [1] Morton fallback count, [2..] scratch
 
-  // global AABB: lo[3], hi[3] values and PointId witnesses
-  DevBuf<double> bounds;
-  DevBuf<uint32_t> bound_ids;
+  DevBuf<double> bounds;  // global AABB: lo[3], hi[3], then its partial results
 
   // LBVH: leaves in (Morton code, PointId) order
   DevBuf<uint64_t> codes;
@@ -65,7 +63,7 @@ struct Context {
   DevBuf<WideNode> wide;      // FP32 two-level copy of the internal nodes (ball and k-NN queries)
   DevBuf<GroupBox> groups;    // wave tree: level 0, 1 and 2 boxes (wave_tree.hpp), relative to centre
   double centre[3] = {0, 0, 0};
-  DevBuf<uint32_t> counter;
+  DevBuf<uint8_t> group_exact;  // the groups' exact boxes with witnesses (lbvh.hip)
   RadixSorter sorter;
   Scanner scanner;
   mhgp_stats stats{};

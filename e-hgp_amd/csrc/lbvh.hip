@@ -19,6 +19,126 @@ namespace mhgp {
 
 namespace {
 
+// Cloud bounds, per workgroup (lower x, y, z, upper x, y, z).
+constexpr int kBoundBlocks = 64;
+constexpr int kBoundBlock = 256;
+__global__ void __launch_bounds__(kBoundBlock) k_bounds(const double *__restrict__ src, int64_t n, double *part) {
+  __shared__ double red[kBoundBlock / 64][6];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  for (int64_t i = (int64_t)blockIdx.x * kBoundBlock + threadIdx.x; i < n; i += (int64_t)kBoundBlocks * kBoundBlock)
+    for (int a = 0; a < 3; ++a) {
+      const double x = src[3 * i + a] + 0.0;  // -0 -> +0
+      v[a] = fmin(v[a], x);
+      v[3 + a] = fmax(v[3 + a], x);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    for (int a = 0; a < 3; ++a) {
+      v[a] = fmin(v[a], __shfl_xor(v[a], o));
+      v[3 + a] = fmax(v[3 + a], __shfl_xor(v[3 + a], o));
+    }
+  if (lane == 0)
+    for (int a = 0; a < 6; ++a) red[wave][a] = v[a];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    double x = red[0][threadIdx.x];
+    for (int w = 1; w < kBoundBlock / 64; ++w)
+      x = threadIdx.x < 3 ? fmin(x, red[w][threadIdx.x]) : fmax(x, red[w][threadIdx.x]);
+    part[6 * blockIdx.x + threadIdx.x] = x;
+  }
+}
+
+__global__ void __launch_bounds__(64) k_bounds_all(const double *__restrict__ part, double *bounds) {
+  static_assert(kBoundBlocks == 64, "one partial per lane");
+  double v[6];
+  for (int a = 0; a < 6; ++a) v[a] = part[6 * threadIdx.x + a];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    for (int a = 0; a < 3; ++a) {
+      v[a] = fmin(v[a], __shfl_xor(v[a], o));
+      v[3 + a] = fmax(v[3 + a], __shfl_xor(v[3 + a], o));
+    }
+  if (threadIdx.x == 0)
+    for (int a = 0; a < 6; ++a) bounds[a] = v[a];
+}
+
+// Canonical order by one sort: a coarse key of 22 + 21 + 21 bits (the
+// coordinates' places between the bounds, monotone in each coordinate), and
+// then the exact lexicographic order within runs of equal x bits.  Points of
+// different x bits are in order; inside a run the key has ordered equal x by
+// y and z already, so only adjacent inversions, which differing x values cause,
+// need the repair below.  Three sorts of the full coordinates (24 passes)
+// remain for clouds with longer runs.
+constexpr int kCoarseShift = 42;
+constexpr int kRunMost = 64;
+constexpr uint32_t kRunMark = 0x80000000u;
+
+__device__ inline uint64_t coarse(double x, double lo, double hi, double most) {
+  const double e = hi - lo, s = e > 0.0 && e < INFINITY ? most / e : 0.0;
+  return (uint64_t)fmin(fmax((x - lo) * s, 0.0), most);
+}
+
+__global__ void k_coarse_keys(const double *__restrict__ src, int64_t n, const double *__restrict__ b, uint64_t *key,
+                              uint32_t *perm) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  key[i] = coarse(src[3 * i] + 0.0, b[0], b[3], 4194303.0) << kCoarseShift |
+           coarse(src[3 * i + 1] + 0.0, b[1], b[4], 2097151.0) << 21 |
+           coarse(src[3 * i + 2] + 0.0, b[2], b[5], 2097151.0);
+  perm[i] = (uint32_t)i;
+}
+
+// Exact lexicographic order of two source points, equal points by index.
+__device__ inline bool source_less(const double *src, uint32_t a, uint32_t b) {
+  for (int k = 0; k < 3; ++k) {
+    const uint64_t x = order_key(dbits(src[3 * (size_t)a + k])), y = order_key(dbits(src[3 * (size_t)b + k]));
+    if (x != y) return x < y;
+  }
+  return a < b;
+}
+
+// Marks the start of every run that holds an adjacent inversion; a run beyond
+// kRunMost points sets status bit 4.  LESS(a, b): the exact order of values.
+template <class LESS>
+__device__ inline void mark_run(const uint64_t *key, int shift, uint32_t *val, int64_t n, int64_t i, uint32_t *status,
+                                LESS &&less) {
+  if (i <= 0 || i >= n) return;
+  const uint64_t r = key[i] >> shift;
+  if (key[i - 1] >> shift != r) return;
+  volatile uint32_t *v = val;  // marks come and go in the top bit
+  if (!less(v[i] & ~kRunMark, v[i - 1] & ~kRunMark)) return;
+  int64_t s = i - 1;
+  while (s > 0 && i - s < kRunMost && key[s - 1] >> shift == r) --s;
+  int64_t e = i + 1;
+  while (e < n && e - s <= kRunMost && key[e] >> shift == r) ++e;
+  if (e - s > kRunMost || (s > 0 && key[s - 1] >> shift == r)) {
+    atomicOr(status, 4u);
+    return;
+  }
+  atomicOr(&val[s], kRunMark);
+}
+
+__global__ void k_mark_runs(const double *__restrict__ src, const uint64_t *__restrict__ key, uint32_t *perm, int64_t n,
+                            uint32_t *status) {
+  mark_run(key, kCoarseShift, perm, n, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, status,
+           [&](uint32_t a, uint32_t b) { return source_less(src, a, b); });
+}
+
+__global__ void k_sort_runs(const double *__restrict__ src, const uint64_t *__restrict__ key, uint32_t *perm,
+                            int64_t n) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n || !(perm[s] & kRunMark)) return;
+  perm[s] &= ~kRunMark;
+  const uint64_t r = key[s] >> kCoarseShift;
+  for (int64_t i = s + 1; i < n && i < s + kRunMost && key[i] >> kCoarseShift == r; ++i) {
+    const uint32_t v = perm[i];
+    int64_t j = i;
+    for (; j > s && source_less(src, v, perm[j - 1]); --j) perm[j] = perm[j - 1];
+    perm[j] = v;
+  }
+}
+
 __global__ void k_order_keys(const double *__restrict__ src, int64_t n, uint64_t *k0,
                              uint64_t *k1, uint64_t *k2, uint32_t *perm) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -35,7 +155,7 @@ __global__ void k_gather_key(const uint64_t *__restrict__ from, const uint32_t *
   if (i < n) to[i] = from[perm[i]];
 }
 
-// After the three stable passes perm lists source indices in canonical order.
+// perm lists source indices in canonical order.
 __global__ void k_canonical(const double *__restrict__ src, const uint32_t *__restrict__ perm,
                             int64_t n, double *X, double *Y, double *Z, uint32_t *source_index,
                             uint32_t *status) {
@@ -56,39 +176,6 @@ __global__ void k_canonical(const double *__restrict__ src, const uint32_t *__re
   double v[3] = {x, y, z};
   for (int a = 0; a < 3; ++a)
     if (!isfinite(v[a])) atomicOr(&status[0], 2u);
-}
-
-// Global AABB with PointId witnesses: the first (smallest) PointId attaining
-// each extremum, as the reference's sequential scan (lbvh.cpp:105-151).
-__global__ void k_bounds(const double *__restrict__ X, const double *__restrict__ Y,
-                         const double *__restrict__ Z, int64_t n, double *bounds,
-                         uint32_t *ids) {
-  __shared__ double sv[6][512];
-  __shared__ uint32_t si[6][512];
-  const int t = threadIdx.x;
-  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  uint32_t w[6] = {kInvalid, kInvalid, kInvalid, kInvalid, kInvalid, kInvalid};
-  for (int64_t i = t; i < n; i += blockDim.x) {
-    double p[3] = {X[i], Y[i], Z[i]};
-    for (int a = 0; a < 3; ++a) {
-      if (p[a] < v[a]) { v[a] = p[a]; w[a] = (uint32_t)i; }
-      if (p[a] > v[3 + a]) { v[3 + a] = p[a]; w[3 + a] = (uint32_t)i; }
-    }
-  }
-  for (int k = 0; k < 6; ++k) { sv[k][t] = v[k]; si[k][t] = w[k]; }
-  __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if (t < off) {
-      for (int k = 0; k < 6; ++k) {
-        double a = sv[k][t], b = sv[k][t + off];
-        uint32_t ia = si[k][t], ib = si[k][t + off];
-        bool take = (k < 3) ? (b < a || (b == a && ib < ia)) : (b > a || (b == a && ib < ia));
-        if (take) { sv[k][t] = b; si[k][t] = ib; }
-      }
-    }
-    __syncthreads();
-  }
-  if (t < 6) { bounds[t] = sv[t][0]; ids[t] = si[t][0]; }
 }
 
 // floor(2^21 (x - l) / (u - l)), certified exactly.
@@ -190,8 +277,7 @@ __device__ inline int delta(const uint64_t *codes, const uint64_t *path, int64_t
 }
 
 __global__ void k_karras(const uint64_t *__restrict__ codes, const uint64_t *__restrict__ path,
-                         int64_t n, Node *nodes, uint32_t *parent_int, uint32_t *parent_leaf,
-                         uint32_t *counter) {
+                         int64_t n, Node *nodes, uint32_t *parent_int, uint32_t *parent_leaf) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n - 1) return;
   const int d = (delta(codes, path, n, i, i + 1) - delta(codes, path, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -220,57 +306,134 @@ __global__ void k_karras(const uint64_t *__restrict__ codes, const uint64_t *__r
   else { nd.right = (uint32_t)(gamma + 1); parent_int[gamma + 1] = (uint32_t)i; }
   for (int a = 0; a < 3; ++a) { nd.lo[a] = 0; nd.hi[a] = 0; }
   nodes[i] = nd;
-  counter[i] = 0;
   if (i == 0) parent_int[0] = kInvalid;
 }
 
-__device__ inline void child_box(uint32_t c, const Node *nodes, const uint32_t *wit,
-                                 const double *LX, const double *LY, const double *LZ,
-                                 const uint32_t *leaf_id, double lo[3], double hi[3],
-                                 uint32_t wl[3], uint32_t wh[3]) {
-  if (c & kLeafBit) {
-    uint32_t p = c & ~kLeafBit;
-    double v[3] = {LX[p], LY[p], LZ[p]};
-    uint32_t id = leaf_id[p];
-    for (int a = 0; a < 3; ++a) { lo[a] = hi[a] = v[a]; wl[a] = wh[a] = id; }
-  } else {
-    // volatile loads: the sibling thread wrote this box before its fence
-    const volatile Node *vn = nodes + c;
-    const volatile uint32_t *vw = wit + 6 * (size_t)c;
+// Box of a set of leaves with its witnesses: per side the extremum and the
+// least PointId attaining it (reference tie rule, lbvh.cpp:46-76).  Any split
+// of the set gives the same box.
+struct Box {
+  double v[6];  // lower x, y, z, upper x, y, z
+  uint32_t w[6];
+  __device__ void clear() {
     for (int a = 0; a < 3; ++a) {
-      lo[a] = vn->lo[a]; hi[a] = vn->hi[a];
-      wl[a] = vw[a]; wh[a] = vw[3 + a];
+      v[a] = INFINITY;
+      v[3 + a] = -INFINITY;
+      w[a] = w[3 + a] = kInvalid;
     }
+  }
+  __device__ void add(int a, double x, uint32_t id) {
+    const bool take = (a < 3 ? x < v[a] : x > v[a]) || (x == v[a] && id < w[a]);
+    v[a] = take ? x : v[a];
+    w[a] = take ? id : w[a];
+  }
+  __device__ void add_leaf(const double *LX, const double *LY, const double *LZ, const uint32_t *leaf_id, int64_t p) {
+    const double x[3] = {LX[p], LY[p], LZ[p]};
+    const uint32_t id = leaf_id[p];
+    for (int a = 0; a < 3; ++a) {
+      add(a, x[a], id);
+      add(3 + a, x[a], id);
+    }
+  }
+  __device__ void add_box(const Box &b) {
+    for (int a = 0; a < 6; ++a) add(a, b.v[a], b.w[a]);
+  }
+  // over the wave, in every lane
+  __device__ void reduce() {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int a = 0; a < 6; ++a) {
+        const double x = __shfl_xor(v[a], o);
+        const uint32_t id = __shfl_xor(w[a], o);
+        add(a, x, id);
+      }
+  }
+};
+
+// Boxes of the wave tree's level-0 and level-1 groups, one workgroup per
+// level-1 group.
+constexpr int kGroupBlock = 1024;
+__global__ void __launch_bounds__(kGroupBlock) k_group_boxes(int64_t n, const double *__restrict__ LX,
+                                                             const double *__restrict__ LY,
+                                                             const double *__restrict__ LZ,
+                                                             const uint32_t *__restrict__ leaf_id, Box *l0, Box *l1) {
+  __shared__ Box box[64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c0 = (n + 63) / 64;
+  for (int j = wave; j < 64; j += kGroupBlock / 64) {
+    const int64_t g = (int64_t)blockIdx.x * 64 + j;
+    Box b;
+    b.clear();
+    if (g < c0) {
+      if (g * 64 + lane < n) b.add_leaf(LX, LY, LZ, leaf_id, g * 64 + lane);
+      b.reduce();
+    }
+    if (lane == 0) {
+      box[j] = b;
+      if (g < c0) l0[g] = b;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    Box b = box[lane];
+    b.reduce();
+    if (lane == 0) l1[blockIdx.x] = b;
   }
 }
 
-__global__ void k_refit(int64_t n, Node *nodes, uint32_t *wit, const uint32_t *__restrict__ parent_int,
-                        const uint32_t *__restrict__ parent_leaf, uint32_t *counter,
-                        const double *__restrict__ LX, const double *__restrict__ LY,
-                        const double *__restrict__ LZ, const uint32_t *__restrict__ leaf_id) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  uint32_t node = parent_leaf[p];
-  while (node != kInvalid) {
-    __threadfence();
-    if (atomicAdd(&counter[node], 1u) == 0) return;  // the sibling subtree is not done yet
-    __threadfence();
-    Node nd = nodes[node];
-    double l0[3], h0[3], l1[3], h1[3];
-    uint32_t wl0[3], wh0[3], wl1[3], wh1[3];
-    child_box(nd.left, nodes, wit, LX, LY, LZ, leaf_id, l0, h0, wl0, wh0);
-    child_box(nd.right, nodes, wit, LX, LY, LZ, leaf_id, l1, h1, wl1, wh1);
-    volatile Node *vn = nodes + node;
-    volatile uint32_t *vw = wit + 6 * (size_t)node;
+// Boxes and witnesses of the internal nodes from their leaf ranges: short
+// ranges leaf by leaf, one node per lane; longer ones by the whole wave from
+// the leaves and groups that make up the range.  No node waits for another
+// (a bottom-up pass with fences between siblings took 97 us at 256 points and
+// 1.44 ms at 200 000).  Bound by the latency of the lane loops.
+constexpr uint32_t kShortRange = 32;
+__global__ void __launch_bounds__(256) k_refit(int64_t n, Node *nodes, uint32_t *wit, const double *__restrict__ LX,
+                                               const double *__restrict__ LY, const double *__restrict__ LZ,
+                                               const uint32_t *__restrict__ leaf_id, const Box *__restrict__ l0,
+                                               const Box *__restrict__ l1) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool valid = i < n - 1;
+  const uint32_t b = valid ? nodes[i].begin : 0u, e = valid ? nodes[i].end : 0u;
+  auto store = [&](int64_t node, const Box &x) {
     for (int a = 0; a < 3; ++a) {
-      bool tl = l1[a] < l0[a] || (l1[a] == l0[a] && wl1[a] < wl0[a]);
-      bool th = h1[a] > h0[a] || (h1[a] == h0[a] && wh1[a] < wh0[a]);
-      vn->lo[a] = tl ? l1[a] : l0[a];
-      vw[a] = tl ? wl1[a] : wl0[a];
-      vn->hi[a] = th ? h1[a] : h0[a];
-      vw[3 + a] = th ? wh1[a] : wh0[a];
+      nodes[node].lo[a] = x.v[a];
+      nodes[node].hi[a] = x.v[3 + a];
     }
-    node = parent_int[node];
+    for (int a = 0; a < 6; ++a) wit[6 * node + a] = x.w[a];
+  };
+  const bool is_short = e - b <= kShortRange;
+  if (valid && is_short) {
+    Box x;
+    x.clear();
+    for (uint32_t p = b; p < e; ++p) x.add_leaf(LX, LY, LZ, leaf_id, p);
+    store(i, x);
+  }
+  for (uint64_t m = __ballot(valid && !is_short); m;) {
+    const int k = __builtin_amdgcn_readfirstlane(__ffsll((long long)m) - 1);
+    m &= m - 1;
+    const uint32_t rb = __builtin_amdgcn_readlane(b, k), re = __builtin_amdgcn_readlane(e, k);
+    Box x;
+    x.clear();
+    // whole level-0 groups [g0, g1), of these whole level-1 groups [h0, h1)
+    const uint32_t g0 = (rb + 63) / 64, g1 = re / 64;
+    if (g0 >= g1) {
+      for (uint32_t p = rb + lane; p < re; p += 64) x.add_leaf(LX, LY, LZ, leaf_id, p);
+    } else {
+      if (rb + lane < g0 * 64) x.add_leaf(LX, LY, LZ, leaf_id, rb + lane);
+      if (g1 * 64 + lane < re) x.add_leaf(LX, LY, LZ, leaf_id, g1 * 64 + lane);
+      const uint32_t h0 = (g0 + 63) / 64, h1 = g1 / 64;
+      if (h0 >= h1) {
+        for (uint32_t g = g0 + lane; g < g1; g += 64) x.add_box(l0[g]);
+      } else {
+        if (g0 + lane < h0 * 64) x.add_box(l0[g0 + lane]);
+        if (h1 * 64 + lane < g1) x.add_box(l0[h1 * 64 + lane]);
+        for (uint32_t h = h0 + lane; h < h1; h += 64) x.add_box(l1[h]);
+      }
+    }
+    x.reduce();
+    if (lane == 0) store(i - lane + k, x);
   }
 }
 
@@ -371,54 +534,19 @@ __global__ void k_wide_nodes(int64_t m, const Node *__restrict__ nodes, const do
   out[i] = w;
 }
 
-// Wave-tree boxes (wave_tree.hpp): one workgroup per level-1 group, its 16
-// waves reducing four level-0 groups each; the level-1 box follows from them
-// in LDS.  Bound by the read of the leaves (24 B each).
-constexpr int kGroupBlock = 1024;
-__global__ void __launch_bounds__(kGroupBlock) k_group_boxes(int64_t n, double cx, double cy, double cz,
-                                                             const double *__restrict__ LX,
-                                                             const double *__restrict__ LY,
-                                                             const double *__restrict__ LZ, GroupBox *l0,
-                                                             GroupBox *l1) {
-  __shared__ float box[64][6];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t c0 = (n + 63) / 64;
-  for (int j = wave; j < 64; j += kGroupBlock / 64) {
-    const int64_t g = (int64_t)blockIdx.x * 64 + j;
-    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    const int64_t p = g * 64 + lane;
-    if (p < n) {
-      const double d[3] = {LX[p] - cx, LY[p] - cy, LZ[p] - cz};
-      for (int a = 0; a < 3; ++a) {
-        v[a] = __double2float_rd(d[a]);
-        v[3 + a] = __double2float_ru(d[a]);
-      }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        v[a] = fminf(v[a], __shfl_xor(v[a], o));
-        v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
-      }
-    if (lane == 0) {
-      for (int a = 0; a < 6; ++a) box[j][a] = v[a];
-      if (g < c0) l0[g] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
-    }
+// Wave-tree boxes (wave_tree.hpp) of levels 0 and 1 from the exact group
+// boxes, in the unit 2^e, relative to the centre and rounded outward.
+__global__ void k_wave_boxes(int64_t count, const Box *__restrict__ in, int e, double cx, double cy, double cz,
+                             GroupBox *out) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= count) return;
+  const double c[3] = {cx, cy, cz};
+  GroupBox b{};
+  for (int a = 0; a < 3; ++a) {
+    b.lo[a] = __double2float_rd(ldexp(in[g].v[a], e) - c[a]);
+    b.hi[a] = __double2float_ru(ldexp(in[g].v[3 + a], e) - c[a]);
   }
-  __syncthreads();
-  if (wave == 0) {
-    float v[6];
-    for (int a = 0; a < 6; ++a) v[a] = box[lane][a];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        v[a] = fminf(v[a], __shfl_xor(v[a], o));
-        v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
-      }
-    if (lane == 0) l1[blockIdx.x] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
-  }
+  out[g] = b;
 }
 
 // Level-2 boxes, one wave per group (clouds of more than 262 144 points).
@@ -502,65 +630,82 @@ void apply_unit_scale(Context &c, const double bounds[6]) {
 
 }  // namespace
 
-void canonicalize_and_build(Context &c) {
+// Canonical order and LBVH; full_sort: by three sorts of the whole
+// coordinates, whatever the runs.  Returns false when that is needed.
+static bool build(Context &c, bool full_sort) {
   const int64_t n = c.n;
-  c.scale_exp = 0;
   hipStream_t s = c.stream;
   const int T = 256;
-  c.X.ensure(n); c.Y.ensure(n); c.Z.ensure(n);
-  c.source_index.ensure(n);
-  c.key0.ensure(n); c.key1.ensure(n); c.key2.ensure(n);
-  c.perm.ensure(n);
-  c.status.ensure(16);
-  c.bounds.ensure(6);
-  c.bound_ids.ensure(6);
+  const dim3 G(blocks_for(n, T)), B256(T);
   MHGP_HIP(hipMemsetAsync(c.status.p, 0, 16 * sizeof(uint32_t), s));
-  hipLaunchKernelGGL(k_order_keys, dim3(blocks_for(n, T)), dim3(T), 0, s, c.src.p, n, c.key0.p,
-                     c.key1.p, c.key2.p, c.perm.p);
-  // stable LSD over (k0, k1, k2): least significant key first
-  c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
-  hipLaunchKernelGGL(k_gather_key, dim3(blocks_for(n, T)), dim3(T), 0, s, c.key1.p, c.perm.p, n,
-                     c.key2.p);
-  c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
-  hipLaunchKernelGGL(k_gather_key, dim3(blocks_for(n, T)), dim3(T), 0, s, c.key0.p, c.perm.p, n,
-                     c.key2.p);
-  c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
-  hipLaunchKernelGGL(k_canonical, dim3(blocks_for(n, T)), dim3(T), 0, s, c.src.p, c.perm.p, n,
-                     c.X.p, c.Y.p, c.Z.p, c.source_index.p, c.status.p);
-  hipLaunchKernelGGL(k_bounds, dim3(1), dim3(512), 0, s, c.X.p, c.Y.p, c.Z.p, n, c.bounds.p,
-                     c.bound_ids.p);
-  c.codes.ensure(n);
-  c.leaf_id.ensure(n);
-  c.leaf_pos.ensure(n);
-  c.LX.ensure(n); c.LY.ensure(n); c.LZ.ensure(n);
-  c.path.ensure(n);
-  hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, T)), dim3(T), 0, s, c.X.p, c.Y.p, c.Z.p, n,
-                     c.bounds.p, c.codes.p, c.leaf_id.p, c.status.p);
-  c.sorter.sort(c.codes.p, c.leaf_id.p, n, 0, 64, s);
-  hipLaunchKernelGGL(k_leaves, dim3(blocks_for(n, T)), dim3(T), 0, s, c.leaf_id.p, c.X.p, c.Y.p,
-                     c.Z.p, c.codes.p, n, c.LX.p, c.LY.p, c.LZ.p, c.leaf_pos.p, c.path.p);
-  const int64_t ni = n > 1 ? n - 1 : 1;
-  c.nodes.ensure(ni);
-  c.parent_int.ensure(ni);
-  c.parent_leaf.ensure(n);
-  c.wit.ensure(6 * ni);
-  c.counter.ensure(ni);
+  hipLaunchKernelGGL(k_bounds, dim3(kBoundBlocks), dim3(kBoundBlock), 0, s, c.src.p, n, c.bounds.p + 6);
+  hipLaunchKernelGGL(k_bounds_all, dim3(1), dim3(64), 0, s, c.bounds.p + 6, c.bounds.p);
+  if (full_sort) {
+    c.key1.ensure(n);
+    c.key2.ensure(n);
+    hipLaunchKernelGGL(k_order_keys, G, B256, 0, s, c.src.p, n, c.key0.p, c.key1.p, c.key2.p, c.perm.p);
+    // stable LSD over (k0, k1, k2): least significant key first
+    c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
+    hipLaunchKernelGGL(k_gather_key, G, B256, 0, s, c.key1.p, c.perm.p, n, c.key2.p);
+    c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
+    hipLaunchKernelGGL(k_gather_key, G, B256, 0, s, c.key0.p, c.perm.p, n, c.key2.p);
+    c.sorter.sort(c.key2.p, c.perm.p, n, 0, 64, s);
+  } else {
+    hipLaunchKernelGGL(k_coarse_keys, G, B256, 0, s, c.src.p, n, c.bounds.p, c.key0.p, c.perm.p);
+    c.sorter.sort(c.key0.p, c.perm.p, n, 0, 64, s);
+    hipLaunchKernelGGL(k_mark_runs, G, B256, 0, s, c.src.p, c.key0.p, c.perm.p, n, c.status.p);
+    hipLaunchKernelGGL(k_sort_runs, G, B256, 0, s, c.src.p, c.key0.p, c.perm.p, n);
+  }
+  hipLaunchKernelGGL(k_canonical, G, B256, 0, s, c.src.p, c.perm.p, n, c.X.p, c.Y.p, c.Z.p, c.source_index.p,
+                     c.status.p);
+  hipLaunchKernelGGL(k_morton, G, B256, 0, s, c.X.p, c.Y.p, c.Z.p, n, c.bounds.p, c.codes.p, c.leaf_id.p,
+                     c.status.p);
+  c.sorter.sort(c.codes.p, c.leaf_id.p, n, 0, 63, s);
+  hipLaunchKernelGGL(k_leaves, G, B256, 0, s, c.leaf_id.p, c.X.p, c.Y.p, c.Z.p, c.codes.p, n, c.LX.p, c.LY.p, c.LZ.p,
+                     c.leaf_pos.p, c.path.p);
+  const int64_t c0 = (n + 63) / 64, c1 = (c0 + 63) / 64;
+  c.group_exact.ensure((c0 + c1) * sizeof(Box));
+  Box *gb = reinterpret_cast<Box *>(c.group_exact.p);
+  hipLaunchKernelGGL(k_group_boxes, dim3(c1), dim3(kGroupBlock), 0, s, n, c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p, gb,
+                     gb + c0);
   if (n > 1) {
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1, T)), dim3(T), 0, s, c.codes.p, c.path.p, n,
-                       c.nodes.p, c.parent_int.p, c.parent_leaf.p, c.counter.p);
-    hipLaunchKernelGGL(k_refit, dim3(blocks_for(n, T)), dim3(T), 0, s, n, c.nodes.p, c.wit.p,
-                       c.parent_int.p, c.parent_leaf.p, c.counter.p, c.LX.p, c.LY.p, c.LZ.p,
-                       c.leaf_id.p);
+    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1, T)), B256, 0, s, c.codes.p, c.path.p, n, c.nodes.p,
+                       c.parent_int.p, c.parent_leaf.p);
+    hipLaunchKernelGGL(k_refit, dim3(blocks_for(n - 1, T)), B256, 0, s, n, c.nodes.p, c.wit.p, c.LX.p, c.LY.p,
+                       c.LZ.p, c.leaf_id.p, gb, gb + c0);
   } else {
     MHGP_HIP(hipMemsetAsync(c.parent_leaf.p, 0xff, sizeof(uint32_t), s));
   }
   MHGP_LAUNCH_CHECK();
   uint32_t st[4];
-  MHGP_HIP(hipMemcpyAsync(st, c.status.p, sizeof(st), hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipStreamSynchronize(s));
+  copy_wait(st, c.status.p, sizeof(st), hipMemcpyDeviceToHost, s);
+  if (st[0] & 4u) return false;
   if (st[0] & 2u) throw std::invalid_argument("a point coordinate is not finite");
   if (st[0] & 1u) throw std::invalid_argument("the cloud contains duplicate geometric points");
   if (st[2]) throw std::runtime_error("an exact Morton bin could not be certified");
+  return true;
+}
+
+void canonicalize_and_build(Context &c) {
+  const int64_t n = c.n, ni = n > 1 ? n - 1 : 1;
+  c.scale_exp = 0;
+  hipStream_t s = c.stream;
+  c.X.ensure(n); c.Y.ensure(n); c.Z.ensure(n);
+  c.source_index.ensure(n);
+  c.key0.ensure(n);
+  c.perm.ensure(n);
+  c.status.ensure(16);
+  c.bounds.ensure(6 * (1 + kBoundBlocks));
+  c.codes.ensure(n);
+  c.leaf_id.ensure(n);
+  c.leaf_pos.ensure(n);
+  c.LX.ensure(n); c.LY.ensure(n); c.LZ.ensure(n);
+  c.path.ensure(n);
+  c.nodes.ensure(ni);
+  c.parent_int.ensure(ni);
+  c.parent_leaf.ensure(n);
+  c.wit.ensure(6 * ni);
+  if (!build(c, false) && !build(c, true)) throw std::runtime_error("the canonical order did not settle");
   double bounds[6];
   copy_wait(bounds, c.bounds.p, sizeof(bounds), hipMemcpyDeviceToHost, s);
   apply_unit_scale(c, bounds);
@@ -572,8 +717,9 @@ void canonicalize_and_build(Context &c) {
   const int64_t c0 = (n + 63) / 64, c1 = (c0 + 63) / 64, c2 = (c1 + 63) / 64;
   c.groups.ensure(c0 + c1 + c2);
   for (int a = 0; a < 3; ++a) c.centre[a] = std::ldexp(0.5 * bounds[a] + 0.5 * bounds[3 + a], c.scale_exp);
-  hipLaunchKernelGGL(k_group_boxes, dim3(c1), dim3(kGroupBlock), 0, s, n, c.centre[0], c.centre[1], c.centre[2],
-                     c.LX.p, c.LY.p, c.LZ.p, c.groups.p, c.groups.p + c0);
+  hipLaunchKernelGGL(k_wave_boxes, dim3(blocks_for(c0 + c1, 256)), dim3(256), 0, s, c0 + c1,
+                     reinterpret_cast<const Box *>(c.group_exact.p), c.scale_exp, c.centre[0], c.centre[1],
+                     c.centre[2], c.groups.p);
   if (c2 > 1)
     hipLaunchKernelGGL(k_group_top, dim3(c2), dim3(64), 0, s, (uint32_t)c1, c.groups.p + c0, c.groups.p + c0 + c1);
   MHGP_LAUNCH_CHECK();

@@ -27,10 +27,10 @@ Context::~Context() {
 }
 
 int64_t device_bytes(const Context &c) {
-  int64_t b = c.src.bytes() + c.X.bytes() * 3 + c.source_index.bytes() + c.key0.bytes() * 3 +
+  int64_t b = c.src.bytes() + c.X.bytes() * 3 + c.source_index.bytes() + c.key0.bytes() + c.key1.bytes() + c.key2.bytes() +
               c.perm.bytes() + c.codes.bytes() + c.leaf_id.bytes() + c.leaf_pos.bytes() +
               c.LX.bytes() * 3 + c.path.bytes() + c.nodes.bytes() + c.parent_int.bytes() +
-              c.parent_leaf.bytes() + c.wit.bytes() + c.counter.bytes() + c.wide.bytes() + c.groups.bytes();
+              c.parent_leaf.bytes() + c.wit.bytes() + c.wide.bytes() + c.groups.bytes() + c.group_exact.bytes();
   if (c.catalog) b += catalog_device_bytes(*c.catalog);
   if (c.emst) b += c.emst->bytes();
   if (c.tower_work) b += c.tower_work->bytes();
@@ -48,12 +48,13 @@ void release_device_state(Context &c) {
   c.catalog.reset();
   for (DevBuf<double> *b : {&c.src, &c.X, &c.Y, &c.Z, &c.bounds, &c.LX, &c.LY, &c.LZ}) b->release();
   for (DevBuf<uint64_t> *b : {&c.key0, &c.key1, &c.key2, &c.codes, &c.path}) b->release();
-  for (DevBuf<uint32_t> *b : {&c.source_index, &c.perm, &c.status, &c.bound_ids, &c.leaf_id, &c.leaf_pos,
-                              &c.parent_int, &c.parent_leaf, &c.wit, &c.counter})
+  for (DevBuf<uint32_t> *b : {&c.source_index, &c.perm, &c.status, &c.leaf_id, &c.leaf_pos,
+                              &c.parent_int, &c.parent_leaf, &c.wit})
     b->release();
   c.nodes.release();
   c.wide.release();
   c.groups.release();
+  c.group_exact.release();
   c.n = 0;
   c.lbvh_ready = false;
 }

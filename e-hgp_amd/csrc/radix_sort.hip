@@ -1,30 +1,39 @@
 // Stable LSD radix sort of (uint64 key, uint32 value) pairs, 8-bit digits.
 //
-// Pass structure (one pass per digit), on tiles of 4 096 keys:
+// Pass structure (one pass per digit), on tiles of 1 024 or 4 096 keys:
 //   1. tile histograms: 64-key groups of equal digits are found with eight
 //      ballots and counted with one LDS atomic per group;
-//   2. multi-block inclusive scan over [digit][tile]; the entry before
-//      (digit, tile) is that tile's base offset for the digit (digit-major,
-//      so equal digits keep tile order);
-//   3. scatter: each of the four waves of a tile ranks its 1 024 keys in
-//      order (64-key chunks, eight ballots, a per-digit running count in
-//      LDS), the tile is reordered by digit in LDS, and the reordered tile is
-//      written out in index order, so the stores of a digit run are
-//      contiguous.  Key order inside a digit is (wave, chunk, lane), the
-//      input order: the pass is stable.
-// Passes whose digit is the same for every key (detected on the device by
-// the scan) copy instead of scattering, so ping-pong buffers stay consistent.
+//   2. base offsets of (digit, tile), digit-major, so equal digits keep tile
+//      order: up to kDirectTiles tiles each scatter workgroup sums the counts
+//      it needs itself; beyond that a multi-block inclusive scan over
+//      [digit][tile] leaves them;
+//   3. scatter: each of the four waves of a tile ranks its keys in order
+//      (64-key chunks, eight ballots, a per-digit running count in LDS), the
+//      tile is reordered by digit in LDS, and the reordered tile is written
+//      out in index order, so the stores of a digit run are contiguous.  Key
+//      order inside a digit is (wave, chunk, lane), the input order: the pass
+//      is stable.
+// Passes whose digit is the same for every key copy instead of scattering, so
+// ping-pong buffers stay consistent.  Up to kSmallSort keys are sorted by one
+// workgroup in LDS (bitonic over (key, index), hence stable).
+//
+// Below a few hundred thousand keys a pass is bound by its launches and by the
+// few workgroups it has: tiles of 1 024 and the two-launch pass took the sorts
+// of a 50 000-point build from four launches and 13 workgroups a pass to two
+// and 49, the one-workgroup sort those of a 256-point build from 128 launches
+// to two (index of 256 points: 0.91 -> 0.29 ms with the rest of the build).
 #include "radix_sort.hpp"
 
 namespace mhgp {
 
 namespace {
 
-constexpr int kTile = 4096;
+constexpr int kDirectTiles = 128;
+constexpr int kSmallSort = 8192;
+constexpr int kSmallBlock = 1024;
 constexpr int kDigits = 256;
 constexpr int kSortBlock = 256;
 constexpr int kWaves = kSortBlock / 64;
-constexpr int kChunks = kTile / kSortBlock;  // 64-key chunks per wave
 
 __device__ inline uint64_t lanes_below() {
   const int lane = (int)(threadIdx.x & 63u);
@@ -42,6 +51,8 @@ __device__ inline uint64_t digit_match(bool valid, uint32_t dig) {
   return match;
 }
 
+// counts: [digit][tile], or [tile][digit] when the scatter sums them itself
+template <int kTile, bool DIRECT>
 __global__ void __launch_bounds__(kSortBlock) rs_histogram(const uint64_t *__restrict__ keys, int64_t n, int shift,
                                                            uint32_t *__restrict__ counts, int tiles) {
   __shared__ uint32_t h[kDigits];
@@ -59,38 +70,38 @@ __global__ void __launch_bounds__(kSortBlock) rs_histogram(const uint64_t *__res
     if (valid && (match & below) == 0) atomicAdd(&h[dig], (uint32_t)__popcll(match));
   }
   __syncthreads();
-  counts[(size_t)t * tiles + blockIdx.x] = h[t];
+  counts[DIRECT ? (size_t)blockIdx.x * kDigits + t : (size_t)t * tiles + blockIdx.x] = h[t];
 }
 
-// flags[0] = 1 when one digit holds every key (the pass is the identity
-// permutation); incl is the inclusive scan of the digit-major counts.
-__global__ void rs_identity(const uint32_t *__restrict__ incl, int64_t n, int tiles, uint32_t *flags) {
-  __shared__ uint32_t full;
-  const int d = threadIdx.x;
-  if (d == 0) full = 0;
-  __syncthreads();
-  const uint32_t lo = d == 0 ? 0u : incl[(size_t)d * tiles - 1];
-  const uint32_t hi = incl[(size_t)(d + 1) * tiles - 1];
-  if (hi - lo == (uint32_t)n) full = 1;
-  __syncthreads();
-  if (d == 0) flags[0] = full;
-}
-
+template <int kTile, bool DIRECT>
 __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restrict__ kin,
                                                          const uint32_t *__restrict__ vin,
                                                          uint64_t *__restrict__ kout,
                                                          uint32_t *__restrict__ vout, int64_t n, int shift,
-                                                         const uint32_t *__restrict__ offsets, int tiles,
-                                                         const uint32_t *__restrict__ flags) {
+                                                         const uint32_t *__restrict__ counts, int tiles) {
+  constexpr int kChunks = kTile / kSortBlock;  // 64-key chunks per wave
   __shared__ uint64_t skey[kTile];
   __shared__ uint32_t sval[kTile];
   __shared__ uint32_t wrun[kWaves][kDigits];  // per wave: running count, then the wave's base
   __shared__ uint32_t lbase[kDigits];         // tile-local start of each digit
   __shared__ uint32_t gbase[kDigits];         // global start of the tile's keys of each digit
-  __shared__ uint32_t wtot[kWaves];
+  __shared__ uint32_t wtot[kWaves], dtot[kWaves];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int64_t base = (int64_t)blockIdx.x * kTile;
-  if (flags[0]) {  // identity pass
+  // digit t: keys of the digit in earlier tiles and in all tiles (DIRECT), or
+  // the scanned bounds of its keys
+  uint32_t in_before = 0, in_all = 0;
+  if (DIRECT) {
+    for (int i = 0; i < tiles; ++i) {
+      const uint32_t c = counts[(size_t)i * kDigits + t];
+      in_before += i < (int)blockIdx.x ? c : 0u;
+      in_all += c;
+    }
+  } else {
+    const uint32_t lo = t == 0 ? 0u : counts[(size_t)t * tiles - 1];
+    in_all = counts[(size_t)(t + 1) * tiles - 1] - lo;
+  }
+  if (__syncthreads_or(in_all == (uint32_t)n)) {  // one digit holds every key: identity pass
     for (int i = t; i < kTile; i += kSortBlock) {
       const int64_t g = base + i;
       if (g < n) {
@@ -144,9 +155,25 @@ __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restr
     if (lane >= d) x += y;
   }
   if (lane == 63) wtot[wave] = x;
-  const size_t e = (size_t)t * tiles + blockIdx.x;
-  gbase[t] = e ? offsets[e - 1] : 0u;
-  __syncthreads();
+  if (DIRECT) {
+    // exclusive scan of the digits' totals
+    uint32_t y = in_all;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t z = __shfl_up(y, (unsigned)d, 64);
+      if (lane >= d) y += z;
+    }
+    if (lane == 63) dtot[wave] = y;
+    __syncthreads();
+    uint32_t digits_before = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) digits_before += w < wave ? dtot[w] : 0u;
+    gbase[t] = digits_before + y - in_all + in_before;
+  } else {
+    const size_t e = (size_t)t * tiles + blockIdx.x;
+    gbase[t] = e ? counts[e - 1] : 0u;
+    __syncthreads();
+  }
   uint32_t before = 0;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) before += w < wave ? wtot[w] : 0u;
@@ -171,25 +198,92 @@ __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restr
   }
 }
 
+// Up to kSmallSort keys in one workgroup: a bitonic sort of (key, index) in
+// LDS, keys beyond n sorting last.
+__global__ void __launch_bounds__(kSmallBlock) rs_small(uint64_t *keys, uint32_t *vals, int n, int padded, int shift,
+                                                        uint64_t mask) {
+  __shared__ uint64_t k[kSmallSort];
+  __shared__ uint16_t at[kSmallSort];
+  for (int i = threadIdx.x; i < padded; i += kSmallBlock) {
+    k[i] = i < n ? (keys[i] >> shift) & mask : ~0ull;
+    at[i] = (uint16_t)i;
+  }
+  __syncthreads();
+  for (int size = 2; size <= padded; size <<= 1)
+    for (int d = size >> 1; d > 0; d >>= 1) {
+      for (int p = threadIdx.x; p < padded / 2; p += kSmallBlock) {
+        const int i = 2 * p - (p & (d - 1)), j = i + d;  // bit d of i clear
+        const bool up = (i & size) == 0;
+        const uint64_t a = k[i], b = k[j];
+        const uint16_t x = at[i], y = at[j];
+        const bool above = a > b || (a == b && x > y);
+        if (above == up) {
+          k[i] = b;
+          k[j] = a;
+          at[i] = y;
+          at[j] = x;
+        }
+      }
+      __syncthreads();
+    }
+  // gather through registers: sources are read before any is overwritten
+  uint64_t kv[kSmallSort / kSmallBlock];
+  uint32_t vv[kSmallSort / kSmallBlock];
+#pragma unroll
+  for (int r = 0; r < kSmallSort / kSmallBlock; ++r) {
+    const int i = threadIdx.x + r * kSmallBlock;
+    if (i < n) {
+      kv[r] = keys[at[i]];
+      vv[r] = vals[at[i]];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kSmallSort / kSmallBlock; ++r) {
+    const int i = threadIdx.x + r * kSmallBlock;
+    if (i < n) {
+      keys[i] = kv[r];
+      vals[i] = vv[r];
+    }
+  }
+}
+
+template <int kTile, bool DIRECT>
+void sort_pass(RadixSorter &S, const uint64_t *ka, const uint32_t *va, uint64_t *kb, uint32_t *vb, int64_t n, int shift,
+               int tiles, hipStream_t stream) {
+  hipLaunchKernelGGL((rs_histogram<kTile, DIRECT>), dim3(tiles), dim3(kSortBlock), 0, stream, ka, n, shift, S.counts.p,
+                     tiles);
+  if (!DIRECT) S.scanner.inclusive(S.counts.p, (int64_t)kDigits * tiles, stream);
+  hipLaunchKernelGGL((rs_scatter<kTile, DIRECT>), dim3(tiles), dim3(kSortBlock), 0, stream, ka, va, kb, vb, n, shift,
+                     S.counts.p, tiles);
+}
+
 }  // namespace
 
 void RadixSorter::sort(uint64_t *keys, uint32_t *vals, int64_t n, int begin_bit, int end_bit,
                        hipStream_t stream) {
   if (n <= 1) return;
-  const int tiles = blocks_for(n, kTile);
+  if (n <= kSmallSort) {
+    int padded = 2;
+    while (padded < n) padded <<= 1;
+    const uint64_t mask = end_bit - begin_bit >= 64 ? ~0ull : (1ull << (end_bit - begin_bit)) - 1ull;
+    hipLaunchKernelGGL(rs_small, dim3(1), dim3(kSmallBlock), 0, stream, keys, vals, (int)n, padded, begin_bit, mask);
+    MHGP_LAUNCH_CHECK();
+    return;
+  }
+  // tiles of 1 024 keys while each scatter can sum their counts, then of 4 096
+  const bool fine = n <= 1024 * kDirectTiles;
+  const int tiles = blocks_for(n, fine ? 1024 : 4096);
   tmp_keys.ensure(n);
   tmp_vals.ensure(n);
   counts.ensure((size_t)kDigits * tiles);
-  flags.ensure(1);
   uint64_t *ka = keys, *kb = tmp_keys.p;
   uint32_t *va = vals, *vb = tmp_vals.p;
   int passes = 0;
   for (int shift = begin_bit; shift < end_bit; shift += 8) {
-    hipLaunchKernelGGL(rs_histogram, dim3(tiles), dim3(kSortBlock), 0, stream, ka, n, shift, counts.p, tiles);
-    scanner.inclusive(counts.p, (int64_t)kDigits * tiles, stream);
-    hipLaunchKernelGGL(rs_identity, dim3(1), dim3(kDigits), 0, stream, counts.p, n, tiles, flags.p);
-    hipLaunchKernelGGL(rs_scatter, dim3(tiles), dim3(kSortBlock), 0, stream, ka, va, kb, vb, n, shift, counts.p,
-                       tiles, flags.p);
+    if (fine) sort_pass<1024, true>(*this, ka, va, kb, vb, n, shift, tiles, stream);
+    else if (tiles <= kDirectTiles) sort_pass<4096, true>(*this, ka, va, kb, vb, n, shift, tiles, stream);
+    else sort_pass<4096, false>(*this, ka, va, kb, vb, n, shift, tiles, stream);
     MHGP_LAUNCH_CHECK();
     std::swap(ka, kb);
     std::swap(va, vb);

@@ -96,3 +96,40 @@ def test_device_snapshot_is_certified_exactly():
             xyz, _ = ctx.canonical_points()
             leaves, nodes, counters = ctx.lbvh_snapshot()
         mhgp.lbvh_certify(xyz, leaves, nodes, counters)
+
+
+def _build_edges():
+    """Sizes around the one-workgroup sort and the sort tiles, and clouds whose
+    coarse canonical keys collide: tight clusters (short runs, repaired), a far
+    outlier that puts every other point into one run and columns of equal x
+    (the sort of the full coordinates), and signed zeros."""
+    for n in (2, 63, 65, 4096, 4097, 8192, 8193):
+        yield f"uniform{n}", workloads.uniform_cloud(n, seed=n)
+    rng = np.random.default_rng(8)
+    centres = rng.random((700, 3))
+    yield "clusters", np.repeat(centres, 13, axis=0) + rng.normal(0.0, 1e-9, size=(9100, 3))
+    far = workloads.uniform_cloud(9000, seed=4)
+    far[17] = [1e12, -1e12, 1e12]
+    yield "outlier", far
+    cols = rng.random((9000, 3))
+    cols[:, 0] = np.floor(cols[:, 0] * 4) / 4 + rng.random(9000) * 1e-12
+    yield "columns", cols
+    zero = workloads.uniform_cloud(300, seed=5) - 0.5
+    zero[:40, 0] = np.where(np.arange(40) % 2, 0.0, -0.0)
+    yield "zeros", zero
+
+
+@pytest.mark.parametrize("name,pts", list(_build_edges()), ids=lambda v: v if isinstance(v, str) else "")
+def test_build_at_its_edges(name, pts):
+    print(f"build edge case {name} n={len(pts)}", flush=True)
+    canon = oracle.canonicalize(pts)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        xyz, src = ctx.canonical_points()
+        assert np.array_equal(xyz, canon)
+        assert np.array_equal(np.asarray(pts)[src] + 0.0, canon)
+        leaves, nodes, counters = ctx.lbvh_snapshot()
+    ref = oracle.lbvh_snapshot(canon)
+    assert np.array_equal(leaves, ref.leaves)
+    assert np.array_equal(nodes, ref.nodes)
+    assert np.array_equal(counters, ref.counters)
