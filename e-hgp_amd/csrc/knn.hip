@@ -29,7 +29,8 @@ constexpr int kKnnBlock = 256;  // four waves, four queries
 // group is tested.  Bound by VALU issue of the insertions and the distance
 // evaluations.  mhgp_knn over 50 000 points, k = 32: 10.4 ms with one thread
 // per query (its list in scratch memory), 1.27 ms here, copies included.
-__global__ void __launch_bounds__(kKnnBlock) k_knn(WaveTree T, int k, uint32_t *out, uint8_t *flags) {
+__global__ void __launch_bounds__(kKnnBlock) k_knn(WaveTree T, int k, uint32_t *out, int stride,
+                                                   uint8_t *flags) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t p = blockIdx.x * (kKnnBlock / 64) + (threadIdx.x >> 6);
   if (p >= T.n) return;
@@ -76,7 +77,7 @@ __global__ void __launch_bounds__(kKnnBlock) k_knn(WaveTree T, int k, uint32_t *
   const uint32_t nx = __shfl_down(bx, 1u);
   const bool tie = (int)lane + 1 < kk && !(bx && nx) && (nd - bd) <= kSlack * nd + kSlackAbs;
   const uint64_t any = __ballot(tie);
-  if ((int)lane < k) out[(int64_t)self * k + lane] = (int)lane < kk ? bi : kInvalid;
+  if ((int)lane < stride) out[(int64_t)self * stride + lane] = (int)lane < min(k, kk) ? bi : kInvalid;
   if (lane == 0) flags[self] = any ? 1 : 0;
 }
 
@@ -326,12 +327,12 @@ void knn_partition(Context &c, const int64_t *num, const int64_t *den, int64_t Q
   }
 }
 
-void knn_all(Context &c, int k, uint32_t *d_out, uint8_t *d_flags, hipStream_t stream) {
-  if (k < 1 || k > 32) throw std::invalid_argument("k must lie in 1..32");
+void knn_all(Context &c, int k, uint32_t *d_out, uint8_t *d_flags, hipStream_t stream, int stride) {
+  if (k < 1 || k > 63) throw std::invalid_argument("k must lie in 1..63");
   if (k >= c.n) throw std::invalid_argument("k must be smaller than the point count");
   hipStream_t s = stream ? stream : c.stream;
   hipLaunchKernelGGL(k_knn, dim3(blocks_for(c.n, kKnnBlock / 64)), dim3(kKnnBlock), 0, s, wave_tree(c), k, d_out,
-                     d_flags);
+                     stride ? stride : k, d_flags);
   MHGP_LAUNCH_CHECK();
 }
 

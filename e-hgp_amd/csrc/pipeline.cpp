@@ -164,6 +164,7 @@ static void knn_exact_one(Context &c, int64_t q, int k, uint32_t *out) {
 }
 
 void knn_host(Context &c, int k, uint32_t *ids_out) {
+  if (k < 1 || k > 32) throw std::invalid_argument("k must lie in 1..32");
   const int64_t n = c.n;
   DevBuf<uint32_t> d_out;
   DevBuf<uint8_t> d_flags;

@@ -4,11 +4,12 @@
 // saddles those of closed rank k+1.  Every strict arm (closed label minus one
 // shell point) is resolved to the minimum of its component:
 //  * the labels of the minima live in an open-addressing hash table;
-//  * an arm that is not a minimum descends: Welzl's algorithm gives the FP64
-//    miniball of the facet, its support and containment are certified with
-//    the predicates of predicates.hpp, an LBVH ball query lists the points of
-//    the closed ball, and the facet trades its least support point for the
-//    least point strictly inside (the miniball strictly shrinks);
+//  * an arm that is not a minimum descends: the FP64 miniball of the facet
+//    (proposed in FP32) has its support and containment certified with the
+//    predicates of predicates.hpp, the points of the closed ball come from a
+//    neighbour list or an LBVH ball query, and the facet trades its least
+//    support point for the least point strictly inside (the miniball strictly
+//    shrinks);
 //  * anything the certified filters cannot decide is flagged for the host's
 //    exact descent.
 #include <chrono>
@@ -29,31 +30,86 @@ namespace {
 
 constexpr int kMaxLabel = 11;
 
-__device__ inline uint64_t label_hash(const uint32_t *ids, int k) {
-  uint64_t h = 0x9e3779b97f4a7c15ull ^ (uint64_t)k;
-  for (int i = 0; i < k; ++i) {
-    h ^= ids[i] + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);
-    h *= 0xff51afd7ed558ccdull;
-    h ^= h >> 33;
-  }
-  return h | 1ull;  // 0 marks an empty slot
+// Hash of a facet: the sum of its points' mixes, so that the hash of a
+// saddle's label minus one point is a subtraction.  The low word picks the
+// slot, the high word (made odd) is the tag stored beside the value.
+__device__ inline uint64_t point_mix(uint32_t id) {
+  uint32_t a = id * 0x9e3779b1u, b = (id ^ 0x5bd1e995u) * 0x85ebca77u;
+  a ^= a >> 15;
+  b ^= b >> 13;
+  a *= 0x2c1b3c6du;
+  b *= 0xc2b2ae3du;
+  return ((uint64_t)(b ^ (b >> 16)) << 32) | (a ^ (a >> 13));
 }
-
-__device__ inline int event_label(const EventRec &e, uint32_t *out) {
-  const int m = e.meta & 0xff, ni = (e.meta >> 16) & 0xff;
-  int k = 0;
-  for (int i = 0; i < m; ++i) out[k++] = e.ids[i];
-  for (int i = 0; i < ni; ++i) out[k++] = e.interior[i];
-  for (int i = 1; i < k; ++i) {  // insertion sort
-    uint32_t v = out[i];
-    int j = i - 1;
-    while (j >= 0 && out[j] > v) { out[j + 1] = out[j]; j--; }
-    out[j + 1] = v;
-  }
-  return k;
-}
+__device__ inline uint64_t hash_slot(uint64_t h, uint64_t mask) { return (h ^ (h >> 19)) & mask & 0xffffffffull; }
+__device__ inline unsigned long long hash_tag(uint64_t h) { return (unsigned long long)((h >> 32) | 1ull) << 32; }
 
 __device__ inline int rank_of(const EventRec &e) { return (e.meta >> 8) & 0xff; }
+
+// Sorted closed label (L points) of a record: the interior is sorted and
+// padded with kInvalid, each support point is bubbled in (static indices, the
+// label stays in registers).  members: bit q set when label[q] is a support
+// point; support ids ascend, so arm j drops the j-th of them.
+template <int L>
+__device__ inline void sorted_label(const EventRec &e, uint32_t (&a)[L], uint32_t &members) {
+#pragma unroll
+  for (int q = 0; q < L; ++q) a[q] = q < kMaxInterior ? e.interior[q] : kInvalid;
+  uint32_t sup[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    sup[i] = e.ids[i];
+    uint32_t x = sup[i];
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      const uint32_t lo = min(a[q], x);
+      x = max(a[q], x);
+      a[q] = lo;
+    }
+  }
+  members = 0;
+#pragma unroll
+  for (int q = 0; q < L; ++q) {
+    bool in = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) in |= a[q] == sup[i];
+    members |= (uint32_t)(in && a[q] != kInvalid) << q;
+  }
+}
+
+// Position of the j-th set bit.
+__device__ inline int nth_bit(uint32_t m, int j) {
+  for (int i = 0; i < j; ++i) m &= m - 1;
+  return __ffs(m) - 1;
+}
+
+// Slots of this thread in a global append list, count of them per thread:
+// one atomic per workgroup (a single counter takes about 10 ns per atomic, so
+// one per wave bound the kernels below).  Every thread of the workgroup calls.
+template <int WAVES>
+__device__ inline unsigned long long block_append(uint32_t count, unsigned long long *counter) {
+  __shared__ uint32_t tot[WAVES];
+  __shared__ unsigned long long base;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t x = count;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, (unsigned)d);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) tot[wave] = x;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    before += w < wave ? tot[w] : 0u;
+    all += tot[w];
+  }
+  if (threadIdx.x == 0 && all) base = atomicAdd(counter, (unsigned long long)all);
+  __syncthreads();
+  const unsigned long long at = all ? base + before + x - count : 0ull;
+  __syncthreads();  // the shared words serve the next call
+  return at;
+}
 
 // Records grouped by closed rank, canonical order kept inside each rank:
 // key = rank (0xff for a degenerate record), value = sorted position.
@@ -74,49 +130,586 @@ __global__ void k_rank_bounds(const uint64_t *__restrict__ keys, int64_t n, uint
   if (i == n - 1 || keys[i + 1] != key) hi[key] = (uint32_t)(i + 1);
 }
 
+// Minima of an order: labels (K ids each) and the hash table, whose slots
+// hold tag << 32 | minimum (0: empty).
+struct MinimaTable {
+  unsigned long long *slots;
+  uint64_t mask;
+  uint32_t *labels;
+};
+
+template <int K>
 __global__ void k_insert_minima(const EventRec *__restrict__ ev, const uint32_t *__restrict__ order,
-                                const uint32_t *__restrict__ pos, int64_t count, int k,
-                                uint32_t *labels, uint64_t *table_keys, uint32_t *table_vals,
-                                uint64_t mask) {
+                                const uint32_t *__restrict__ pos, int64_t count, MinimaTable T) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= count) return;
-  uint32_t lab[kMaxLabel];
-  int kk = event_label(ev[order[pos[i]]], lab);
-  for (int q = 0; q < k; ++q) labels[(size_t)i * k + q] = q < kk ? lab[q] : kInvalid;
-  uint64_t h = label_hash(lab, k);
-  uint64_t slot = h & mask;
-  while (true) {
-    unsigned long long prev = atomicCAS((unsigned long long *)&table_keys[slot], 0ull, (unsigned long long)h);
-    if (prev == 0ull) { table_vals[slot] = (uint32_t)i; return; }
-    slot = (slot + 1) & mask;
+  uint32_t lab[K], members;
+  sorted_label<K>(ev[order[pos[i]]], lab, members);
+  uint64_t h = 0;
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    T.labels[(size_t)i * K + q] = lab[q];
+    h += point_mix(lab[q]);
   }
+  uint64_t slot = hash_slot(h, T.mask);
+  const unsigned long long mine = hash_tag(h) | (unsigned long long)(uint32_t)i;
+  while (atomicCAS(&T.slots[slot], 0ull, mine) != 0ull) slot = (slot + 1) & T.mask;
 }
 
-__device__ int64_t lookup(const uint32_t *F, int k, const uint64_t *table_keys, const uint32_t *table_vals,
-                          uint64_t mask, const uint32_t *labels) {
-  uint64_t h = label_hash(F, k);
-  uint64_t slot = h & mask;
+// The minimum with facet F (sorted, hash h), or -1.
+template <int K>
+__device__ inline int64_t lookup(const MinimaTable &T, const uint32_t (&F)[K], uint64_t h) {
+  uint64_t slot = hash_slot(h, T.mask);
+  const unsigned long long tag = hash_tag(h);
   while (true) {
-    uint64_t key = table_keys[slot];
-    if (key == 0) return -1;
-    if (key == h) {
-      uint32_t v = ((volatile uint32_t *)table_vals)[slot];
+    const unsigned long long s = T.slots[slot];
+    if (s == 0ull) return -1;
+    if ((s & 0xffffffff00000000ull) == tag) {
+      const uint32_t v = (uint32_t)s;
       bool same = true;
-      for (int q = 0; q < k; ++q) same &= labels[(size_t)v * k + q] == F[q];
+#pragma unroll
+      for (int q = 0; q < K; ++q) same &= T.labels[(size_t)v * K + q] == F[q];
       if (same) return v;
     }
-    slot = (slot + 1) & mask;
+    slot = (slot + 1) & T.mask;
   }
 }
 
+// Saddles of an order, read once from their records: sorted labels (K + 1
+// ids), support members, arm counts, exact class and level.
+struct Saddles {
+  uint32_t *label;      // K + 1 per saddle
+  uint16_t *members;
+  uint32_t *base;       // first arm (after the scan of the arm counts)
+};
+
+template <int K>
+__global__ void k_saddles(const EventRec *__restrict__ ev, const uint32_t *__restrict__ order,
+                          const uint32_t *__restrict__ cls, const uint32_t *__restrict__ pos, int64_t count, Saddles D,
+                          uint32_t *sizes, uint32_t *out_cls, double *out_level) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= count) return;
+  const EventRec &e = ev[order[pos[i]]];
+  uint32_t lab[K + 1], members;
+  sorted_label<K + 1>(e, lab, members);
+#pragma unroll
+  for (int q = 0; q <= K; ++q) D.label[(size_t)i * (K + 1) + q] = lab[q];
+  D.members[i] = (uint16_t)members;
+  sizes[i] = e.meta & 0xff;
+  out_cls[i] = cls[pos[i]];
+  out_level[i] = e.level;
+}
+
+// Facet of an arm: the saddle's label without position `at`.
+template <int K>
+__device__ inline void drop_point(const uint32_t (&L)[K + 1], int at, uint32_t (&F)[K]) {
+#pragma unroll
+  for (int q = 0; q < K; ++q) F[q] = q < at ? L[q] : L[q + 1];
+}
+
+template <int K>
+__device__ inline void load_label(const Saddles &D, uint32_t s, uint32_t (&L)[K + 1]) {
+#pragma unroll
+  for (int q = 0; q <= K; ++q) L[q] = D.label[(size_t)s * (K + 1) + q];
+}
+
+struct ArmParams {
+  Saddles sad;
+  const uint32_t *sizes;       // inclusive scan of the arm counts
+  int64_t saddles;
+  MinimaTable table;
+  const double *X, *Y, *Z;
+  const WideNode *wide;
+  const double *LX, *LY, *LZ;
+  const uint32_t *leaf_id;
+  const uint32_t *leaf_pos;
+  uint32_t *carrier;  // per arm: minimum index, or kInvalid (host)
+  // nearest neighbours of every PointId (a row of kNearRow ids, nearest first,
+  // kInvalid past the list) and the FP64 squared distance to the last of them
+  // (infinite when the list holds every other point); nn == nullptr: none
+  const uint32_t *nn;
+  const double *nn_d2;
+};
+
+constexpr int kNearK = 63;    // a wave's neighbour list without its tie probe
+constexpr int kNearRow = 64;
+
+// Facets to descend, deduplicated: a slot holds tag << 32 | saddle << 2 | arm
+// of the saddle; an arm whose facet equals a stored one takes that arm's
+// carrier after the descents.  The probe length is bounded; an arm that finds
+// no slot simply descends itself.
+struct FacetSet {
+  unsigned long long *slots;
+  uint64_t mask;
+  uint32_t *alias_arm, *alias_rep;
+  unsigned long long *alias_count;
+};
+
+// One thread per saddle: each arm's facet is a minimum (hash hit), equals a
+// facet already claimed, or is queued for the descents (saddle << 2 | arm, with
+// the Morton position of its least point, so that the descents run in spatial
+// order).  Bound by the random reads of the tables; a thread per arm built
+// every label up to four times and its two appends per wave serialised on
+// their counters (order 10 of the
+// 50 000-point tower, 20.6 M arms: 6.9 ms, 2.1 here).
+constexpr int kArmBlock = 256;
+template <int K>
+__global__ void __launch_bounds__(kArmBlock) k_arm_lookup(ArmParams A, FacetSet D, uint32_t *queue, uint64_t *qkey,
+                                                          unsigned long long *qcount) {
+  const int64_t s = (int64_t)blockIdx.x * kArmBlock + threadIdx.x;
+  uint32_t ndesc = 0, nalias = 0, desc = 0, rep[4] = {}, key[4] = {}, base = 0;
+  uint32_t alias = 0;
+  if (s < A.saddles) {
+    base = A.sad.base[s];
+    uint32_t L[K + 1];
+    load_label<K>(A.sad, (uint32_t)s, L);
+    const uint32_t members = A.sad.members[s];
+    uint64_t whole = 0;
+#pragma unroll
+    for (int q = 0; q <= K; ++q) whole += point_mix(L[q]);
+    uint32_t left = members;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (!left) continue;
+      const int at = __ffs(left) - 1;
+      left &= left - 1;
+      uint32_t F[K];
+      drop_point<K>(L, at, F);
+      if (K == 1) {  // order one: the arm is a point, its own minimum
+        A.carrier[base + j] = F[0];
+        continue;
+      }
+      uint32_t gone = L[0];
+#pragma unroll
+      for (int q = 1; q <= K; ++q) gone = q == at ? L[q] : gone;
+      const uint64_t h = whole - point_mix(gone);
+      const int64_t hit = lookup<K>(A.table, F, h);
+      A.carrier[base + j] = hit >= 0 ? (uint32_t)hit : kInvalid;
+      if (hit >= 0) continue;
+      // claim the facet
+      const unsigned long long tag = hash_tag(h), mine = tag | (unsigned long long)((uint32_t)s << 2 | (uint32_t)j);
+      uint64_t slot = hash_slot(h, D.mask);
+      bool same = false;
+      uint32_t other = 0;
+      for (int probe = 0; probe < 64; ++probe) {
+        const unsigned long long cur = atomicCAS(&D.slots[slot], 0ull, mine);
+        if (cur == 0ull) break;
+        if ((cur & 0xffffffff00000000ull) == tag) {
+          other = (uint32_t)cur;
+          uint32_t M[K + 1], G[K];
+          load_label<K>(A.sad, other >> 2, M);
+          drop_point<K>(M, nth_bit(A.sad.members[other >> 2], (int)(other & 3u)), G);
+          same = true;
+#pragma unroll
+          for (int q = 0; q < K; ++q) same &= G[q] == F[q];
+          if (same) break;
+        }
+        slot = (slot + 1) & D.mask;
+      }
+      if (same) {
+        alias |= 1u << j;
+        rep[j] = A.sad.base[other >> 2] + (other & 3u);
+        nalias++;
+      } else {
+        desc |= 1u << j;
+        key[j] = A.leaf_pos[F[0]];
+        ndesc++;
+      }
+    }
+  }
+  if (K == 1) return;
+  unsigned long long ai = block_append<kArmBlock / 64>(nalias, D.alias_count);
+  unsigned long long di = block_append<kArmBlock / 64>(ndesc, qcount);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if ((alias >> j) & 1u) {
+      D.alias_arm[ai] = base + j;
+      D.alias_rep[ai] = rep[j];
+      ai++;
+    }
+    if ((desc >> j) & 1u) {
+      queue[di] = (uint32_t)s << 2 | (uint32_t)j;
+      qkey[di] = key[j];
+      di++;
+    }
+  }
+}
+
+__global__ void k_alias_carriers(const uint32_t *__restrict__ alias_arm, const uint32_t *__restrict__ alias_rep,
+                                 uint64_t count, uint32_t *carrier) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) carrier[alias_arm[i]] = carrier[alias_rep[i]];
+}
+
+__device__ inline V3 P3(const double *X, const double *Y, const double *Z, uint32_t id) { return {X[id], Y[id], Z[id]}; }
+
+// Sphere of a miniball support (2..4 points) in one form for every size: the
+// scaled power a p.p - p.b of a point relative to the first support point, with
+// its magnitude bound (predicates.hpp), and the centre.
+struct SupSphere {
+  double a, aA;
+  V3 b, bA;
+  V3 off;  // centre relative to the first support point
+  // certified well-centred support of m points (relative to the first)
+  __device__ bool init(int m, const V3 &p1, const V3 &p2, const V3 &p3) {
+    if (m == 2) {
+      a = aA = 1.0;
+      b = p1;
+      bA = vabs(p1);
+      if (!(dot(p1, p1) > 0)) return false;
+    } else if (m == 3) {
+      TriSphere t;
+      if (t.init(p1, p2) <= 0) return false;
+      a = t.D;
+      aA = t.DA;
+      b = t.g;
+      bA = t.gA;
+    } else if (m == 4) {
+      TetSphere t;
+      if (t.init(p1, p2, p3) <= 0) return false;
+      a = t.V;
+      aA = t.VA;
+      b = t.N;
+      bA = t.NA;
+    } else {
+      return false;
+    }
+    const double h = 0.5 / a;
+    off = {b.x * h, b.y * h, b.z * h};
+    return true;
+  }
+  // certified position of a point relative to the first support point
+  __device__ int side(const V3 &p) const {
+    const double pp = dot(p, p);
+    const int s = cert_sign(a * pp - dot(p, b), aA * pp + dot(vabs(p), bA));
+    return a > 0 ? s : -s;
+  }
+};
+
+// Support of the smallest ball holding K points, by walking a centre: T are
+// points on the ball's boundary; the centre moves towards its projection onto
+// their affine hull (the ball shrinks) until another point is met, which joins
+// T, or the projection is reached; there the point of T with the most negative
+// barycentric coordinate leaves, and without one the ball is the smallest.
+// Every lane does the same work per move, unlike Welzl's nested restarts.
+// FP32: the result is a proposal, certified in FP64 by the caller.  Returns the
+// size of the support (positions in at[]), 0 when the walk does not settle.
+template <int K>
+__device__ inline int walk_miniball(const float (&x)[K], const float (&y)[K], const float (&z)[K], int (&at)[4]) {
+  float cx = 0.f, cy = 0.f, cz = 0.f;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    cx += x[i];
+    cy += y[i];
+    cz += z[i];
+  }
+  cx *= 1.0f / K;
+  cy *= 1.0f / K;
+  cz *= 1.0f / K;
+  float far = -1.f;
+  float tx[4] = {}, ty[4] = {}, tz[4] = {};
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const float dx = x[i] - cx, dy = y[i] - cy, dz = z[i] - cz, d = dx * dx + dy * dy + dz * dz;
+    const bool take = d > far;
+    far = take ? d : far;
+    at[0] = take ? i : at[0];
+    tx[0] = take ? x[i] : tx[0];
+    ty[0] = take ? y[i] : ty[0];
+    tz[0] = take ? z[i] : tz[0];
+  }
+  int m = 1;
+  uint32_t in = 1u << at[0];
+#pragma unroll 1
+  for (int it = 0; it < 24; ++it) {
+    const float wx = cx - tx[0], wy = cy - ty[0], wz = cz - tz[0];
+    float la = 0.f, lb = 0.f, lc = 0.f;
+    const float ux = tx[1] - tx[0], uy = ty[1] - ty[0], uz = tz[1] - tz[0];
+    const float vx = tx[2] - tx[0], vy = ty[2] - ty[0], vz = tz[2] - tz[0];
+    float qx = tx[0], qy = ty[0], qz = tz[0];
+    if (m == 2) {
+      la = (wx * ux + wy * uy + wz * uz) * __builtin_amdgcn_rcpf(ux * ux + uy * uy + uz * uz);
+    } else if (m >= 3) {
+      // solved with the normal of the first three points
+      const float nx = uy * vz - uz * vy, ny = uz * vx - ux * vz, nz = ux * vy - uy * vx;
+      if (m == 3) {
+        const float in2 = __builtin_amdgcn_rcpf(nx * nx + ny * ny + nz * nz);
+        // w x v . n and u x w . n
+        la = ((wy * vz - wz * vy) * nx + (wz * vx - wx * vz) * ny + (wx * vy - wy * vx) * nz) * in2;
+        lb = ((uy * wz - uz * wy) * nx + (uz * wx - ux * wz) * ny + (ux * wy - uy * wx) * nz) * in2;
+      } else {
+        const float ex = tx[3] - tx[0], ey = ty[3] - ty[0], ez = tz[3] - tz[0];
+        const float id = __builtin_amdgcn_rcpf(ex * nx + ey * ny + ez * nz);
+        lc = (wx * nx + wy * ny + wz * nz) * id;
+        const float rx = wx - lc * ex, ry = wy - lc * ey, rz = wz - lc * ez;
+        const float in2 = __builtin_amdgcn_rcpf(nx * nx + ny * ny + nz * nz);
+        la = ((ry * vz - rz * vy) * nx + (rz * vx - rx * vz) * ny + (rx * vy - ry * vx) * nz) * in2;
+        lb = ((uy * rz - uz * ry) * nx + (uz * rx - ux * rz) * ny + (ux * ry - uy * rx) * nz) * in2;
+      }
+    }
+    float step = 1.0f;
+    int hit = -1;
+    float hx = 0.f, hy = 0.f, hz = 0.f;
+    if (m < 4) {
+      qx += la * ux + lb * vx;
+      qy += la * uy + lb * vy;
+      qz += la * uz + lb * vz;
+      const float dx = qx - cx, dy = qy - cy, dz = qz - cz;
+      const float ww = wx * wx + wy * wy + wz * wz;
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        const float px = cx - x[i], py = cy - y[i], pz = cz - z[i];
+        // 2 d . (t0 - p), the rate at which p nears the boundary
+        const float rate = 2.0f * (dx * (px - wx) + dy * (py - wy) + dz * (pz - wz));
+        const float gap = ww - (px * px + py * py + pz * pz);
+        const float t = fmaxf(gap, 0.0f) * __builtin_amdgcn_rcpf(rate);
+        const bool take = rate > 0.0f && t < step && !((in >> i) & 1u);
+        step = take ? t : step;
+        hit = take ? i : hit;
+        hx = take ? x[i] : hx;
+        hy = take ? y[i] : hy;
+        hz = take ? z[i] : hz;
+      }
+      cx += step * dx;
+      cy += step * dy;
+      cz += step * dz;
+    }
+    if (hit >= 0) {
+#pragma unroll
+      for (int q = 1; q < 4; ++q) {
+        const bool here = q == m;
+        tx[q] = here ? hx : tx[q];
+        ty[q] = here ? hy : ty[q];
+        tz[q] = here ? hz : tz[q];
+        at[q] = here ? hit : at[q];
+      }
+      in |= 1u << hit;
+      m++;
+      continue;
+    }
+    const float l[4] = {1.0f - la - lb - lc, la, lb, lc};
+    float least = -1e-5f;
+    int out = -1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool take = q < m && l[q] < least;
+      least = take ? l[q] : least;
+      out = take ? q : out;
+    }
+    if (out < 0) return m;
+    // the last of T takes the place of the one that leaves
+    float ex = tx[0], ey = ty[0], ez = tz[0];
+    int ei = at[0], oi = at[0];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      const bool last = q == m - 1;
+      ex = last ? tx[q] : ex;
+      ey = last ? ty[q] : ey;
+      ez = last ? tz[q] : ez;
+      ei = last ? at[q] : ei;
+      oi = q == out ? at[q] : oi;
+    }
+    in &= ~(1u << oi);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool here = q == out;
+      tx[q] = here ? ex : tx[q];
+      ty[q] = here ? ey : ty[q];
+      tz[q] = here ? ez : tz[q];
+      at[q] = here ? ei : at[q];
+    }
+    m--;
+  }
+  return 0;
+}
+
+// Descents advance one or more steps per round for every arm still
+// descending.  Item state lives in SoA arrays of capacity cap: facet ids
+// F[q * cap + i] (sorted, not a minimum) and origin arm.
+struct DescentItems {
+  uint32_t *F, *origin;
+  uint64_t cap;
+};
+// counters of a round
+enum { D_OUT = 0, D_SLOW = 1, D_STEPS = 2 };
+
+// One descent step of facet F (sorted ids): F := F - y + x, where x is the
+// least point strictly inside the facet's miniball and y its least support
+// point (the miniball strictly shrinks).  Points inside come from the
+// neighbour list of the facet point nearest the centre: every point of the
+// ball lies within sqrt(R2) + |c - f| of f, so the list holds them all when
+// that radius stays below the distance to its last entry (with margins far
+// above the FP64 rounding), and its walk ends at the first entry beyond it.
+// False: the certified filters or the list cannot decide the step.
+template <int K>
+__device__ inline bool descent_step(const ArmParams &A, uint32_t (&F)[K]) {
+  int at[4] = {0, 0, 0, 0};
+  int m;
+  {
+    const V3 o = P3(A.X, A.Y, A.Z, F[0]);
+    float x[K], y[K], z[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const V3 p = sub(P3(A.X, A.Y, A.Z, F[i]), o);
+      x[i] = (float)p.x;
+      y[i] = (float)p.y;
+      z[i] = (float)p.z;
+    }
+    m = walk_miniball<K>(x, y, z, at);
+  }
+  if (m < 2) return false;
+  uint32_t sid[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sid[j] = F[0];
+#pragma unroll
+    for (int i = 1; i < K; ++i) sid[j] = at[j] == i ? F[i] : sid[j];
+    if (j >= m) sid[j] = kInvalid;
+  }
+  const V3 o = P3(A.X, A.Y, A.Z, sid[0]);
+  const V3 p1 = sub(P3(A.X, A.Y, A.Z, sid[1]), o);
+  const V3 p2 = m > 2 ? sub(P3(A.X, A.Y, A.Z, sid[2]), o) : p1;
+  const V3 p3 = m > 3 ? sub(P3(A.X, A.Y, A.Z, sid[3]), o) : p1;
+  SupSphere S;
+  if (!S.init(m, p1, p2, p3)) return false;
+  // every facet point must be certainly inside, or a support point
+  bool ok = true;
+  double best = INFINITY;
+  uint32_t f = F[0];
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const V3 p = sub(P3(A.X, A.Y, A.Z, F[i]), o);
+    bool on = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) on |= sid[j] == F[i];
+    ok = ok && (on || S.side(p) < 0);
+    const V3 d = sub(p, S.off);
+    const double d2 = dot(d, d);
+    f = d2 < best ? F[i] : f;
+    best = fmin(best, d2);
+  }
+  if (!ok || !A.nn) return false;
+  const double R2 = dot(S.off, S.off) * (1.0 + 1e-9) + 1e-300;
+  const double rho = (sqrt(R2) + sqrt(best)) * (1.0 + 1e-9) + 1e-150, rho2 = rho * rho;
+  if (!(rho2 < A.nn_d2[f] * (1.0 - 1e-9))) return false;
+  uint32_t xin = kInvalid;
+  bool undecided = false;
+  const V3 pf = sub(P3(A.X, A.Y, A.Z, f), o);
+  const uint4 *row = reinterpret_cast<const uint4 *>(A.nn + (size_t)f * kNearRow);
+  bool more = true;
+#pragma unroll 1
+  for (int j = 0; more && j < kNearRow / 4; ++j) {
+    const uint4 r = row[j];
+    const uint32_t id4[4] = {r.x, r.y, r.z, r.w};
+    V3 p4[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p4[q] = sub(P3(A.X, A.Y, A.Z, id4[q] == kInvalid ? f : id4[q]), o);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t id = id4[q];
+      const V3 e = sub(p4[q], pf), d = sub(p4[q], S.off);
+      more = more && id != kInvalid && !(dot(e, e) > rho2 * (1.0 + 1e-9));  // ascending from here on
+      if (id == kInvalid || dot(d, d) > R2) continue;
+      bool member = false;
+#pragma unroll
+      for (int i = 0; i < K; ++i) member |= F[i] == id;
+      if (member) continue;
+      const int sd = S.side(p4[q]);
+      xin = sd < 0 ? min(xin, id) : xin;
+      undecided |= sd == 0;
+    }
+  }
+  if (undecided || xin == kInvalid) return false;
+  uint32_t y = sid[0];
+#pragma unroll
+  for (int j = 1; j < 4; ++j) y = min(y, sid[j]);
+  // F - y + xin, kept sorted: close the gap, bubble xin in
+  bool gone = false;
+#pragma unroll
+  for (int q = 0; q + 1 < K; ++q) {
+    gone |= F[q] == y;
+    F[q] = gone ? F[q + 1] : F[q];
+  }
+  F[K - 1] = kInvalid;
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    const uint32_t lo = min(F[q], xin);
+    xin = max(F[q], xin);
+    F[q] = lo;
+  }
+  return true;
+}
+
+// One round of the descents: up to `steps` steps per item, each followed by
+// the lookup of the new facet; what still descends goes to `out`, what the
+// step leaves open to `slow`.  queue != nullptr: the first round, whose items
+// are queued arms.  Bound by the gathers of the neighbours' coordinates and
+// the FP64 predicates; Welzl's miniball and a tree traversal per step, with
+// the facet in scratch memory, took 66 ms of the 50 000-point tower at 0.22
+// lane utilisation (order 10: 28 ms, 7 here).
+constexpr int kDescentBlock = 256;
+template <int K>
+__global__ void __launch_bounds__(kDescentBlock) k_descend(ArmParams A, const uint32_t *queue, DescentItems in,
+                                                           uint32_t n_in, DescentItems out, DescentItems slow,
+                                                           int steps, unsigned long long *counters) {
+  const uint64_t i = (uint64_t)blockIdx.x * kDescentBlock + threadIdx.x;
+  bool next = false, open = false;
+  uint32_t F[K], origin = 0, done = 0;
+  if (i < n_in) {
+    if (queue) {
+      const uint32_t code = queue[i], s = code >> 2;
+      uint32_t L[K + 1];
+      load_label<K>(A.sad, s, L);
+      drop_point<K>(L, nth_bit(A.sad.members[s], (int)(code & 3u)), F);
+      origin = A.sad.base[s] + (code & 3u);
+    } else {
+      origin = in.origin[i];
+#pragma unroll
+      for (int q = 0; q < K; ++q) F[q] = in.F[q * in.cap + i];
+    }
+    next = true;
+#pragma unroll 1
+    for (int t = 0; next && t < steps; ++t) {
+      if (!descent_step<K>(A, F)) {
+        next = false;
+        open = true;
+        break;
+      }
+      done++;
+      uint64_t h = 0;
+#pragma unroll
+      for (int q = 0; q < K; ++q) h += point_mix(F[q]);
+      const int64_t hit = lookup<K>(A.table, F, h);
+      if (hit >= 0) {
+        A.carrier[origin] = (uint32_t)hit;
+        next = false;
+      }
+    }
+  }
+  const unsigned long long at = block_append<kDescentBlock / 64>(next ? 1u : 0u, counters + D_OUT);
+  if (next) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) out.F[q * out.cap + at] = F[q];
+    out.origin[at] = origin;
+  }
+  (void)block_append<kDescentBlock / 64>(done, counters + D_STEPS);
+  const unsigned long long sl = block_append<kDescentBlock / 64>(open ? 1u : 0u, counters + D_SLOW);
+  if (open) {
+#pragma unroll
+    for (int q = 0; q < K; ++q) slow.F[q * slow.cap + sl] = F[q];
+    slow.origin[sl] = origin;
+  }
+}
+
+// The steps the fast path leaves open, one thread each with the facet in
+// scratch memory: Welzl's miniball in FP64, certified containment, and an LBVH
+// ball query for the points inside.
 struct Ball {
   V3 c;
   double r2;
   int m;
   uint32_t sup[4];  // indices into the facet
 };
-
-__device__ inline V3 P3(const double *X, const double *Y, const double *Z, uint32_t id) { return {X[id], Y[id], Z[id]}; }
 
 // circumball of 0..4 facet points with centre in their affine hull (FP64);
 // point i of the facet is pts[i * stride]
@@ -192,7 +785,7 @@ __device__ bool welzl(const V3 *pts, int stride, int n, Ball &out) {
 // Sphere of a miniball support (1..4 canonical ids), built once per descent
 // step; side() is the certified position of a point (0: on a support point
 // or undecided, which sends the arm to the host).
-struct SupSphere {
+struct SlowSphere {
   int m;
   uint32_t sid[4];
   V3 o;
@@ -223,151 +816,13 @@ struct SupSphere {
   }
 };
 
-struct ArmParams {
-  const EventRec *ev;
-  const uint32_t *order;
-  const uint32_t *saddle_pos;  // sorted positions of the saddles of this order
-  const uint32_t *arm_base;    // first arm of each saddle (exclusive scan of sizes)
-  const uint32_t *arm_saddle;  // saddle of each arm
-  int64_t arms;
-  int k;
-  const uint64_t *table_keys;
-  const uint32_t *table_vals;
-  uint64_t mask;
-  const uint32_t *labels;
-  const double *X, *Y, *Z;
-  const WideNode *wide;
-  const double *LX, *LY, *LZ;
-  const uint32_t *leaf_id;
-  const uint32_t *leaf_pos;
-  int64_t n;
-  uint32_t *carrier;  // per arm: minimum index, or kInvalid (host)
-  unsigned long long *steps;
-  // nearest neighbours of every PointId (kNearK ids, nearest first) and the
-  // FP64 squared distance to the last of them; nn == nullptr: none
-  const uint32_t *nn;
-  const double *nn_d2;
-};
-
-constexpr int kNearK = 32;
-
-constexpr int kArmBlock = 64;
-constexpr int kArmStack = 40;  // LBVH depth is 18 at 50k points, 32 at 200k; overflow goes to the host
-
-// Facet of an arm: the saddle's closed label without the arm's shell point.
-// hint (optional) receives the saddle's other shell points, kInvalid padded:
-// the likely support of the facet's miniball.
-__device__ inline void arm_facet(const ArmParams &A, int64_t arm, uint32_t *F, uint32_t *hint = nullptr) {
-  const uint32_t s = A.arm_saddle[arm];
-  const int j = (int)(arm - A.arm_base[s]);
-  const EventRec &e = A.ev[A.order[A.saddle_pos[s]]];
-  uint32_t L[kMaxLabel];
-  const int len = event_label(e, L);
-  int f = 0;
-  for (int i = 0; i < len; ++i)
-    if (L[i] != e.ids[j]) F[f++] = L[i];
-  if (hint) {
-    const int m = e.meta & 0xff;
-    int h = 0;
-    for (int q = 0; q < m; ++q)
-      if (q != j) hint[h++] = e.ids[q];
-    while (h < 4) hint[h++] = kInvalid;
-  }
-}
-
-// Facets to descend, deduplicated: a slot holds (32 hash bits | 1) << 32 |
-// arm; an arm whose facet equals a stored arm's takes that arm's carrier
-// after the descents.  The probe length is bounded; an arm that finds no slot
-// simply descends itself.
-struct FacetSet {
-  unsigned long long *slots;
-  uint64_t mask;
-  uint32_t *alias_arm, *alias_rep;
-  unsigned long long *alias_count;
-};
-
-__device__ inline bool same_facet(const ArmParams &A, int64_t other, const uint32_t *F) {
-  uint32_t G[kMaxLabel];
-  arm_facet(A, other, G);
-  bool same = true;
-  for (int q = 0; q < A.k; ++q) same &= G[q] == F[q];
-  return same;
-}
-
-// Returns the arm already holding this facet, or -1 (this arm descends).
-__device__ inline int64_t facet_claim(const ArmParams &A, const FacetSet &D, int64_t arm, const uint32_t *F) {
-  const uint64_t h = label_hash(F, A.k);
-  const unsigned long long tag = ((h >> 32) | 1ull) << 32;
-  const unsigned long long mine = tag | (unsigned long long)(uint32_t)arm;
-  uint64_t slot = h & D.mask;
-  for (int probe = 0; probe < 64; ++probe) {
-    unsigned long long cur = atomicCAS(&D.slots[slot], 0ull, mine);
-    if (cur == 0ull) return -1;
-    if ((cur & 0xffffffff00000000ull) == tag) {
-      const int64_t other = (int64_t)(cur & 0xffffffffull);
-      if (same_facet(A, other, F)) return other;
-    }
-    slot = (slot + 1) & D.mask;
-  }
-  return -1;
-}
-
-// One thread per strict arm: the facet is a minimum (hash hit) or the arm
-// is queued for descents (once per distinct facet).  Splitting the two keeps
-// the descending lanes of a wave together.  Queued arms carry the Morton
-// position of their facet's least point, so the descents can run in spatial
-// order.
-__global__ void k_arm_lookup(ArmParams A, FacetSet D, uint32_t *queue, uint64_t *qkey,
-                             unsigned long long *qcount) {
-  const int64_t arm = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool descend = false, aliased = false;
-  int64_t rep = -1;
-  uint32_t F[kMaxLabel];
-  if (arm < A.arms) {
-    arm_facet(A, arm, F);
-    if (A.k == 1) {  // order one: the arm is a point, its own minimum
-      A.carrier[arm] = F[0];
-    } else {
-      const int64_t hit = lookup(F, A.k, A.table_keys, A.table_vals, A.mask, A.labels);
-      A.carrier[arm] = hit >= 0 ? (uint32_t)hit : kInvalid;
-      if (hit < 0) {
-        rep = facet_claim(A, D, arm, F);
-        aliased = rep >= 0;
-        descend = !aliased;
-      }
-    }
-  }
-  const unsigned long long ai = wave_append(aliased, D.alias_count);
-  if (aliased) {
-    D.alias_arm[ai] = (uint32_t)arm;
-    D.alias_rep[ai] = (uint32_t)rep;
-  }
-  // wave-aggregated append to the descent queue
-  const uint64_t mask = __ballot(descend);
-  if (!mask) return;
-  const int lane = (int)(threadIdx.x & 63u);
-  const int leader = __ffsll((unsigned long long)mask) - 1;
-  unsigned long long at = 0;
-  if (lane == leader) at = atomicAdd(qcount, (unsigned long long)__popcll(mask));
-  at = __shfl(at, leader);
-  if (descend) {
-    const unsigned long long pos = at + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull));
-    queue[pos] = (uint32_t)arm;
-    qkey[pos] = A.leaf_pos[F[0]];
-  }
-}
-
-__global__ void k_alias_carriers(const uint32_t *__restrict__ alias_arm, const uint32_t *__restrict__ alias_rep,
-                                 uint64_t count, uint32_t *carrier) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) carrier[alias_arm[i]] = carrier[alias_rep[i]];
-}
+constexpr int kSlowBlock = 64;
+constexpr int kSlowStack = 40;  // LBVH depth is 18 at 50k points, 32 at 200k; overflow goes to the host
 
 // Trade the miniball's least support point for the least point strictly
 // inside; false leaves the arm to the host (shell points, or no point inside:
 // a minimum missing from the table).
-__device__ bool finish_step(const Ball &b, const uint32_t *sid, int k, uint32_t *F, uint32_t *hint, uint32_t xin,
-                            bool undecided) {
+__device__ bool finish_step(const Ball &b, const uint32_t *sid, int k, uint32_t *F, uint32_t xin, bool undecided) {
   if (undecided || xin == kInvalid) return false;
   uint32_t y = sid[0];
   for (int i = 1; i < b.m; ++i) y = min(y, sid[i]);
@@ -382,42 +837,19 @@ __device__ bool finish_step(const Ball &b, const uint32_t *sid, int k, uint32_t 
   }
   if (!placed) G[w++] = xin;
   for (int i = 0; i < k; ++i) F[i] = G[i];
-  // the next miniball's likely support: this one's, y traded for xin
-  for (int h = 0; h < 4; ++h) hint[h] = h < b.m ? (sid[h] == y ? xin : sid[h]) : kInvalid;
   return true;
 }
 
-// One descent step of facet F (sorted ids) with the likely support hint:
-// F := F - y + x, where x is the least point strictly inside the facet's
-// miniball and y its least support point.  false: the certified filters
-// cannot decide the step (the host descends the arm).  stk is the lane's
-// traversal stack in LDS (stride kArmBlock).
-__device__ bool descent_step(const ArmParams &A, uint32_t *F, uint32_t *hint, uint32_t *stk, int lane) {
-  const int k = A.k;
-  // miniball of the facet; the likely support goes first, so that Welzl's
-  // outer loop mostly meets points already inside
-  uint32_t ord[kMaxLabel];
-  int no = 0;
-  for (int h = 0; h < 4; ++h) {
-    bool in = hint[h] != kInvalid;
-    if (in) {
-      in = false;
-      for (int i = 0; i < k; ++i) in |= F[i] == hint[h];
-    }
-    if (in) ord[no++] = hint[h];
-  }
-  for (int i = 0; i < k; ++i) {
-    bool hinted = false;
-    for (int h = 0; h < 4; ++h) hinted |= hint[h] == F[i];
-    if (!hinted) ord[no++] = F[i];
-  }
+// stk is the lane's traversal stack in LDS (stride kSlowBlock).  False: the
+// certified filters cannot decide the step (the host descends the arm).
+__device__ bool slow_step(const ArmParams &A, int k, uint32_t *F, uint32_t *stk, int lane) {
   V3 pts[kMaxLabel];
-  for (int i = 0; i < k; ++i) pts[i] = P3(A.X, A.Y, A.Z, ord[i]);
+  for (int i = 0; i < k; ++i) pts[i] = P3(A.X, A.Y, A.Z, F[i]);
   Ball b;
   if (!welzl(pts, 1, k, b)) return false;
   uint32_t sid[4];
-  for (int i = 0; i < b.m; ++i) sid[i] = ord[b.sup[i]];
-  SupSphere S;
+  for (int i = 0; i < b.m; ++i) sid[i] = F[b.sup[i]];
+  SlowSphere S;
   if (S.init(A.X, A.Y, A.Z, sid, b.m) <= 0) return false;
   // every facet point must be certainly inside, or a support point
   bool ok = true;
@@ -432,34 +864,6 @@ __device__ bool descent_step(const ArmParams &A, uint32_t *F, uint32_t *hint, ui
   bool undecided = false;
   const double q[3] = {b.c.x, b.c.y, b.c.z};
   const double R2 = b.r2 * (1.0 + 1e-9) + 1e-300;
-  if (A.nn) {
-    // every point of the ball lies within sqrt(R2) + |c - f| of a facet point
-    // f; when that radius stays below the distance to f's last listed
-    // neighbour, f's neighbour list holds all of them and replaces the
-    // traversal (with margins far above the FP64 rounding)
-    uint32_t f = F[0];
-    double best = INFINITY;
-    for (int i = 0; i < k; ++i) {
-      const double dx = A.X[F[i]] - q[0], dy = A.Y[F[i]] - q[1], dz = A.Z[F[i]] - q[2];
-      const double d2 = dx * dx + dy * dy + dz * dz;
-      if (d2 < best) { best = d2; f = F[i]; }
-    }
-    const double rho = (sqrt(R2) + sqrt(best)) * (1.0 + 1e-9) + 1e-150;
-    if (rho * rho < A.nn_d2[f] * (1.0 - 1e-9)) {
-      for (int j = 0; j < kNearK && !undecided; ++j) {
-        const uint32_t id = A.nn[(size_t)f * kNearK + j];
-        const double dx = A.X[id] - q[0], dy = A.Y[id] - q[1], dz = A.Z[id] - q[2];
-        if (dx * dx + dy * dy + dz * dz > R2) continue;
-        bool inF = false;
-        for (int i = 0; i < k; ++i) inF |= F[i] == id;
-        if (inF) continue;
-        const int sd = S.side(A.X, A.Y, A.Z, id);
-        if (sd < 0) xin = min(xin, id);
-        else if (sd == 0) undecided = true;
-      }
-      return finish_step(b, sid, k, F, hint, xin, undecided);
-    }
-  }
   // FP32 pruning against outward-rounded child boxes: the radius is
   // inflated by the rounding of the query point and of the FP32 arithmetic
   // (a non-finite bound prunes nothing)
@@ -472,7 +876,7 @@ __device__ bool descent_step(const ArmParams &A, uint32_t *F, uint32_t *hint, ui
   stk[lane] = 0;
   sp = 1;
   while (sp && !undecided) {
-    const WideNode &N = A.wide[stk[(--sp) * kArmBlock + lane]];
+    const WideNode &N = A.wide[stk[(--sp) * kSlowBlock + lane]];
     for (int c = 0; c < 4; ++c) {
       float d2 = 0.f;
       for (int a = 0; a < 3; ++a) {
@@ -492,84 +896,57 @@ __device__ bool descent_step(const ArmParams &A, uint32_t *F, uint32_t *hint, ui
         const int sd = S.side(A.X, A.Y, A.Z, id);
         if (sd < 0) xin = min(xin, id);
         else if (sd == 0) undecided = true;
-      } else if (sp < kArmStack) {
-        stk[(sp++) * kArmBlock + lane] = x;
+      } else if (sp < kSlowStack) {
+        stk[(sp++) * kSlowBlock + lane] = x;
       } else {
         undecided = true;
       }
     }
   }
-  return finish_step(b, sid, k, F, hint, xin, undecided);
+  return finish_step(b, sid, k, F, xin, undecided);
 }
 
-// Descents advance one step per round for every arm still descending, so the
-// lanes of a wave do equal work.  Item state lives in SoA arrays of
-// capacity cap: facet ids F[q * cap + i], hint H[h * cap + i], origin arm.
-struct DescentItems {
-  uint32_t *F, *H, *origin;
-  uint64_t cap;
-};
-
-// Round 0 takes the queued arms (their facets are not minima); later rounds
-// first look their facet up among the minima.
-__global__ void __launch_bounds__(kArmBlock) k_descend_round(ArmParams A, int round, const uint32_t *queue,
-                                                             DescentItems in, uint32_t n_in, DescentItems out,
-                                                             unsigned long long *n_out) {
-  __shared__ uint32_t stk[kArmStack * kArmBlock];
+template <int K>
+__global__ void __launch_bounds__(kSlowBlock) k_descend_slow(ArmParams A, DescentItems in, uint32_t n_in,
+                                                             DescentItems out, unsigned long long *counters) {
+  __shared__ uint32_t stk[kSlowStack * kSlowBlock];
   const int lane = threadIdx.x;
-  const uint64_t i = (uint64_t)blockIdx.x * kArmBlock + lane;
-  const int k = A.k;
-  bool next = false;
-  uint32_t F[kMaxLabel], hint[4], origin = 0;
+  const uint64_t i = (uint64_t)blockIdx.x * kSlowBlock + lane;
+  bool next = false, stepped = false;
+  uint32_t origin = 0, F[K];
   if (i < n_in) {
-    if (round == 0) {
-      origin = queue[i];
-      arm_facet(A, origin, F, hint);
+    origin = in.origin[i];
+    uint32_t G[K];
+    for (int q = 0; q < K; ++q) G[q] = in.F[q * in.cap + i];
+    stepped = slow_step(A, K, G, stk, lane);
+    if (stepped) {
+      uint64_t h = 0;
+      for (int q = 0; q < K; ++q) {
+        F[q] = G[q];
+        h += point_mix(F[q]);
+      }
+      const int64_t hit = lookup<K>(A.table, F, h);
+      if (hit >= 0) A.carrier[origin] = (uint32_t)hit;
+      else next = true;
     } else {
-      origin = in.origin[i];
-      for (int q = 0; q < k; ++q) F[q] = in.F[q * in.cap + i];
-      for (int h = 0; h < 4; ++h) hint[h] = in.H[h * in.cap + i];
-    }
-    int64_t hit = -1;
-    if (round > 0) hit = lookup(F, k, A.table_keys, A.table_vals, A.mask, A.labels);
-    if (hit >= 0) {
-      A.carrier[origin] = (uint32_t)hit;
-    } else if (round >= 4096 || !descent_step(A, F, hint, stk, lane)) {
       A.carrier[origin] = kInvalid;  // the host descends this arm
-    } else {
-      next = true;
     }
   }
-  const unsigned long long at = wave_append(next, n_out);
+  const unsigned long long at = wave_append(next, counters + D_OUT);
   if (next) {
-    for (int q = 0; q < k; ++q) out.F[q * out.cap + at] = F[q];
-    for (int h = 0; h < 4; ++h) out.H[h * out.cap + at] = hint[h];
+    for (int q = 0; q < K; ++q) out.F[q * out.cap + at] = F[q];
     out.origin[at] = origin;
   }
+  (void)wave_append(stepped, counters + D_STEPS);
 }
 
-__global__ void k_arm_owner(const uint32_t *__restrict__ base, const uint32_t *__restrict__ sizes_incl,
+__global__ void k_arm_owner(uint32_t *__restrict__ base, const uint32_t *__restrict__ sizes_incl,
                             int64_t count, uint32_t *arm_saddle) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= count) return;
-  const uint32_t b = base[i], e = sizes_incl[i];
+  const uint32_t b = i ? sizes_incl[i - 1] : 0u, e = sizes_incl[i];
+  base[i] = b;
   for (uint32_t a = b; a < e; ++a) arm_saddle[a] = (uint32_t)i;
-}
-
-__global__ void k_arm_sizes(const EventRec *__restrict__ ev, const uint32_t *__restrict__ order,
-                            const uint32_t *__restrict__ pos, int64_t count, uint32_t *sizes) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) sizes[i] = ev[order[pos[i]]].meta & 0xff;
-}
-
-__global__ void k_saddle_meta(const EventRec *__restrict__ ev, const uint32_t *__restrict__ order,
-                              const uint32_t *__restrict__ cls, const uint32_t *__restrict__ pos,
-                              int64_t count, uint32_t *out_cls, double *out_level) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const EventRec &e = ev[order[pos[i]]];
-  out_cls[i] = cls[pos[i]];
-  out_level[i] = e.level;
 }
 
 // Closed labels (support then interior, kInvalid padded to 11) and supports
@@ -706,9 +1083,10 @@ __global__ void k_edge_list(const uint32_t *__restrict__ arm_saddle, const uint3
 // Boruvka round, part 1: least edge (by index) leaving each component.  The
 // edges still joining two components are appended to the next round's list
 // (li == nullptr: the list is the full edge list, li[i] = i).
-__global__ void k_msf_best(int64_t L, const uint32_t *__restrict__ lu, const uint32_t *__restrict__ lv,
+constexpr int kMsfBlock = 1024;
+__global__ void __launch_bounds__(kMsfBlock) k_msf_best(int64_t L, const uint32_t *__restrict__ lu, const uint32_t *__restrict__ lv,
                            const uint32_t *__restrict__ li, const uint32_t *__restrict__ comp, uint32_t *best,
-                           uint32_t *ou, uint32_t *ov, uint32_t *oi, uint32_t *count) {
+                           uint32_t *ou, uint32_t *ov, uint32_t *oi, unsigned long long *count) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t u = 0, v = 0, idx = 0, cu = 0, cv = 0;
   if (i < L) {
@@ -725,16 +1103,8 @@ __global__ void k_msf_best(int64_t L, const uint32_t *__restrict__ lu, const uin
     if (idx < best[cu]) atomicMin(&best[cu], idx);
     if (idx < best[cv]) atomicMin(&best[cv], idx);
   }
-  // wave-aggregated append
-  const uint64_t mask = __ballot(live);
-  if (!mask) return;
-  const int lane = (int)(threadIdx.x & 63u);
-  const int leader = __ffsll((unsigned long long)mask) - 1;
-  uint32_t at = 0;
-  if (lane == leader) at = atomicAdd(count, (uint32_t)__popcll(mask));
-  at = __shfl(at, leader);
+  const uint64_t pos = block_append<kMsfBlock / 64>(live ? 1u : 0u, count);
   if (live) {
-    const uint32_t pos = at + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
     ou[pos] = u;
     ov[pos] = v;
     oi[pos] = idx;
@@ -874,21 +1244,24 @@ __global__ void k_raw_of_dense(int64_t M, const uint32_t *__restrict__ dense, ui
   if (dense[m] != prev) out[prev] = (uint32_t)m;
 }
 
-// FP64 squared distance from every point to the last of its listed neighbours;
-// 0 (the list is never used) when a slot is empty.
-__global__ void k_nn_last_d2(int64_t n, const uint32_t *__restrict__ nn, const double *__restrict__ X,
+// FP64 squared distance from every point to the last of its `listed`
+// neighbours; infinite when the list holds every other point.
+__global__ void k_nn_last_d2(int64_t n, int listed, const uint32_t *__restrict__ nn, const double *__restrict__ X,
                              const double *__restrict__ Y, const double *__restrict__ Z, double *d2) {
   int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  bool whole = true;
-  for (int j = 0; j < kNearK; ++j) whole &= nn[p * kNearK + j] < (uint64_t)n;
-  const uint32_t q = nn[p * kNearK + kNearK - 1];
-  if (!whole) {
-    d2[p] = 0.0;
+  const uint32_t q = nn[p * kNearRow + listed - 1];
+  if (listed == n - 1 || q >= (uint64_t)n) {
+    d2[p] = q >= (uint64_t)n ? 0.0 : INFINITY;  // 0: never used
     return;
   }
   const double dx = X[q] - X[p], dy = Y[q] - Y[p], dz = Z[q] - Z[p];
   d2[p] = dx * dx + dy * dy + dz * dz;
+}
+
+__global__ void k_give_up(const uint32_t *__restrict__ origin, uint32_t n, uint32_t *carrier) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) carrier[origin[i]] = kInvalid;
 }
 
 __global__ void k_gather_u32(const uint32_t *__restrict__ src, const uint32_t *__restrict__ idx, int64_t n,
@@ -920,7 +1293,8 @@ void tower_vm_store(Context &c, hipStream_t s, uint32_t first_pos, const std::ve
 }
 
 void tower_prefetch_neighbours(Context &c) {
-  if (c.n <= kNearK) return;
+  if (c.n < 2) return;
+  const int listed = (int)std::min<int64_t>(kNearK, c.n - 1);
   if (!c.tower_work) c.tower_work = std::make_unique<TowerWork>();
   TowerWork &W = *c.tower_work;
   if (!W.vm_stream) MHGP_HIP(hipStreamCreateWithFlags(&W.vm_stream, hipStreamNonBlocking));
@@ -928,15 +1302,15 @@ void tower_prefetch_neighbours(Context &c) {
     MHGP_HIP(hipEventCreateWithFlags(&W.nn_start, hipEventDisableTiming));
     MHGP_HIP(hipEventCreateWithFlags(&W.nn_done, hipEventDisableTiming));
   }
-  W.nn.ensure((size_t)c.n * kNearK);
+  W.nn.ensure((size_t)c.n * kNearRow);
   W.nn_d2.ensure(c.n);
   W.nn_flags.ensure(c.n);
   // the side stream starts after the context stream's work so far (the LBVH)
   MHGP_HIP(hipEventRecord(W.nn_start, c.stream));
   MHGP_HIP(hipStreamWaitEvent(W.vm_stream, W.nn_start, 0));
-  knn_all(c, kNearK, W.nn.p, W.nn_flags.p, W.vm_stream);
-  hipLaunchKernelGGL(k_nn_last_d2, dim3(blocks_for(c.n, 256)), dim3(256), 0, W.vm_stream, c.n, W.nn.p, c.X.p,
-                     c.Y.p, c.Z.p, W.nn_d2.p);
+  knn_all(c, listed, W.nn.p, W.nn_flags.p, W.vm_stream, kNearRow);
+  hipLaunchKernelGGL(k_nn_last_d2, dim3(blocks_for(c.n, 256)), dim3(256), 0, W.vm_stream, c.n, listed, W.nn.p,
+                     c.X.p, c.Y.p, c.Z.p, W.nn_d2.p);
   MHGP_LAUNCH_CHECK();
   MHGP_HIP(hipEventRecord(W.nn_done, W.vm_stream));
   W.nn_pending = true;
@@ -957,7 +1331,7 @@ void tower_rank_index(Context &c) {
   // neighbour lists of the points, for the descents' ball queries: started
   // beside the level order, or computed here
   W.nn_ready = false;
-  if (c.n > kNearK) {
+  if (c.n >= 2) {
     if (!W.nn_pending) tower_prefetch_neighbours(c);
     MHGP_HIP(hipStreamWaitEvent(s, W.nn_done, 0));
     W.nn_pending = false;
@@ -978,6 +1352,24 @@ void tower_rank_index(Context &c) {
     if (W.rank_lo[r] > W.rank_hi[r] || W.rank_hi[r] > (uint64_t)n) throw std::runtime_error("malformed rank index");
 }
 
+// Calls f.template operator()<K>() for K = k.
+template <class F>
+void with_order(int k, F &&f) {
+  switch (k) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    default: throw std::logic_error("tower order beyond 10");
+  }
+}
+
 void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, TowerOrderData &out) {
   CatalogBuffers &B = *c.catalog;
   hipStream_t s = W.stream;
@@ -993,54 +1385,56 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   out.minima = M;
   uint64_t cap = 1;
   while (cap < 2ull * M + 16) cap <<= 1;
-  auto &tkeys = W.tkeys;
-  auto &tvals = W.tvals, &labels = W.labels;
-  tkeys.ensure(cap);
-  tvals.ensure(cap);
+  auto &slots = W.slots;
+  auto &labels = W.labels;
+  slots.ensure(cap);
   labels.ensure((size_t)M * k + 1);
-  MHGP_HIP(hipMemsetAsync(tkeys.p, 0, cap * 8, s));
+  const MinimaTable table{(unsigned long long *)slots.p, cap - 1, labels.p};
+  hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for((int64_t)cap, 256)), dim3(256), 0, s, slots.p, (int64_t)cap, 0ull);
   if (M)
-    hipLaunchKernelGGL(k_insert_minima, dim3(blocks_for(M, 256)), dim3(256), 0, s, B.events.p, B.order.p,
-                       minima_pos, (int64_t)M, k, labels.p, tkeys.p, tvals.p, cap - 1);
+    with_order(k, [&](auto K) {
+      hipLaunchKernelGGL((k_insert_minima<K.value>), dim3(blocks_for(M, 256)), dim3(256), 0, s, B.events.p, B.order.p,
+                         minima_pos, (int64_t)M, table);
+    });
   out.saddles = S;
   if (S == 0) return;
+  if (S >= (1u << 30)) throw CapacityError("an order of the tower has more saddles than the arm codes hold");
   auto &sizes = W.sizes, &carrier = W.carrier, &scls = W.scls;
   auto &slev = W.slev;
-  auto &steps = W.steps;
   sizes.ensure(S);
-  hipLaunchKernelGGL(k_arm_sizes, dim3(blocks_for(S, 256)), dim3(256), 0, s, B.events.p, B.order.p,
-                     saddle_pos, (int64_t)S, sizes.p);
+  scls.ensure(S);
+  slev.ensure(S);
+  W.members.ensure(S);
+  // the saddles' labels; the pool's words serve the spanning forest later
+  auto &base = W.base;
+  base.ensure(S);
+  const Saddles sad{W.slab.ensure((size_t)S * (k + 1)), W.members.p, base.p};
+  with_order(k, [&](auto K) {
+    hipLaunchKernelGGL((k_saddles<K.value>), dim3(blocks_for(S, 256)), dim3(256), 0, s, B.events.p, B.order.p, B.cls.p,
+                       saddle_pos, (int64_t)S, sad, sizes.p, scls.p, slev.p);
+  });
   W.scanner.inclusive(sizes.p, S, s);
   uint32_t arms = 0;
   copy_wait(&arms, sizes.p + S - 1, 4, hipMemcpyDeviceToHost, s);
   ph[1] = ph[2] = ph[3] = clk::now();
-  // exclusive bases: shift the inclusive scan by one
-  auto &base = W.base;
-  base.ensure(S);
-  MHGP_HIP(hipMemsetAsync(base.p, 0, 4, s));
-  if (S > 1) MHGP_HIP(hipMemcpyAsync(base.p + 1, sizes.p, (S - 1) * 4, hipMemcpyDeviceToDevice, s));
   carrier.ensure(arms);
   auto &arm_saddle = W.arm_saddle;
   arm_saddle.ensure(arms);
+  // exclusive bases (the inclusive scan shifted by one) and the arms' saddles
   hipLaunchKernelGGL(k_arm_owner, dim3(blocks_for(S, 256)), dim3(256), 0, s, base.p, sizes.p, (int64_t)S,
                      arm_saddle.p);
-  steps.ensure(1);
-  MHGP_HIP(hipMemsetAsync(steps.p, 0, 8, s));
   ArmParams A{};
-  A.ev = B.events.p; A.order = B.order.p; A.saddle_pos = saddle_pos; A.arm_base = base.p;
-  A.arm_saddle = arm_saddle.p; A.arms = arms; A.k = k;
-  A.table_keys = tkeys.p; A.table_vals = tvals.p; A.mask = cap - 1; A.labels = labels.p;
+  A.sad = sad;
+  A.sizes = sizes.p;
+  A.saddles = S;
+  A.table = table;
   A.X = c.X.p; A.Y = c.Y.p; A.Z = c.Z.p;
-  A.wide = c.wide.p; A.LX = c.LX.p; A.LY = c.LY.p; A.LZ = c.LZ.p; A.leaf_id = c.leaf_id.p; A.leaf_pos = c.leaf_pos.p; A.n = c.n;
+  A.wide = c.wide.p; A.LX = c.LX.p; A.LY = c.LY.p; A.LZ = c.LZ.p; A.leaf_id = c.leaf_id.p; A.leaf_pos = c.leaf_pos.p;
   A.carrier = carrier.p;
-  A.steps = (unsigned long long *)steps.p;
   A.nn = R.nn_ready ? R.nn.p : nullptr;
   A.nn_d2 = R.nn_ready ? R.nn_d2.p : nullptr;
   auto &queue = W.queue;
-  auto &qcount = W.qcount;
   queue.ensure(arms);
-  qcount.ensure(1);
-  MHGP_HIP(hipMemsetAsync(qcount.p, 0, 8, s));
   W.clock.start(s);
   auto &qkey = W.qkey;
   qkey.ensure(arms);
@@ -1050,44 +1444,61 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   W.facet_slots.ensure(fcap);
   W.alias_arm.ensure(arms);
   W.alias_rep.ensure(arms);
-  W.alias_count.ensure(1);
+  W.dcount.ensure(4);
   hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for((int64_t)fcap, 256)), dim3(256), 0, s, W.facet_slots.p,
                      (int64_t)fcap, 0ull);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(256), 0, s, W.alias_count.p, (int64_t)1, 0ull);
-  const FacetSet D{(unsigned long long *)W.facet_slots.p, fcap - 1, W.alias_arm.p, W.alias_rep.p,
-                   (unsigned long long *)W.alias_count.p};
-  hipLaunchKernelGGL(k_arm_lookup, dim3(blocks_for(arms, 256)), dim3(256), 0, s, A, D, queue.p, qkey.p,
-                     (unsigned long long *)qcount.p);
-  uint64_t nq = 0, na = 0;
-  MHGP_HIP(hipMemcpyAsync(&nq, qcount.p, 8, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipMemcpyAsync(&na, W.alias_count.p, 8, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipStreamSynchronize(s));
+  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, W.dcount.p, (int64_t)4, 0ull);
+  unsigned long long *counters = (unsigned long long *)W.dcount.p;
+  const FacetSet D{(unsigned long long *)W.facet_slots.p, fcap - 1, W.alias_arm.p, W.alias_rep.p, counters + 1};
+  with_order(k, [&](auto K) {
+    hipLaunchKernelGGL((k_arm_lookup<K.value>), dim3(blocks_for(S, kArmBlock)), dim3(kArmBlock), 0, s, A, D, queue.p,
+                       qkey.p, counters);
+  });
+  uint64_t got[4] = {0, 0, 0, 0};
+  copy_wait(got, W.dcount.p, 16, hipMemcpyDeviceToHost, s);
+  const uint64_t nq = got[0], na = got[1];
   ph[2] = ph[3] = clk::now();
-  if (nq > 1) {  // spatial order: neighbouring lanes walk neighbouring nodes
+  if (nq > 1) {  // spatial order: neighbouring lanes read neighbouring lists
     int bits = 8;
     while (bits < 32 && (1ll << bits) < c.n) bits += 8;
     W.sorter.sort(qkey.p, queue.p, (int64_t)nq, 0, bits, s);
   }
-  uint64_t steps_total = 0;
-  if (nq) {
-    DescentItems items[2];
-    for (int q = 0; q < 2; ++q) {
-      W.dF[q].ensure((size_t)kMaxLabel * nq);
-      W.dH[q].ensure(4 * nq);
+  uint64_t steps_total = 0, slow_total = 0;
+  if (nq && k >= 2) {
+    DescentItems items[3];  // two rounds' items, and what the fast steps leave open
+    for (int q = 0; q < 3; ++q) {
+      W.dF[q].ensure((size_t)k * nq);
       W.dO[q].ensure(nq);
-      items[q] = DescentItems{W.dF[q].p, W.dH[q].p, W.dO[q].p, nq};
+      items[q] = DescentItems{W.dF[q].p, W.dO[q].p, nq};
     }
-    W.dcount.ensure(1);
     uint32_t active = (uint32_t)nq;
     for (int round = 0; active > 0; ++round) {
       const int q = round & 1;
-      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, W.dcount.p, (int64_t)1, 0ull);
-      hipLaunchKernelGGL(k_descend_round, dim3(blocks_for(active, kArmBlock)), dim3(kArmBlock), 0, s, A, round,
-                         queue.p, items[q ^ 1], active, items[q], (unsigned long long *)W.dcount.p);
-      uint64_t nxt = 0;
-      copy_wait(&nxt, W.dcount.p, 8, hipMemcpyDeviceToHost, s);
-      steps_total += nxt;
-      active = (uint32_t)nxt;
+      if (round > 4096) {  // the host descends what is left
+        hipLaunchKernelGGL(k_give_up, dim3(blocks_for(active, 256)), dim3(256), 0, s, items[q ^ 1].origin, active,
+                           carrier.p);
+        break;
+      }
+      // a small round is bound by its launch and wait, not by idle lanes:
+      // several steps in one
+      const int steps = active <= 1u << 17 ? 8 : 1;
+      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, W.dcount.p, (int64_t)4, 0ull);
+      with_order(k, [&](auto K) {
+        hipLaunchKernelGGL((k_descend<K.value>), dim3(blocks_for(active, kDescentBlock)), dim3(kDescentBlock), 0, s, A,
+                           round == 0 ? queue.p : nullptr, items[q ^ 1], active, items[q], items[2], steps, counters);
+      });
+      copy_wait(got, W.dcount.p, 24, hipMemcpyDeviceToHost, s);
+      const uint32_t slow = (uint32_t)got[D_SLOW];
+      if (slow) {
+        with_order(k, [&](auto K) {
+          hipLaunchKernelGGL((k_descend_slow<K.value>), dim3(blocks_for(slow, kSlowBlock)), dim3(kSlowBlock), 0, s, A,
+                             items[2], slow, items[q], counters);
+        });
+        copy_wait(got, W.dcount.p, 24, hipMemcpyDeviceToHost, s);
+        slow_total += slow;
+      }
+      steps_total += got[D_STEPS];
+      active = (uint32_t)got[D_OUT];
     }
     ph[3] = clk::now();
   }
@@ -1101,10 +1512,6 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   // algorithmic bytes: each saddle record and its order/position entries read
   // once, each arm's carrier written once and one hash probe (key + value)
   W.arm_bytes += (int64_t)S * ((int64_t)sizeof(EventRec) + 8) + (int64_t)arms * (4 + 12);
-  scls.ensure(S);
-  slev.ensure(S);
-  hipLaunchKernelGGL(k_saddle_meta, dim3(blocks_for(S, 256)), dim3(256), 0, s, B.events.p, B.order.p, B.cls.p,
-                     saddle_pos, (int64_t)S, scls.p, slev.p);
   // drop the saddles that cannot change the contraction (unless the host
   // must descend some arms: then every saddle goes down as it is)
   const int64_t minima_n = k == 1 ? c.n : (int64_t)M;
@@ -1141,7 +1548,7 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
     hipLaunchKernelGGL(k_attach, gs, tb, 0, s, (int64_t)S, base.p, sizes.p, carrier.p, first.p, all_owned, attach.p);
     hipLaunchKernelGGL(k_attach_roots, gm, tb, 0, s, minima_n, attach.p, rep.p, err.p);
     // star edges between the representatives of owned carriers, in arm (= level) order
-    auto &eflag = W.eflag, &eu = W.eu, &ev = W.ev, &es = W.es;
+    auto &eflag = W.eflag;
     eflag.ensure(arms);
     hipLaunchKernelGGL(k_edge_flags, ga, tb, 0, s, arm_saddle.p, base.p, sizes.p, carrier.p, first.p, rep.p,
                        all_owned, (int64_t)arms, eflag.p);
@@ -1151,63 +1558,61 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
     copy_wait(&E, eflag.p + arms - 1, 4, hipMemcpyDeviceToHost, s);
     if (bad) throw std::runtime_error("tower attachment forest is cyclic");
     ph[5] = ph[6] = clk::now();
-    eu.ensure(E);
-    ev.ensure(E);
-    es.ensure(E);
+    // edges and two rounds' lists, in the pool that held the saddles' labels
+    uint32_t *pool = W.slab.ensure(9 * (size_t)E);
+    uint32_t *eu = pool, *ev = eu + E, *es = ev + E;
+    uint32_t *Lu[2] = {es + E, es + 4 * (size_t)E}, *Lv[2] = {Lu[0] + E, Lu[1] + E}, *Li[2] = {Lv[0] + E, Lv[1] + E};
     hipLaunchKernelGGL(k_edge_list, ga, tb, 0, s, arm_saddle.p, base.p, sizes.p, carrier.p, first.p, rep.p,
-                       all_owned, eflag.p, (int64_t)arms, eu.p, ev.p, es.p);
+                       all_owned, eflag.p, (int64_t)arms, eu, ev, es);
     // Boruvka spanning forest of the minima over the star edges
     auto &comp = W.comp, &comp2 = W.comp2, &best = W.best, &hook = W.hook, &msf = W.msf;
-    auto &mcount = W.mcount, &changed = W.changed, &live_n = W.live_n;
-    auto &Lu = W.Lu, &Lv = W.Lv, &Li = W.Li;
-    for (int q = 0; q < 2; ++q) {
-      Lu[q].ensure(E);
-      Lv[q].ensure(E);
-      Li[q].ensure(E);
-    }
-    live_n.ensure(1);
+    auto &mcount = W.mcount;
+    auto &live_n = W.live_n;
+    live_n.ensure(2);
     comp.ensure(minima_n);
     comp2.ensure(minima_n);
     best.ensure(minima_n);
     hook.ensure(minima_n);
     msf.ensure(E + 1);
     mcount.ensure(S);
-    changed.ensure(1);
     const dim3 ge(blocks_for(E + 1, 256));
     hipLaunchKernelGGL(k_identity, gm, tb, 0, s, comp.p, minima_n);
     hipLaunchKernelGGL(k_fill_u32, gm, tb, 0, s, best.p, minima_n, kInvalid);
     hipLaunchKernelGGL(k_fill_u32, gm, tb, 0, s, hook.p, minima_n, kInvalid);
     hipLaunchKernelGGL(k_fill_u32, ge, tb, 0, s, msf.p, (int64_t)E, 0u);
     hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(S, 256)), tb, 0, s, mcount.p, (int64_t)S, 0u);
-    const uint32_t *lu = eu.p, *lv = ev.p, *li = nullptr;
+    const uint32_t *lu = eu, *lv = ev, *li = nullptr;
     uint32_t live = E;
     msf_edges = E;
     for (int round = 0; live > 0; ++round) {
       if (round > 64) throw std::runtime_error("spanning forest of the tower did not converge");
       msf_rounds = round + 1;
       const int q = round & 1;
-      hipLaunchKernelGGL(k_fill_u32, dim3(1), tb, 0, s, changed.p, (int64_t)1, 0u);
-      hipLaunchKernelGGL(k_fill_u32, dim3(1), tb, 0, s, live_n.p, (int64_t)1, 0u);
-      hipLaunchKernelGGL(k_msf_best, dim3(blocks_for(live, 256)), tb, 0, s, (int64_t)live, lu, lv, li, comp.p,
-                         best.p, Lu[q].p, Lv[q].p, Li[q].p, live_n.p);
-      hipLaunchKernelGGL(k_msf_hook, gm, tb, 0, s, minima_n, eu.p, ev.p, comp.p, best.p, hook.p, msf.p, changed.p);
+      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, live_n.p, (int64_t)2, 0ull);
+      hipLaunchKernelGGL(k_msf_best, dim3(blocks_for(live, kMsfBlock)), dim3(kMsfBlock), 0, s, (int64_t)live, lu, lv, li, comp.p,
+                         best.p, Lu[q], Lv[q], Li[q], (unsigned long long *)live_n.p);
+      hipLaunchKernelGGL(k_msf_hook, gm, tb, 0, s, minima_n, eu, ev, comp.p, best.p, hook.p, msf.p,
+                         (uint32_t *)(live_n.p + 1));
       hipLaunchKernelGGL(k_msf_apply, gm, tb, 0, s, minima_n, comp.p, best.p, hook.p);
-      hipLaunchKernelGGL(k_msf_flatten, gm, tb, 0, s, minima_n, comp.p, comp2.p, err.p);
+      hipLaunchKernelGGL(k_msf_flatten, gm, tb, 0, s, minima_n, comp.p, comp2.p, (uint32_t *)(live_n.p + 1) + 1);
       std::swap(comp.p, comp2.p);
       std::swap(comp.cap, comp2.cap);
-      uint32_t flags[3] = {0, 0, 0};
-      MHGP_HIP(hipMemcpyAsync(&flags[0], changed.p, 4, hipMemcpyDeviceToHost, s));
-      MHGP_HIP(hipMemcpyAsync(&flags[2], live_n.p, 4, hipMemcpyDeviceToHost, s));
-      copy_wait(&flags[1], err.p, 4, hipMemcpyDeviceToHost, s);
-      if (flags[1]) throw std::runtime_error("spanning forest of the tower: cyclic hook forest");
-      if (!flags[0]) break;
-      live = flags[2];
-      lu = Lu[q].p;
-      lv = Lv[q].p;
-      li = Li[q].p;
+      // live edges; hooked anything, cyclic forest
+      struct {
+        uint64_t live;
+        uint32_t changed, cyclic;
+      } r;
+      static_assert(sizeof r == 16, "round result layout");
+      copy_wait(&r, live_n.p, sizeof r, hipMemcpyDeviceToHost, s);
+      if (r.cyclic) throw std::runtime_error("spanning forest of the tower: cyclic hook forest");
+      if (!r.changed) break;
+      live = (uint32_t)r.live;
+      lu = Lu[q];
+      lv = Lv[q];
+      li = Li[q];
     }
     ph[6] = clk::now();
-    if (E) hipLaunchKernelGGL(k_msf_count, ge, tb, 0, s, (int64_t)E, msf.p, es.p, mcount.p);
+    if (E) hipLaunchKernelGGL(k_msf_count, ge, tb, 0, s, (int64_t)E, msf.p, es, mcount.p);
     // keep births, multifusions and shared levels
     hipLaunchKernelGGL(k_reduce_saddles, gs, tb, 0, s, (int64_t)S, base.p, sizes.p, carrier.p, scls.p, first.p,
                        mcount.p, all_owned, keep.p, kept.p);
@@ -1271,10 +1676,10 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   out.steps = (int64_t)st;
   if (std::getenv("MHGP_TIMING"))
     std::fprintf(stderr,
-                 "[mhgp] arms order %2d: %u saddles, %u arms, %llu descending, %llu steps, %u forest edges in %d "
+                 "[mhgp] arms order %2d: %u saddles, %u arms, %llu descending, %llu steps (%llu slow), %u forest edges in %d "
                  "rounds, %u kept | ms: setup %.2f lookup %.2f descents %.2f first %.2f edges %.2f forest %.2f "
                  "tail %.2f\n",
-                 k, S, arms, (unsigned long long)nq, (unsigned long long)st, msf_edges, msf_rounds, S2,
+                 k, S, arms, (unsigned long long)nq, (unsigned long long)st, (unsigned long long)slow_total, msf_edges, msf_rounds, S2,
                  std::chrono::duration<double, std::milli>(ph[1] - ph[0]).count(),
                  std::chrono::duration<double, std::milli>(ph[2] - ph[1]).count(),
                  std::chrono::duration<double, std::milli>(ph[3] - ph[2]).count(),

@@ -60,17 +60,17 @@ struct TowerWork {
   DevBuf<uint64_t> rank_keys;
   DevBuf<uint32_t> rank_vals, rank_bounds;
   uint32_t rank_lo[256] = {}, rank_hi[256] = {};
-  DevBuf<uint32_t> tvals, labels;
-  DevBuf<uint64_t> tkeys, steps, qcount, qkey, facet_slots, alias_count;
-  DevBuf<uint32_t> alias_arm, alias_rep, dF[2], dH[2], dO[2];
-  DevBuf<uint64_t> dcount;
+  // the minima's hash table and labels, the saddles' labels (a pool whose
+  // words then serve the spanning forest) and support members
+  DevBuf<uint64_t> slots, qkey, facet_slots, dcount, live_n;
+  DevBuf<uint32_t> labels, slab;
+  DevBuf<uint16_t> members;
+  DevBuf<uint32_t> alias_arm, alias_rep, dF[3], dO[3];
   DevBuf<uint32_t> sizes, carrier, scls, base, arm_saddle, queue;
   DevBuf<double> slev, c_lev;
   DevBuf<uint32_t> first, keep, kept, flag1, c_cls, c_base, c_car;
-  DevBuf<uint32_t> eflag, eu, ev, es;
-  DevBuf<uint32_t> comp, comp2, best, hook, msf, mcount, changed, err, live_n;
-  DevBuf<uint32_t> Lu[2], Lv[2], Li[2];
-  DevBuf<uint32_t> attach, rep, dense, slab, ssup;
+  DevBuf<uint32_t> eflag, comp, comp2, best, hook, msf, mcount, err;
+  DevBuf<uint32_t> attach, rep, dense, ssup;
   // vertical maps: per record (rank-index position) the contraction element
   // of its first arm's carrier as a saddle of the order below (first lane
   // only), the gather scratch, and the dense -> raw minimum map of a lane
@@ -83,13 +83,16 @@ struct TowerWork {
   bool nn_ready = false;
   int64_t bytes() const {
     int64_t b = 0;
-    for (const DevBuf<uint32_t> *x : {&rank_vals, &rank_bounds, &tvals, &labels, &sizes, &carrier, &scls,
-                                      &base, &arm_saddle, &queue, &first, &keep, &kept, &flag1, &c_cls, &c_base,
-                                      &c_car, &eflag, &eu, &ev, &es, &comp, &comp2, &best, &hook, &msf, &mcount,
-                                      &changed, &err, &live_n, &Lu[0], &Lu[1], &Lv[0], &Lv[1], &Li[0], &Li[1],
-                                      &attach, &rep, &dense, &slab, &ssup, &vm_elem, &vm_idx, &vm_out, &raw_dense, &alias_arm, &alias_rep, &dF[0], &dF[1], &dH[0], &dH[1], &dO[0], &dO[1]})
+    for (const DevBuf<uint32_t> *x :
+         {&rank_vals, &rank_bounds, &labels, &slab,   &alias_arm, &alias_rep, &dF[0],     &dF[1],  &dF[2],  &dO[0],
+          &dO[1],     &dO[2],       &sizes,  &carrier, &scls,      &base,      &arm_saddle, &queue,  &first,  &keep,
+          &kept,      &flag1,       &c_cls,  &c_base,  &c_car,     &eflag,     &comp,       &comp2,  &best,   &hook,
+          &msf,       &mcount,      &err,    &attach,  &rep,       &dense,     &ssup,       &vm_elem, &vm_idx, &vm_out,
+          &raw_dense, &nn})
       b += (int64_t)x->bytes();
-    return b + (int64_t)(nn.bytes() + nn_d2.bytes() + nn_flags.bytes()) + (int64_t)(rank_keys.bytes() + qkey.bytes() + facet_slots.bytes() + alias_count.bytes() + dcount.bytes() + tkeys.bytes() + steps.bytes() + qcount.bytes() + slev.bytes() + c_lev.bytes());
+    for (const DevBuf<uint64_t> *x : {&rank_keys, &slots, &qkey, &facet_slots, &dcount, &live_n})
+      b += (int64_t)x->bytes();
+    return b + (int64_t)(members.bytes() + nn_flags.bytes() + nn_d2.bytes() + slev.bytes() + c_lev.bytes());
   }
 };
 
