@@ -403,6 +403,8 @@ void contract_order(int k, int64_t n, TowerOrderData &D, Forest &F) {
 // later than m's level <= L.  So the target is the owner at L of c's class:
 // the node that first owned the class of c's contraction element, raised
 // through its ancestors while their level is <= L.
+//
+// (tower_vm_targets answers the same on the device for large pairs.)
 static void vertical_order(const Forest &S, const Forest &T, const std::vector<uint32_t> &elem,
                            std::vector<int64_t> &target) {
   const size_t m = S.order.size(), tm = T.order.size();
@@ -533,9 +535,20 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
       W0.vm_out.ensure(most);
     }
   }
+  const auto t0 = std::chrono::steady_clock::now();
+  auto since = [&] { return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count(); };
   auto vertical_pair = [&](int o) {
+    const double v0 = since();
     const Forest &S = forests[o - 1];
     const uint32_t base = W0.rank_lo[o], span = W0.rank_hi[o] - base;
+    {
+      std::lock_guard<std::mutex> g(vm_gather_mu);
+      MHGP_HIP(hipSetDevice(c.device));
+      if (tower_vm_targets(c, S, forests[o - 2], base, span, forests[o - 1].vtarget)) {
+        if (tm.on) std::fprintf(stderr, "[mhgp] vertical %2d: from %.1f done %.1f ms\n", o, v0, since());
+        return;
+      }
+    }
     std::vector<uint32_t> pos(S.order.size());
     for (size_t i = 0; i < S.order.size(); ++i) {
       const int32_t d = S.rep_elem[i];
@@ -551,7 +564,9 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
       std::lock_guard<std::mutex> g(vm_gather_mu);
       tower_vm_gather(c, pos, elem);
     }
+    const double v1 = since();
     vertical_order(forests[o - 1], forests[o - 2], elem, forests[o - 1].vtarget);
+    if (tm.on) std::fprintf(stderr, "[mhgp] vertical %2d: from %.1f gathered %.1f done %.1f ms\n", o, v0, v1, since());
   };
   auto after_contract = [&](int k) {
     int ready[2], nready = 0;
@@ -577,6 +592,7 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
     for (int k = next_k.fetch_sub(1); k >= 1; k = next_k.fetch_sub(1)) {
       TowerOrderData &D = Ds[k - 1];
       tower_order_device(c, W, W0, k, D);
+      if (tm.on) std::fprintf(stderr, "[mhgp] device %2d done %.1f ms\n", k, since());
       {
         std::lock_guard<std::mutex> g(mu);
         T.descent_steps += D.steps;
@@ -620,7 +636,9 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
       std::lock_guard<std::mutex> g(mu);
       workers.emplace_back([&, k] {
         try {
+          const double c0 = since();
           contract_order(k, n, Ds[k - 1], forests[k - 1]);
+          if (tm.on) std::fprintf(stderr, "[mhgp] contract %2d: from %.1f to %.1f ms\n", k, c0, since());
           after_contract(k);
         } catch (...) {
           errors[k - 1] = std::current_exception();

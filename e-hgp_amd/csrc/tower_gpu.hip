@@ -22,6 +22,7 @@
 #include "supports.hpp"
 #include "traverse.hpp"
 #include "tower_gpu.hpp"
+#include "tower_state.hpp"
 #include "wave.hpp"
 
 namespace mhgp {
@@ -1173,10 +1174,21 @@ __global__ void k_msf_count(int64_t E, const uint32_t *__restrict__ msf, const u
   if (i < E && msf[i]) atomicAdd(&mcount[es[i]], 1u);
 }
 
+// Whether arm a's contraction element (its carrier's representative; the
+// carrier itself without representatives) differs from those of the saddle's
+// arms before it: the others join nothing new, the host never sees them.
+__device__ inline bool first_of_class(const uint32_t *carrier, const uint32_t *rep, uint32_t b, uint32_t a) {
+  const uint32_t c = rep ? rep[carrier[a]] : carrier[a];
+  for (uint32_t x = b; x < a; ++x)
+    if ((rep ? rep[carrier[x]] : carrier[x]) == c) return false;
+  return true;
+}
+
 __global__ void k_reduce_saddles(int64_t S, const uint32_t *__restrict__ base, const uint32_t *__restrict__ incl,
                                  const uint32_t *__restrict__ carrier, const uint32_t *__restrict__ cls,
                                  const uint32_t *__restrict__ first, const uint32_t *__restrict__ mcount,
-                                 int all_owned, uint32_t *keep, uint32_t *kept_arms) {
+                                 const uint32_t *__restrict__ rep, int all_owned, uint32_t *keep,
+                                 uint32_t *kept_arms) {
   int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S) return;
   const uint32_t b = base[s], e = incl[s];
@@ -1189,7 +1201,9 @@ __global__ void k_reduce_saddles(int64_t S, const uint32_t *__restrict__ base, c
     k = !any_owned;  // no owned carrier: a birth
   }
   keep[s] = k ? 1u : 0u;
-  kept_arms[s] = k ? e - b : 0u;
+  uint32_t distinct = 0;
+  for (uint32_t a = b; k && a < e; ++a) distinct += first_of_class(carrier, rep, b, a);
+  kept_arms[s] = distinct;
 }
 
 __global__ void k_attach_roots(int64_t M, uint32_t *attach, uint32_t *rep, uint32_t *err) {
@@ -1217,11 +1231,13 @@ __global__ void k_compact_saddles(int64_t S, const uint32_t *__restrict__ kpos, 
   const uint32_t prev = s ? kpos[s - 1] : 0u;
   if (kpos[s] == prev) return;  // dropped
   const uint32_t b = base[s], e = incl[s];
-  const uint32_t p = prev, nb = kinc[s] - (e - b);
+  const uint32_t p = prev;
+  uint32_t nb = s ? kinc[s - 1] : 0u;
   o_cls[p] = scls[s];
   o_lev[p] = slev[s];
   o_base[p] = nb;
-  for (uint32_t a = b; a < e; ++a) o_car[nb + (a - b)] = rep ? dense[rep[carrier[a]]] - 1u : carrier[a];
+  for (uint32_t a = b; a < e; ++a)
+    if (first_of_class(carrier, rep, b, a)) o_car[nb++] = rep ? dense[rep[carrier[a]]] - 1u : carrier[a];
 }
 
 // Vertical maps: the order-k contraction element (dense representative id;
@@ -1264,6 +1280,58 @@ __global__ void k_give_up(const uint32_t *__restrict__ origin, uint32_t n, uint3
   if (i < n) carrier[origin[i]] = kInvalid;
 }
 
+// Vertical maps of a large order pair: targets by ancestor doubling.  up[0] is
+// the parent of every node of the order below (-1: none); level j holds the
+// 2^j-th ancestor.
+__global__ void k_double_up(int64_t n, const int32_t *__restrict__ below, int32_t *above) {
+  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= n) return;
+  const int32_t p = below[x];
+  above[x] = p < 0 ? -1 : below[p];
+}
+
+// Node i (level class L) starts at the node that first owned the class of
+// its element and climbs to that node's highest ancestor at or below L
+// (levels never decrease towards a root).
+struct VerticalPair {
+  const int64_t *s_cls;      // order o: level class per node
+  const int32_t *s_rep;      // representative element per node
+  const uint32_t *s_raw;     // raw minimum of each element (null: identity)
+  int64_t s_nodes, s_raws;
+  uint32_t base, span;       // rank-index range of order o's minima
+  const uint32_t *elem;      // element of the order below per rank-index position
+  const int64_t *t_cls;      // order o - 1
+  const int32_t *t_acq;      // per element: node that first owned its class
+  const int64_t *t_acq_cls;  // and its level class
+  int64_t t_nodes, t_elems;
+  const int32_t *up;         // levels x t_nodes
+  int levels;
+};
+
+__global__ void k_vertical(VerticalPair V, int64_t *target, uint32_t *error) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= V.s_nodes) return;
+  const int64_t L = V.s_cls[i];
+  int64_t x = -1;
+  const int32_t r = V.s_rep[i];
+  if (r >= 0 && (!V.s_raw || r < V.s_raws)) {
+    const uint32_t raw = V.s_raw ? V.s_raw[r] : (uint32_t)r;
+    if (raw < V.span) {
+      const uint32_t e = V.elem[V.base + raw];
+      if (e < (uint64_t)V.t_elems && V.t_acq[e] >= 0 && V.t_acq[e] < V.t_nodes && V.t_acq_cls[e] <= L) x = V.t_acq[e];
+    }
+  }
+  if (x < 0) {
+    *error = 1u;
+    return;
+  }
+  for (int j = V.levels - 1; j >= 0; --j) {
+    const int32_t a = V.up[(int64_t)j * V.t_nodes + x];
+    if (a >= 0 && V.t_cls[a] <= L) x = a;
+  }
+  target[i] = x;
+}
+
 __global__ void k_gather_u32(const uint32_t *__restrict__ src, const uint32_t *__restrict__ idx, int64_t n,
                              uint32_t *out) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1285,6 +1353,47 @@ void tower_vm_gather(Context &c, const std::vector<uint32_t> &pos, std::vector<u
   hipLaunchKernelGGL(k_gather_u32, dim3(blocks_for(q, 256)), dim3(256), 0, s, R.vm_elem.p, R.vm_idx.p, q, R.vm_out.p);
   MHGP_LAUNCH_CHECK();
   copy_wait(out.data(), R.vm_out.p, q * 4, hipMemcpyDeviceToHost, s);
+}
+
+bool tower_vm_targets(Context &c, const Forest &S, const Forest &T, uint32_t base, uint32_t span,
+                      std::vector<int64_t> &target) {
+  const int64_t m = (int64_t)S.order.size(), tm = (int64_t)T.order.size(), te = (int64_t)T.acq_node.size();
+  if (m < kVerticalOnDevice || tm < 2) return false;
+  TowerWork &R = *c.tower_work;
+  if (!R.vm_stream) MHGP_HIP(hipStreamCreateWithFlags(&R.vm_stream, hipStreamNonBlocking));
+  hipStream_t s = R.vm_stream;
+  int levels = 1;
+  while ((1ll << levels) < tm) ++levels;
+  const int64_t raws = (int64_t)S.raw_of_dense.size();
+  // eight-byte words, then four-byte ones
+  R.vm_long.ensure((size_t)(2 * m + tm + te));
+  R.vm_int.ensure((size_t)(m + raws + te + levels * tm + 1));
+  int64_t *s_cls = R.vm_long.p, *d_target = s_cls + m, *t_cls = d_target + m, *t_acq_cls = t_cls + tm;
+  int32_t *s_rep = R.vm_int.p, *s_raw = s_rep + m, *t_acq = s_raw + raws, *up = t_acq + te, *err = up + levels * tm;
+  auto put = [&](void *d, const void *h, size_t bytes) {
+    if (bytes) MHGP_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
+  };
+  put(s_cls, S.level_class.data(), m * 8);
+  put(t_cls, T.level_class.data(), tm * 8);
+  put(t_acq_cls, T.acq_cls.data(), te * 8);
+  put(s_rep, S.rep_elem.data(), m * 4);
+  put(s_raw, S.raw_of_dense.data(), raws * 4);
+  put(t_acq, T.acq_node.data(), te * 4);
+  put(up, T.parent.data(), tm * 4);
+  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, (uint32_t *)err, (int64_t)1, 0u);
+  for (int j = 1; j < levels; ++j)
+    hipLaunchKernelGGL(k_double_up, dim3(blocks_for(tm, 256)), dim3(256), 0, s, tm, up + (int64_t)(j - 1) * tm,
+                       up + (int64_t)j * tm);
+  const VerticalPair V{s_cls, s_rep, raws ? (const uint32_t *)s_raw : nullptr, m, raws, base, span, R.vm_elem.p,
+                       t_cls, t_acq, t_acq_cls, tm, te, up, levels};
+  hipLaunchKernelGGL(k_vertical, dim3(blocks_for(m, 256)), dim3(256), 0, s, V, d_target, (uint32_t *)err);
+  MHGP_LAUNCH_CHECK();
+  target.resize(m);
+  uint32_t bad = 0;
+  MHGP_HIP(hipMemcpyAsync(&bad, err, 4, hipMemcpyDeviceToHost, s));
+  copy_wait(target.data(), d_target, m * 8, hipMemcpyDeviceToHost, s);
+  if (bad) throw std::runtime_error("vertical map: the order below holds no owned class at the node's level");
+  return true;
 }
 
 void tower_vm_store(Context &c, hipStream_t s, uint32_t first_pos, const std::vector<uint32_t> &elems) {
@@ -1614,17 +1723,16 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
     ph[6] = clk::now();
     if (E) hipLaunchKernelGGL(k_msf_count, ge, tb, 0, s, (int64_t)E, msf.p, es, mcount.p);
     // keep births, multifusions and shared levels
+    const uint32_t *d_rep = k >= 2 ? rep.p : nullptr, *d_dense = nullptr;  // order one keeps point ids: every point is born
     hipLaunchKernelGGL(k_reduce_saddles, gs, tb, 0, s, (int64_t)S, base.p, sizes.p, carrier.p, scls.p, first.p,
-                       mcount.p, all_owned, keep.p, kept.p);
-    const uint32_t *d_rep = nullptr, *d_dense = nullptr;
+                       mcount.p, d_rep, all_owned, keep.p, kept.p);
     uint32_t Mdense = (uint32_t)minima_n;
-    if (k >= 2) {  // order one keeps point ids: every point is born
+    if (k >= 2) {
       dense.ensure(minima_n);
       hipLaunchKernelGGL(k_fill_u32, gm, tb, 0, s, dense.p, minima_n, 0u);
       hipLaunchKernelGGL(k_flag_used, gs, tb, 0, s, (int64_t)S, keep.p, base.p, sizes.p, carrier.p, rep.p, dense.p);
       W.scanner.inclusive(dense.p, minima_n, s);
       copy_wait(&Mdense, dense.p + minima_n - 1, 4, hipMemcpyDeviceToHost, s);
-      d_rep = rep.p;
       d_dense = dense.p;
       // dense id -> raw minimum, for the vertical maps out of this order
       W.raw_dense.ensure(Mdense + 1);

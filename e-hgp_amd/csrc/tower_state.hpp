@@ -17,6 +17,7 @@ struct Forest {
   std::vector<double> level;
   std::vector<int64_t> child_offset{0};
   std::vector<int64_t> children;
+  std::vector<int32_t> parent;  // -1: root
   // Vertical maps.  Contraction elements are the order's minima (points at
   // order one, dense representatives otherwise): per element, the node that
   // first owned its class and that node's level class there; per node, an
@@ -36,6 +37,8 @@ struct Forest {
     level_class.push_back(cls);
     level.push_back(lev);
     children.insert(children.end(), kids, kids + nk);
+    for (size_t i = 0; i < nk; ++i) parent[kids[i]] = (int32_t)parent.size();
+    parent.push_back(-1);
     child_offset.push_back((int64_t)children.size());
     return (int64_t)order.size() - 1;
   }
@@ -48,6 +51,7 @@ struct Forest {
     kind.reserve(nodes);
     level_class.reserve(nodes);
     level.reserve(nodes);
+    parent.reserve(nodes);
     child_offset.reserve(nodes + 1);
     children.reserve(2 * nodes);
   }

@@ -268,3 +268,36 @@ def test_order_one_cuts_equal_emst_components():
                     mine.setdefault(int(lab[p]), set()).add(p)
                 assert sorted(map(sorted, groups.values())) == sorted(map(sorted, mine.values())), (cls, closed)
                 assert sorted(mine) == sorted(int(r) for r in roots)
+
+
+def test_vertical_maps_of_large_orders_climb_and_commute():
+    """Order pairs of more than 65 536 nodes take their vertical targets from
+    the device: every target lies at or below its node's level while its parent
+    lies above it, and the maps commute with the forests (a child's target is
+    below its parent's)."""
+    pts = workloads.jittered_lattice(40_000, side=35, sigma=0.1, seed=3)
+    print("vertical maps: lattice n=40000 k=3", flush=True)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        ctx.emst()
+        ctx.supports(3, fetch=False)
+        tw = ctx.tower(3)
+    order, cls, vert, off, kids = (tw[k] for k in ("order", "level_class", "vertical", "child_offset", "children"))
+    assert np.count_nonzero(order == 3) > 65_536
+    parent = np.full(len(order), -1, dtype=np.int64)
+    parent[kids] = np.repeat(np.arange(len(order)), np.diff(off))
+    up = np.flatnonzero(order >= 2)
+    t = vert[up]
+    assert np.all(order[t] == order[up] - 1) and np.all(cls[t] <= cls[up])
+    p = parent[t]
+    assert np.all((p < 0) | (cls[np.maximum(p, 0)] > cls[up]))
+    # commuting: climbing a child's target to its parent's level gives the parent's target
+    child = up[parent[up] >= 0]
+    x, want, level = vert[child].copy(), vert[parent[child]], cls[parent[child]]
+    while True:
+        q = parent[x]
+        move = (q >= 0) & (cls[np.maximum(q, 0)] <= level)
+        if not move.any():
+            break
+        x = np.where(move, q, x)
+    assert np.array_equal(x, want)
