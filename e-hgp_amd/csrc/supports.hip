@@ -50,7 +50,7 @@ namespace mhgp {
 
 int64_t catalog_device_bytes(const CatalogBuffers &b) {
   return b.radius.bytes() + b.gcount.bytes() + b.goff.bytes() + b.glist.bytes() + b.region.bytes() +
-         b.lists.bytes() + b.big.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
+         b.lists.bytes() + b.big.bytes() + b.rescans.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
          b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.scratch.bytes() + b.anchors.bytes() +
          b.total.bytes() + b.run_count.bytes() + b.run_pos.bytes() + b.run_gidx.bytes() + b.run_new.bytes() +
          b.run_link.bytes() + b.run_rec.bytes();
@@ -77,6 +77,7 @@ enum { L_WIDEN = 0, L_WIDE = 1, L_BIG = 2, L_SMALL = 3, L_MID = 4, L_LARGE = 5, 
 constexpr int kListCount = 8;    // counters: list lengths
 constexpr int kOpenCount = 16;   // counters: open anchors, their largest region
 constexpr int kOpenLargest = 17;
+constexpr int kRescanMost = 18;  // longest rescan list of a launch
 constexpr int kCounters = 24;
 
 // Regions of the global-memory path are enumerated face by face in
@@ -106,11 +107,14 @@ struct Params {
   uint64_t fallback_cap;
   uint32_t *fb_region;
   uint64_t fb_region_cap;
-  unsigned long long *counters;  // [0] events [1] fallbacks [2] region words [3] candidates [4] queue errors
+  struct Rescan *rescans;        // sides of faces left to k_rescan
+  uint64_t rescan_cap;
+  unsigned long long *counters;  // [0] events [1] fallbacks [2] region words [3] candidates [4] rescans
                                  // [5] FP64 [6] FP32 operations, then the lists' lengths and the open anchors
   const uint32_t *anchors;
   uint32_t anchor_count;
   int probe;                     // 1: stop once the region is in the slab
+  int ascending;                 // 1: the slabs' regions are in increasing distance
   double *scratch;
   uint64_t slab_doubles;
   uint32_t gcap;                 // gathered points a slab holds
@@ -139,12 +143,14 @@ struct Work {
   float *rho;        // certificate radius per cell (FP32, rounded up)
   uint32_t *ridx;    // gathered index of each region slot (until the points are compacted)
   uint64_t *rmask;  // 6 words per member
-  uint32_t *kidx;
+  uint16_t *kidx;    // candidate vertices (region slots)
   float4 *fc;       // FP32 offset and distance per gathered point (certificate and masks)
   uint32_t *cand;   // candidate supports classified (LDS, flushed once per anchor)
   unsigned long long *flops;  // FP64 operations of the certified predicates (LDS, flushed once per anchor; null: not counted)
-  float *fx, *fy, *fz;        // FP32 copies of the region's coordinates (LDS path only)
+  float *fx, *fy, *fz, *fw;   // FP32 copies of the region's coordinates and distances from the anchor
   unsigned long long *flops32;  // FP32 operations of the tests (as flops; null: not counted)
+  bool ascending;             // the region is in increasing distance: scans end at a sphere's diameter
+  uint32_t slab;              // the anchor's index in its launch
 };
 
 // FP64 operations (add, subtract, multiply; a fused multiply-add counts two)
@@ -168,26 +174,21 @@ __device__ inline void add_flops(const Work &w, uint64_t v) {
 // roots count one each.
 constexpr uint32_t kF32Cover = 16;      // one point against one cell (certificate)
 constexpr uint32_t kF32Mask = 16;       // one point against one cell (membership)
-constexpr uint32_t kF32Pencil = 19;     // Pencil::outside, per slot
+constexpr uint32_t kF32Pencil = 15;     // Pencil::outside, per slot
 constexpr uint32_t kF32Cell = 28;       // one shared cell of a face (face_interval)
-constexpr uint32_t kF32FacePoint = 31;  // TriSphereF::eval and two certified signs
+constexpr uint32_t kF32FacePoint = 24;  // TriSphereF::eval and two certified signs
 constexpr uint32_t kF32Key = 16;        // key_bounds_32
-constexpr uint32_t kF32PairSide = 17;   // PairSphereF::side
-constexpr uint32_t kF32TetSide = 20;    // TetSphereF::side
+constexpr uint32_t kF32PairSide = 13;   // SphereF::place of a pair
+constexpr uint32_t kF32TetSide = 13;    // SphereF::place of a tetrahedron
 __device__ inline void add_flops32(const Work &w, uint64_t v) {
   if (w.flops32 && v) atomicAdd(w.flops32, (unsigned long long)v);
 }
 
 __device__ inline V3 gpt(const Work &w, uint32_t i) { return {w.gx[i], w.gy[i], w.gz[i]}; }
 
-// Interior id lists are written and sorted with static indices only, so
-// they stay in registers: an append is a select over the slots, the sort an
-// odd-even transposition network (unused slots hold kInvalid and sort last).
-__device__ inline void put_static(uint32_t (&a)[kMaxInterior], int pos, uint32_t v) {
-#pragma unroll
-  for (int j = 0; j < kMaxInterior; ++j) a[j] = j == pos ? v : a[j];
-}
-
+// Interior id lists are sorted with static indices only, so they stay in
+// registers: an odd-even transposition network (unused slots hold kInvalid and
+// sort last).
 __device__ inline void sort_static(uint32_t (&a)[kMaxInterior], int n) {
 #pragma unroll
   for (int j = 0; j < kMaxInterior; ++j) a[j] = j < n ? a[j] : kInvalid;
@@ -202,7 +203,7 @@ __device__ inline void sort_static(uint32_t (&a)[kMaxInterior], int n) {
   }
 }
 
-__device__ void emit_event(const Params &P, uint32_t u, const uint32_t *sup, int m, int nint,
+__device__ __attribute__((always_inline)) inline void emit_event(const Params &P, uint32_t u, const uint32_t *sup, int m, int nint,
                            const uint32_t *interior, double level, double lerr) {
   const unsigned long long slot = wave_append(true, &P.counters[0]);
   if (slot >= P.event_cap) return;
@@ -219,7 +220,7 @@ __device__ void emit_event(const Params &P, uint32_t u, const uint32_t *sup, int
 }
 
 // Queues undecided work and, once per anchor, its region for the host.
-__device__ void emit_fallback(const Params &P, const Work &w, uint32_t u, uint32_t kind,
+__device__ __attribute__((always_inline)) inline void emit_fallback(const Params &P, const Work &w, uint32_t u, uint32_t kind,
                               const uint32_t *ids, int m, uint32_t M, uint32_t *region_slot) {
   if (*region_slot == kInvalid) {
     uint32_t expected = kInvalid;
@@ -241,8 +242,6 @@ __device__ void emit_fallback(const Params &P, const Work &w, uint32_t u, uint32
   f.pad = 0;
 }
 
-// Certified classification of the region against a candidate sphere.
-// Returns 1 event, 0 not critical, -1 undecided (host).
 // FP32 certification of a sign: v against its magnitude bound a.  With
 // the coordinates, the coefficients and the at most ~9 roundings of a chain
 // in FP32 (the FP64 coefficients rounded to nearest), |v32 - v| < 1e-6 a
@@ -254,83 +253,117 @@ __device__ inline int cert32(float v, float a) {
   return !(a > 1e-30f) ? 0 : (v > e ? 1 : (v < -e ? -1 : 0));
 }
 
-// Pair and tetrahedron side tests in FP32 on the region's FP32 coordinates.
-struct PairSphereF {
-  float a[3];
-  __device__ int side(float x, float y, float z) const {
-    const float v = x * (x - a[0]) + y * (y - a[1]) + z * (z - a[2]);
-    const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
-    const float va = ax * (ax + fabsf(a[0])) + ay * (ay + fabsf(a[1])) + az * (az + fabsf(a[2]));
-    return cert32(v, va);
+// A candidate sphere through the anchor in FP32: the scaled power
+// a |p|^2 - p.b of a point, with the magnitude bound |p| (aA |p| + bA) (the
+// norms bound the sums of magnitudes).  reach: no point farther from the
+// anchor is inside (the sphere passes through the anchor, so its diameter with
+// a margin for the FP32 estimate; infinite when the region is not in
+// increasing distance).
+struct SphereF {
+  float a, aA, b[3], bA, reach;
+  __device__ void test(float x, float y, float z, float w, float &v, float &va) const {
+    v = a * (w * w) - (x * b[0] + y * b[1] + z * b[2]);
+    va = w * (aA * w + bA);
   }
 };
-struct TetSphereF {
-  float V, VA, N[3], NA[3];
-  int sg;  // sign of the FP64 volume (certified nonzero)
-  __device__ int side(float x, float y, float z) const {
-    const float pp = x * x + y * y + z * z;
-    const float Q = V * pp - (x * N[0] + y * N[1] + z * N[2]);
-    const float QA = VA * pp + (fabsf(x) * NA[0] + fabsf(y) * NA[1] + fabsf(z) * NA[2]);
-    return sg * cert32(Q, QA);
-  }
-};
-__device__ inline PairSphereF to_f32(const PairSphere &s) {
-  return {{(float)s.a.x, (float)s.a.y, (float)s.a.z}};
+__device__ inline float norm_up(double x, double y, double z) {
+  return (float)sqrt(x * x + y * y + z * z) * (1.0f + 1e-6f);
 }
-__device__ inline TetSphereF to_f32(const TetSphere &t) {
-  return {(float)t.V, (float)t.VA, {(float)t.N.x, (float)t.N.y, (float)t.N.z},
-          {(float)t.NA.x, (float)t.NA.y, (float)t.NA.z}, t.V > 0 ? 1 : -1};
+__device__ inline SphereF to_f32(const PairSphere &s, bool ascending) {
+  const float l = norm_up(s.a.x, s.a.y, s.a.z);
+  return {1.0f, 1.0f, {(float)s.a.x, (float)s.a.y, (float)s.a.z}, l, ascending ? l * (1.0f + 1e-4f) + 1e-30f : INFINITY};
+}
+__device__ inline SphereF to_f32(const TetSphere &t, bool ascending) {
+  // diameter |N| / |V|; both hold 12 digits at worst below their magnitude
+  // bounds (their signs are certified), hence the wide margin
+  const double sg = t.V > 0 ? 1.0 : -1.0;
+  const double d = sqrt(dot(t.N, t.N)) * __builtin_amdgcn_rcp(fabs(t.V));
+  return {(float)(sg * t.V), (float)t.VA, {(float)(sg * t.N.x), (float)(sg * t.N.y), (float)(sg * t.N.z)},
+          norm_up(t.NA.x, t.NA.y, t.NA.z), ascending ? (float)d * 1.05f + 1e-30f : INFINITY};
 }
 
+// Up to kMaxInterior region slots, 16 bits each, 2 per word.
+constexpr int kPacked = (kMaxInterior + 1) / 2;
+__device__ inline void put_packed(uint32_t (&pk)[kPacked], int n, uint32_t slot) {
+  const uint32_t word = (uint32_t)n >> 1, shift = ((uint32_t)n & 1u) * 16u;
+#pragma unroll
+  for (int k = 0; k < kPacked; ++k) pk[k] |= (uint32_t)k == word ? slot << shift : 0u;
+}
+__device__ inline void unpack_ids(const Work &w, const uint32_t (&pk)[kPacked], int n, uint32_t (&ids)[kMaxInterior]) {
+#pragma unroll
+  for (int j = 0; j < kMaxInterior; ++j) ids[j] = j < n ? w.gid[(pk[j / 2] >> ((j % 2) * 16)) & 0xFFFFu] : kInvalid;
+}
+
+// Certified classification of the region against a candidate sphere through
+// the anchor and m - 1 region points (slots skip).  FP32 for 64 slots at a time
+// into two bit masks (inside, undecided), FP64 for the undecided; the inside
+// slots are packed.  Returns 1 event, 0 not critical, -1 undecided (host).
+// Bound by VALU issue; collecting the ids point by point over the whole region
+// took 24 of the enumeration's 73 ms for the 50 000-point lattice, this about 5.
 template <class S>
-__device__ int classify(const Params &P, const Work &w, uint32_t M, const S &sph,
-                        const uint32_t *skip, int m, uint32_t (&interior)[kMaxInterior], int &nint) {
+__device__ __attribute__((always_inline)) inline int classify(const Params &P, const Work &w, uint32_t M, const S &sph,
+                        const uint32_t *skip, int m, uint32_t (&interior)[kPacked], int &nint) {
   nint = 0;
+#pragma unroll
+  for (int k = 0; k < kPacked; ++k) interior[k] = 0;
   const int cap = P.s_max - m;
   int undecided = 0;
   constexpr uint32_t per = sizeof(S) == sizeof(PairSphere) ? kFlopPairSide : kFlopTetSide;
   constexpr uint32_t per32 = sizeof(S) == sizeof(PairSphere) ? kF32PairSide : kF32TetSide;
   uint32_t evals = 0, evals32 = 0;
-  // FP32 first where the region has FP32 copies; FP64 for what it leaves open
-  const bool f32 = w.fx != nullptr;
-  const auto s32 = to_f32(sph);
-  for (uint32_t s = 0; s < M; ++s) {
-    const uint32_t gi = s;
-    bool on_support = false;
-    for (int k = 0; k < m - 1; ++k) on_support |= (gi == skip[k]);
-    if (on_support) continue;
-    int side = f32 ? s32.side(w.fx[gi], w.fy[gi], w.fz[gi]) : 0;
-    evals32 += f32;
-    if (side == 0) {
-      side = sph.side(gpt(w, gi));
-      evals++;
+  const SphereF f = to_f32(sph, w.ascending);
+  bool over = false;
+#pragma unroll 1
+  for (uint32_t s0 = 0; s0 < M; s0 += 64) {
+    if (w.fw[s0] > f.reach) break;
+    const uint32_t cn = min(64u, M - s0);
+    uint64_t in = 0, open = 0;
+#pragma unroll 4
+    for (uint32_t j = 0; j < cn; ++j) {
+      float v, va;
+      f.test(w.fx[s0 + j], w.fy[s0 + j], w.fz[s0 + j], w.fw[s0 + j], v, va);
+      const float e = fmaxf(1e-5f * va, 1e-35f);
+      in |= (uint64_t)(v < -e) << j;
+      open |= (uint64_t)(!(fabsf(v) > e)) << j;
     }
-    if (side < 0) {
-      put_static(interior, nint, w.gid[gi]);
-      nint++;
-      if (nint > cap) {
-        add_flops(w, (uint64_t)evals * per);
-        add_flops32(w, (uint64_t)evals32 * per32);
-        return 0;
+    evals32 += cn;
+    for (int k = 0; k < m - 1; ++k)
+      if (skip[k] - s0 < cn) {
+        in &= ~(1ull << (skip[k] - s0));
+        open &= ~(1ull << (skip[k] - s0));
       }
-    } else if (side == 0) {
-      undecided++;
+    while (open) {
+      const uint32_t j = (uint32_t)(__ffsll((long long)open) - 1);
+      open &= open - 1;
+      const int side = sph.side(gpt(w, s0 + j));
+      evals++;
+      in |= (uint64_t)(side < 0) << j;
+      undecided += side == 0;
+    }
+    if (nint + __popcll(in) > cap) {
+      over = true;
+      break;
+    }
+    while (in) {
+      put_packed(interior, nint, s0 + (uint32_t)(__ffsll((long long)in) - 1));
+      in &= in - 1;
+      nint++;
     }
   }
   add_flops(w, (uint64_t)evals * per);
   add_flops32(w, (uint64_t)evals32 * per32);
-  return undecided ? -1 : 1;
+  return over ? 0 : undecided ? -1 : 1;
 }
 
 
-__device__ void process_pair(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
+__device__ __attribute__((always_inline)) inline void process_pair(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
                              uint32_t *region_slot) {
   PairSphere sph;
   sph.init(gpt(w, vi));
-  uint32_t interior[kMaxInterior];
+  uint32_t packed[kPacked];
   int nint;
   uint32_t skip[1] = {vi};
-  int r = classify(P, w, M, sph, skip, 2, interior, nint);
+  int r = classify(P, w, M, sph, skip, 2, packed, nint);
   uint32_t vid = w.gid[vi];
   if (r == 0) return;
   atomicAdd(w.cand, 1u);
@@ -338,11 +371,13 @@ __device__ void process_pair(const Params &P, const Work &w, uint32_t u, uint32_
     emit_fallback(P, w, u, 2, &vid, 2, M, region_slot);
     return;
   }
+  uint32_t interior[kMaxInterior];
+  unpack_ids(w, packed, nint, interior);
   sort_static(interior, nint);
   emit_event(P, u, &vid, 2, nint, interior, sph.level(), 8 * kCert);
 }
 
-__device__ void process_tet(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi, uint32_t wi,
+__device__ __attribute__((always_inline)) inline void process_tet(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi, uint32_t wi,
                             uint32_t zi, uint32_t *region_slot) {
   TetSphere t;
   int wc = t.init(gpt(w, vi), gpt(w, wi), gpt(w, zi));
@@ -351,54 +386,40 @@ __device__ void process_tet(const Params &P, const Work &w, uint32_t u, uint32_t
   if (wc < 0) return;
   atomicAdd(w.cand, 1u);
   if (wc == 0) { emit_fallback(P, w, u, 4, ids, 4, M, region_slot); return; }
-  uint32_t interior[kMaxInterior];
+  uint32_t packed[kPacked];
   int nint;
   uint32_t skip[3] = {vi, wi, zi};
-  int r = classify(P, w, M, t, skip, 4, interior, nint);
+  int r = classify(P, w, M, t, skip, 4, packed, nint);
   if (r == 0) return;
   if (r < 0) { emit_fallback(P, w, u, 4, ids, 4, M, region_slot); return; }
+  uint32_t interior[kMaxInterior];
+  unpack_ids(w, packed, nint, interior);
   sort_static(interior, nint);
   emit_event(P, u, ids, 4, nint, interior, t.level(), t.level_err());
 }
 
-// Smallest sweep keys of the outside points ahead of one side: tau with its
-// error bound and the region slot.  Insertion runs over static indices, so
-// the list stays in registers.
+// Smallest upper bounds of the sweep keys of the outside points ahead of one
+// side.  Insertion runs over static indices, so the list stays in registers.
 struct SweepList {
   static constexpr int kCap = 8;  // >= s_max - 3 for s_max <= 11
   double hi[kCap];                // upper key bounds, ascending
-  float err[kCap];                // key error bounds (key = hi - err)
-  uint32_t slot[kCap];
-  double evicted_lo;  // smallest lower key bound of a point not in the list
   __device__ void init() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) { hi[j] = INFINITY; err[j] = 0.f; slot[j] = kInvalid; }
-    evicted_lo = INFINITY;
+    for (int j = 0; j < kCap; ++j) hi[j] = INFINITY;
   }
-  __device__ void insert(double t, double e, uint32_t s) {
-    const double h = t + e;
-    if (!(h < hi[kCap - 1])) {
-      evicted_lo = fmin(evicted_lo, t - e);
-      return;
-    }
-    evicted_lo = fmin(evicted_lo, hi[kCap - 1] - 2.0 * (double)err[kCap - 1]);
-    const float ef = (float)e * (1.0f + 1e-6f);
+  __device__ void insert(double t, double e) {
+    double h = t + e;
 #pragma unroll
-    for (int j = kCap - 1; j > 0; --j) {
-      const bool shift = h < hi[j - 1];
-      const bool place = !shift && h < hi[j];
-      hi[j] = shift ? hi[j - 1] : (place ? h : hi[j]);
-      err[j] = shift ? err[j - 1] : (place ? ef : err[j]);
-      slot[j] = shift ? slot[j - 1] : (place ? s : slot[j]);
+    for (int j = 0; j < kCap; ++j) {
+      const double lo = fmin(hi[j], h);
+      h = fmax(hi[j], h);
+      hi[j] = lo;
     }
-    if (h < hi[0]) { hi[0] = h; err[0] = ef; slot[0] = s; }
   }
-  // upper key bound of the need-th entry (need in 1..kCap)
-  __device__ double threshold(int need) const {
-    double r = INFINITY;
+  __device__ void pop() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) r = (j == need - 1) ? hi[j] : r;
-    return r;
+    for (int j = 0; j + 1 < kCap; ++j) hi[j] = hi[j + 1];
+    hi[kCap - 1] = INFINITY;
   }
 };
 
@@ -541,22 +562,20 @@ __device__ inline void key_bounds_f(double tau, double terr, float &hf, float &l
 // underflow then adds at most ~1e-37, far below the threshold).  Undecided
 // points take the FP64 path.
 struct TriSphereF {
-  float D, DA, g[3], gA[3], n[3], nA[3];
+  float D, DA, g[3], gA, n[3], nA;  // gA, nA: norms, which bound the sums of magnitudes
   __device__ void init(const TriSphere &f) {
     D = (float)f.D;
     DA = (float)f.DA;
     g[0] = (float)f.g.x; g[1] = (float)f.g.y; g[2] = (float)f.g.z;
-    gA[0] = (float)f.gA.x; gA[1] = (float)f.gA.y; gA[2] = (float)f.gA.z;
+    gA = norm_up(f.gA.x, f.gA.y, f.gA.z);
     n[0] = (float)f.n.x; n[1] = (float)f.n.y; n[2] = (float)f.n.z;
-    nA[0] = (float)f.nA.x; nA[1] = (float)f.nA.y; nA[2] = (float)f.nA.z;
+    nA = norm_up(f.nA.x, f.nA.y, f.nA.z);
   }
-  __device__ void eval(float x, float y, float z, float &P, float &PA, float &H, float &HA) const {
-    const float pp = x * x + y * y + z * z;
-    const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
-    P = D * pp - (x * g[0] + y * g[1] + z * g[2]);
-    PA = DA * pp + (ax * gA[0] + ay * gA[1] + az * gA[2]);
+  __device__ void eval(float x, float y, float z, float w, float &P, float &PA, float &H, float &HA) const {
+    P = D * (w * w) - (x * g[0] + y * g[1] + z * g[2]);
+    PA = w * (DA * w + gA);
     H = x * n[0] + y * n[1] + z * n[2];
-    HA = ax * nA[0] + ay * nA[1] + az * nA[2];
+    HA = w * nA;
   }
 };
 // Key interval of a point whose FP32 signs are certified: the true P lies
@@ -585,11 +604,6 @@ __device__ inline void key_bounds_32(float Pv, float PA, float H, float HA, floa
   lf = lo;
 }
 
-// Apexes of one side of a face: the outside points ahead of the side whose
-// sweep key is among the s_max-3 smallest (fewer when inside points are
-// already ahead), each checked against the inside points behind the side.
-// One pass over the region fills the side's sweep list; the candidates are
-// packed into a mask before any tetrahedron is classified.
 // The part of a face's pencil that can be critical: spheres through u, v, w
 // with centres c3 + t n, t in an interval [tl, tu] (face_interval).  A point's
 // power against such a sphere is linear in t, so a point outside both end
@@ -600,8 +614,9 @@ __device__ inline void key_bounds_32(float Pv, float PA, float H, float HA, floa
 struct Pencil {
   float l[3], u[3];  // twice the end centres
   float a;           // infinite: every point is kept
-  __device__ bool outside(float x, float y, float z) const {
-    const float pp = x * x + y * y + z * z;
+  float reach;       // no point farther from the anchor is in any of the spheres (as SphereF::reach)
+  __device__ bool outside(float x, float y, float z, float w) const {
+    const float pp = w * w;
     const float dl = x * l[0] + y * l[1] + z * l[2], du = x * u[0] + y * u[1] + z * u[2];
     return pp * 0.999f - a > fmaxf(dl, du);
   }
@@ -609,9 +624,10 @@ struct Pencil {
 
 // Ends of the pencil for t in [lo, hi] x r3 (r3: the face's circumradius);
 // lo = -infinity: not restricted.
-__device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi) {
+__device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi, bool ascending) {
   Pencil c{};
   c.a = INFINITY;
+  c.reach = INFINITY;
   if (!(lo > -INFINITY)) return c;
   const double s = 1.0 / f.D;
   const V3 k = {f.g.x * s, f.g.y * s, f.g.z * s};  // twice the circumcentre
@@ -626,7 +642,9 @@ __device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi) {
     ll += cl[i] * cl[i];
     uu += cu[i] * cu[i];
   }
-  c.a = (float)(1e-8 * fmax(ll, uu)) + 1e-34f;
+  const double m2 = fmax(ll, uu);  // the larger sphere's squared diameter
+  c.a = (float)(1e-8 * m2) + 1e-34f;
+  if (ascending) c.reach = (float)sqrt(m2) * (1.0f + 1e-4f) + 1e-30f;
   return c;
 }
 
@@ -643,7 +661,7 @@ __device__ inline uint64_t pencil_chunk(const Work &w, const Pencil &c, uint32_t
 #pragma unroll 4
   for (uint32_t j = 0; j < cn; ++j) {
     const uint32_t gi = s0 + j;
-    const bool keep = !c.outside(w.fx[gi], w.fy[gi], w.fz[gi]);
+    const bool keep = !c.outside(w.fx[gi], w.fy[gi], w.fz[gi], w.fw[gi]);
     in |= (uint64_t)keep << j;
   }
   if (vi - s0 < cn) in &= ~(1ull << (vi - s0));
@@ -652,148 +670,38 @@ __device__ inline uint64_t pencil_chunk(const Work &w, const Pencil &c, uint32_t
   return in;
 }
 
-// Per-wave work queues of the face phase (LDS).  The first pass of every
-// face runs one face per lane; the per-side passes and the tetrahedra it
-// leads to are queued and then taken one per lane, so the lanes of a wave
-// run passes of equal length instead of waiting for the face with the most
-// apexes.  A full queue falls back to doing the work in place.
-constexpr uint32_t kSideQ = 64;
+// Per-wave work queue of the face phase (LDS).  The pass of every face runs
+// one face per lane; the tetrahedra it leads to are queued and then taken one
+// per lane, so the lanes of a wave run scans of equal length instead of
+// waiting for the face with the most apexes.  A full queue falls back to doing the work in place.
 constexpr uint32_t kTetQ = 256;
 struct WaveQueues {
-  uint32_t *side;    // vi | wi << 10 | side << 20 | cin << 21 (region slots, < 1024)
-  float *side_lo, *side_hi;  // the face's pencil interval: the side pass rebuilds exactly the face pass's pencil
-  uint32_t *tet;     // vi | wi << 10 | zi << 20
-  uint32_t *nside, *ntet;
+  uint32_t *tet;     // vi | wi << 10 | zi << 20 (region slots, < 1024)
+  uint32_t *ntet;
 };
 
-__device__ void process_tet(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi, uint32_t wi,
-                            uint32_t zi, uint32_t *region_slot);
+// A side of a face whose apexes its face's list does not decide (near-equal
+// keys past its end, a few thousand in 25 million records): the face by its
+// PointIds with its pencil interval, and the inside points ahead of the side.
+// Settled by k_rescan from the anchor's slab; in the enumeration kernel the
+// FP64 passes of these sides cost 160 spilled registers.
+struct Rescan {
+  uint32_t anchor;  // slab of the launch
+  uint32_t v, w;
+  uint32_t side;    // side | cin << 1
+  float lo, hi;
+};
 
-__device__ void face_side_apexes(const Params &P, const Work &w, uint32_t u, uint32_t M, const TriSphere &f,
-                                 const Pencil &pen, uint32_t vi, uint32_t wi, uint32_t wid, int side,
-                                 int cin_side, int K, uint32_t *region_slot, WaveQueues *q) {
-  const int need = K - cin_side;  // slots left for points swept before z
-  if (need <= 0) return;
-  SweepList top;
-  BehindList beh;
-  top.init();
-  beh.init();
-  bool undecided = false;
-  uint32_t tests = 0, evals = 0;
-  // a point outside every feasible sphere of the pencil can neither be an
-  // apex nor be swept before one (dropping it only loosens the threshold)
-#pragma unroll 1
-  for (uint32_t s0 = 0; s0 < M; s0 += 64) {
-    uint64_t in = pencil_chunk(w, pen, s0, M, vi, wi, tests);
-#pragma unroll 1
-    while (in) {
-      const uint32_t s = s0 + (uint32_t)(__ffsll((long long)in) - 1);
-      in &= in - 1;
-      const V3 p = gpt(w, s);
-      evals++;
-      double Pw, PA, H, HA;
-      f.power(p, Pw, PA);
-      f.height(p, H, HA);
-      const int sp = cert_sign(Pw, PA), sh = cert_sign(H, HA);
-      undecided |= sp == 0 || sh == 0;
-      const bool ahead = side == 0 ? sh > 0 : sh < 0;
-      double tau, terr;
-      sweep_key(Pw, PA, H, HA, tau, terr);
-      if (sp < 0) {
-        // inside the triangle's sphere, behind this side: inside the
-        // pencil's spheres until the sweep key reaches -tau
-        if (!ahead) beh.insert(-tau - terr);
-      } else if (ahead) {
-        top.insert(tau, terr, s);
-      }
-    }
-  }
-  add_flops(w, (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
-  add_flops32(w, (uint64_t)tests * kF32Pencil);
-  // the face pass certified every sign with the same arithmetic
-  if (undecided) return;
-  const double thr = top.threshold(need);
-  // evicted_lo stays +inf while no point has left or missed the list (every
-  // candidate is then listed, also when fewer than `need` are: thr = +inf)
+// Apexes of one side among the FP32 list its face's first pass filled: bit j
+// for entry j.  rescan: a point left or missed the list with a lower bound
+// within the threshold, so the side takes its own passes instead.
+__device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF &top, const BehindListF &beh, bool &rescan) {
+  rescan = false;
+  if (cin_side >= K) return 0;
+  const float thr = top.threshold(K - cin_side);
   if (top.evicted_lo != INFINITY && top.evicted_lo <= thr) {
-    // a point outside the list may still qualify (near-equal keys): full scan
-    tests = evals = 0;
-#pragma unroll 1
-    for (uint32_t s = 0; s < M; ++s) {
-      const uint32_t zi = s;
-      if (zi == vi || zi == wi || w.gid[zi] <= wid) continue;
-      const V3 p = gpt(w, zi);
-      tests++;
-      if (pen.outside(w.fx[zi], w.fy[zi], w.fz[zi])) continue;
-      evals++;
-      double Pw, PA, H, HA;
-      f.power(p, Pw, PA);
-      f.height(p, H, HA);
-      if (cert_sign(Pw, PA) <= 0) continue;
-      const int sh = cert_sign(H, HA);
-      if ((side == 0 && sh <= 0) || (side == 1 && sh >= 0)) continue;
-      double tau, terr;
-      sweep_key(Pw, PA, H, HA, tau, terr);
-      if (tau - terr > thr) continue;
-      if (cin_side + beh.count_above(tau + terr) >= K) continue;
-      process_tet(P, w, u, M, vi, wi, zi, region_slot);
-    }
-    add_flops(w, (uint64_t)evals * (kFlopFacePoint + kFlopSweepKey));
-    add_flops32(w, (uint64_t)tests * kF32Pencil);
-    return;
-  }
-  uint32_t cand = 0;
-#pragma unroll
-  for (int j = 0; j < SweepList::kCap; ++j) {
-    const double terr = (double)top.err[j], h = top.hi[j];
-    // inside points behind: counted while their key exceeds z's
-    const bool ok = top.slot[j] != kInvalid && h - 2.0 * terr <= thr && cin_side + beh.count_above(h) < K;
-    cand |= ok ? (1u << j) : 0u;
-  }
-  while (cand) {
-    const int j = __ffs(cand) - 1;
-    cand &= cand - 1;
-    uint32_t slot = 0;  // selected by static index, the list stays in registers
-#pragma unroll
-    for (int q = 0; q < SweepList::kCap; ++q) slot = q == j ? top.slot[q] : slot;
-    const uint32_t zi = slot;
-    if (w.gid[zi] <= wid) continue;
-    if (q) {
-      const uint32_t at = atomicAdd(q->ntet, 1u);
-      if (at < kTetQ) {
-        q->tet[at] = vi | (wi << 10) | (zi << 20);
-        continue;
-      }
-    }
-    process_tet(P, w, u, M, vi, wi, zi, region_slot);
-  }
-}
-
-// Apexes of one side from the FP32 lists its face's first pass filled (the
-// tail of face_side_apexes).  When a point left or missed the list with a
-// lower bound within the threshold, the side takes its own pass instead
-// (queued, with the full scan that case needs).
-__device__ inline void fused_side(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi, uint32_t wi,
-                                  uint32_t wid, int side, int cin_side, int K, const SweepListF &top,
-                                  const BehindListF &beh, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
-  const int need = K - cin_side;
-  const float thr = top.threshold(need);
-  if (top.evicted_lo != INFINITY && top.evicted_lo <= thr) {
-    if (q) {
-      const uint32_t at = atomicAdd(q->nside, 1u);
-      if (at < kSideQ) {
-        q->side[at] = vi | (wi << 10) | ((uint32_t)side << 20) | ((uint32_t)cin_side << 21);
-        q->side_lo[at] = lo;
-        q->side_hi[at] = hi;
-        return;
-      }
-    }
-    // in place (global-memory path, full queue): the face's sphere rebuilt
-    // (same arithmetic, same values), then the side's own pass
-    TriSphere f;
-    f.init(gpt(w, vi), gpt(w, wi));
-    face_side_apexes(P, w, u, M, f, face_pencil(f, lo, hi), vi, wi, wid, side, cin_side, K, region_slot, q);
-    return;
+    rescan = true;
+    return 0;
   }
   uint32_t cand = 0;
 #pragma unroll
@@ -803,35 +711,21 @@ __device__ inline void fused_side(const Params &P, const Work &w, uint32_t u, ui
                     cin_side + beh.count_above(top.hi[j]) < K;
     cand |= ok ? (1u << j) : 0u;
   }
-  while (cand) {
-    const int j = __ffs(cand) - 1;
-    cand &= cand - 1;
-    uint32_t ent = 0;  // selected by static index, the list stays in registers
-#pragma unroll
-    for (int qq = 0; qq < SweepListF::kCap; ++qq) ent = qq == j ? top.ent[qq] : ent;
-    const uint32_t zi = entry_slot(ent);
-    if (w.gid[zi] <= wid) continue;
-    if (q) {
-      const uint32_t at = atomicAdd(q->ntet, 1u);
-      if (at < kTetQ) {
-        q->tet[at] = vi | (wi << 10) | (zi << 20);
-        continue;
-      }
-    }
-    process_tet(P, w, u, M, vi, wi, zi, region_slot);
-  }
+  return cand;
 }
 
 // Face (u, v, w): its triangle event, then the apexes of each side.  One
 // pass certifies every side and insideness, builds the triangle's interior,
 // counts the inside points ahead of each side and fills both sides' sweep
-// lists, from which the apexes follow (fused_side).  QUEUED (LDS paths):
-// tetrahedra and rescans go to the wave's queues; otherwise in place.  The
-// pass runs on the region's FP32 copies (FP64 only for the points whose FP32
+// lists, from which the apexes follow (apex_mask): the outside points ahead of
+// the side whose sweep key is among the s_max - 3 smallest (fewer when inside
+// points are already ahead), each checked against the inside points behind.
+// QUEUED (LDS paths): tetrahedra go to the wave's queue; otherwise in place.
+// The pass runs on the region's FP32 copies (FP64 only for the points whose FP32
 // signs are not certified) and sees the points that some sphere of the face's
 // pencil within [lo, hi] (face_interval; n oriented as v x w) can hold.
 template <bool QUEUED>
-__device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
+__device__ __attribute__((always_inline)) inline void process_face(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
                              uint32_t wi, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
   // the sphere is built from its points in PointId order, so its FP64 level
   // (and every later tetrahedron's) does not depend on the enumeration order
@@ -849,7 +743,7 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   const uint32_t wid = ids[1];
   const int smax = P.s_max;
   const int K = smax - 3;  // an apex must be among the first K points swept
-  const Pencil pen = face_pencil(f, lo, hi);
+  const Pencil pen = face_pencil(f, lo, hi, w.ascending);
   // the triangle's own sphere (t = 0) is critical only within the interval;
   // a side that the interval does not reach has no apexes
   const bool tri = lo <= 0.0f && hi >= 0.0f;
@@ -858,9 +752,9 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   // inside the triangle's sphere, ahead of side 0 / 1
   int cin0 = hi < 0.0f ? K : 0, cin1 = lo > 0.0f ? K : 0;
   int total_in = 0;
-  // region slots of the first 8 inside points, 16 bits each, 2 per word (a
-  // triangle event has at most s_max - 3 <= 8 interior points)
-  uint32_t tri_pk[4] = {0u, 0u, 0u, 0u};
+  // region slots of the first inside points (a triangle event has at most
+  // s_max - 3 <= 8)
+  uint32_t tri_pk[kPacked] = {};
   uint32_t evals = 0;
   SweepListF top0, top1;  // outside points ahead of side 0 / 1
   BehindListF beh0, beh1;  // inside points behind side 0 / 1
@@ -874,6 +768,7 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   f32.init(f);
 #pragma unroll 1
   for (uint32_t s0 = 0; s0 < M; s0 += 64) {
+    if (w.fw[s0] > pen.reach) break;
     uint64_t in = pencil_chunk(w, pen, s0, M, vi, wi, tests32);
 #pragma unroll 1
     while (in) {
@@ -881,7 +776,7 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
       in &= in - 1;
       float hf = 0.0f, lf = 0.0f;
       float P32, PA32, H32, HA32;
-      f32.eval(w.fx[gi], w.fy[gi], w.fz[gi], P32, PA32, H32, HA32);
+      f32.eval(w.fx[gi], w.fy[gi], w.fz[gi], w.fw[gi], P32, PA32, H32, HA32);
       int sp = cert32(P32, PA32), sh = cert32(H32, HA32);
       evals32++;
       if (sp != 0 && sh != 0) {
@@ -921,11 +816,7 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
         else beh0.insert(-hf);
       }
       if (sp > 0) continue;
-      if (total_in < 8) {
-        const uint32_t word = (uint32_t)total_in >> 1, shift = ((uint32_t)total_in & 1u) * 16u;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) tri_pk[k] |= (uint32_t)k == word ? gi << shift : 0u;
-      }
+      if (total_in < kMaxInterior) put_packed(tri_pk, total_in, gi);
       total_in++;
       cin0 += sh > 0;
       cin1 += sh < 0;
@@ -945,9 +836,7 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
   } else if (wc > 0 && total_in + 3 <= smax) {
     atomicAdd(w.cand, 1u);
     uint32_t tri_int[kMaxInterior];
-#pragma unroll
-    for (int j = 0; j < kMaxInterior; ++j)
-      tri_int[j] = j < 8 && j < total_in ? w.gid[(tri_pk[j / 2] >> ((j % 2) * 16)) & 0xFFFFu] : kInvalid;
+    unpack_ids(w, tri_pk, total_in, tri_int);
     sort_static(tri_int, total_in);
     emit_event(P, u, ids, 3, total_in, tri_int, tri_level, tri_level_err);
   } else if (wc == 0 && total_in + 3 <= smax) {
@@ -955,28 +844,36 @@ __device__ void process_face(const Params &P, const Work &w, uint32_t u, uint32_
     return;
   }
   if (K <= 0) return;
+  bool rescan[2];
+  uint32_t cand = apex_mask(cin0, K, top0, beh0, rescan[0]);
+  cand |= apex_mask(cin1, K, top1, beh1, rescan[1]) << SweepListF::kCap;
   // queued on the LDS paths, in place on the global-memory path
-  WaveQueues *qq = QUEUED ? q : nullptr;
-  if (cin0 < K) fused_side(P, w, u, M, vi, wi, wid, 0, cin0, K, top0, beh0, lo, hi, region_slot, qq);
-  if (cin1 < K) fused_side(P, w, u, M, vi, wi, wid, 1, cin1, K, top1, beh1, lo, hi, region_slot, qq);
-}
-
-// A queued side of a face: the face's sphere rebuilt (same arithmetic, same
-// values), then the side's pass.
-__device__ void side_item(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t item, float lo, float hi,
-                          uint32_t *region_slot, WaveQueues *q) {
-  const uint32_t vi = item & 1023u, wi = (item >> 10) & 1023u, side = (item >> 20) & 1u, cin_side = item >> 21;
-  TriSphere f;
-  f.init(gpt(w, vi), gpt(w, wi));
-  add_flops(w, kFlopTriInit);
-  face_side_apexes(P, w, u, M, f, face_pencil(f, lo, hi), vi, wi, w.gid[wi], (int)side, (int)cin_side, P.s_max - 3,
-                   region_slot, q);
-}
-
-__device__ void tet_item(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t item,
-                         uint32_t *region_slot) {
-  const uint32_t vi = item & 1023u, wi = (item >> 10) & 1023u, zi = item >> 20;
-  process_tet(P, w, u, M, vi, wi, zi, region_slot);
+  while (cand) {
+    const int j = __ffs(cand) - 1;
+    cand &= cand - 1;
+    uint32_t ent = 0;  // selected by static index, the lists stay in registers
+#pragma unroll
+    for (int e = 0; e < SweepListF::kCap; ++e) {
+      ent = e == j ? top0.ent[e] : ent;
+      ent = e + SweepListF::kCap == j ? top1.ent[e] : ent;
+    }
+    const uint32_t zi = entry_slot(ent);
+    if (w.gid[zi] <= wid) continue;
+    if (QUEUED) {
+      const uint32_t at = atomicAdd(q->ntet, 1u);
+      if (at < kTetQ) {
+        q->tet[at] = vi | (wi << 10) | (zi << 20);
+        continue;
+      }
+    }
+    process_tet(P, w, u, M, vi, wi, zi, region_slot);
+  }
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    if (!rescan[side]) continue;
+    const unsigned long long at = atomicAdd(&P.counters[4], 1ull);
+    if (at < P.rescan_cap) P.rescans[at] = Rescan{w.slab, ids[0], ids[1], (uint32_t)side | ((uint32_t)(side ? cin1 : cin0) << 1), lo, hi};
+  }
 }
 
 // Cell direction and angular radius in FP32, rounded so that the cell only
@@ -1172,7 +1069,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       const uint32_t s = s0 + t;
       const bool above = s < M && w.gid[min(s, M - 1)] > u;
       const uint64_t m = __ballot(above);
-      if (above) w.kidx[k + (uint32_t)__popcll(m & ((1ull << t) - 1ull))] = s;
+      if (above) w.kidx[k + (uint32_t)__popcll(m & ((1ull << t) - 1ull))] = (uint16_t)s;
       k += (uint32_t)__popcll(m);
     }
     if (t == 0) sK = k;
@@ -1181,6 +1078,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     w.fx[s] = (float)w.gx[s];
     w.fy[s] = (float)w.gy[s];
     w.fz[s] = (float)w.gz[s];
+    w.fw[s] = (float)sqrt(w.gx[s] * w.gx[s] + w.gy[s] * w.gy[s] + w.gz[s] * w.gz[s]);
   }
   __syncthreads();
   const uint32_t Kc = sK;
@@ -1198,24 +1096,24 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   // takes 64 candidate faces at a time: first passes one per lane, then the
   // queued sides and tetrahedra one per lane (LDS path; the global-memory
   // path works in place).
-  __shared__ uint32_t q_side[WAVES][kSideQ];
-  __shared__ float q_side_lo[WAVES][kSideQ], q_side_hi[WAVES][kSideQ];
+  __shared__ uint32_t q_pair[WAVES][128];
   __shared__ uint32_t q_face[WAVES][128];
   __shared__ float q_key[WAVES][128], q_lo[WAVES][128], q_hi[WAVES][128];
   __shared__ uint32_t q_tet[WAVES][kTetQ];
-  __shared__ uint32_t q_n[WAVES][2];
+  __shared__ uint32_t q_n[WAVES];
   const int wave = t >> 6, lane = t & 63, nwaves = (int)(blockDim.x >> 6);
-  WaveQueues wq{q_side[wave], q_side_lo[wave], q_side_hi[wave], q_tet[wave], &q_n[wave][0], &q_n[wave][1]};
+  WaveQueues wq{q_tet[wave], &q_n[wave]};
   WaveQueues *q = BIG ? nullptr : &wq;
-  if (lane == 0) { q_n[wave][0] = 0; q_n[wave][1] = 0; }
+  if (lane == 0) q_n[wave] = 0;
   wave_sync();
   // candidate face fidx -> region slots of (v, w): the pair (i < j) of the
   // strictly lower triangle
   auto face_of = [&](uint64_t fidx, uint32_t &si, uint32_t &sj) {
-    uint64_t j = (uint64_t)((1.0 + sqrt(1.0 + 8.0 * (double)fidx)) * 0.5);
-    while (j * (j - 1) / 2 > fidx) j--;
-    while ((j + 1) * j / 2 <= fidx) j++;
-    const uint64_t i = fidx - j * (j - 1) / 2;
+    const uint32_t f = (uint32_t)fidx;  // at most 2048 x 2047 / 2
+    uint32_t j = (uint32_t)((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * (float)f)) * 0.5f);
+    while (j * (j - 1) / 2 > f) j--;
+    while ((j + 1) * j / 2 <= f) j++;
+    const uint32_t i = f - j * (j - 1) / 2;
     si = w.kidx[i];
     sj = w.kidx[j];
   };
@@ -1229,36 +1127,51 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false>(P, w, u, M, si, sj, lo, hi, &sregion, q);
     }
   } else {
-    // Each wave first collects up to 128 feasible faces in its LDS list with
-    // their pencil intervals (the faces without one cost only the test),
-    // orders them by the extent of their pencils, then runs the first passes
+    // Each wave lists the candidate faces that share a cell (q_pair), takes 64
+    // of them at a time through the interval test, so that its lanes are full
+    // (about half of the candidates share none), and collects up to 128
+    // feasible faces with their pencil intervals; it orders them by the extent of their pencils, then runs the first passes
     // of the 64 largest one per lane (lanes of similar work), then the queued
-    // sides and tetrahedra; the smaller ones wait for the next round.
-    uint32_t nf = 0;  // faces in the wave's list (uniform)
+    // tetrahedra; the smaller ones wait for the next round.
+    uint32_t nf = 0, np = 0;  // faces and candidates in the wave's lists (uniform)
     uint64_t cbase = ((uint64_t)part * nwaves + wave) * 64;
     const uint64_t cstride = (uint64_t)parts * nwaves * 64;
     for (;;) {
-      while (nf <= 64 && cbase < F) {
-        const uint64_t fidx = cbase + lane;
+      while (nf <= 64 && (np || cbase < F)) {
+        while (np < 64 && cbase < F) {
+          const uint64_t fidx = cbase + lane;
+          bool share = false;
+          uint32_t si = 0, sj = 0;
+          if (fidx < F) {
+            face_of(fidx, si, sj);
+            for (int k = 0; k < 6; ++k) share |= (w.rmask[6 * si + k] & w.rmask[6 * sj + k]) != 0;
+          }
+          const uint64_t m = __ballot(share);
+          if (share) q_pair[wave][np + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = si | (sj << 10);
+          np += (uint32_t)__popcll(m);
+          cbase += cstride;
+        }
+        wave_sync();
+        const uint32_t got = min(np, 64u);
+        np -= got;
         bool ok = false;
-        uint32_t si = 0, sj = 0;
+        uint32_t fv = 0;
         float key = 0.0f, lo = 0.0f, hi = 0.0f;
-        if (fidx < F) {
-          face_of(fidx, si, sj);
-          ok = face_interval(P, w, si, sj, lo, hi, key);
+        if ((uint32_t)lane < got) {
+          fv = q_pair[wave][np + lane];
+          ok = face_interval(P, w, fv & 1023u, fv >> 10, lo, hi, key);
         }
         const uint64_t m = __ballot(ok);
         if (ok) {
           const uint32_t at = nf + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-          q_face[wave][at] = si | (sj << 10);
+          q_face[wave][at] = fv;
           q_key[wave][at] = key;
           q_lo[wave][at] = lo;
           q_hi[wave][at] = hi;
         }
         nf += (uint32_t)__popcll(m);
-        cbase += cstride;
+        wave_sync();  // the list's words are read before the next ones take them
       }
-      if (nf == 0) break;
       wave_sync();
       if (nf > 64) {
         // rank sort of the list by key (ties by position), ascending
@@ -1303,21 +1216,21 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
         process_face<true>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
       }
       wave_sync();
-      const uint32_t ns = min(q_n[wave][0], kSideQ);
-      for (uint32_t it = lane; it < ns; it += 64)
-        side_item(P, w, u, M, q_side[wave][it], q_side_lo[wave][it], q_side_hi[wave][it], &sregion, q);
-      wave_sync();
       // whole rounds of 64 tetrahedra (the top of the queue); the rest waits
-      // for the next round's, so that the lanes stay busy
-      const uint32_t nt = min(q_n[wave][1], kTetQ);
-      const uint32_t full = nt & ~63u;
-      for (uint32_t it = nt - full + lane; it < nt; it += 64) tet_item(P, w, u, M, q_tet[wave][it], &sregion);
+      // for the next round's, so that the lanes stay busy, or ends the anchor
+      const bool last = nf == 0 && np == 0 && cbase >= F;
+      const uint32_t nt = min(q_n[wave], kTetQ);
+      const uint32_t full = last ? nt : nt & ~63u;
+#pragma unroll 1
+      for (uint32_t it = nt - full + lane; it < nt; it += 64) {
+        const uint32_t item = q_tet[wave][it];
+        process_tet(P, w, u, M, item & 1023u, (item >> 10) & 1023u, item >> 20, &sregion);
+      }
+      if (last) break;
       wave_sync();
-      if (lane == 0) { q_n[wave][0] = 0; q_n[wave][1] = nt - full; }
+      if (lane == 0) q_n[wave] = nt - full;
       wave_sync();
     }
-    const uint32_t nt = min(q_n[wave][1], kTetQ);
-    for (uint32_t it = lane; it < nt; it += 64) tet_item(P, w, u, M, q_tet[wave][it], &sregion);
   }
   __syncthreads();
   if (t == 0) {
@@ -1751,19 +1664,21 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
   w.rmask = (uint64_t *)(slab + slab_masks(G));
   w.gid = (uint32_t *)(slab + slab_ids(G));
   w.ridx = w.gid + G;
-  w.kidx = w.ridx + G;
+  w.kidx = reinterpret_cast<uint16_t *>(w.ridx + G);
   w.fc = reinterpret_cast<float4 *>(slab + big_fc_offset(G));
   // the FP32 region copies take the FP32 offsets' area once the region is
-  // compacted (4G floats hold 3G)
+  // compacted (4G floats)
   w.fx = reinterpret_cast<float *>(w.fc);
   w.fy = w.fx + G;
   w.fz = w.fy + G;
+  w.fw = w.fz + G;
   __shared__ uint32_t cand;
   __shared__ unsigned long long flops;
   if (threadIdx.x == 0) { cand = 0; flops = 0; }
   __syncthreads();
   w.cand = &cand;
   w.flops = P.count_flops ? &flops : nullptr;
+  w.slab = a;
   anchor_work(P, w, u, a);
 }
 
@@ -1779,6 +1694,14 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
 // asks for about kRegionParts workgroups in all, a few per CU slot so that
 // the longest ones do not end it alone.  A 2 003-point mixture's catalogue:
 // 885 -> 332 ms.
+//
+// VALU bound: of 58 ms for the 50 000-point lattice K 10 (25 million records)
+// about 27 are the faces' passes, 18 the pairs of vertices that share a cell
+// and their intervals, 4 the tetrahedra, and 7 the loads, pairs and queues.
+// Its registers were what held it back (FP64 state of rare passes spilled 160
+// of them); with those passes in k_rescan, scans that end at a sphere's
+// diameter and id lists read from bit masks: 73 -> 58 ms, K 4 19.3 -> 18.3 ms,
+// the mixture's catalogue 75.6 -> 67.2 ms.
 constexpr uint32_t kRegionParts = 4096;
 template <int RCAP, int WAVES, int PER_SIMD>
 __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P, const uint32_t *__restrict__ list) {
@@ -1794,24 +1717,178 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   __shared__ uint32_t gid[RCAP];
   __shared__ float rho[kCells];
   __shared__ uint64_t rmask[6 * RCAP];
-  __shared__ uint32_t kidx[RCAP];
-  __shared__ float fx[RCAP], fy[RCAP], fz[RCAP];
+  __shared__ uint16_t kidx[RCAP];
+  __shared__ float fx[RCAP], fy[RCAP], fz[RCAP], fw[RCAP];
   __shared__ uint32_t cand, sK, sregion;
   __shared__ unsigned long long flops, flops32;
   const int t = threadIdx.x;
-  for (uint32_t i = t; i < M; i += blockDim.x) {
-    gx[i] = slab[i];
-    gy[i] = slab[G + i];
-    gz[i] = slab[2 * G + i];
-    gid[i] = sgid[i];
+  if (P.ascending) {
+    for (uint32_t i = t; i < M; i += blockDim.x) {
+      gx[i] = slab[i];
+      gy[i] = slab[G + i];
+      gz[i] = slab[2 * G + i];
+      gid[i] = sgid[i];
+    }
+    for (uint32_t i = t; i < 6 * M; i += blockDim.x) rmask[i] = smask[i];
+  } else {
+    // into increasing distance from the anchor (the same in every workgroup)
+    constexpr int kPer = (RCAP + 64 * WAVES - 1) / (64 * WAVES);
+    for (uint32_t i = t; i < M; i += blockDim.x) {
+      const double x = slab[i], y = slab[G + i], z = slab[2 * G + i];
+      gx[i] = x * x + y * y + z * z;
+    }
+    __syncthreads();
+    uint32_t rank[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const uint32_t i = t + r * 64 * WAVES;
+      const double d = i < M ? gx[i] : 0.0;
+      rank[r] = 0;
+      for (uint32_t j = 0; j < M; ++j) rank[r] += gx[j] < d || (gx[j] == d && j < i);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const uint32_t i = t + r * 64 * WAVES, q = rank[r];
+      if (i >= M) continue;
+      gx[q] = slab[i];
+      gy[q] = slab[G + i];
+      gz[q] = slab[2 * G + i];
+      gid[q] = sgid[i];
+      for (int k = 0; k < 6; ++k) rmask[6 * q + k] = smask[6 * (uint64_t)i + k];
+    }
   }
-  for (uint32_t i = t; i < 6 * M; i += blockDim.x) rmask[i] = smask[i];
   for (int c = t; c < kCells; c += blockDim.x) rho[c] = reinterpret_cast<const float *>(slab + 3 * G)[c];
   if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; flops32 = 0; }
   __syncthreads();
-  Work w{gx, gy, gz, gid, rho, kidx, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz,
-         P.count_flops ? &flops32 : nullptr};
+  Work w{gx, gy, gz, gid, rho, nullptr, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz, fw,
+         P.count_flops ? &flops32 : nullptr, true, a};
   anchor_faces<false, true, WAVES>(P, w, u, M, &sK, &sregion);
+}
+
+// Sides of faces left by the enumeration of one launch, one per wave, in FP64
+// over the anchor's slab (lanes over the points that the pencil can hold): a
+// first scan finds the side's key threshold and the inside points behind it, a
+// second one the apexes, each classified against the whole region.  The face
+// pass has certified every sign with the same arithmetic.  Few sides come here
+// (0 to a few hundred of a catalogue), so their latency counts: M / 64 steps
+// a scan.  The grid is fixed; the number of sides is read on the device.
+constexpr int kRescanBlocks = 1024;
+__global__ void __launch_bounds__(64) k_rescan(Params P) {
+  const unsigned long long count = min(P.counters[4], (unsigned long long)P.rescan_cap);
+  const uint64_t G = P.gcap;
+  const int K = P.s_max - 3, lane = threadIdx.x;
+  unsigned long long evals = 0, cands = 0;
+  for (unsigned long long it = blockIdx.x; it < count; it += kRescanBlocks) {
+    const Rescan r = P.rescans[it];
+    const uint32_t u = P.anchors[r.anchor], M = P.region[u], side = r.side & 1u;
+    const int cin = (int)(r.side >> 1), need = K - cin;
+    if (need <= 0) continue;
+    double *slab = P.scratch + (uint64_t)r.anchor * P.slab_doubles;
+    Work w{};
+    w.gx = slab;
+    w.gy = slab + G;
+    w.gz = slab + 2 * G;
+    w.gid = (uint32_t *)(slab + slab_ids(G));
+    const V3 o = {P.X[u], P.Y[u], P.Z[u]};
+    const V3 pv = sub({P.X[r.v], P.Y[r.v], P.Z[r.v]}, o), pw = sub({P.X[r.w], P.Y[r.w], P.Z[r.w]}, o);
+    TriSphere f;
+    f.init(pv, pw);
+    const Pencil pen = face_pencil(f, r.lo, r.hi, false);
+    uint32_t region_slot = kInvalid;
+    // sign of the power and whether ahead of the side; false: not in the pencil
+    auto key = [&](uint32_t s, int &sp, bool &ahead, double &tau, double &terr) {
+      const uint32_t id = w.gid[s];
+      if (id == r.v || id == r.w) return false;
+      const V3 p = gpt(w, s);
+      if (pen.outside((float)p.x, (float)p.y, (float)p.z, (float)sqrt(p.x * p.x + p.y * p.y + p.z * p.z))) return false;
+      evals++;
+      double Pw, PA, H, HA;
+      f.power(p, Pw, PA);
+      f.height(p, H, HA);
+      sp = cert_sign(Pw, PA);
+      const int sh = cert_sign(H, HA);
+      ahead = side == 0 ? sh > 0 : sh < 0;
+      sweep_key(Pw, PA, H, HA, tau, terr);
+      return true;
+    };
+    SweepList top;
+    BehindList beh;
+    top.init();
+    beh.init();
+    for (uint32_t s = lane; s < M; s += 64) {
+      int sp;
+      bool ahead;
+      double tau, terr;
+      if (!key(s, sp, ahead, tau, terr)) continue;
+      // inside the triangle's sphere and behind this side: inside the
+      // pencil's spheres until the sweep key reaches -tau
+      if (sp < 0 && !ahead) beh.insert(-tau - terr);
+      else if (sp > 0 && ahead) top.insert(tau, terr);
+    }
+    // the need-th smallest upper bound over the lanes' lists
+    double thr = INFINITY;
+    for (int k = 0; k < need; ++k) {
+      thr = top.hi[0];
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) thr = fmin(thr, __shfl_xor(thr, d));
+      const uint64_t who = __ballot(top.hi[0] == thr);
+      if (lane == __ffsll((long long)who) - 1) top.pop();
+    }
+    for (uint32_t s0 = 0; s0 < M; s0 += 64) {
+      const uint32_t s = s0 + lane;
+      int sp = 0;
+      bool ahead = false;
+      double tau = 0, terr = 0;
+      const bool apex = s < M && key(s, sp, ahead, tau, terr) && sp > 0 && ahead && w.gid[min(s, M - 1)] > r.w &&
+                        !(tau - terr > thr);
+      for (uint64_t todo = __ballot(apex); todo; todo &= todo - 1) {
+        const int j = __ffsll((long long)todo) - 1;
+        // inside points behind: counted while their key exceeds z's
+        int ahead_of = beh.count_above(__shfl(tau + terr, j));
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) ahead_of += __shfl_xor(ahead_of, d);
+        if (cin + ahead_of >= K) continue;
+        const uint32_t id = w.gid[s0 + j];
+        TetSphere t;
+        const int wc = t.init(pv, pw, gpt(w, s0 + j));
+        if (wc < 0) continue;
+        cands++;
+        const uint32_t ids[3] = {r.v, r.w, id};
+        uint32_t interior[kMaxInterior];
+#pragma unroll
+        for (int k = 0; k < kMaxInterior; ++k) interior[k] = kInvalid;
+        int nint = 0;
+        bool open = wc == 0;
+        for (uint32_t q0 = 0; wc > 0 && q0 < M && nint + 4 <= P.s_max; q0 += 64) {
+          const uint32_t q = min(q0 + lane, M - 1), x = w.gid[q];
+          int sd = 1;
+          if (q0 + lane < M && x != r.v && x != r.w && x != id) sd = t.side(gpt(w, q));
+          open |= __ballot(sd == 0) != 0;
+          for (uint64_t in = __ballot(sd < 0); in; in &= in - 1) {
+            const uint32_t y = __shfl(x, __ffsll((long long)in) - 1);
+#pragma unroll
+            for (int k = 0; k < kMaxInterior; ++k) interior[k] = k == nint ? y : interior[k];
+            nint++;
+          }
+        }
+        if (nint + 4 > P.s_max) continue;
+        sort_static(interior, nint);
+        if (lane == 0) {
+          if (open) emit_fallback(P, w, u, 4, ids, 4, M, &region_slot);
+          else emit_event(P, u, ids, 4, nint, interior, t.level(), t.level_err());
+        }
+      }
+    }
+  }
+  if (lane == 0 && cands) atomicAdd(&P.counters[3], cands);
+  if (P.count_flops && evals) atomicAdd(&P.counters[5], evals * (kFlopFacePoint + kFlopSweepKey));
+}
+
+// The list starts again; its longest length is kept for the host.
+__global__ void k_rescans_done(Params P) {
+  P.counters[kRescanMost] = max(P.counters[kRescanMost], P.counters[4]);
+  P.counters[4] = 0;
 }
 
 // Ball count / emit around every anchor of the list: one wave per anchor over
@@ -2056,6 +2133,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   uint64_t event_cap = std::max<uint64_t>(1024, (uint64_t)n * (smax >= 11 ? 640 : 64 * smax));
   uint64_t fb_cap = std::max<uint64_t>(4096, (uint64_t)n / 4);
   uint64_t reg_cap = std::max<uint64_t>(1 << 20, (uint64_t)n * 64);
+  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n);
   uint64_t ctr[kCounters];
   int64_t widened = 0;
   // The record queues have a fixed capacity per launch; records past it are
@@ -2067,7 +2145,8 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     // the record queues are the catalogue's large, data-sized allocation
     const int64_t more = (int64_t)(event_cap - std::min<uint64_t>(event_cap, B.events.cap)) * (int64_t)sizeof(EventRec) +
                          (int64_t)(fb_cap - std::min<uint64_t>(fb_cap, B.fallbacks.cap)) * (int64_t)sizeof(FallbackRec) +
-                         (int64_t)(reg_cap - std::min<uint64_t>(reg_cap, B.fb_region.cap)) * 4;
+                         (int64_t)(reg_cap - std::min<uint64_t>(reg_cap, B.fb_region.cap)) * 4 +
+                         (int64_t)(rescan_cap - std::min<uint64_t>(rescan_cap, B.rescans.cap / sizeof(Rescan))) * (int64_t)sizeof(Rescan);
     if (device_bytes(c) + more > c.capacity_bytes)
       throw CapacityError("the catalogue's record queues (" + std::to_string(event_cap) + " records) exceed the " +
                           "context's device capacity of " + std::to_string(c.capacity_bytes) + " bytes");
@@ -2075,6 +2154,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   B.events.ensure(event_cap);
   B.fallbacks.ensure(fb_cap);
   B.fb_region.ensure(reg_cap);
+  B.rescans.ensure(rescan_cap * sizeof(Rescan));
   MHGP_HIP(hipMemsetAsync(B.counters.p, 0, kCounters * 8, s));
   widened = 0;
   Params P{};
@@ -2090,6 +2170,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   P.events = B.events.p; P.event_cap = event_cap;
   P.fallbacks = B.fallbacks.p; P.fallback_cap = fb_cap;
   P.fb_region = B.fb_region.p; P.fb_region_cap = reg_cap;
+  P.rescans = reinterpret_cast<Rescan *>(B.rescans.p); P.rescan_cap = rescan_cap;
   P.counters = (unsigned long long *)B.counters.p;
   P.count_flops = c.count_flops ? 1 : 0;
   P.region_limit = std::min<uint32_t>(c.region_limit, kBigRegionMax);
@@ -2114,6 +2195,12 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
         hipLaunchKernelGGL((k_anchor_region<kRegionCap, 4, 3>), grid, dim3(256), 0, s, Q, list(l));
       MHGP_LAUNCH_CHECK();
     }
+  };
+  // the sides that a launch's enumeration left, before its slabs are reused
+  auto settle = [&](const Params &Q) {
+    hipLaunchKernelGGL(k_rescan, dim3(kRescanBlocks), dim3(64), 0, s, Q);
+    hipLaunchKernelGGL(k_rescans_done, dim3(1), dim3(1), 0, s, Q);
+    MHGP_LAUNCH_CHECK();
   };
   // scratch for slabs: 8 GiB, 1 GiB in a context with a device capacity; and
   // at most a quarter of the device memory still free (other contexts on the
@@ -2143,6 +2230,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
       Q.gcap = g;
       Q.scratch = B.scratch.p;
       Q.slab_doubles = slab;
+      Q.ascending = 1;
       clear_lists(L_SMALL, kLists);
       if (wide)
         hipLaunchKernelGGL(k_anchor_probe<kGatherCapWide>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
@@ -2151,6 +2239,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
       MHGP_LAUNCH_CHECK();
       read_counters();
       enumerate(Q);
+      settle(Q);
     }
   };
   // anchors in Morton order: neighbouring workgroups share cache lines
@@ -2223,10 +2312,14 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
           if (probe) clear_lists(L_SMALL, kLists);
           hipLaunchKernelGGL(k_anchor_big, dim3(bn), dim3(kBlock), 0, s, Q);
           MHGP_LAUNCH_CHECK();
+          if (!probe) settle(Q);
           if (probe) {
             read_counters();
             // test hook: every region through the slab enumeration
-            if (force_path != 2) enumerate(Q);
+            if (force_path != 2) {
+              enumerate(Q);
+              settle(Q);
+            }
             for (int l = force_path == 2 ? L_SMALL : L_SLAB; l <= L_SLAB; ++l) {
               std::vector<uint32_t> at(ctr[kListCount + l]);
               if (!at.empty()) copy_wait(at.data(), list(l), at.size() * 4, hipMemcpyDeviceToHost, s);
@@ -2270,16 +2363,18 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   }
   tm.mark("catalogue big anchors");
   read_counters();
-  if (ctr[4]) throw std::runtime_error("face side queue overflow");
-  if (ctr[0] <= event_cap && ctr[1] <= fb_cap && ctr[2] <= reg_cap) break;
-  if (attempt >= 2) throw CapacityError("catalogue record queues did not settle after regrowth");
+  if (tm.on) std::fprintf(stderr, "[mhgp] sides left to the rescans, most in a launch: %llu\n", (unsigned long long)ctr[kRescanMost]);
+  if (ctr[0] <= event_cap && ctr[1] <= fb_cap && ctr[2] <= reg_cap && ctr[kRescanMost] <= rescan_cap) break;
+  // a launch that ran out of rescans has also counted too few records
+  if (attempt >= 3) throw CapacityError("catalogue record queues did not settle after regrowth");
   const uint64_t ev2 = std::max(event_cap, ctr[0] + ctr[0] / 8), fb2 = std::max(fb_cap, ctr[1] + ctr[1] / 8),
                  rg2 = std::max(reg_cap, ctr[2] + ctr[2] / 8);
+  rescan_cap = std::max(rescan_cap, ctr[kRescanMost] + ctr[kRescanMost] / 8);
   size_t free_b = 0, total_b = 0;
   MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
   const uint64_t more = (ev2 - std::min<uint64_t>(ev2, B.events.cap)) * sizeof(EventRec) +
                         (fb2 - std::min<uint64_t>(fb2, B.fallbacks.cap)) * sizeof(FallbackRec) +
-                        (rg2 - std::min<uint64_t>(rg2, B.fb_region.cap)) * 4;
+                        (rg2 - std::min<uint64_t>(rg2, B.fb_region.cap)) * 4 + rescan_cap * sizeof(Rescan);
   if (more > free_b / 10 * 9)
     throw CapacityError("the catalogue needs " + std::to_string(ctr[0]) + " record slots, more than the device can hold");
   event_cap = ev2;

@@ -48,6 +48,7 @@ struct CatalogBuffers {
   DevBuf<uint32_t> glist;         // gathered ids
   DevBuf<uint32_t> region;        // region size of a probed anchor
   DevBuf<uint32_t> lists;         // anchors by what comes next for them (supports.hip)
+  DevBuf<uint8_t> rescans;        // sides of faces left to the rescan kernel
   DevBuf<uint32_t> big;           // anchors of a global-memory launch
   DevBuf<EventRec> events;
   DevBuf<FallbackRec> fallbacks;

@@ -129,6 +129,17 @@ def test_catalog_big_paths_small(path, monkeypatch):
     _compare(workloads.uniform_cloud(40, seed=34), 4, f"uniform40-k4-{path}")
 
 
+@pytest.mark.parametrize("path", ["", "region", "slabs"])
+@pytest.mark.parametrize("sigma,n,k", [(1e-4, 64, 10), (1e-6, 110, 10), (1e-6, 100, 4)])
+def test_catalog_nearly_cospherical(path, sigma, n, k, monkeypatch):
+    """Lattices displaced by less than FP32 key bounds can tell apart: most
+    sides of faces hold more near-equal sweep keys than a face's list, so
+    their apexes come from the sides' own FP64 passes (and their list outgrows
+    its first capacity)."""
+    monkeypatch.setenv("MHGP_TEST_ANCHOR_PATH", path)
+    _compare(workloads.jittered_lattice(n, side=5, sigma=sigma, seed=36), k, f"lattice{n}-{sigma}-{path}")
+
+
 def test_big_regions_give_a_conditional_catalogue():
     """Anchors whose candidate region exceeds the enumeration bound are left
     open: the catalogue reports status conditional with their count and
