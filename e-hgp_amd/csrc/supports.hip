@@ -51,7 +51,7 @@ namespace mhgp {
 int64_t catalog_device_bytes(const CatalogBuffers &b) {
   return b.radius.bytes() + b.gcount.bytes() + b.goff.bytes() + b.glist.bytes() + b.region.bytes() +
          b.lists.bytes() + b.big.bytes() + b.rescans.bytes() + b.events.bytes() + b.fallbacks.bytes() + b.fb_region.bytes() +
-         b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.scratch.bytes() + b.anchors.bytes() +
+         b.counters.bytes() + b.cells.bytes() + b.cellf.bytes() + b.strips.bytes() + b.scratch.bytes() + b.anchors.bytes() +
          b.total.bytes() + b.run_count.bytes() + b.run_pos.bytes() + b.run_gidx.bytes() + b.run_new.bytes() +
          b.run_link.bytes() + b.run_rec.bytes();
 }
@@ -73,11 +73,12 @@ __device__ inline void wave_sync() {
 // pass: gathers to widen, gathers beyond the small probe, gathers beyond LDS.
 // The others hold the probed anchors of one launch (their index in it, which
 // is also their slab's) by the size of their region.
-enum { L_WIDEN = 0, L_WIDE = 1, L_BIG = 2, L_SMALL = 3, L_MID = 4, L_LARGE = 5, L_SLAB = 6, kLists = 7 };
+enum { L_WIDEN = 0, L_WIDE = 1, L_BIG = 2, L_TINY = 3, L_LITTLE = 4, L_SMALL = 5, L_MID = 6, L_LARGE = 7, L_SLAB = 8,
+       kLists = 9 };
 constexpr int kListCount = 8;    // counters: list lengths
-constexpr int kOpenCount = 16;   // counters: open anchors, their largest region
-constexpr int kOpenLargest = 17;
-constexpr int kRescanMost = 18;  // longest rescan list of a launch
+constexpr int kOpenCount = 17;   // counters: open anchors, their largest region
+constexpr int kOpenLargest = 18;
+constexpr int kRescanMost = 19;  // longest rescan list of a launch
 constexpr int kCounters = 24;
 
 // Regions of the global-memory path are enumerated face by face in
@@ -96,6 +97,7 @@ struct Params {
   double *radius;
   const double *cells;           // 8 doubles per cell
   const float *cellf;            // 8 floats per cell: the FP32 cell (see cell_f)
+  const uint64_t *strips;        // kStrips x 8: cells a great circle can meet (k_strips)
   double blo[3], bhi[3];         // cloud AABB
   int s_max;
   uint32_t *region;              // region size of a probed anchor
@@ -114,6 +116,7 @@ struct Params {
   const uint32_t *anchors;
   uint32_t anchor_count;
   int probe;                     // 1: stop once the region is in the slab
+  uint32_t one_wave, two_waves;  // regions up to these sizes take workgroups of one and of two waves
   int ascending;                 // 1: the slabs' regions are in increasing distance
   double *scratch;
   uint64_t slab_doubles;
@@ -151,6 +154,7 @@ struct Work {
   unsigned long long *flops32;  // FP32 operations of the tests (as flops; null: not counted)
   bool ascending;             // the region is in increasing distance: scans end at a sphere's diameter
   uint32_t slab;              // the anchor's index in its launch
+  const float4 *cell;         // LDS: direction and cosine of the 64 cells of a cube face, in its frame
 };
 
 // FP64 operations (add, subtract, multiply; a fused multiply-add counts two)
@@ -959,6 +963,45 @@ __device__ inline float cell_radius(const Params &P, int c, float bk, double ux,
   return rf;
 }
 
+// Axis cell of a great circle with normal m (or -m): kStripSide^2 cells on each
+// of three cube faces.  Of the 15 cells that a pair of the 50 000-point lattice
+// shares, its lanes' longest walks (4 to 6 times that) bound face_interval;
+// dropping those that the pencil's circle misses by one 64-byte row halves
+// them: K 10 53.1 -> 46.3 ms, K 4 13.6 -> 12.8 ms (the walk itself on a table
+// of one cube face in LDS: 2.5 and 0.7 ms before that).
+constexpr int kStripSide = 16;
+constexpr int kStrips = 3 * kStripSide * kStripSide;
+__device__ inline uint32_t strip_of(float mx, float my, float mz) {
+  const float ax = fabsf(mx), ay = fabsf(my), az = fabsf(mz);
+  const bool fy = ay > ax && ay >= az, fz = az > ax && az > ay;
+  const float m = fz ? mz : fy ? my : mx, a = fz ? mx : fy ? mz : my, b = fz ? my : fy ? mx : mz;
+  const float r = __builtin_amdgcn_rcpf(m) * (0.5f * kStripSide);
+  const int i = min(max((int)(a * r + 0.5f * kStripSide), 0), kStripSide - 1);
+  const int j = min(max((int)(b * r + 0.5f * kStripSide), 0), kStripSide - 1);
+  return (uint32_t)(((fz ? 2 : fy ? 1 : 0) * kStripSide + i) * kStripSide + j);
+}
+
+// For every axis cell of strip_of (a workgroup) the direction cells (its
+// threads) that a great circle with its normal there can meet, six words of
+// eight: |angle(g, m) - 90 degrees| at most the two cells' radii and 2e-3, which
+// covers the lowered cosines of face_interval and the rounding of the axis.
+__global__ void k_strips(const double *__restrict__ cells, uint64_t *__restrict__ strips) {
+  const int f = blockIdx.x / (kStripSide * kStripSide), i = blockIdx.x / kStripSide % kStripSide, j = blockIdx.x % kStripSide;
+  auto axis = [&](double s, double t) {
+    const double a = 2.0 * s / kStripSide - 1.0, b = 2.0 * t / kStripSide - 1.0, q = 1.0 / sqrt(1.0 + a * a + b * b);
+    return f == 0 ? V3{q, a * q, b * q} : f == 1 ? V3{b * q, q, a * q} : V3{a * q, b * q, q};
+  };
+  const V3 m = axis(i + 0.5, j + 0.5);
+  double least = 1.0;
+  for (int c = 0; c < 4; ++c) least = fmin(least, dot(m, axis(i + c / 2, j + c % 2)));
+  const double radius = acos(least) + 2e-3;
+  const double *g = cells + 8 * threadIdx.x;
+  // |g.m| <= sin(delta + radius), the sum below 90 degrees
+  const bool met = fabs(dot(m, V3{g[0], g[1], g[2]})) <= g[4] * cos(radius) + g[3] * sin(radius);
+  const uint64_t word = __ballot(met);
+  if (threadIdx.x % 64 == 0) strips[8 * blockIdx.x + threadIdx.x / 64] = word;
+}
+
 // Face (u, v, w) of region slots si, sj: the part of its pencil of spheres
 // that the certificate leaves.  A critical sphere through the three points has
 // its centre at c3 + t n (n the unit normal along v x w, t = s r3), its
@@ -972,7 +1015,8 @@ __device__ inline float cell_radius(const Params &P, int c, float bk, double ux,
 // the cells' cosines lowered by 1e-4 cover (a cell only grows), and the radius
 // bound carries 2e-5.  Where a cell holds (nearly) the normal itself the roots
 // are unbounded and its interval is taken as that whole side.  An
-// ill-conditioned face is not restricted (lo = -infinity).
+// ill-conditioned face is not restricted (lo = -infinity).  The cells of the
+// six cube faces are one table in the frame of their face (w.cell).
 // key: the squared radius of the larger end sphere (it only orders the faces
 // into waves of similar work).
 __device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si, uint32_t sj, float &lo, float &hi,
@@ -1003,9 +1047,15 @@ __device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si
   if (!(fabsf(cx) <= 1.001f && fabsf(nx) <= 1.001f && ir3 > 1e-30f && ir3 < 1e30f)) return true;  // out of FP32's range
   float l = INFINITY, h = -INFINITY;
   uint32_t cells = 0;
+  // only the cells that the pencil's great circle can meet (of the others, q < 0)
+  const uint64_t *strip = P.strips + 8 * strip_of(cy * nz - cz * ny, cz * nx - cx * nz, cx * ny - cy * nx);
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
-    uint64_t mm = sh[k];
+    uint64_t mm = sh[k] & strip[k];
+    // c and n in the frame of cube face k
+    const float sg = k % 2 ? -1.0f : 1.0f;
+    const float kc[3] = {sg * (k < 2 ? cx : k < 4 ? cy : cz), k < 2 ? cy : k < 4 ? cz : cx, k < 2 ? cz : k < 4 ? cx : cy};
+    const float kn[3] = {sg * (k < 2 ? nx : k < 4 ? ny : nz), k < 2 ? ny : k < 4 ? nz : nx, k < 2 ? nz : k < 4 ? nx : ny};
     while (mm) {
       const int c = 64 * k + __ffsll((long long)mm) - 1;
       mm &= mm - 1;
@@ -1013,9 +1063,9 @@ __device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si
       const float ratio = w.rho[c] * ir3;
       const float sc2 = ratio * ratio * (1.0f + 2e-5f) - (1.0f - 1e-5f);
       if (sc2 < 0.0f) continue;
-      const CellF cf = cell_f(P.cellf + 8 * c);
-      const float ga = cf.dx * cx + cf.dy * cy + cf.dz * cz, gn = cf.dx * nx + cf.dy * ny + cf.dz * nz;
-      const float cd = cf.cosd - 1e-4f, kk = cd * cd;
+      const float4 cf = w.cell[c & 63];
+      const float ga = cf.x * kc[0] + cf.y * kc[1] + cf.z * kc[2], gn = cf.x * kn[0] + cf.y * kn[1] + cf.z * kn[2];
+      const float cd = cf.w - 1e-4f, kk = cd * cd;
       const float q = ga * ga + gn * gn - kk, den = kk - gn * gn;
       if (q < 0.0f) continue;
       const float sc = __builtin_amdgcn_sqrtf(sc2);
@@ -1445,7 +1495,7 @@ __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t 
     return;
   }
   P.region[u] = M;
-  if (M) list_add(P, M <= kRegionCap ? L_SMALL : M <= kRegionCapWide ? L_MID : M <= kRegionCapHuge ? L_LARGE : L_SLAB, a);
+  if (M) list_add(P, M <= P.one_wave ? L_TINY : M <= P.two_waves ? L_LITTLE : M <= kRegionCap ? L_SMALL : M <= kRegionCapWide ? L_MID : M <= kRegionCapHuge ? L_LARGE : L_SLAB, a);
 }
 
 // Certificate and region of one anchor per workgroup, gathers of up to GCAP
@@ -1679,15 +1729,26 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
   w.cand = &cand;
   w.flops = P.count_flops ? &flops : nullptr;
   w.slab = a;
+  __shared__ float4 cell[64];
+  if (threadIdx.x < 64) cell[threadIdx.x] = *reinterpret_cast<const float4 *>(P.cellf + 8 * threadIdx.x);
+  w.cell = cell;
   anchor_work(P, w, u, a);
 }
 
 // Enumeration of probed regions that fit LDS: the region (coordinates,
 // PointIds, masks) and cell radii are loaded from the anchor's slab, and the
-// face phase runs on them with the wave queues.  Three sizes: up to 384 points
-// (three workgroups per CU at 168 VGPRs), up to 640 (two) and up to 1 023 (one;
-// region slots stay below 1 024, as the packed queue items need).  list:
-// the launch's slabs with such a region.
+// face phase runs on them with the wave queues.  Sizes: up to 384 points
+// (three workgroups of four waves per CU at 168 VGPRs), up to 640 (two) and up
+// to 1 023 (one of eight waves; region slots stay below 1 024, as the packed
+// queue items need).  list: the launch's slabs with such a region.
+//
+// In launches of many anchors small regions take one wave (up to 96 points) or
+// two (up to 180, the most of which six workgroups share a CU): a wave's 64
+// lanes fill from its own share of an anchor's faces, of which a K 4 lattice
+// has 89 in all, and the last rounds of fewer waves are less often part empty.
+// 50 000-point lattice: K 10 57.7 -> 53.6 ms, K 4 18.3 -> 14.3 ms.  With fewer
+// anchors than the CUs hold waves of one launch after another loses more (1 000
+// points 2.05 -> 3.2 ms), hence the rule by the launch's anchors.
 //
 // One workgroup per anchor left the chip idle wherever tens of anchors held
 // large regions (43 anchors: 313 ms, each workgroup alone on its CU): a launch
@@ -1703,6 +1764,7 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
 // diameter and id lists read from bit masks: 73 -> 58 ms, K 4 19.3 -> 18.3 ms,
 // the mixture's catalogue 75.6 -> 67.2 ms.
 constexpr uint32_t kRegionParts = 4096;
+constexpr uint32_t kSmallRegionLaunch = 8192;  // anchors of a launch that splits off the small regions
 template <int RCAP, int WAVES, int PER_SIMD>
 __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P, const uint32_t *__restrict__ list) {
   const uint32_t a = list[blockIdx.x];
@@ -1719,9 +1781,11 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   __shared__ uint64_t rmask[6 * RCAP];
   __shared__ uint16_t kidx[RCAP];
   __shared__ float fx[RCAP], fy[RCAP], fz[RCAP], fw[RCAP];
+  __shared__ float4 cell[64];
   __shared__ uint32_t cand, sK, sregion;
   __shared__ unsigned long long flops, flops32;
   const int t = threadIdx.x;
+  if (t < 64) cell[t] = *reinterpret_cast<const float4 *>(P.cellf + 8 * t);
   if (P.ascending) {
     for (uint32_t i = t; i < M; i += blockDim.x) {
       gx[i] = slab[i];
@@ -1762,7 +1826,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; flops32 = 0; }
   __syncthreads();
   Work w{gx, gy, gz, gid, rho, nullptr, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz, fw,
-         P.count_flops ? &flops32 : nullptr, true, a};
+         P.count_flops ? &flops32 : nullptr, true, a, cell};
   anchor_faces<false, true, WAVES>(P, w, u, M, &sK, &sregion);
 }
 
@@ -2110,6 +2174,9 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     const std::vector<float> cf = make_cells_f(cells);
     B.cellf.ensure(8 * kCells);
     copy_wait(B.cellf.p, cf.data(), cf.size() * 4, hipMemcpyHostToDevice, s);
+    B.strips.ensure(8 * kStrips);
+    hipLaunchKernelGGL(k_strips, dim3(kStrips), dim3(kCells), 0, s, B.cells.p, B.strips.p);
+    MHGP_LAUNCH_CHECK();
   }
   // Test hook (MHGP_TEST_ANCHOR_PATH): "region" sends every anchor through
   // the big path's probe and LDS region kernels, "slabs" through the
@@ -2162,6 +2229,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   P.gcount = B.gcount.p; P.goff = B.goff.p; P.radius = B.radius.p;
   P.cells = B.cells.p;
   P.cellf = B.cellf.p;
+  P.strips = B.strips.p;
   for (int a = 0; a < 3; ++a) { P.blo[a] = bounds[a]; P.bhi[a] = bounds[3 + a]; }
   P.s_max = smax;
   P.region = B.region.p;
@@ -2183,7 +2251,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   // enumerates the regions of one probe launch (ctr holds its list lengths),
   // the largest first
   auto enumerate = [&](const Params &Q) {
-    for (int l = L_LARGE; l >= L_SMALL; --l) {
+    for (int l = L_LARGE; l >= L_TINY; --l) {
       const uint32_t m = (uint32_t)ctr[kListCount + l];
       if (!m) continue;
       const dim3 grid(m, std::clamp<uint32_t>(kRegionParts / m, 1, 64));
@@ -2191,6 +2259,10 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
         hipLaunchKernelGGL((k_anchor_region<kRegionCapHuge, 8, 2>), grid, dim3(512), 0, s, Q, list(l));
       else if (l == L_MID)
         hipLaunchKernelGGL((k_anchor_region<kRegionCapWide, 4, 2>), grid, dim3(256), 0, s, Q, list(l));
+      else if (l == L_TINY)
+        hipLaunchKernelGGL((k_anchor_region<kRegionCapTiny, 1, 3>), grid, dim3(64), 0, s, Q, list(l));
+      else if (l == L_LITTLE)
+        hipLaunchKernelGGL((k_anchor_region<kRegionCapLittle, 2, 3>), grid, dim3(128), 0, s, Q, list(l));
       else
         hipLaunchKernelGGL((k_anchor_region<kRegionCap, 4, 3>), grid, dim3(256), 0, s, Q, list(l));
       MHGP_LAUNCH_CHECK();
@@ -2231,7 +2303,11 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
       Q.scratch = B.scratch.p;
       Q.slab_doubles = slab;
       Q.ascending = 1;
-      clear_lists(L_SMALL, kLists);
+      if (Q.anchor_count >= kSmallRegionLaunch) {
+        Q.one_wave = kRegionCapTiny;
+        Q.two_waves = kRegionCapLittle;
+      }
+      clear_lists(L_TINY, kLists);
       if (wide)
         hipLaunchKernelGGL(k_anchor_probe<kGatherCapWide>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
       else
@@ -2309,7 +2385,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
           Params Q = P;
           Q.anchors = B.big.p + b0; Q.anchor_count = bn; Q.probe = probe;
           Q.scratch = B.scratch.p; Q.slab_doubles = slab_of(g); Q.gcap = g;
-          if (probe) clear_lists(L_SMALL, kLists);
+          if (probe) clear_lists(L_TINY, kLists);
           hipLaunchKernelGGL(k_anchor_big, dim3(bn), dim3(kBlock), 0, s, Q);
           MHGP_LAUNCH_CHECK();
           if (!probe) settle(Q);
@@ -2320,7 +2396,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
               enumerate(Q);
               settle(Q);
             }
-            for (int l = force_path == 2 ? L_SMALL : L_SLAB; l <= L_SLAB; ++l) {
+            for (int l = force_path == 2 ? L_TINY : L_SLAB; l <= L_SLAB; ++l) {
               std::vector<uint32_t> at(ctr[kListCount + l]);
               if (!at.empty()) copy_wait(at.data(), list(l), at.size() * 4, hipMemcpyDeviceToHost, s);
               for (uint32_t i : at) {

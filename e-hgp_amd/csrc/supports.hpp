@@ -9,6 +9,7 @@ namespace mhgp {
 
 constexpr int kCells = 384;      // 6 cube faces x 8 x 8 direction cells
 constexpr int kGatherCap = 600;  // gathered neighbours the probe holds in LDS
+constexpr uint32_t kRegionCapTiny = 96, kRegionCapLittle = 180;  // members that one and two waves hold in LDS
 constexpr int kRegionCap = 384;  // region members the smallest enumeration holds in LDS
 constexpr uint32_t kRegionLimitMax = 2048;  // largest candidate region any path enumerates
 constexpr int kGatherCapWide = 1024;  // the same for the wide probe and the next enumeration
@@ -56,6 +57,7 @@ struct CatalogBuffers {
   DevBuf<uint64_t> counters;      // events, fallbacks, region words, candidates, operations, list lengths
   DevBuf<double> cells;           // per cell: dir xyz, cos d, sin d, chord
   DevBuf<float> cellf;            // per cell: the FP32 cell of the certificate and the masks
+  DevBuf<uint64_t> strips;        // cells that a great circle can meet, by its axis
   DevBuf<double> scratch;         // slabs: the regions of probed anchors
   DevBuf<uint32_t> anchors;       // anchor list of the current launch
   // canonical order on the device: records (device emitted + host settled),
