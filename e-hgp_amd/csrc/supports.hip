@@ -150,7 +150,7 @@ struct Work {
   float4 *fc;       // FP32 offset and distance per gathered point (certificate and masks)
   uint32_t *cand;   // candidate supports classified (LDS, flushed once per anchor)
   unsigned long long *flops;  // FP64 operations of the certified predicates (LDS, flushed once per anchor; null: not counted)
-  float *fx, *fy, *fz, *fw;   // FP32 copies of the region's coordinates and distances from the anchor
+  float4 *f;                  // FP32 copies of the region's coordinates and distances from the anchor
   unsigned long long *flops32;  // FP32 operations of the tests (as flops; null: not counted)
   bool ascending;             // the region is in increasing distance: scans end at a sphere's diameter
   uint32_t slab;              // the anchor's index in its launch
@@ -258,16 +258,18 @@ __device__ inline int cert32(float v, float a) {
 }
 
 // A candidate sphere through the anchor in FP32: the scaled power
-// a |p|^2 - p.b of a point, with the magnitude bound |p| (aA |p| + bA) (the
-// norms bound the sums of magnitudes).  reach: no point farther from the
+// v = a |p|^2 - p.b of a point, and 1e-5 of its magnitude bound
+// |p| (aA |p| + bA) (the norms bound the sums of magnitudes) plus 1e-35; a
+// larger |v| certifies the sign (cert32).  reach: no point farther from the
 // anchor is inside (the sphere passes through the anchor, so its diameter with
 // a margin for the FP32 estimate; infinite when the region is not in
 // increasing distance).
 struct SphereF {
-  float a, aA, b[3], bA, reach;
-  __device__ void test(float x, float y, float z, float w, float &v, float &va) const {
-    v = a * (w * w) - (x * b[0] + y * b[1] + z * b[2]);
-    va = w * (aA * w + bA);
+  float a, aE, b[3], bE, reach;
+  __device__ void test(const float4 &p, float &v, float &e) const {
+    const float pp = p.w * p.w;
+    v = a * pp - (p.x * b[0] + p.y * b[1] + p.z * b[2]);
+    e = aE * pp + (bE * p.w + 1e-35f);
   }
 };
 __device__ inline float norm_up(double x, double y, double z) {
@@ -275,23 +277,28 @@ __device__ inline float norm_up(double x, double y, double z) {
 }
 __device__ inline SphereF to_f32(const PairSphere &s, bool ascending) {
   const float l = norm_up(s.a.x, s.a.y, s.a.z);
-  return {1.0f, 1.0f, {(float)s.a.x, (float)s.a.y, (float)s.a.z}, l, ascending ? l * (1.0f + 1e-4f) + 1e-30f : INFINITY};
+  return {1.0f, 1e-5f, {(float)s.a.x, (float)s.a.y, (float)s.a.z}, 1e-5f * l, ascending ? l * (1.0f + 1e-4f) + 1e-30f : INFINITY};
 }
 __device__ inline SphereF to_f32(const TetSphere &t, bool ascending) {
   // diameter |N| / |V|; both hold 12 digits at worst below their magnitude
   // bounds (their signs are certified), hence the wide margin
   const double sg = t.V > 0 ? 1.0 : -1.0;
   const double d = sqrt(dot(t.N, t.N)) * __builtin_amdgcn_rcp(fabs(t.V));
-  return {(float)(sg * t.V), (float)t.VA, {(float)(sg * t.N.x), (float)(sg * t.N.y), (float)(sg * t.N.z)},
-          norm_up(t.NA.x, t.NA.y, t.NA.z), ascending ? (float)d * 1.05f + 1e-30f : INFINITY};
+  return {(float)(sg * t.V), (float)(1e-5 * t.VA), {(float)(sg * t.N.x), (float)(sg * t.N.y), (float)(sg * t.N.z)},
+          1e-5f * norm_up(t.NA.x, t.NA.y, t.NA.z), ascending ? (float)d * 1.05f + 1e-30f : INFINITY};
 }
 
-// Up to kMaxInterior region slots, 16 bits each, 2 per word.
+// Bits of a test over n <= 32 slots, slot 0 first, shifted in from below (one
+// add with carry each) and turned round.
+__device__ inline uint32_t shift_in(uint32_t bits, bool b) { return bits + bits + (b ? 1u : 0u); }
+__device__ inline uint32_t in_order(uint32_t bits, uint32_t n) { return __builtin_bitreverse32(bits) >> (32u - n); }
+
+// Up to kMaxInterior region slots, 16 bits each, 2 per word; the newest lowest.
 constexpr int kPacked = (kMaxInterior + 1) / 2;
-__device__ inline void put_packed(uint32_t (&pk)[kPacked], int n, uint32_t slot) {
-  const uint32_t word = (uint32_t)n >> 1, shift = ((uint32_t)n & 1u) * 16u;
+__device__ inline void push_packed(uint32_t (&pk)[kPacked], uint32_t slot) {
 #pragma unroll
-  for (int k = 0; k < kPacked; ++k) pk[k] |= (uint32_t)k == word ? slot << shift : 0u;
+  for (int k = kPacked - 1; k > 0; --k) pk[k] = __builtin_amdgcn_alignbit(pk[k], pk[k - 1], 16);
+  pk[0] = pk[0] << 16 | slot;
 }
 __device__ inline void unpack_ids(const Work &w, const uint32_t (&pk)[kPacked], int n, uint32_t (&ids)[kMaxInterior]) {
 #pragma unroll
@@ -299,7 +306,7 @@ __device__ inline void unpack_ids(const Work &w, const uint32_t (&pk)[kPacked], 
 }
 
 // Certified classification of the region against a candidate sphere through
-// the anchor and m - 1 region points (slots skip).  FP32 for 64 slots at a time
+// the anchor and m - 1 region points (slots skip).  FP32 for 32 slots at a time
 // into two bit masks (inside, undecided), FP64 for the undecided; the inside
 // slots are packed.  Returns 1 event, 0 not critical, -1 undecided (host).
 // Bound by VALU issue; collecting the ids point by point over the whole region
@@ -318,38 +325,39 @@ __device__ __attribute__((always_inline)) inline int classify(const Params &P, c
   const SphereF f = to_f32(sph, w.ascending);
   bool over = false;
 #pragma unroll 1
-  for (uint32_t s0 = 0; s0 < M; s0 += 64) {
-    if (w.fw[s0] > f.reach) break;
-    const uint32_t cn = min(64u, M - s0);
-    uint64_t in = 0, open = 0;
+  for (uint32_t s0 = 0; s0 < M; s0 += 32) {
+    if (w.f[s0].w > f.reach) break;
+    const uint32_t cn = min(32u, M - s0);
+    uint32_t in = 0, open = 0;
 #pragma unroll 4
     for (uint32_t j = 0; j < cn; ++j) {
-      float v, va;
-      f.test(w.fx[s0 + j], w.fy[s0 + j], w.fz[s0 + j], w.fw[s0 + j], v, va);
-      const float e = fmaxf(1e-5f * va, 1e-35f);
-      in |= (uint64_t)(v < -e) << j;
-      open |= (uint64_t)(!(fabsf(v) > e)) << j;
+      float v, e;
+      f.test(w.f[s0 + j], v, e);
+      in = shift_in(in, v < -e);
+      open = shift_in(open, !(fabsf(v) > e));
     }
+    in = in_order(in, cn);
+    open = in_order(open, cn);
     evals32 += cn;
     for (int k = 0; k < m - 1; ++k)
       if (skip[k] - s0 < cn) {
-        in &= ~(1ull << (skip[k] - s0));
-        open &= ~(1ull << (skip[k] - s0));
+        in &= ~(1u << (skip[k] - s0));
+        open &= ~(1u << (skip[k] - s0));
       }
     while (open) {
-      const uint32_t j = (uint32_t)(__ffsll((long long)open) - 1);
+      const uint32_t j = (uint32_t)(__ffs((int)open) - 1);
       open &= open - 1;
       const int side = sph.side(gpt(w, s0 + j));
       evals++;
-      in |= (uint64_t)(side < 0) << j;
+      in |= (uint32_t)(side < 0) << j;
       undecided += side == 0;
     }
-    if (nint + __popcll(in) > cap) {
+    if (nint + __popc(in) > cap) {
       over = true;
       break;
     }
     while (in) {
-      put_packed(interior, nint, s0 + (uint32_t)(__ffsll((long long)in) - 1));
+      push_packed(interior, s0 + (uint32_t)(__ffs((int)in) - 1));
       in &= in - 1;
       nint++;
     }
@@ -449,76 +457,54 @@ struct BehindList {
   }
 };
 
-// The same two lists in FP32, filled for both sides during a face's first
-// pass: key bounds rounded outwards (lo down, hi up), so that every
-// threshold test below stays conservative (wider intervals only admit more
-// apex candidates, which are classified exactly).
-//
-// An entry keeps its upper bound and one word with the region slot (low 11
-// bits, regions of up to 2048 points) and the interval's width, rounded up
-// to a 21-bit float (the FP32 width's bit pattern rounded up past its 10
-// lowest bits); its lower bound is
-// hi - width, rounded down.  Listed entries have finite upper bounds (an
-// infinite one never enters the list).  The upper bounds stay sorted with
-// one median-of-three per entry.
-__device__ inline uint32_t pack_entry(float h, float l, uint32_t slot) {
-  // the rounded difference widened past its rounding error
-  float gap = (h - l) * (1.0f + 2.4e-7f) + 1e-37f;
-  if (!(gap >= 0.0f)) gap = INFINITY;
-  return (((__float_as_uint(gap) + 1023u) >> 10) << 11) | slot;
-}
-__device__ inline float entry_lo(float h, uint32_t e) {
-  const float d = h - __uint_as_float((e >> 11) << 10);
-  return d - fabsf(d) * 2.4e-7f - 1e-37f;
-}
-__device__ inline uint32_t entry_slot(uint32_t e) { return e & 2047u; }
-
+// The same two lists in 32-bit fixed point, filled for both sides during a
+// face's pass without a branch: a point of the other side goes in as the
+// weakest value.  Keys are scaled so that the end of the face's pencil is
+// kLimit; a point whose key lies past it cannot be an apex.  An entry of the
+// sweep list is the key's upper bound, above SB bits of region slot, so that
+// one median of three per entry keeps bound and slot in order; its lower bound
+// is the entry less the face's widest interval.  All bounds err outwards: a
+// wider interval only admits more apex candidates, which are classified
+// exactly, or sends a side to k_rescan.
+__device__ inline uint32_t umed3(uint32_t a, uint32_t b, uint32_t c) { return max(min(a, b), min(max(a, b), c)); }
+template <int SB>
 struct SweepListF {
   static constexpr int kCap = 8;  // >= s_max - 3 for s_max <= 11
-  float hi[kCap];                 // upper key bounds, ascending
-  uint32_t ent[kCap];             // slot and width (pack_entry); kInvalid: empty
-  float evicted_lo;  // smallest lower key bound of a point not in the list
+  static constexpr float kLimit = (float)((1u << (32 - SB)) - 8u);
+  uint32_t hi[kCap];  // entries, ascending; kInvalid: empty
+  uint32_t evicted;   // smallest entry that left or missed the list
   __device__ void init() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) { hi[j] = INFINITY; ent[j] = kInvalid; }
-    evicted_lo = INFINITY;
+    for (int j = 0; j < kCap; ++j) hi[j] = kInvalid;
+    evicted = kInvalid;
   }
-  __device__ void insert(float h, float l, uint32_t s) {
-    if (!(h < hi[kCap - 1])) {
-      evicted_lo = fminf(evicted_lo, l);
-      return;
-    }
-    if (ent[kCap - 1] != kInvalid) evicted_lo = fminf(evicted_lo, entry_lo(hi[kCap - 1], ent[kCap - 1]));
-    const uint32_t e = pack_entry(h, l, s);
+  __device__ void insert(uint32_t e) {
+    evicted = min(evicted, max(hi[kCap - 1], e));
 #pragma unroll
-    for (int j = kCap - 1; j > 0; --j) {
-      ent[j] = h < hi[j - 1] ? ent[j - 1] : (h < hi[j] ? e : ent[j]);
-      hi[j] = __builtin_amdgcn_fmed3f(hi[j - 1], h, hi[j]);
-    }
-    ent[0] = h < hi[0] ? e : ent[0];
-    hi[0] = fminf(hi[0], h);
+    for (int j = kCap - 1; j > 0; --j) hi[j] = umed3(hi[j - 1], e, hi[j]);
+    hi[0] = min(hi[0], e);
   }
-  __device__ float threshold(int need) const {
-    float r = INFINITY;
+  __device__ uint32_t threshold(int need) const {
+    uint32_t r = kInvalid;
 #pragma unroll
     for (int j = 0; j < kCap; ++j) r = (j == need - 1) ? hi[j] : r;
-    return r;
+    return r >> SB;
   }
 };
 struct BehindListF {
   static constexpr int kCap = 4;
-  float v[kCap];
+  uint32_t v[kCap];
   __device__ void init() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) v[j] = -INFINITY;
+    for (int j = 0; j < kCap; ++j) v[j] = 0;
   }
-  __device__ void insert(float x) {
+  __device__ void insert(uint32_t x) {
     // descending: the median of the entry above, x and the entry
 #pragma unroll
-    for (int j = kCap - 1; j > 0; --j) v[j] = __builtin_amdgcn_fmed3f(v[j - 1], x, v[j]);
-    v[0] = fmaxf(v[0], x);
+    for (int j = kCap - 1; j > 0; --j) v[j] = umed3(v[j - 1], x, v[j]);
+    v[0] = max(v[0], x);
   }
-  __device__ int count_above(float x) const {
+  __device__ int count_above(uint32_t x) const {
     int c = 0;
 #pragma unroll
     for (int j = 0; j < kCap; ++j) c += v[j] > x;
@@ -575,37 +561,25 @@ struct TriSphereF {
     n[0] = (float)f.n.x; n[1] = (float)f.n.y; n[2] = (float)f.n.z;
     nA = norm_up(f.nA.x, f.nA.y, f.nA.z);
   }
-  __device__ void eval(float x, float y, float z, float w, float &P, float &PA, float &H, float &HA) const {
-    P = D * (w * w) - (x * g[0] + y * g[1] + z * g[2]);
-    PA = w * (DA * w + gA);
-    H = x * n[0] + y * n[1] + z * n[2];
-    HA = w * nA;
+  __device__ void eval(const float4 &p, float &P, float &PA, float &H, float &HA) const {
+    P = D * (p.w * p.w) - (p.x * g[0] + p.y * g[1] + p.z * g[2]);
+    PA = p.w * (DA * p.w + gA);
+    H = p.x * n[0] + p.y * n[1] + p.z * n[2];
+    HA = p.w * nA;
   }
 };
 // Key interval of a point whose FP32 signs are certified: the true P lies
 // within 1e-6 PA of P32 and |H| within 1e-6 HA of |H32| (< |H32| / 10), so
 // tau = P / |H| lies between the quotients of the extreme values; the
 // roundings of the sums, the reciprocals (1 ulp) and the products stay
-// inside the final 1e-6 widening.
+// inside the final 1e-6 widening.  lf is a lower bound for P > 0 only.
 __device__ inline void key_bounds_32(float Pv, float PA, float H, float HA, float &hf, float &lf) {
   const float ah = fabsf(H), eP = 1e-6f * PA, eH = 1e-6f * HA;
   const float rlo = __builtin_amdgcn_rcpf(ah + eH), rhi = __builtin_amdgcn_rcpf(ah - eH);
-  float lo, hi;
-  if (Pv > 0.0f) {
-    lo = (Pv - eP) * rlo;
-    hi = (Pv + eP) * rhi;
-  } else {
-    lo = (Pv - eP) * rhi;
-    hi = (Pv + eP) * rlo;
-  }
-  lo = lo - 1e-6f * fabsf(lo) - 1e-37f;
-  hi = hi + 1e-6f * fabsf(hi) + 1e-37f;
-  if (!(fabsf(lo) < INFINITY && fabsf(hi) < INFINITY)) {
-    lo = -INFINITY;
-    hi = INFINITY;
-  }
-  hf = hi;
-  lf = lo;
+  lf = (Pv - eP) * rlo;
+  hf = (Pv + eP) * (Pv > 0.0f ? rhi : rlo);
+  lf = lf - 1e-6f * fabsf(lf) - 1e-37f;
+  hf = hf + 1e-6f * fabsf(hf) + 1e-37f;
 }
 
 // The part of a face's pencil that can be critical: spheres through u, v, w
@@ -619,10 +593,10 @@ struct Pencil {
   float l[3], u[3];  // twice the end centres
   float a;           // infinite: every point is kept
   float reach;       // no point farther from the anchor is in any of the spheres (as SphereF::reach)
-  __device__ bool outside(float x, float y, float z, float w) const {
-    const float pp = w * w;
-    const float dl = x * l[0] + y * l[1] + z * l[2], du = x * u[0] + y * u[1] + z * u[2];
-    return pp * 0.999f - a > fmaxf(dl, du);
+  double end;        // sweep key of the farther end, a little past it (0: unrestricted)
+  __device__ bool outside(const float4 &p) const {
+    const float dl = p.x * l[0] + p.y * l[1] + p.z * l[2], du = p.x * u[0] + p.y * u[1] + p.z * u[2];
+    return p.w * p.w * 0.999f - a > fmaxf(dl, du);
   }
 };
 
@@ -632,11 +606,13 @@ __device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi, boo
   Pencil c{};
   c.a = INFINITY;
   c.reach = INFINITY;
+  c.end = 0.0;
   if (!(lo > -INFINITY)) return c;
   const double s = 1.0 / f.D;
   const V3 k = {f.g.x * s, f.g.y * s, f.g.z * s};  // twice the circumcentre
   const double q = sqrt(dot(k, k) * s);            // 2 r3 / |n|
   const double l = lo * q, h = hi * q;
+  c.end = fmax(fabs(l), fabs(h)) * f.D * (1.0 + 1e-3);
   const double cl[3] = {k.x + l * f.n.x, k.y + l * f.n.y, k.z + l * f.n.z};
   const double cu[3] = {k.x + h * f.n.x, k.y + h * f.n.y, k.z + h * f.n.z};
   double ll = 0, uu = 0;
@@ -660,14 +636,14 @@ __device__ inline Pencil face_pencil(const TriSphere &f, float lo, float hi, boo
 // tests32 counts the slots tested (the face's own vertices excluded).
 __device__ inline uint64_t pencil_chunk(const Work &w, const Pencil &c, uint32_t s0, uint32_t M, uint32_t vi,
                                         uint32_t wi, uint32_t &tests32) {
-  const uint32_t cn = min(64u, M - s0);
-  uint64_t in = 0;
+  const uint32_t cn = min(64u, M - s0), c0 = min(cn, 32u);
+  uint32_t lo = 0, hi = 0;
 #pragma unroll 4
-  for (uint32_t j = 0; j < cn; ++j) {
-    const uint32_t gi = s0 + j;
-    const bool keep = !c.outside(w.fx[gi], w.fy[gi], w.fz[gi], w.fw[gi]);
-    in |= (uint64_t)keep << j;
-  }
+  for (uint32_t j = 0; j < c0; ++j) lo = shift_in(lo, !c.outside(w.f[s0 + j]));
+#pragma unroll 4
+  for (uint32_t j = c0; j < cn; ++j) hi = shift_in(hi, !c.outside(w.f[s0 + j]));
+  uint64_t in = in_order(lo, c0);
+  if (cn > 32) in |= (uint64_t)in_order(hi, cn - 32) << 32;
   if (vi - s0 < cn) in &= ~(1ull << (vi - s0));
   if (wi - s0 < cn) in &= ~(1ull << (wi - s0));
   tests32 += cn;
@@ -696,23 +672,25 @@ struct Rescan {
   float lo, hi;
 };
 
-// Apexes of one side among the FP32 list its face's first pass filled: bit j
-// for entry j.  rescan: a point left or missed the list with a lower bound
-// within the threshold, so the side takes its own passes instead.
-__device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF &top, const BehindListF &beh, bool &rescan) {
+// Apexes of one side among the FP32 list its face's pass filled: bit j for
+// entry j.  rescan: a point left or missed the list with a lower bound within
+// the threshold, so the side takes its own passes instead.
+template <int SB>
+__device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF<SB> &top, const BehindListF &beh,
+                                     uint32_t widest, bool &rescan) {
   rescan = false;
   if (cin_side >= K) return 0;
-  const float thr = top.threshold(K - cin_side);
-  if (top.evicted_lo != INFINITY && top.evicted_lo <= thr) {
+  const uint32_t thr = top.threshold(K - cin_side) + widest;
+  if (top.evicted != kInvalid && (top.evicted >> SB) <= thr) {
     rescan = true;
     return 0;
   }
   uint32_t cand = 0;
 #pragma unroll
-  for (int j = 0; j < SweepListF::kCap; ++j) {
+  for (int j = 0; j < SweepListF<SB>::kCap; ++j) {
     // inside points behind: counted while their key exceeds z's
-    const bool ok = top.ent[j] != kInvalid && entry_lo(top.hi[j], top.ent[j]) <= thr &&
-                    cin_side + beh.count_above(top.hi[j]) < K;
+    const uint32_t h = top.hi[j] >> SB;
+    const bool ok = top.hi[j] != kInvalid && h <= thr && cin_side + beh.count_above(h) < K;
     cand |= ok ? (1u << j) : 0u;
   }
   return cand;
@@ -728,7 +706,7 @@ __device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF &top,
 // The pass runs on the region's FP32 copies (FP64 only for the points whose FP32
 // signs are not certified) and sees the points that some sphere of the face's
 // pencil within [lo, hi] (face_interval; n oriented as v x w) can hold.
-template <bool QUEUED>
+template <bool QUEUED, int SB>
 __device__ __attribute__((always_inline)) inline void process_face(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
                              uint32_t wi, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
   // the sphere is built from its points in PointId order, so its FP64 level
@@ -760,33 +738,35 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
   // s_max - 3 <= 8)
   uint32_t tri_pk[kPacked] = {};
   uint32_t evals = 0;
-  SweepListF top0, top1;  // outside points ahead of side 0 / 1
+  SweepListF<SB> top0, top1;  // outside points ahead of side 0 / 1
   BehindListF beh0, beh1;  // inside points behind side 0 / 1
   top0.init();
   top1.init();
   beh0.init();
   beh1.init();
   constexpr uint32_t kFlopPoint = kFlopFacePoint + kFlopSweepKey;
-  uint32_t tests32 = 0, evals32 = 0, keys32 = 0;  // FP32 work
+  uint32_t tests32 = 0, evals32 = 0;  // FP32 work
+  constexpr float kLimit = SweepListF<SB>::kLimit;
+  const double per_key = kLimit / pen.end;
+  const float scale = per_key < 1e37 ? (float)per_key : 0.0f;  // 0: all keys are equal
+  uint32_t widest = 0;                                          // widest key interval
+  const int tri_limit = tri ? smax - 2 : 0;  // inside points that exclude the triangle
   TriSphereF f32;
   f32.init(f);
 #pragma unroll 1
   for (uint32_t s0 = 0; s0 < M; s0 += 64) {
-    if (w.fw[s0] > pen.reach) break;
+    if (w.f[s0].w > pen.reach) break;
     uint64_t in = pencil_chunk(w, pen, s0, M, vi, wi, tests32);
 #pragma unroll 1
     while (in) {
       const uint32_t gi = s0 + (uint32_t)(__ffsll((long long)in) - 1);
       in &= in - 1;
-      float hf = 0.0f, lf = 0.0f;
-      float P32, PA32, H32, HA32;
-      f32.eval(w.fx[gi], w.fy[gi], w.fz[gi], w.fw[gi], P32, PA32, H32, HA32);
-      int sp = cert32(P32, PA32), sh = cert32(H32, HA32);
+      float hf, lf, P32, PA32, H32, HA32;
+      f32.eval(w.f[gi], P32, PA32, H32, HA32);
+      bool outer = P32 > 0.0f, above = H32 > 0.0f;
       evals32++;
-      if (sp != 0 && sh != 0) {
-        key_bounds_32(P32, PA32, H32, HA32, hf, lf);
-        keys32++;
-      } else {
+      key_bounds_32(P32, PA32, H32, HA32, hf, lf);
+      if (cert32(P32, PA32) == 0 || cert32(H32, HA32) == 0) {
         const V3 p = gpt(w, gi);
         evals++;
         double Pw, PA, H, HA;
@@ -796,44 +776,50 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
         f64.init(gpt(w, vi), gpt(w, wi));
         f64.power(p, Pw, PA);
         f64.height(p, H, HA);
-        sp = cert_sign(Pw, PA);
-        sh = cert_sign(H, HA);
+        const int sp = cert_sign(Pw, PA), sh = cert_sign(H, HA);
         // every sign the side passes use is certified here, before anything is emitted
         if (sp == 0 || sh == 0) {
           add_flops(w, (uint64_t)evals * kFlopPoint);
-          add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+          add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * (kF32FacePoint + kF32Key));
           emit_fallback(P, w, u, 3, ids, 3, M, region_slot);
           return;
         }
         double tau, terr;
         sweep_key(Pw, PA, H, HA, tau, terr);
         key_bounds_f(tau, terr, hf, lf);
+        outer = sp > 0;
+        above = sh > 0;
+        if (!outer) hf = fminf(hf, 0.0f);  // a key interval that reaches past 0: weakest
       }
-      if (sp > 0) {
-        // outside: ahead of side 0 when sh > 0, of side 1 otherwise
-        if (sh > 0) top0.insert(hf, lf, gi);
-        else top1.insert(hf, lf, gi);
-      } else {
-        // inside: behind side 1 when sh > 0, behind side 0 otherwise; -hf
-        // is a lower bound of -tau - terr
-        if (sh > 0) beh1.insert(-hf);
-        else beh0.insert(-hf);
-      }
-      if (sp > 0) continue;
-      if (total_in < kMaxInterior) put_packed(tri_pk, total_in, gi);
+      // fixed point, the multiplication's rounding and the truncation within 2
+      const uint32_t h = (uint32_t)fminf(fabsf(hf * scale), kLimit);
+      // outside: ahead of side 0 when above, of side 1 otherwise
+      const float ls = lf * scale;
+      const bool ahead = outer && !(ls >= kLimit);
+      const uint32_t e = (h + 2u) << SB | gi, width = h + 4u - (uint32_t)__builtin_amdgcn_fmed3f(ls, 0.0f, kLimit);
+      widest = max(widest, ahead ? width : 0u);
+      top0.insert(ahead && above ? e : kInvalid);
+      top1.insert(ahead && !above ? e : kInvalid);
+      // inside: behind side 1 when above, behind side 0 otherwise; -hf is a
+      // lower bound of -tau - terr
+      const uint32_t x = outer ? 0u : max(h, 2u) - 2u;
+      beh0.insert(above ? 0u : x);
+      beh1.insert(above ? x : 0u);
+      if (outer) continue;
+      push_packed(tri_pk, gi);
       total_in++;
-      cin0 += sh > 0;
-      cin1 += sh < 0;
+      cin0 += above;
+      cin1 += !above;
       // both sides saturated and the triangle out of rank: nothing left here
-      if (cin0 >= K && cin1 >= K && (!tri || total_in + 3 > smax)) {
+      if (cin0 >= K && cin1 >= K && total_in >= tri_limit) {
         add_flops(w, (uint64_t)evals * kFlopPoint);
-        add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+        add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * (kF32FacePoint + kF32Key));
         return;
       }
     }
   }
   add_flops(w, (uint64_t)evals * kFlopPoint);
-  add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * kF32FacePoint + (uint64_t)keys32 * kF32Key);
+  add_flops32(w, (uint64_t)tests32 * kF32Pencil + (uint64_t)evals32 * (kF32FacePoint + kF32Key));
   // triangle event
   if (!tri) {
     // not critical by the certificate
@@ -849,19 +835,19 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
   }
   if (K <= 0) return;
   bool rescan[2];
-  uint32_t cand = apex_mask(cin0, K, top0, beh0, rescan[0]);
-  cand |= apex_mask(cin1, K, top1, beh1, rescan[1]) << SweepListF::kCap;
+  uint32_t cand = apex_mask(cin0, K, top0, beh0, widest, rescan[0]);
+  cand |= apex_mask(cin1, K, top1, beh1, widest, rescan[1]) << SweepListF<SB>::kCap;
   // queued on the LDS paths, in place on the global-memory path
   while (cand) {
     const int j = __ffs(cand) - 1;
     cand &= cand - 1;
     uint32_t ent = 0;  // selected by static index, the lists stay in registers
 #pragma unroll
-    for (int e = 0; e < SweepListF::kCap; ++e) {
-      ent = e == j ? top0.ent[e] : ent;
-      ent = e + SweepListF::kCap == j ? top1.ent[e] : ent;
+    for (int e = 0; e < SweepListF<SB>::kCap; ++e) {
+      ent = e == j ? top0.hi[e] : ent;
+      ent = e + SweepListF<SB>::kCap == j ? top1.hi[e] : ent;
     }
-    const uint32_t zi = entry_slot(ent);
+    const uint32_t zi = ent & ((1u << SB) - 1u);
     if (w.gid[zi] <= wid) continue;
     if (QUEUED) {
       const uint32_t at = atomicAdd(q->ntet, 1u);
@@ -1103,7 +1089,7 @@ __device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si
 // the faces, and takes its share of them and of the pairs.  The workgroups
 // beyond one per kSplitFaces candidate faces have nothing to do.
 constexpr uint64_t kSplitFaces = 2048;
-template <bool BIG, bool SPLIT, int WAVES>
+template <bool BIG, bool SPLIT, int WAVES, int SB>
 __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t *sK_,
                              uint32_t *sregion_) {
   uint32_t &sK = *sK_;
@@ -1125,10 +1111,8 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
     if (t == 0) sK = k;
   }
   for (uint32_t s = t; s < M; s += blockDim.x) {
-    w.fx[s] = (float)w.gx[s];
-    w.fy[s] = (float)w.gy[s];
-    w.fz[s] = (float)w.gz[s];
-    w.fw[s] = (float)sqrt(w.gx[s] * w.gx[s] + w.gy[s] * w.gy[s] + w.gz[s] * w.gz[s]);
+    const V3 p = gpt(w, s);
+    w.f[s] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)sqrt(dot(p, p)));
   }
   __syncthreads();
   const uint32_t Kc = sK;
@@ -1148,7 +1132,8 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
   // path works in place).
   __shared__ uint32_t q_pair[WAVES][128];
   __shared__ uint32_t q_face[WAVES][128];
-  __shared__ float q_key[WAVES][128], q_lo[WAVES][128], q_hi[WAVES][128];
+  __shared__ uint32_t q_key[WAVES][128];  // key (a positive float) with its low 7 bits the position: no ties
+  __shared__ float q_lo[WAVES][128], q_hi[WAVES][128];
   __shared__ uint32_t q_tet[WAVES][kTetQ];
   __shared__ uint32_t q_n[WAVES];
   const int wave = t >> 6, lane = t & 63, nwaves = (int)(blockDim.x >> 6);
@@ -1174,7 +1159,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       uint32_t si, sj;
       face_of(fidx, si, sj);
       float lo, hi, key;
-      if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false>(P, w, u, M, si, sj, lo, hi, &sregion, q);
+      if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false, SB>(P, w, u, M, si, sj, lo, hi, &sregion, q);
     }
   } else {
     // Each wave lists the candidate faces that share a cell (q_pair), takes 64
@@ -1215,7 +1200,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
         if (ok) {
           const uint32_t at = nf + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
           q_face[wave][at] = fv;
-          q_key[wave][at] = key;
+          q_key[wave][at] = (__float_as_uint(key) & ~127u) | at;
           q_lo[wave][at] = lo;
           q_hi[wave][at] = hi;
         }
@@ -1224,28 +1209,22 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       }
       wave_sync();
       if (nf > 64) {
-        // rank sort of the list by key (ties by position), ascending
-        uint32_t fv[2], rk[2];
-        float lv[2], hv[2], kv[2];
+        // rank sort of the list by key, ascending
+        uint32_t fv[2], kv[2], rk[2] = {0, 0};
+        float lv[2], hv[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t i = (uint32_t)lane + 64u * h;
-          fv[h] = 0;
-          rk[h] = 0;
-          lv[h] = hv[h] = kv[h] = 0.0f;
-          if (i < nf) {
-            const float ki = q_key[wave][i];
-            kv[h] = ki;
-            fv[h] = q_face[wave][i];
-            lv[h] = q_lo[wave][i];
-            hv[h] = q_hi[wave][i];
-            uint32_t r = 0;
-            for (uint32_t j = 0; j < nf; ++j) {
-              const float kj = q_key[wave][j];
-              r += kj < ki || (kj == ki && j < i);
-            }
-            rk[h] = r;
-          }
+          const bool has = i < nf;
+          kv[h] = has ? q_key[wave][i] : ~0u;
+          fv[h] = has ? q_face[wave][i] : 0;
+          lv[h] = has ? q_lo[wave][i] : 0.0f;
+          hv[h] = has ? q_hi[wave][i] : 0.0f;
+        }
+        for (uint32_t j = 0; j < nf; ++j) {
+          const uint32_t kj = q_key[wave][j];
+          rk[0] += kj < kv[0];
+          rk[1] += kj < kv[1];
         }
         wave_sync();
 #pragma unroll
@@ -1254,7 +1233,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
             q_face[wave][rk[h]] = fv[h];
             q_lo[wave][rk[h]] = lv[h];
             q_hi[wave][rk[h]] = hv[h];
-            q_key[wave][rk[h]] = kv[h];
+            q_key[wave][rk[h]] = (kv[h] & ~127u) | rk[h];
           }
         wave_sync();
       }
@@ -1263,7 +1242,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if ((uint32_t)lane < take) {
         const uint32_t fv = q_face[wave][nf + lane];
         const uint32_t si = fv & 1023u, sj = fv >> 10;
-        process_face<true>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
+        process_face<true, SB>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
       }
       wave_sync();
       // whole rounds of 64 tetrahedra (the top of the queue); the rest waits
@@ -1476,7 +1455,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
     if (t == 0) probed(P, u, a, M);
     return;
   }
-  anchor_faces<true, false, kBlock / 64>(P, w, u, M, &sK, &sregion);
+  anchor_faces<true, false, kBlock / 64, 11>(P, w, u, M, &sK, &sregion);
 }
 
 // Slab of one probed anchor (in doubles), for G gathered points:
@@ -1718,10 +1697,7 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
   w.fc = reinterpret_cast<float4 *>(slab + big_fc_offset(G));
   // the FP32 region copies take the FP32 offsets' area once the region is
   // compacted (4G floats)
-  w.fx = reinterpret_cast<float *>(w.fc);
-  w.fy = w.fx + G;
-  w.fz = w.fy + G;
-  w.fw = w.fz + G;
+  w.f = w.fc;
   __shared__ uint32_t cand;
   __shared__ unsigned long long flops;
   if (threadIdx.x == 0) { cand = 0; flops = 0; }
@@ -1756,13 +1732,16 @@ __global__ void __launch_bounds__(kBlock) k_anchor_big(Params P) {
 // the longest ones do not end it alone.  A 2 003-point mixture's catalogue:
 // 885 -> 332 ms.
 //
-// VALU bound: of 58 ms for the 50 000-point lattice K 10 (25 million records)
-// about 27 are the faces' passes, 18 the pairs of vertices that share a cell
-// and their intervals, 4 the tetrahedra, and 7 the loads, pairs and queues.
-// Its registers were what held it back (FP64 state of rare passes spilled 160
-// of them); with those passes in k_rescan, scans that end at a sphere's
-// diameter and id lists read from bit masks: 73 -> 58 ms, K 4 19.3 -> 18.3 ms,
-// the mixture's catalogue 75.6 -> 67.2 ms.
+// Bound by VALU issue: 14 G wave instructions for the 50 000-point lattice K 10
+// (25 million records), 23 of the launches' 28 ms; about 4.5 G in the points of
+// the faces' passes (39 million wave steps), 2.8 G in the interval walks (55
+// million), 1.8 G in the pencil tests (143 million slots), 1.3 G in the
+// tetrahedra.  FP64 state of rare passes spilled 160 registers (k_rescan has
+// them now).  Scans that end at a sphere's diameter and id lists read from bit
+// masks: 73 -> 58 ms for the whole enumeration with its probes; sweep lists of
+// one word per entry, filled without branches, bits shifted in by add with
+// carry and a rank sort without ties: 46 -> 39 ms, 1 000 points 1.75 -> 1.55 ms,
+// uniform 8 000 points K 8 8.5 -> 6.5 ms.
 constexpr uint32_t kRegionParts = 4096;
 constexpr uint32_t kSmallRegionLaunch = 8192;  // anchors of a launch that splits off the small regions
 template <int RCAP, int WAVES, int PER_SIMD>
@@ -1780,7 +1759,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   __shared__ float rho[kCells];
   __shared__ uint64_t rmask[6 * RCAP];
   __shared__ uint16_t kidx[RCAP];
-  __shared__ float fx[RCAP], fy[RCAP], fz[RCAP], fw[RCAP];
+  __shared__ float4 f[RCAP];
   __shared__ float4 cell[64];
   __shared__ uint32_t cand, sK, sregion;
   __shared__ unsigned long long flops, flops32;
@@ -1825,9 +1804,9 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   for (int c = t; c < kCells; c += blockDim.x) rho[c] = reinterpret_cast<const float *>(slab + 3 * G)[c];
   if (t == 0) { cand = 0; sK = 0; sregion = kInvalid; flops = 0; flops32 = 0; }
   __syncthreads();
-  Work w{gx, gy, gz, gid, rho, nullptr, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, fx, fy, fz, fw,
+  Work w{gx, gy, gz, gid, rho, nullptr, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, f,
          P.count_flops ? &flops32 : nullptr, true, a, cell};
-  anchor_faces<false, true, WAVES>(P, w, u, M, &sK, &sregion);
+  anchor_faces<false, true, WAVES, RCAP <= 256 ? 8 : RCAP <= 512 ? 9 : 10>(P, w, u, M, &sK, &sregion);
 }
 
 // Sides of faces left by the enumeration of one launch, one per wave, in FP64
@@ -1837,7 +1816,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
 // pass has certified every sign with the same arithmetic.  Few sides come here
 // (0 to a few hundred of a catalogue), so their latency counts: M / 64 steps
 // a scan.  The grid is fixed; the number of sides is read on the device.
-constexpr int kRescanBlocks = 1024;
+constexpr int kRescanBlocks = 4096;
 __global__ void __launch_bounds__(64) k_rescan(Params P) {
   const unsigned long long count = min(P.counters[4], (unsigned long long)P.rescan_cap);
   const uint64_t G = P.gcap;
@@ -1865,7 +1844,7 @@ __global__ void __launch_bounds__(64) k_rescan(Params P) {
       const uint32_t id = w.gid[s];
       if (id == r.v || id == r.w) return false;
       const V3 p = gpt(w, s);
-      if (pen.outside((float)p.x, (float)p.y, (float)p.z, (float)sqrt(p.x * p.x + p.y * p.y + p.z * p.z))) return false;
+      if (pen.outside(make_float4((float)p.x, (float)p.y, (float)p.z, (float)sqrt(dot(p, p))))) return false;
       evals++;
       double Pw, PA, H, HA;
       f.power(p, Pw, PA);
@@ -2200,7 +2179,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   uint64_t event_cap = std::max<uint64_t>(1024, (uint64_t)n * (smax >= 11 ? 640 : 64 * smax));
   uint64_t fb_cap = std::max<uint64_t>(4096, (uint64_t)n / 4);
   uint64_t reg_cap = std::max<uint64_t>(1 << 20, (uint64_t)n * 64);
-  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n);
+  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n * 16);
   uint64_t ctr[kCounters];
   int64_t widened = 0;
   // The record queues have a fixed capacity per launch; records past it are
