@@ -273,7 +273,7 @@ void contract_order(int k, int64_t n, TowerOrderData &D, Forest &F) {
     if ((int64_t)D.carrier[a] >= M) throw std::runtime_error("an arm's carrier lies outside the order's minima");
   std::vector<Cell> cell(M);
   for (int64_t x = 0; x < M; ++x) cell[x] = {(uint32_t)x, -1};
-  F.reserve(k == 1 ? (size_t)n + D.saddles / 8 : D.saddles / 8);
+  F.reserve((k == 1 ? (size_t)n : 0) + D.saddles, D.arms);
   F.acq_node.assign(M, -1);
   F.acq_cls.assign(M, -1);
   if (k == 1)
@@ -495,11 +495,17 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
   const int K = (int)std::min<int64_t>(k_max, n);
   if (!c.tower) c.tower = std::make_unique<TowerState>();
   TowerState &T = *c.tower;
+  // The forests take the storage of the context's last tower, unless that was
+  // of a cloud more than four times as large: 3.4 million nodes are 200 MB, and
+  // returning and faulting them in again was most of a contraction's time.
+  std::vector<Forest> forests;
+  if (T.points <= 4 * n) forests.swap(T.forests);
   T = TowerState{};
+  for (Forest &F : forests) F.clear();
+  forests.resize(K);
   std::unique_ptr<Descender> desc;  // host exact descents, built on demand
   std::vector<double> xyz;
   std::vector<TowerOrderData> Ds(K);
-  std::vector<Forest> forests(K);
   std::vector<std::exception_ptr> errors(K);
   std::vector<std::thread> workers;
   struct Joiner {
@@ -694,6 +700,7 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
   T.forests = std::move(forests);
   T.descent_steps += desc ? desc->steps : 0;
   T.orders = K;
+  T.points = n;
   T.level_exp = -2 * c.scale_exp;
   T.status = 0;
   T.valid = true;

@@ -3,6 +3,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <functional>
 #include <thread>
 #include <vector>
 
@@ -45,7 +46,22 @@ struct Forest {
   int64_t add(int32_t o, int32_t k, int64_t cls, double lev, const std::vector<int64_t> &kids) {
     return add(o, k, cls, lev, kids.data(), kids.size());
   }
-  void reserve(size_t nodes) {
+  // empty again, with its storage
+  void clear() {
+    order.clear();
+    kind.clear();
+    level_class.clear();
+    level.clear();
+    child_offset.assign(1, 0);
+    children.clear();
+    parent.clear();
+    acq_node.clear();
+    acq_cls.clear();
+    rep_elem.clear();
+    raw_of_dense.clear();
+    vtarget.clear();
+  }
+  void reserve(size_t nodes, size_t kids) {
     rep_elem.reserve(nodes);
     order.reserve(nodes);
     kind.reserve(nodes);
@@ -53,13 +69,14 @@ struct Forest {
     level.reserve(nodes);
     parent.reserve(nodes);
     child_offset.reserve(nodes + 1);
-    children.reserve(2 * nodes);
+    children.reserve(kids);
   }
 };
 
 struct TowerState {
   bool valid = false;
   std::vector<Forest> forests;  // order k at index k - 1
+  int64_t points = 0;           // of the cloud the forests were built from
   int64_t node_count = 0, child_count = 0;
   int64_t descent_steps = 0;
   int32_t orders = 0;
@@ -67,39 +84,48 @@ struct TowerState {
   int level_exp = 0;  // levels are reported times 2^level_exp (device unit -> input unit)
 
   // The tower as one node list: orders ascending, node ids and child offsets
-  // shifted by the nodes and children of the orders below (one thread per
-  // order, each writes its own ranges).
+  // shifted by the nodes and children of the orders below (each order writes
+  // its own ranges).
   void copy_out(int32_t *order, int32_t *kind, int64_t *level_class, double *level, int64_t *child_offset,
                 int64_t *children) const {
     child_offset[0] = 0;
-    std::vector<std::thread> th;
-    int64_t nb = 0, cb = 0;
-    for (const Forest &F : forests) {
-      const int lexp = level_exp;
-      th.emplace_back([&F, nb, cb, lexp, order, kind, level_class, level, child_offset, children] {
-        const size_t m = F.order.size();
-        std::copy(F.order.begin(), F.order.end(), order + nb);
-        std::copy(F.kind.begin(), F.kind.end(), kind + nb);
-        std::copy(F.level_class.begin(), F.level_class.end(), level_class + nb);
-        for (size_t i = 0; i < m; ++i) level[nb + (int64_t)i] = std::ldexp(F.level[i], lexp);
-        for (size_t i = 1; i <= m; ++i) child_offset[nb + (int64_t)i] = cb + F.child_offset[i];
-        for (size_t j = 0; j < F.children.size(); ++j) children[cb + (int64_t)j] = nb + F.children[j];
-      });
-      nb += (int64_t)F.order.size();
-      cb += (int64_t)F.children.size();
-    }
-    for (auto &t : th) t.join();
+    each_order([=](const Forest &F, int64_t nb, int64_t cb, int64_t) {
+      const size_t m = F.order.size();
+      std::copy(F.order.begin(), F.order.end(), order + nb);
+      std::copy(F.kind.begin(), F.kind.end(), kind + nb);
+      std::copy(F.level_class.begin(), F.level_class.end(), level_class + nb);
+      for (size_t i = 0; i < m; ++i) level[nb + (int64_t)i] = std::ldexp(F.level[i], level_exp);
+      for (size_t i = 1; i <= m; ++i) child_offset[nb + (int64_t)i] = cb + F.child_offset[i];
+      for (size_t j = 0; j < F.children.size(); ++j) children[cb + (int64_t)j] = nb + F.children[j];
+    });
   }
 
   // Vertical targets as global node ids (orders ascending), -1 at order one.
   void copy_vertical(int64_t *target) const {
-    int64_t nb = 0, below = 0;
-    for (const Forest &F : forests) {
+    each_order([=](const Forest &F, int64_t nb, int64_t, int64_t below) {
       for (size_t i = 0; i < F.order.size(); ++i)
         target[nb + (int64_t)i] = (F.vtarget.empty() || F.vtarget[i] < 0) ? -1 : below + F.vtarget[i];
+    });
+  }
+
+ private:
+  // f(forest, nodes below it, children below it, nodes below the order below)
+  // for every order, a thread each: the outputs are fresh memory, and one
+  // thread's page faults bound the copy (3.4 million nodes).  A small tower is
+  // copied before its threads would have started.
+  template <class F>
+  void each_order(F f) const {
+    std::vector<std::thread> th;
+    int64_t nb = 0, cb = 0, below = 0;
+    const bool small = node_count < 1 << 15;
+    for (const Forest &G : forests) {
+      if (small) f(G, nb, cb, below);
+      else th.emplace_back(f, std::cref(G), nb, cb, below);
       below = nb;
-      nb += (int64_t)F.order.size();
+      nb += (int64_t)G.order.size();
+      cb += (int64_t)G.children.size();
     }
+    for (auto &t : th) t.join();
   }
 };
 
