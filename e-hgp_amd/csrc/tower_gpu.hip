@@ -995,10 +995,6 @@ __global__ void k_fill_u64(uint64_t *p, int64_t n, uint64_t v) {
   if (i < n) p[i] = v;
 }
 
-__global__ void k_identity(uint32_t *p, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (uint32_t)i;
-}
 
 __global__ void k_first_touch(const uint32_t *__restrict__ arm_saddle, const uint32_t *__restrict__ carrier,
                               int64_t arms, int64_t minima, uint32_t *first, uint32_t *invalid) {
@@ -1009,7 +1005,9 @@ __global__ void k_first_touch(const uint32_t *__restrict__ arm_saddle, const uin
     *invalid = 1u;
     return;
   }
-  atomicMin(&first[c], arm_saddle[a]);
+  // arms come in saddle order, so a plain read first spares most atomics
+  const uint32_t s = arm_saddle[a];
+  if (s < first[c]) atomicMin(&first[c], s);
 }
 
 __device__ inline bool carrier_owned(const uint32_t *first, uint32_t c, uint32_t s, int all_owned) {
@@ -1035,65 +1033,104 @@ __global__ void k_attach(int64_t S, const uint32_t *__restrict__ base, const uin
   }
 }
 
-// Star edge of arm a: an owned carrier on a representative that neither the
-// saddle's first owned carrier nor an earlier owned arm has.
-__device__ inline bool arm_edge(const uint32_t *base, const uint32_t *incl, const uint32_t *carrier,
-                                const uint32_t *first, const uint32_t *rep, uint32_t s, uint32_t a, int all_owned,
-                                uint32_t &r0, uint32_t &r) {
-  const uint32_t c = carrier[a];
-  if (!carrier_owned(first, c, s, all_owned)) return false;
-  r = rep[c];
-  uint32_t x = base[s];
-  while (!carrier_owned(first, carrier[x], s, all_owned)) ++x;  // a itself is owned
-  if (x == a) return false;
-  r0 = rep[carrier[x]];
-  if (r == r0) return false;
-  for (++x; x < a; ++x)
-    if (carrier_owned(first, carrier[x], s, all_owned) && rep[carrier[x]] == r) return false;
-  (void)incl;
-  return true;
+// Star edges of a saddle, in arm order: from the representative of its first
+// owned carrier to each other representative of an owned carrier.  f(r0, r);
+// returns their number (at most 3).
+//
+// A thread per saddle reads each of its up to four carriers once.  A thread
+// per arm had to look through the arms before it again, 3.6 arms a saddle, and
+// the scan ran over the arms: for 20.6 million arms 1.5 ms,
+// now 1.2 ms.
+template <class F>
+__device__ inline uint32_t star_edges(const uint32_t *base, const uint32_t *incl, const uint32_t *carrier,
+                                      const uint32_t *first, const uint32_t *rep, uint32_t s, int all_owned, F f) {
+  const uint32_t b = base[s], e = incl[s];
+  uint32_t seen[4], n = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q) {
+    if (b + q >= e) continue;
+    const uint32_t c = carrier[b + q];
+    if (!carrier_owned(first, c, s, all_owned)) continue;
+    const uint32_t r = rep[c];
+    bool known = false;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) known |= k < n && seen[k] == r;
+    if (known) continue;
+    if (n) f(seen[0], r, n - 1);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) seen[k] = k == n ? r : seen[k];
+    n++;
+  }
+  return n ? n - 1 : 0;
 }
 
-__global__ void k_edge_flags(const uint32_t *__restrict__ arm_saddle, const uint32_t *__restrict__ base,
-                             const uint32_t *__restrict__ incl, const uint32_t *__restrict__ carrier,
-                             const uint32_t *__restrict__ first, const uint32_t *__restrict__ rep, int all_owned,
-                             int64_t arms, uint32_t *flag) {
-  int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= arms) return;
-  uint32_t r0, r;
-  flag[a] = arm_edge(base, incl, carrier, first, rep, arm_saddle[a], (uint32_t)a, all_owned, r0, r) ? 1u : 0u;
+__global__ void k_edge_counts(int64_t S, const uint32_t *__restrict__ base, const uint32_t *__restrict__ incl,
+                              const uint32_t *__restrict__ carrier, const uint32_t *__restrict__ first,
+                              const uint32_t *__restrict__ rep, int all_owned, uint32_t *count) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= S) return;
+  count[s] = star_edges(base, incl, carrier, first, rep, (uint32_t)s, all_owned, [](uint32_t, uint32_t, uint32_t) {});
 }
 
-__global__ void k_edge_list(const uint32_t *__restrict__ arm_saddle, const uint32_t *__restrict__ base,
-                            const uint32_t *__restrict__ incl, const uint32_t *__restrict__ carrier,
-                            const uint32_t *__restrict__ first, const uint32_t *__restrict__ rep, int all_owned,
-                            const uint32_t *__restrict__ scan, int64_t arms, uint32_t *eu, uint32_t *ev,
-                            uint32_t *es) {
-  int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= arms) return;
-  const uint32_t prev = a ? scan[a - 1] : 0u;
-  if (scan[a] == prev) return;
-  const uint32_t s = arm_saddle[a];
-  uint32_t r0 = 0, r = 0;
-  arm_edge(base, incl, carrier, first, rep, s, (uint32_t)a, all_owned, r0, r);
-  eu[prev] = r0;
-  ev[prev] = r;
-  es[prev] = s;
+// scan: the saddles' edge counts, inclusive
+__global__ void k_edge_list(int64_t S, const uint32_t *__restrict__ base, const uint32_t *__restrict__ incl,
+                            const uint32_t *__restrict__ carrier, const uint32_t *__restrict__ first,
+                            const uint32_t *__restrict__ rep, int all_owned, const uint32_t *__restrict__ scan,
+                            uint32_t *eu, uint32_t *ev, uint32_t *es) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= S) return;
+  const uint32_t at = s ? scan[s - 1] : 0u;
+  if (scan[s] == at) return;
+  star_edges(base, incl, carrier, first, rep, (uint32_t)s, all_owned, [&](uint32_t r0, uint32_t r, uint32_t j) {
+    eu[at + j] = r0;
+    ev[at + j] = r;
+    es[at + j] = (uint32_t)s;
+  });
+}
+
+// Edge lists from this length on contract their first quarter first: forest of
+// 6.4 million edges (order 10 of a 50 000-point lattice) 5.0 -> 3.0 ms; a
+// twelfth or a sixteenth and a quarter first were slower (tower 45.9, 46.9 and
+// 48.3 ms).  Shorter lists are bound by launches and waits: three launches a
+// round and two rounds a wait, 70 000 edges 0.55 -> 0.27 ms.
+constexpr uint32_t kMsfSplit = 1u << 20;
+
+// Counters of one Boruvka round
+struct MsfRound {
+  unsigned long long live;  // edges that still joined two components
+  uint32_t changed, cyclic;
+};
+constexpr int kMsfRounds = 256;
+
+__global__ void k_msf_init(int64_t M, int64_t E, int64_t S, uint32_t *comp, uint32_t *best, uint32_t *msf,
+                           uint32_t *mcount, MsfRound *rounds) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < M) {
+    comp[i] = (uint32_t)i;
+    best[i] = kInvalid;
+  }
+  if (i < E) msf[i] = 0u;
+  if (i < S) mcount[i] = 0u;
+  if (i < kMsfRounds) rounds[i] = MsfRound{0ull, 0u, 0u};
 }
 
 // Boruvka round, part 1: least edge (by index) leaving each component.  The
-// edges still joining two components are appended to the next round's list
-// (li == nullptr: the list is the full edge list, li[i] = i).
+// edges still joining two components are appended to the next round's list.
+// The list holds L edges, or *live of them when given (at most L); li ==
+// nullptr: it is the edge list from `base` on, edge i at base + i.
 constexpr int kMsfBlock = 1024;
-__global__ void __launch_bounds__(kMsfBlock) k_msf_best(int64_t L, const uint32_t *__restrict__ lu, const uint32_t *__restrict__ lv,
-                           const uint32_t *__restrict__ li, const uint32_t *__restrict__ comp, uint32_t *best,
-                           uint32_t *ou, uint32_t *ov, uint32_t *oi, unsigned long long *count) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kMsfBlock) k_msf_best(int64_t L, const unsigned long long *live_in, const uint32_t *__restrict__ lu,
+                           const uint32_t *__restrict__ lv, const uint32_t *__restrict__ li, uint32_t base,
+                           const uint32_t *__restrict__ comp, uint32_t *best, uint32_t *ou, uint32_t *ov, uint32_t *oi,
+                           MsfRound *round) {
+  if (live_in) L = min(L, (int64_t)*live_in);
+  if ((int64_t)blockIdx.x * kMsfBlock >= L) return;
+  const int64_t i = (int64_t)blockIdx.x * kMsfBlock + threadIdx.x;
   uint32_t u = 0, v = 0, idx = 0, cu = 0, cv = 0;
   if (i < L) {
     u = lu[i];
     v = lv[i];
-    idx = li ? li[i] : (uint32_t)i;
+    idx = li ? li[i] : base + (uint32_t)i;
     cu = comp[u];
     cv = comp[v];
   }
@@ -1104,7 +1141,7 @@ __global__ void __launch_bounds__(kMsfBlock) k_msf_best(int64_t L, const uint32_
     if (idx < best[cu]) atomicMin(&best[cu], idx);
     if (idx < best[cv]) atomicMin(&best[cv], idx);
   }
-  const uint64_t pos = block_append<kMsfBlock / 64>(live ? 1u : 0u, count);
+  const uint64_t pos = block_append<kMsfBlock / 64>(live ? 1u : 0u, &round->live);
   if (live) {
     ou[pos] = u;
     ov[pos] = v;
@@ -1113,29 +1150,27 @@ __global__ void __launch_bounds__(kMsfBlock) k_msf_best(int64_t L, const uint32_
 }
 
 // Part 2: every component root hooks along its least edge, which is a forest
-// edge; of a pair choosing the same edge the smaller root stays a root.
-// comp is only read here; the hooks are applied by the next kernel.
+// edge; of a pair choosing the same edge the smaller root stays a root.  next
+// takes the hook forest over all minima.
 __global__ void k_msf_hook(int64_t M, const uint32_t *__restrict__ eu, const uint32_t *__restrict__ ev,
-                           const uint32_t *__restrict__ comp, const uint32_t *__restrict__ best, uint32_t *hook,
-                           uint32_t *msf, uint32_t *changed) {
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M || comp[m] != (uint32_t)m) return;
-  const uint32_t i = best[m];
-  if (i == kInvalid) return;
-  const uint32_t cu = comp[eu[i]], cv = comp[ev[i]];
-  const uint32_t other = cu == (uint32_t)m ? cv : cu;
-  msf[i] = 1u;
-  if (best[other] == i && (uint32_t)m < other) return;
-  hook[m] = other;
-  *changed = 1u;
-}
-
-__global__ void k_msf_apply(int64_t M, uint32_t *comp, uint32_t *best, uint32_t *hook) {
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M || comp[m] != (uint32_t)m) return;
-  if (hook[m] != kInvalid) comp[m] = hook[m];
-  hook[m] = kInvalid;
-  best[m] = kInvalid;
+                           const uint32_t *__restrict__ comp, const uint32_t *__restrict__ best, uint32_t *next,
+                           uint32_t *msf, MsfRound *round) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= M) return;
+  uint32_t to = comp[m];
+  if (to == (uint32_t)m) {
+    const uint32_t i = best[m];
+    if (i != kInvalid) {
+      const uint32_t cu = comp[eu[i]], cv = comp[ev[i]];
+      const uint32_t other = cu == (uint32_t)m ? cv : cu;
+      msf[i] = 1u;
+      if (best[other] != i || (uint32_t)m > other) {
+        to = other;
+        round->changed = 1u;
+      }
+    }
+  }
+  next[m] = to;
 }
 
 // Root of m in a forest of parent pointers (a root points to itself, or
@@ -1161,11 +1196,13 @@ __device__ inline uint32_t forest_root(uint32_t *parent, uint32_t m, bool nil_ro
   return x;
 }
 
-// Roots of the hook forest into the next round's component array.
-__global__ void k_msf_flatten(int64_t M, uint32_t *comp, uint32_t *next, uint32_t *err) {
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Part 3: roots of the hook forest into the component array; the least edges
+// start again.
+__global__ void k_msf_flatten(int64_t M, uint32_t *hooks, uint32_t *comp, uint32_t *best, MsfRound *round) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= M) return;
-  next[m] = forest_root(comp, (uint32_t)m, false, M, err);
+  comp[m] = forest_root(hooks, (uint32_t)m, false, M, &round->cyclic);
+  best[m] = kInvalid;
 }
 
 __global__ void k_msf_count(int64_t E, const uint32_t *__restrict__ msf, const uint32_t *__restrict__ es,
@@ -1646,7 +1683,7 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   if (!any_invalid) {
     const dim3 tb(256);
     const int all_owned = k == 1 ? 1 : 0;
-    const dim3 gm(blocks_for(minima_n, 256)), gs(blocks_for(S, 256)), ga(blocks_for(arms, 256));
+    const dim3 gm(blocks_for(minima_n, 256)), gs(blocks_for(S, 256));
     // attachment forest of the fresh minima and its representatives
     auto &attach = W.attach, &rep = W.rep, &dense = W.dense, &err = W.err;
     attach.ensure(minima_n);
@@ -1658,68 +1695,66 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
     hipLaunchKernelGGL(k_attach_roots, gm, tb, 0, s, minima_n, attach.p, rep.p, err.p);
     // star edges between the representatives of owned carriers, in arm (= level) order
     auto &eflag = W.eflag;
-    eflag.ensure(arms);
-    hipLaunchKernelGGL(k_edge_flags, ga, tb, 0, s, arm_saddle.p, base.p, sizes.p, carrier.p, first.p, rep.p,
-                       all_owned, (int64_t)arms, eflag.p);
-    W.scanner.inclusive(eflag.p, arms, s);
+    eflag.ensure(S);
+    hipLaunchKernelGGL(k_edge_counts, gs, tb, 0, s, (int64_t)S, base.p, sizes.p, carrier.p, first.p, rep.p, all_owned,
+                       eflag.p);
+    W.scanner.inclusive(eflag.p, S, s);
     uint32_t E = 0, bad = 0;
     MHGP_HIP(hipMemcpyAsync(&bad, err.p, 4, hipMemcpyDeviceToHost, s));
-    copy_wait(&E, eflag.p + arms - 1, 4, hipMemcpyDeviceToHost, s);
+    copy_wait(&E, eflag.p + S - 1, 4, hipMemcpyDeviceToHost, s);
     if (bad) throw std::runtime_error("tower attachment forest is cyclic");
     ph[5] = ph[6] = clk::now();
     // edges and two rounds' lists, in the pool that held the saddles' labels
     uint32_t *pool = W.slab.ensure(9 * (size_t)E);
     uint32_t *eu = pool, *ev = eu + E, *es = ev + E;
     uint32_t *Lu[2] = {es + E, es + 4 * (size_t)E}, *Lv[2] = {Lu[0] + E, Lu[1] + E}, *Li[2] = {Lv[0] + E, Lv[1] + E};
-    hipLaunchKernelGGL(k_edge_list, ga, tb, 0, s, arm_saddle.p, base.p, sizes.p, carrier.p, first.p, rep.p,
-                       all_owned, eflag.p, (int64_t)arms, eu, ev, es);
-    // Boruvka spanning forest of the minima over the star edges
-    auto &comp = W.comp, &comp2 = W.comp2, &best = W.best, &hook = W.hook, &msf = W.msf;
+    hipLaunchKernelGGL(k_edge_list, gs, tb, 0, s, (int64_t)S, base.p, sizes.p, carrier.p, first.p, rep.p, all_owned,
+                       eflag.p, eu, ev, es);
+    // Boruvka spanning forest of the minima over the star edges.  Edges are in
+    // level order, so of a long list a prefix is contracted first: most of the
+    // rest then lies within components and only passes the filter once,
+    // instead of through several rounds.  Two rounds share a wait; the second
+    // takes its list's length from the device.
+    auto &comp = W.comp, &hooks = W.comp2, &best = W.best, &msf = W.msf;
     auto &mcount = W.mcount;
-    auto &live_n = W.live_n;
-    live_n.ensure(2);
+    auto &rounds = W.rounds;
+    rounds.ensure(kMsfRounds * sizeof(MsfRound));
+    MsfRound *slot = reinterpret_cast<MsfRound *>(rounds.p);
     comp.ensure(minima_n);
-    comp2.ensure(minima_n);
+    hooks.ensure(minima_n);
     best.ensure(minima_n);
-    hook.ensure(minima_n);
     msf.ensure(E + 1);
     mcount.ensure(S);
     const dim3 ge(blocks_for(E + 1, 256));
-    hipLaunchKernelGGL(k_identity, gm, tb, 0, s, comp.p, minima_n);
-    hipLaunchKernelGGL(k_fill_u32, gm, tb, 0, s, best.p, minima_n, kInvalid);
-    hipLaunchKernelGGL(k_fill_u32, gm, tb, 0, s, hook.p, minima_n, kInvalid);
-    hipLaunchKernelGGL(k_fill_u32, ge, tb, 0, s, msf.p, (int64_t)E, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(S, 256)), tb, 0, s, mcount.p, (int64_t)S, 0u);
-    const uint32_t *lu = eu, *lv = ev, *li = nullptr;
-    uint32_t live = E;
+    hipLaunchKernelGGL(k_msf_init, dim3(blocks_for(std::max<int64_t>({minima_n, E, S, kMsfRounds}), 256)), tb, 0, s,
+                       minima_n, (int64_t)E, (int64_t)S, comp.p, best.p, msf.p, mcount.p, slot);
     msf_edges = E;
-    for (int round = 0; live > 0; ++round) {
-      if (round > 64) throw std::runtime_error("spanning forest of the tower did not converge");
-      msf_rounds = round + 1;
-      const int q = round & 1;
-      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, live_n.p, (int64_t)2, 0ull);
-      hipLaunchKernelGGL(k_msf_best, dim3(blocks_for(live, kMsfBlock)), dim3(kMsfBlock), 0, s, (int64_t)live, lu, lv, li, comp.p,
-                         best.p, Lu[q], Lv[q], Li[q], (unsigned long long *)live_n.p);
-      hipLaunchKernelGGL(k_msf_hook, gm, tb, 0, s, minima_n, eu, ev, comp.p, best.p, hook.p, msf.p,
-                         (uint32_t *)(live_n.p + 1));
-      hipLaunchKernelGGL(k_msf_apply, gm, tb, 0, s, minima_n, comp.p, best.p, hook.p);
-      hipLaunchKernelGGL(k_msf_flatten, gm, tb, 0, s, minima_n, comp.p, comp2.p, (uint32_t *)(live_n.p + 1) + 1);
-      std::swap(comp.p, comp2.p);
-      std::swap(comp.cap, comp2.cap);
-      // live edges; hooked anything, cyclic forest
-      struct {
-        uint64_t live;
-        uint32_t changed, cyclic;
-      } r;
-      static_assert(sizeof r == 16, "round result layout");
-      copy_wait(&r, live_n.p, sizeof r, hipMemcpyDeviceToHost, s);
-      if (r.cyclic) throw std::runtime_error("spanning forest of the tower: cyclic hook forest");
-      if (!r.changed) break;
-      live = (uint32_t)r.live;
-      lu = Lu[q];
-      lv = Lv[q];
-      li = Li[q];
+    const uint32_t prefix = E >= kMsfSplit ? E / 4 : E;
+    int used = 0;
+    for (uint32_t lo = 0, hi = prefix; lo < E; lo = hi, hi = E) {
+      const uint32_t *lu = eu + lo, *lv = ev + lo, *li = nullptr;
+      uint32_t live = hi - lo;
+      while (live > 0) {
+        if (used + 2 > kMsfRounds) throw std::runtime_error("spanning forest of the tower did not converge");
+        for (int q = 0; q < 2; ++q) {
+          MsfRound *r = slot + used + q;
+          hipLaunchKernelGGL(k_msf_best, dim3(blocks_for(live, kMsfBlock)), dim3(kMsfBlock), 0, s, (int64_t)live,
+                             q ? &r[-1].live : nullptr, lu, lv, li, lo, comp.p, best.p, Lu[q], Lv[q], Li[q], r);
+          hipLaunchKernelGGL(k_msf_hook, gm, tb, 0, s, minima_n, eu, ev, comp.p, best.p, hooks.p, msf.p, r);
+          hipLaunchKernelGGL(k_msf_flatten, gm, tb, 0, s, minima_n, hooks.p, comp.p, best.p, r);
+          lu = Lu[q];
+          lv = Lv[q];
+          li = Li[q];
+        }
+        MsfRound got[2];
+        copy_wait(got, slot + used, sizeof got, hipMemcpyDeviceToHost, s);
+        used += 2;
+        if (got[0].cyclic || got[1].cyclic) throw std::runtime_error("spanning forest of the tower: cyclic hook forest");
+        if (!got[0].changed || !got[1].changed) break;
+        live = (uint32_t)got[1].live;
+      }
     }
+    msf_rounds = used;
     ph[6] = clk::now();
     if (E) hipLaunchKernelGGL(k_msf_count, ge, tb, 0, s, (int64_t)E, msf.p, es, mcount.p);
     // keep births, multifusions and shared levels

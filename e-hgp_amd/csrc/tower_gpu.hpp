@@ -62,14 +62,14 @@ struct TowerWork {
   uint32_t rank_lo[256] = {}, rank_hi[256] = {};
   // the minima's hash table and labels, the saddles' labels (a pool whose
   // words then serve the spanning forest) and support members
-  DevBuf<uint64_t> slots, qkey, facet_slots, dcount, live_n;
+  DevBuf<uint64_t> slots, qkey, facet_slots, dcount;
   DevBuf<uint32_t> labels, slab;
   DevBuf<uint16_t> members;
   DevBuf<uint32_t> alias_arm, alias_rep, dF[3], dO[3];
   DevBuf<uint32_t> sizes, carrier, scls, base, arm_saddle, queue;
   DevBuf<double> slev, c_lev;
   DevBuf<uint32_t> first, keep, kept, flag1, c_cls, c_base, c_car;
-  DevBuf<uint32_t> eflag, comp, comp2, best, hook, msf, mcount, err;
+  DevBuf<uint32_t> eflag, comp, comp2, best, msf, mcount, err;
   DevBuf<uint32_t> attach, rep, dense, ssup;
   // vertical maps: per record (rank-index position) the contraction element
   // of its first arm's carrier as a saddle of the order below (first lane
@@ -81,20 +81,20 @@ struct TowerWork {
   // last listed one (first lane only)
   DevBuf<uint32_t> nn;
   DevBuf<double> nn_d2;
-  DevBuf<uint8_t> nn_flags;
+  DevBuf<uint8_t> nn_flags, rounds;
   bool nn_ready = false;
   int64_t bytes() const {
     int64_t b = 0;
     for (const DevBuf<uint32_t> *x :
          {&rank_vals, &rank_bounds, &labels, &slab,   &alias_arm, &alias_rep, &dF[0],     &dF[1],  &dF[2],  &dO[0],
           &dO[1],     &dO[2],       &sizes,  &carrier, &scls,      &base,      &arm_saddle, &queue,  &first,  &keep,
-          &kept,      &flag1,       &c_cls,  &c_base,  &c_car,     &eflag,     &comp,       &comp2,  &best,   &hook,
+          &kept,      &flag1,       &c_cls,  &c_base,  &c_car,     &eflag,     &comp,       &comp2,  &best,
           &msf,       &mcount,      &err,    &attach,  &rep,       &dense,     &ssup,       &vm_elem, &vm_idx, &vm_out,
           &raw_dense, &nn})
       b += (int64_t)x->bytes();
-    for (const DevBuf<uint64_t> *x : {&rank_keys, &slots, &qkey, &facet_slots, &dcount, &live_n})
+    for (const DevBuf<uint64_t> *x : {&rank_keys, &slots, &qkey, &facet_slots, &dcount})
       b += (int64_t)x->bytes();
-    return b + (int64_t)(members.bytes() + nn_flags.bytes() + nn_d2.bytes() + slev.bytes() + c_lev.bytes() +
+    return b + (int64_t)(members.bytes() + nn_flags.bytes() + rounds.bytes() + nn_d2.bytes() + slev.bytes() + c_lev.bytes() +
                          vm_long.bytes() + vm_int.bytes());
   }
 };
