@@ -140,32 +140,6 @@ void supports(Context &c, int k_max, mhgp_catalog_info *info) {
   B.valid = true;
 }
 
-void supports_fetch(Context &c, uint32_t *ids, uint32_t *meta, uint32_t *interior, double *level,
-                    int64_t *level_class) {
-  if (!c.catalog || !c.catalog->valid) throw StateError("no catalogue has been built");
-  CatalogBuffers &B = *c.catalog;
-  const int64_t n = B.count;
-  std::vector<EventRec> ev(n);
-  std::vector<uint32_t> order(n), cls(n);
-  if (n) {
-    copy_wait(ev.data(), B.events.p, n * sizeof(EventRec), hipMemcpyDeviceToHost, c.stream);
-    copy_wait(order.data(), B.order.p, n * 4, hipMemcpyDeviceToHost, c.stream);
-    copy_wait(cls.data(), B.cls.p, n * 4, hipMemcpyDeviceToHost, c.stream);
-  }
-  const int width = std::max(B.s_max - 1, 1);
-  for (int64_t i = 0; i < n; ++i) {
-    const EventRec &e = ev[order[i]];
-    if (ids)
-      for (int k = 0; k < 4; ++k) ids[4 * i + k] = e.ids[k];
-    if (meta) meta[i] = e.meta;
-    const int nint = (int)((e.meta >> 16) & 0xFFu);
-    if (interior)
-      for (int k = 0; k < width; ++k) interior[width * i + k] = k < nint ? e.interior[k] : kInvalid;
-    if (level) level[i] = std::ldexp(e.level, -2 * c.scale_exp);
-    if (level_class) level_class[i] = cls[i];
-  }
-}
-
 }  // namespace mhgp
 
 namespace mhgp {

@@ -315,4 +315,71 @@ void order_catalogue(Context &c, CatalogBuffers &B) {
   tm.mark("catalogue level classes");
 }
 
+// Records in canonical order as the fetch's arrays, staged one behind the
+// other: ids (4 words), level and level class (8 bytes each), meta, interior
+// (width words).  The host did this record by record at random in the
+// downloaded 72-byte records: the 2 003-point mixture's catalogue with its
+// fetch 62.5 ms, now 39.9 ms (the copies out bound it); of 256 points K 3, 4 790
+// records, 1 215 and 1 160 us.
+__global__ void k_export(const EventRec *__restrict__ ev, const uint32_t *__restrict__ order,
+                         const uint32_t *__restrict__ cls, int64_t first, int64_t n, int width, int level_exp,
+                         uint4 *ids, double *level, int64_t *level_class, uint32_t *meta, uint32_t *interior) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const EventRec &e = ev[order[first + i]];
+  const uint32_t m = e.meta;
+  ids[i] = make_uint4(e.ids[0], e.ids[1], e.ids[2], e.ids[3]);
+  level[i] = ldexp(e.level, level_exp);
+  level_class[i] = (int64_t)cls[first + i];
+  meta[i] = m;
+  const int nint = (int)((m >> 16) & 0xFFu);
+  for (int k = 0; k < width; ++k) interior[(int64_t)width * i + k] = k < nint ? e.interior[k] : kInvalid;
+}
+
+// The staging takes the enumeration's slab memory, in pieces of what that
+// holds.  A piece of up to kExportPinned bytes goes through page-locked memory
+// in one copy (five copies into pageable memory cost more than the piece).
+constexpr size_t kExportPinned = 1u << 20;
+void supports_fetch(Context &c, uint32_t *ids, uint32_t *meta, uint32_t *interior, double *level,
+                    int64_t *level_class) {
+  if (!c.catalog || !c.catalog->valid) throw StateError("no catalogue has been built");
+  CatalogBuffers &B = *c.catalog;
+  const int64_t n = B.count;
+  if (!n) return;
+  hipStream_t s = c.stream;
+  const int width = std::max(B.s_max - 1, 1);
+  const size_t rec = 16 + 8 + 8 + 4 + 4 * (size_t)width;
+  const int64_t most = std::max<int64_t>(1, (int64_t)(B.scratch.bytes() / rec));
+  B.scratch.ensure(rec);
+  for (int64_t first = 0; first < n; first += most) {
+    const int64_t m = std::min(most, n - first);
+    char *d = reinterpret_cast<char *>(B.scratch.p);
+    const size_t o_level = (size_t)m * 16, o_cls = o_level + (size_t)m * 8, o_meta = o_cls + (size_t)m * 8,
+                 o_int = o_meta + (size_t)m * 4, bytes = o_int + (size_t)m * 4 * width;
+    hipLaunchKernelGGL(k_export, dim3(blocks_for(m, 256)), dim3(256), 0, s, B.events.p, B.order.p, B.cls.p, first, m,
+                       width, -2 * c.scale_exp, reinterpret_cast<uint4 *>(d), reinterpret_cast<double *>(d + o_level),
+                       reinterpret_cast<int64_t *>(d + o_cls), reinterpret_cast<uint32_t *>(d + o_meta),
+                       reinterpret_cast<uint32_t *>(d + o_int));
+    MHGP_LAUNCH_CHECK();
+    const struct {
+      void *to;
+      size_t from, bytes;
+    } parts[5] = {{ids ? ids + 4 * first : nullptr, 0, (size_t)m * 16},
+                  {level ? level + first : nullptr, o_level, (size_t)m * 8},
+                  {level_class ? level_class + first : nullptr, o_cls, (size_t)m * 8},
+                  {meta ? meta + first : nullptr, o_meta, (size_t)m * 4},
+                  {interior ? interior + (int64_t)width * first : nullptr, o_int, (size_t)m * 4 * width}};
+    if (bytes <= kExportPinned) {
+      char *h = (char *)B.pinned.ensure(kExportPinned);
+      copy_wait(h, d, bytes, hipMemcpyDeviceToHost, s);
+      for (const auto &p : parts)
+        if (p.to) std::memcpy(p.to, h + p.from, p.bytes);
+    } else {
+      for (const auto &p : parts)
+        if (p.to) MHGP_HIP(hipMemcpyAsync(p.to, d + p.from, p.bytes, hipMemcpyDeviceToHost, s));
+      MHGP_HIP(hipStreamSynchronize(s));
+    }
+  }
+}
+
 }  // namespace mhgp

@@ -72,6 +72,7 @@ struct CatalogBuffers {
   DevBuf<uint64_t> total;         // gathered entries of a pass
   DevBuf<uint64_t> run_count;     // open runs, runs left to the host
   DevBuf<uint32_t> run_pos, run_gidx, run_new, run_link;
+  PinnedBuf pinned;               // small results on their way to the caller
   DevBuf<EventRec> run_rec;       // records of the runs ordered on the host
   int64_t open_runs = 0;          // runs the FP64 intervals left open
   int64_t host_runs = 0;          // of those, runs ordered exactly on the host

@@ -219,6 +219,29 @@ def test_context_capacity_refuses_and_recovers():
     assert np.array_equal(cat.ids, ref.ids) and np.array_equal(cat.level_class, ref.level_class)
 
 
+@pytest.mark.parametrize("n,k,capacity", [(40, 2, 0), (600, 4, 32 << 20), (600, 8, 48 << 20)])
+def test_fetch_in_one_piece_and_in_several(n, k, capacity):
+    """The fetch's arrays are staged in the enumeration's slab memory: one
+    small piece through page-locked memory, or pieces of what a context with a
+    device capacity left for slabs.  Same arrays as the flat records of an
+    unbounded context, which the oracle tests pin."""
+    pts = workloads.uniform_cloud(n, seed=41)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        ref = ctx.supports_raw(k)
+        cat = ctx.supports(k)
+    with mhgp.Context(0, capacity_bytes=capacity) as ctx:
+        ctx.upload(pts)
+        got = ctx.supports_raw(k)
+        print(f"fetch n={n} k={k}: {len(got['meta'])} records, {ctx.device_bytes()} bytes", flush=True)
+    for key in ("ids", "meta", "interior", "level", "level_class"):
+        assert np.array_equal(got[key], ref[key]), key
+    nint = (ref["meta"] >> 16) & 0xFF
+    for i in range(0, len(nint), max(1, len(nint) // 500)):
+        row = ref["interior"][i]
+        assert tuple(row[: nint[i]]) == cat.interior[i] and np.all(row[nint[i]:] == 0xFFFFFFFF)
+
+
 def test_reused_context_one_point_cloud_has_an_empty_catalogue():
     """A context that held a cloud and then takes a one-point cloud returns an
     empty catalogue (no records left over from the earlier cloud)."""
