@@ -39,6 +39,40 @@ struct FallbackRec {
   uint32_t pad;
 };
 
+// Streams beside a context's own, for launches between a fork and a join.
+struct SideStreams {
+  static constexpr int kCount = 2;
+  hipStream_t stream[kCount] = {};
+  hipEvent_t forked = nullptr, done[kCount] = {};
+  SideStreams() = default;
+  SideStreams(const SideStreams &) = delete;
+  SideStreams &operator=(const SideStreams &) = delete;
+  ~SideStreams() {
+    for (int i = 0; i < kCount; ++i) {
+      if (stream[i]) (void)hipStreamDestroy(stream[i]);
+      if (done[i]) (void)hipEventDestroy(done[i]);
+    }
+    if (forked) (void)hipEventDestroy(forked);
+  }
+  // the first `count` streams go on from what s holds now
+  void fork(hipStream_t s, int count) {
+    if (!forked) MHGP_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
+    MHGP_HIP(hipEventRecord(forked, s));
+    for (int i = 0; i < count; ++i) {
+      if (!stream[i]) MHGP_HIP(hipStreamCreateWithFlags(&stream[i], hipStreamNonBlocking));
+      if (!done[i]) MHGP_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
+      MHGP_HIP(hipStreamWaitEvent(stream[i], forked, 0));
+    }
+  }
+  // s waits for them
+  void join(hipStream_t s, int count) {
+    for (int i = 0; i < count; ++i) {
+      MHGP_HIP(hipEventRecord(done[i], stream[i]));
+      MHGP_HIP(hipStreamWaitEvent(s, done[i], 0));
+    }
+  }
+};
+
 struct CatalogBuffers {
   bool valid = false;
   int k_max = 0;
@@ -77,6 +111,7 @@ struct CatalogBuffers {
   int64_t open_runs = 0;          // runs the FP64 intervals left open
   int64_t host_runs = 0;          // of those, runs ordered exactly on the host
   mhgp_catalog_info info{};
+  SideStreams sides;              // declared last: gone before the buffers they use
 };
 
 int64_t catalog_device_bytes(const CatalogBuffers &b);

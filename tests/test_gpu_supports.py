@@ -129,8 +129,8 @@ def test_catalog_big_paths_small(path, monkeypatch):
     _compare(workloads.uniform_cloud(40, seed=34), 4, f"uniform40-k4-{path}")
 
 
-@pytest.mark.parametrize("path", ["", "region", "slabs"])
-@pytest.mark.parametrize("sigma,n,k", [(1e-4, 64, 10), (1e-6, 110, 10), (1e-6, 100, 4)])
+@pytest.mark.parametrize("path,sigma,n,k", [("", 1e-4, 64, 10), ("region", 1e-4, 64, 10), ("slabs", 1e-4, 64, 10),
+                                            ("", 1e-6, 110, 10), ("", 1e-6, 100, 4)])
 def test_catalog_nearly_cospherical(path, sigma, n, k, monkeypatch):
     """Lattices displaced by less than FP32 key bounds can tell apart: most
     sides of faces hold more near-equal sweep keys than a face's list, so
