@@ -437,34 +437,70 @@ __global__ void __launch_bounds__(256) k_refit(int64_t n, Node *nodes, uint32_t 
   }
 }
 
-// Postorder index and depth of every node (internal i < n-1, leaf n-1+p).
+// Canonical points in the input unit (an exact power of two), interleaved.
+__global__ void k_points_out(int64_t n, const double *__restrict__ X, const double *__restrict__ Y,
+                             const double *__restrict__ Z, int exponent, double *out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  out[3 * i] = ldexp(X[i], exponent);
+  out[3 * i + 1] = ldexp(Y[i], exponent);
+  out[3 * i + 2] = ldexp(Z[i], exponent);
+}
+
+// Snapshot leaves (code, PointId) and, of the runs of equal codes, their
+// number (totals[1]) and the longest (totals[2]).  Codes ascend: a run's end
+// is found by doubling steps and halving.
+__global__ void k_leaves_out(int64_t n, const uint64_t *__restrict__ codes, const uint32_t *__restrict__ leaf_id,
+                             ulonglong2 *leaves, unsigned long long *totals) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const uint64_t c = codes[p];
+  leaves[p] = make_ulonglong2(c, leaf_id[p]);
+  if (p + 1 >= n || codes[p + 1] != c || (p > 0 && codes[p - 1] == c)) return;
+  int64_t last = p + 1, step = 2;  // the last known position of the run
+  while (last + step < n && codes[last + step] == c) {
+    last += step;
+    step *= 2;
+  }
+  for (; step > 0; step /= 2)
+    if (last + step < n && codes[last + step] == c) last += step;
+  atomicAdd(&totals[1], 1ull);
+  atomicMax(&totals[2], (unsigned long long)(last - p + 1));
+}
+
+// Postorder index of every node (internal i < n-1, leaf n-1+p), and the
+// largest depth (totals[0]).
 __global__ void k_postorder(int64_t n, const Node *__restrict__ nodes,
                             const uint32_t *__restrict__ parent_int,
                             const uint32_t *__restrict__ parent_leaf, uint64_t *post,
-                            uint32_t *depth) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 2 * n - 1) return;
-  if (n == 1) { post[0] = 0; depth[0] = 0; return; }
-  bool leaf = t >= n - 1;
-  uint32_t cur = leaf ? (uint32_t)(t - (n - 1)) | kLeafBit : (uint32_t)t;
-  uint32_t par = leaf ? parent_leaf[t - (n - 1)] : parent_int[t];
-  uint64_t w = 0;
+                            unsigned long long *totals) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t dep = 0;
-  while (par != kInvalid) {
-    const Node &P = nodes[par];
-    if (P.right == cur) {
-      w += 1;
-    } else {
-      uint32_t r = P.right;
-      uint64_t leaves_r = (r & kLeafBit) ? 1 : (uint64_t)(nodes[r].end - nodes[r].begin);
-      w += 2 * leaves_r;
+  if (t < 2 * n - 1) {
+    const bool leaf = t >= n - 1;
+    uint32_t cur = leaf ? (uint32_t)(t - (n - 1)) | kLeafBit : (uint32_t)t;
+    uint32_t par = n == 1 ? kInvalid : leaf ? parent_leaf[t - (n - 1)] : parent_int[t];
+    uint64_t w = 0;
+    while (par != kInvalid) {
+      const Node &P = nodes[par];
+      if (P.right == cur) {
+        w += 1;
+      } else {
+        uint32_t r = P.right;
+        uint64_t leaves_r = (r & kLeafBit) ? 1 : (uint64_t)(nodes[r].end - nodes[r].begin);
+        w += 2 * leaves_r;
+      }
+      dep++;
+      cur = par;
+      par = parent_int[par];
     }
-    dep++;
-    cur = par;
-    par = parent_int[par];
+    post[t] = (uint64_t)(2 * n - 2) - w;
   }
-  post[t] = (uint64_t)(2 * n - 2) - w;
-  depth[t] = dep;
+  // one atomic per wave, and only of a depth not known yet
+  uint32_t most = dep;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d));
+  if (threadIdx.x % 64 == 0 && most > totals[0]) atomicMax(&totals[0], (unsigned long long)most);
 }
 
 __global__ void k_snapshot(int64_t n, const Node *__restrict__ nodes, const uint32_t *__restrict__ wit,
@@ -732,41 +768,46 @@ WaveTree wave_tree(const Context &c) {
           {c.centre[0], c.centre[1], c.centre[2]}, c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p};
 }
 
-void export_snapshot(Context &c, uint64_t *leaves, uint64_t *nodes_out, uint64_t *counters) {
+void canonical_points(Context &c, double *xyz_out, uint32_t *source_index_out) {
   const int64_t n = c.n;
   hipStream_t s = c.stream;
-  const int T = 256;
-  DevBuf<uint64_t> post, out;
-  DevBuf<uint32_t> depth;
-  post.ensure(2 * n - 1);
-  depth.ensure(2 * n - 1);
-  out.ensure(10 * (2 * n - 1));
-  hipLaunchKernelGGL(k_postorder, dim3(blocks_for(2 * n - 1, T)), dim3(T), 0, s, n, c.nodes.p,
-                     c.parent_int.p, c.parent_leaf.p, post.p, depth.p);
-  hipLaunchKernelGGL(k_snapshot, dim3(blocks_for(2 * n - 1, T)), dim3(T), 0, s, n, c.nodes.p,
-                     c.wit.p, c.leaf_id.p, post.p, out.p);
-  MHGP_LAUNCH_CHECK();
-  std::vector<uint64_t> codes(n);
-  std::vector<uint32_t> ids(n), dep(2 * n - 1);
-  MHGP_HIP(hipMemcpyAsync(codes.data(), c.codes.p, n * 8, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipMemcpyAsync(ids.data(), c.leaf_id.p, n * 4, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipMemcpyAsync(dep.data(), depth.p, (2 * n - 1) * 4, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipMemcpyAsync(nodes_out, out.p, 10 * (2 * n - 1) * 8, hipMemcpyDeviceToHost, s));
-  MHGP_HIP(hipStreamSynchronize(s));
-  uint64_t groups = 0, maxg = 0, maxd = 0;
-  for (int64_t p = 0; p < n; ++p) { leaves[2 * p] = codes[p]; leaves[2 * p + 1] = ids[p]; }
-  for (int64_t b = 0; b < n;) {
-    int64_t e = b + 1;
-    while (e < n && codes[e] == codes[b]) e++;
-    if (e - b > 1) { groups++; maxg = std::max<uint64_t>(maxg, e - b); }
-    b = e;
+  if (source_index_out)
+    MHGP_HIP(hipMemcpyAsync(source_index_out, c.source_index.p, n * 4, hipMemcpyDeviceToHost, s));
+  if (xyz_out && n) {
+    // the uploaded points' buffer is free once the index stands
+    c.src.ensure(3 * n);
+    hipLaunchKernelGGL(k_points_out, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, c.X.p, c.Y.p, c.Z.p, -c.scale_exp, c.src.p);
+    MHGP_LAUNCH_CHECK();
+    MHGP_HIP(hipMemcpyAsync(xyz_out, c.src.p, n * 24, hipMemcpyDeviceToHost, s));
   }
-  for (auto d : dep) maxd = std::max<uint64_t>(maxd, d);
+  MHGP_HIP(hipStreamSynchronize(s));
+}
+
+void export_snapshot(Context &c, uint64_t *leaves, uint64_t *nodes_out, uint64_t *counters) {
+  const int64_t n = c.n, m = 2 * n - 1;
+  hipStream_t s = c.stream;
+  const int T = 256;
+  // leaves, nodes, postorder, totals; kept by the context unless its device
+  // memory is bounded
+  DevBuf<uint64_t> own;
+  DevBuf<uint64_t> &buf = c.capacity_bytes > 0 ? own : c.snapshot;
+  buf.ensure(2 * n + 10 * m + m + 4);
+  uint64_t *d_leaves = buf.p, *d_nodes = d_leaves + 2 * n, *post = d_nodes + 10 * m, *totals = post + m;
+  MHGP_HIP(hipMemsetAsync(totals, 0, 24, s));
+  hipLaunchKernelGGL(k_postorder, dim3(blocks_for(m, T)), dim3(T), 0, s, n, c.nodes.p, c.parent_int.p,
+                     c.parent_leaf.p, post, (unsigned long long *)totals);
+  hipLaunchKernelGGL(k_snapshot, dim3(blocks_for(m, T)), dim3(T), 0, s, n, c.nodes.p, c.wit.p, c.leaf_id.p, post,
+                     d_nodes);
+  hipLaunchKernelGGL(k_leaves_out, dim3(blocks_for(n, T)), dim3(T), 0, s, n, c.codes.p, c.leaf_id.p,
+                     reinterpret_cast<ulonglong2 *>(d_leaves), (unsigned long long *)totals);
+  MHGP_LAUNCH_CHECK();
+  uint64_t got[3];
+  MHGP_HIP(hipMemcpyAsync(leaves, d_leaves, n * 16, hipMemcpyDeviceToHost, s));
+  MHGP_HIP(hipMemcpyAsync(nodes_out, d_nodes, 10 * m * 8, hipMemcpyDeviceToHost, s));
+  copy_wait(got, totals, 24, hipMemcpyDeviceToHost, s);
   counters[0] = n;
-  counters[1] = 2 * n - 1;
-  counters[2] = maxd;
-  counters[3] = groups;
-  counters[4] = maxg;
+  counters[1] = m;
+  for (int i = 0; i < 3; ++i) counters[2 + i] = got[i];
 }
 
 }  // namespace mhgp

@@ -30,7 +30,7 @@ int64_t device_bytes(const Context &c) {
   int64_t b = c.src.bytes() + c.X.bytes() * 3 + c.source_index.bytes() + c.key0.bytes() + c.key1.bytes() + c.key2.bytes() +
               c.perm.bytes() + c.codes.bytes() + c.leaf_id.bytes() + c.leaf_pos.bytes() +
               c.LX.bytes() * 3 + c.path.bytes() + c.nodes.bytes() + c.parent_int.bytes() +
-              c.parent_leaf.bytes() + c.wit.bytes() + c.wide.bytes() + c.groups.bytes() + c.group_exact.bytes();
+              c.parent_leaf.bytes() + c.wit.bytes() + c.wide.bytes() + c.groups.bytes() + c.group_exact.bytes() + c.snapshot.bytes();
   if (c.catalog) b += catalog_device_bytes(*c.catalog);
   if (c.emst) b += c.emst->bytes();
   if (c.tower_work) b += c.tower_work->bytes();
@@ -47,7 +47,7 @@ void release_device_state(Context &c) {
   c.emst.reset();
   c.catalog.reset();
   for (DevBuf<double> *b : {&c.src, &c.X, &c.Y, &c.Z, &c.bounds, &c.LX, &c.LY, &c.LZ}) b->release();
-  for (DevBuf<uint64_t> *b : {&c.key0, &c.key1, &c.key2, &c.codes, &c.path}) b->release();
+  for (DevBuf<uint64_t> *b : {&c.key0, &c.key1, &c.key2, &c.codes, &c.path, &c.snapshot}) b->release();
   for (DevBuf<uint32_t> *b : {&c.source_index, &c.perm, &c.status, &c.leaf_id, &c.leaf_pos,
                               &c.parent_int, &c.parent_leaf, &c.wit})
     b->release();
@@ -95,25 +95,6 @@ void upload_device(Context &c, const double *d_xyz, int64_t n) {
 
 void require_cloud(const Context &c) {
   if (!c.lbvh_ready || c.n <= 0) throw StateError("no cloud has been uploaded");
-}
-
-void canonical_points(Context &c, double *xyz_out, uint32_t *source_index_out) {
-  const int64_t n = c.n;
-  std::vector<double> x(n), y(n), z(n);
-  MHGP_HIP(hipMemcpyAsync(x.data(), c.X.p, n * 8, hipMemcpyDeviceToHost, c.stream));
-  MHGP_HIP(hipMemcpyAsync(y.data(), c.Y.p, n * 8, hipMemcpyDeviceToHost, c.stream));
-  MHGP_HIP(hipMemcpyAsync(z.data(), c.Z.p, n * 8, hipMemcpyDeviceToHost, c.stream));
-  if (source_index_out)
-    MHGP_HIP(hipMemcpyAsync(source_index_out, c.source_index.p, n * 4, hipMemcpyDeviceToHost, c.stream));
-  MHGP_HIP(hipStreamSynchronize(c.stream));
-  // back to the input unit (an exact power of two)
-  const int e = -c.scale_exp;
-  if (xyz_out)
-    for (int64_t i = 0; i < n; ++i) {
-      xyz_out[3 * i] = std::ldexp(x[i], e);
-      xyz_out[3 * i + 1] = std::ldexp(y[i], e);
-      xyz_out[3 * i + 2] = std::ldexp(z[i], e);
-    }
 }
 
 static HostMirror &mirror(Context &c) {

@@ -133,3 +133,32 @@ def test_build_at_its_edges(name, pts):
     assert np.array_equal(leaves, ref.leaves)
     assert np.array_equal(nodes, ref.nodes)
     assert np.array_equal(counters, ref.counters)
+
+
+@pytest.mark.parametrize("runs", [[], [2], [3, 2], [5, 700, 2, 64], [4097]])
+def test_snapshot_totals_of_equal_codes(runs):
+    """The snapshot's collision totals (runs of equal codes, the longest) and
+    canonical points against the fetched arrays: runs of many lengths, each a
+    cluster within one Morton cell, beside points that share no cell."""
+    rng = workloads.SplitMix64(77 + len(runs)).numpy_rng()
+    parts = [rng.uniform(0.0, 1.0, size=(300, 3))]
+    for r in runs:
+        parts.append(rng.uniform(0.1, 0.9, size=(1, 3)) + rng.uniform(0.0, 1e-12, size=(r, 3)))
+    pts = np.concatenate(parts)
+    print(f"snapshot totals: runs {runs}", flush=True)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        leaves, nodes, counters = ctx.lbvh_snapshot()
+        xyz, source = ctx.canonical_points()
+    _, lengths = np.unique(leaves[:, 0], return_counts=True)
+    long = lengths[lengths > 1]
+    assert list(counters[:2]) == [len(xyz), 2 * len(xyz) - 1]
+    assert counters[3] == len(long) and counters[4] == (long.max() if len(long) else 0)
+    assert np.array_equal(xyz, pts[source])
+    # depth from the postorder nodes' children
+    depth = np.zeros(len(nodes), dtype=np.int64)
+    for i in range(len(nodes) - 1, -1, -1):
+        for child in nodes[i, 6:8]:
+            if child != 0xFFFFFFFFFFFFFFFF:
+                depth[int(child)] = depth[i] + 1
+    assert counters[2] == depth.max()
