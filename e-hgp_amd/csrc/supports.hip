@@ -1340,9 +1340,9 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
   uint32_t covers = 0;  // point-cell tests (FP32 count)
   for (int c = t; c < kCells; c += blockDim.x) {
     const CellF cf = cell_f(P.cellf + 8 * c);
-    float best[kCoverCap];
+    float best[kCoverCap];  // the last need_cover of them; the others stay below
 #pragma unroll
-    for (int j = 0; j < kCoverCap; ++j) best[j] = INFINITY;
+    for (int j = 0; j < kCoverCap; ++j) best[j] = j < kCoverCap - need_cover ? -INFINITY : INFINITY;
     for (uint32_t i = 0; i < G; ++i) {
       const float4 q = w.fc[i];
       if (!(q.w > kTinyLen)) continue;  // skipping a point only enlarges the radius
@@ -1356,13 +1356,10 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
       const float r = q.w * __builtin_amdgcn_rcpf(2.0f * cs);
       if (!(r < best[kCoverCap - 1])) continue;
 #pragma unroll
-      for (int j = kCoverCap - 1; j > 0; --j) best[j] = r < best[j - 1] ? best[j - 1] : (r < best[j] ? r : best[j]);
+      for (int j = kCoverCap - 1; j > 0; --j) best[j] = __builtin_amdgcn_fmed3f(best[j - 1], r, best[j]);
       best[0] = fminf(best[0], r);
     }
-    float bk = INFINITY;
-#pragma unroll
-    for (int j = 0; j < kCoverCap; ++j) bk = j == need_cover - 1 ? best[j] : bk;
-    w.rho[c] = cell_radius(P, c, bk, ux, uy, uz);
+    w.rho[c] = cell_radius(P, c, best[kCoverCap - 1], ux, uy, uz);
   }
   add_flops32(w, (uint64_t)covers * kF32Cover);
   __syncthreads();
@@ -1489,7 +1486,11 @@ __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t 
 // share a CU than when one kernel did both, and the enumeration is split over
 // as many workgroups as its size asks for.  VALU bound.  Against one kernel per
 // anchor (two LDS sizes): catalogue of a 2 003-point mixture 332 -> 116 ms,
-// pipeline of 17 117 points K 4 19.3 -> 17.0 ms.
+// pipeline of 17 117 points K 4 19.3 -> 17.0 ms.  A scan that ends with the
+// certificate's own radius (the (s_max - 1)-th) instead of the tenth: K 4 12.65
+// -> 10.6 ms for 50 000 points' enumeration; four points at a time without
+// branches: 10.65 -> 9.1 ms, K 10 38.3 -> 35.2 ms, catalogue of 256 points K 3
+// 1.10 -> 1.03 ms.
 constexpr int kProbeBlock = kCells;
 template <int GCAP>
 __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
@@ -1550,6 +1551,7 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
       fc[rank[r]] = mine[r];
       gid[rank[r]] = id[r];
     }
+  if (t < 4 && G + t < G4) fc[G + t] = make_float4(0.f, 0.f, 0.f, INFINITY);
   __syncthreads();
   // 1. direction-cell certificate (FP32; every rounding errs towards larger
   // radii): a point at distance l covers at radius >= l / 2 (up to the FP32
@@ -1560,31 +1562,37 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
   const CellF cf = cell_f(P.cellf + 8 * c);
   float rho;
   {
+    // the last s_max - 1 entries are the least radii, the others stay below:
+    // the scan ends with the certificate's own radius
     float best[kCoverCap];
 #pragma unroll
-    for (int j = 0; j < kCoverCap; ++j) best[j] = INFINITY;
+    for (int j = 0; j < kCoverCap; ++j) best[j] = j < kCoverCap - (P.s_max - 1) ? -INFINITY : INFINITY;
     uint32_t covers = 0;
-    for (uint32_t i = 0; i < G; ++i) {
-      const float4 q = fc[i];
-      if (!(q.w > kTinyLen)) continue;  // skipping a point only enlarges the radius
-      if (q.w * 0.49999f > best[kCoverCap - 1]) break;
-      covers++;
-      const float ct = (q.x * cf.dx + q.y * cf.dy + q.z * cf.dz) * __builtin_amdgcn_rcpf(q.w);
-      if (ct <= 0.0f) continue;
-      const float st = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - ct * ct));
-      const float cs = ct * cf.cosd - st * cf.sind;  // cos(theta + delta)
-      if (cs < 0.01f) continue;  // ill-conditioned cover: skipped
-      const float r = q.w * __builtin_amdgcn_rcpf(2.0f * cs);
-      if (!(r < best[kCoverCap - 1])) continue;
+    // four points at a time, for the latency of a launch of few anchors
+    for (uint32_t i = 0; i < G; i += 4) {
+      if (fc[i].w * 0.49999f > best[kCoverCap - 1]) break;
+      covers += 4;
+      float r[4];
 #pragma unroll
-      for (int j = kCoverCap - 1; j > 0; --j) best[j] = __builtin_amdgcn_fmed3f(best[j - 1], r, best[j]);
-      best[0] = fminf(best[0], r);
+      for (int k = 0; k < 4; ++k) {
+        const float4 q = fc[i + k];
+        const float ct = (q.x * cf.dx + q.y * cf.dy + q.z * cf.dz) * __builtin_amdgcn_rcpf(q.w);
+        const float st = __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - ct * ct));
+        const float cs = ct * cf.cosd - st * cf.sind;  // cos(theta + delta)
+        // skipping a point (lost to underflow, ill-conditioned) only enlarges the radius
+        const bool covering = q.w > kTinyLen && ct > 0.0f && cs >= 0.01f;
+        r[k] = covering ? q.w * __builtin_amdgcn_rcpf(2.0f * cs) : INFINITY;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (!(r[k] < best[kCoverCap - 1])) continue;
+#pragma unroll
+        for (int j = kCoverCap - 1; j > 0; --j) best[j] = __builtin_amdgcn_fmed3f(best[j - 1], r[k], best[j]);
+        best[0] = fminf(best[0], r[k]);
+      }
     }
     if (P.count_flops) atomicAdd(&flops32, (unsigned long long)covers * kF32Cover);
-    float bk = INFINITY;
-#pragma unroll
-    for (int j = 0; j < kCoverCap; ++j) bk = j == P.s_max - 2 ? best[j] : bk;
-    rho = cell_radius(P, c, bk, ux, uy, uz);
+    rho = cell_radius(P, c, best[kCoverCap - 1], ux, uy, uz);
   }
   float m = rho;
 #pragma unroll
@@ -1604,26 +1612,27 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
   // only be included too often
   {
     uint32_t tests = 0;
+    const float reach = 2.0f * rho * (1.0f + 1e-5f);
     bool open = true;  // points up to the word's limit
     for (uint32_t i0 = 0; i0 < G; i0 += 64) {
       uint64_t word = 0;
       const uint32_t n = min(64u, G - i0);
-      for (uint32_t j = 0; open && j < n; ++j) {
-        const float4 q = fc[i0 + j];
-        bool in = true;  // distance lost to underflow: member everywhere
-        if (q.w > kTinyLen) {
-          if (q.w > wlim) {
-            open = false;
-            break;
-          }
-          tests++;
+      for (uint32_t j = 0; open && j < n; j += 4) {
+        if (fc[i0 + j].w > wlim) {
+          open = false;
+          break;
+        }
+        tests += 4;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+          const float4 q = fc[i0 + j + k];
           const float ct = (q.x * cf.dx + q.y * cf.dy + q.z * cf.dz) * __builtin_amdgcn_rcpf(q.w);
           const float cm = ct >= cf.cosd ? 1.0f  // cos(max(theta - delta, 0))
                                          : ct * cf.cosd + __builtin_amdgcn_sqrtf(fmaxf(0.0f, 1.0f - ct * ct)) * cf.sind;
-          in = q.w <= 2.0f * rho * (cm + 1e-5f) * (1.0f + 1e-5f);
+          // distance lost to underflow: member everywhere
+          const uint64_t b = __ballot(q.w <= reach * (cm + 1e-5f) || !(q.w > kTinyLen));
+          word = (uint32_t)lane == j + k ? b : word;
         }
-        const uint64_t b = __ballot(in);
-        word = (uint32_t)lane == j ? b : word;
       }
       if (i0 + lane < G) rmask[6 * (i0 + lane) + wave] = word;
     }
