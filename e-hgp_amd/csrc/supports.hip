@@ -69,16 +69,17 @@ __device__ inline void wave_sync() {
 }
 
 // Lists the probes append to (B.lists, kLists rows of n entries; their lengths
-// are counters[kListCount ..]).  The first three hold PointIds for a later
-// pass: gathers to widen, gathers beyond the small probe, gathers beyond LDS.
+// are counters[kListCount ..]).  The first four hold PointIds for a later
+// pass: gathers to widen, gathers beyond the small probe, those beyond the next
+// one, gathers (and regions) beyond LDS.
 // The others hold the probed anchors of one launch (their index in it, which
 // is also their slab's) by the size of their region.
-enum { L_WIDEN = 0, L_WIDE = 1, L_BIG = 2, L_TINY = 3, L_LITTLE = 4, L_SMALL = 5, L_MID = 6, L_LARGE = 7, L_SLAB = 8,
-       kLists = 9 };
+enum { L_WIDEN = 0, L_WIDE = 1, L_WIDER = 2, L_BIG = 3, L_TINY = 4, L_LITTLE = 5, L_SMALL = 6, L_MID = 7, L_LARGE = 8, L_SLAB = 9,
+       kLists = 10 };
 constexpr int kListCount = 8;    // counters: list lengths
-constexpr int kOpenCount = 17;   // counters: open anchors, their largest region
-constexpr int kOpenLargest = 18;
-constexpr int kRescanMost = 19;  // longest rescan list of a launch
+constexpr int kOpenCount = 18;   // counters: open anchors, their largest region
+constexpr int kOpenLargest = 19;
+constexpr int kRescanMost = 20;  // longest rescan list of a launch
 constexpr int kCounters = 24;
 
 // Regions of the global-memory path are enumerated face by face in
@@ -1491,14 +1492,20 @@ __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t 
 // -> 10.6 ms for 50 000 points' enumeration; four points at a time without
 // branches: 10.65 -> 9.1 ms, K 10 38.3 -> 35.2 ms, catalogue of 256 points K 3
 // 1.10 -> 1.03 ms.
+//
+// SLAB: the masks are built in the slab instead of LDS (98 KB for 2 048 points;
+// 48 KB then remain, three workgroups a CU).  Such gathers took the
+// global-memory kernel, whose 256 lanes scan all points for 384 cells and whose
+// regions are not in increasing distance: 2 003-point mixture, 1 531 such
+// anchors, catalogue 29.8 -> 26.0 ms.
 constexpr int kProbeBlock = kCells;
-template <int GCAP>
+template <int GCAP, bool SLAB>
 __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
   constexpr int kPer = (GCAP + kProbeBlock - 1) / kProbeBlock;
   constexpr int kWaves = kProbeBlock / 64;
   __shared__ __align__(16) float4 fc[GCAP];   // FP32 offset and distance (rounded up), ascending
   __shared__ uint32_t gid[GCAP];
-  __shared__ __align__(16) uint64_t rmask[6 * GCAP];
+  __shared__ __align__(16) uint64_t lmask[SLAB ? GCAP / 2 : 6 * GCAP];
   __shared__ float wmax[kWaves];
   __shared__ uint32_t wcount[kPer][kWaves];
   __shared__ unsigned long long flops32;
@@ -1508,15 +1515,21 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
   const uint32_t u = P.anchors[a];
   const uint32_t G = P.gcount[u];
   if (G > (uint32_t)GCAP) {
-    if (t == 0) list_add(P, GCAP < kGatherCapWide && G <= (uint32_t)kGatherCapWide ? L_WIDE : L_BIG, u);
+    if (t == 0) list_add(P, G <= (uint32_t)kGatherCapWide ? L_WIDE : G <= (uint32_t)kGatherCapSlab ? L_WIDER : L_BIG, u);
     return;
   }
   if (t == 0) flops32 = 0;
+  double *slab = P.scratch + (uint64_t)a * P.slab_doubles;
+  const uint64_t S = P.gcap;
+  float *srho = reinterpret_cast<float *>(slab + 3 * S);
+  uint64_t *smask = reinterpret_cast<uint64_t *>(slab + slab_masks(S));
+  uint32_t *sgid = reinterpret_cast<uint32_t *>(slab + slab_ids(S));
+  uint64_t *rmask = SLAB ? smask : lmask;
   const uint64_t off = P.goff[u];
   const double ux = P.X[u], uy = P.Y[u], uz = P.Z[u];
   const double Rg = P.radius[u];  // before the first barrier: one lane may widen it below
   // load, ranked by distance (the keys sit in the mask area until the masks come)
-  float *key = reinterpret_cast<float *>(rmask);
+  float *key = reinterpret_cast<float *>(lmask);
   float4 mine[kPer];
   uint32_t id[kPer];
 #pragma unroll
@@ -1651,11 +1664,6 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
     if (lane == 0) wcount[r][wave] = (uint32_t)__popcll(bits[r]);
   }
   __syncthreads();
-  double *slab = P.scratch + (uint64_t)a * P.slab_doubles;
-  const uint64_t S = P.gcap;
-  float *srho = reinterpret_cast<float *>(slab + 3 * S);
-  uint64_t *smask = reinterpret_cast<uint64_t *>(slab + slab_masks(S));
-  uint32_t *sgid = reinterpret_cast<uint32_t *>(slab + slab_ids(S));
   srho[c] = rho;
   uint32_t M = 0;
 #pragma unroll
@@ -1665,14 +1673,23 @@ __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {
       if (w < wave) slot += wcount[r][w];
       M += wcount[r][w];
     }
-    if (!((bits[r] >> lane) & 1)) continue;
+    const bool member = (bits[r] >> lane) & 1;
     slot += (uint32_t)__popcll(bits[r] & ((1ull << lane) - 1ull));
-    const uint32_t i = t + r * kProbeBlock, v = gid[i];
-    slab[slot] = P.X[v] - ux;
-    slab[S + slot] = P.Y[v] - uy;
-    slab[2 * S + slot] = P.Z[v] - uz;
-    sgid[slot] = v;
-    for (int k = 0; k < 6; ++k) smask[6 * (uint64_t)slot + k] = rmask[6 * i + k];
+    const uint32_t i = t + r * kProbeBlock;
+    uint64_t row[6];
+    if (member)
+      for (int k = 0; k < 6; ++k) row[k] = rmask[6 * i + k];
+    // in the slab the rows move to the front of where they are: every row of
+    // the chunk is read before one is written
+    if (SLAB) __syncthreads();
+    if (member) {
+      const uint32_t v = gid[i];
+      slab[slot] = P.X[v] - ux;
+      slab[S + slot] = P.Y[v] - uy;
+      slab[2 * S + slot] = P.Z[v] - uz;
+      sgid[slot] = v;
+      for (int k = 0; k < 6; ++k) smask[6 * (uint64_t)slot + k] = row[k];
+    }
   }
   if (t == 0) {
     // a region beyond the LDS enumerations is probed again on its own slab
@@ -2285,8 +2302,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   // Probes `count` anchors of the device list in chunks whose slabs fit the
   // chunk budget (2 GiB; under a capacity a quarter of what it leaves, at
   // least 1 MiB), each chunk enumerated before the next one takes its slabs.
-  auto probe_lds = [&](const uint32_t *anchors, uint32_t count, bool wide) {
-    const uint32_t g = wide ? kGatherCapWide : kGatherCap;
+  auto probe_lds = [&](const uint32_t *anchors, uint32_t count, uint32_t g) {
     const uint64_t slab = probe_slab_doubles(g);
     uint64_t budget = 2ull << 30;
     if (c.capacity_bytes > 0)
@@ -2307,10 +2323,13 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
         Q.two_waves = kRegionCapLittle;
       }
       clear_lists(L_TINY, kLists);
-      if (wide)
-        hipLaunchKernelGGL(k_anchor_probe<kGatherCapWide>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
+      const dim3 grid(Q.anchor_count), block(kProbeBlock);
+      if (g == kGatherCap)
+        hipLaunchKernelGGL((k_anchor_probe<kGatherCap, false>), grid, block, 0, s, Q);
+      else if (g == kGatherCapWide)
+        hipLaunchKernelGGL((k_anchor_probe<kGatherCapWide, false>), grid, block, 0, s, Q);
       else
-        hipLaunchKernelGGL(k_anchor_probe<kGatherCap>, dim3(Q.anchor_count), dim3(kProbeBlock), 0, s, Q);
+        hipLaunchKernelGGL((k_anchor_probe<kGatherCapSlab, true>), grid, block, 0, s, Q);
       MHGP_LAUNCH_CHECK();
       read_counters();
       enumerate(Q);
@@ -2336,11 +2355,11 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     clear_lists(0, kLists);
     c.anchor_clock.start(s);
     if (!force_path) {
-      probe_lds(B.anchors.p, cnt, false);
-      if (const uint32_t wc = (uint32_t)ctr[kListCount + L_WIDE]) {
-        probe_lds(list(L_WIDE), wc, true);
-        if (tm.on) std::fprintf(stderr, "[mhgp] wide anchors: %u\n", wc);
-      }
+      probe_lds(B.anchors.p, cnt, kGatherCap);
+      const uint32_t wide = (uint32_t)ctr[kListCount + L_WIDE], wider = (uint32_t)ctr[kListCount + L_WIDER];
+      if (wide) probe_lds(list(L_WIDE), wide, kGatherCapWide);
+      if (wider) probe_lds(list(L_WIDER), wider, kGatherCapSlab);
+      if (tm.on && (wide || wider)) std::fprintf(stderr, "[mhgp] wide anchors: %u, wider: %u\n", wide, wider);
     }
     c.anchor_clock.stop(s);
     tm.mark("catalogue anchors");

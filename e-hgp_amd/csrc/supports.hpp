@@ -13,6 +13,7 @@ constexpr uint32_t kRegionCapTiny = 96, kRegionCapLittle = 180;  // members that
 constexpr int kRegionCap = 384;  // region members the smallest enumeration holds in LDS
 constexpr uint32_t kRegionLimitMax = 2048;  // largest candidate region any path enumerates
 constexpr int kGatherCapWide = 1024;  // the same for the wide probe and the next enumeration
+constexpr int kGatherCapSlab = 2048;  // the same with the masks in the slab
 constexpr int kRegionCapWide = 640;
 constexpr int kMaxInterior = 10; // s_max - 2 for s_max <= 11 (K_max <= 10)
 

@@ -140,6 +140,25 @@ def test_catalog_nearly_cospherical(path, sigma, n, k, monkeypatch):
     _compare(workloads.jittered_lattice(n, side=5, sigma=sigma, seed=36), k, f"lattice{n}-{sigma}-{path}")
 
 
+@pytest.mark.parametrize("n,k", [(1100, 4), (2300, 3)])
+def test_wide_gathers_agree_with_the_global_memory_path(n, k, monkeypatch):
+    """Gathers of 1 025 to 2 048 points build their masks in the slab, larger
+    ones take the global-memory probe: an anisotropic mixture whose gathers
+    reach most of the cloud, against the same catalogue with every anchor
+    through the global-memory probe."""
+    pts = workloads.gaussian_mixture(n, blobs=3, noise_fraction=0.15, box=10.0, snap_bits=None, seed=43)
+    print(f"wide gathers: mixture n={n} k={k}", flush=True)
+    got = []
+    for path in ("", "region"):
+        monkeypatch.setenv("MHGP_TEST_ANCHOR_PATH", path)
+        with mhgp.Context(0) as ctx:
+            ctx.upload(pts)
+            got.append(ctx.supports_raw(k))
+    for key in ("ids", "meta", "interior", "level", "level_class"):
+        assert np.array_equal(got[0][key], got[1][key]), key
+    assert got[0]["info"].status == 0 and len(got[0]["meta"]) > n
+
+
 def test_big_regions_give_a_conditional_catalogue():
     """Anchors whose candidate region exceeds the enumeration bound are left
     open: the catalogue reports status conditional with their count and
