@@ -14,14 +14,14 @@
 //      order inside a digit is (wave, chunk, lane), the input order: the pass
 //      is stable.
 // Passes whose digit is the same for every key copy instead of scattering, so
-// ping-pong buffers stay consistent.  Up to kSmallSort keys are sorted by one
-// workgroup in LDS (bitonic over (key, index), hence stable).
+// ping-pong buffers stay consistent.  Up to kSmallSort keys are placed by
+// counting the keys before each (rs_rank).
 //
 // Below a few hundred thousand keys a pass is bound by its launches and by the
 // few workgroups it has: tiles of 1 024 and the two-launch pass took the sorts
 // of a 50 000-point build from four launches and 13 workgroups a pass to two
-// and 49, the one-workgroup sort those of a 256-point build from 128 launches
-// to two (index of 256 points: 0.91 -> 0.29 ms with the rest of the build).
+// and 49, the sort by counting those of a 256-point build from 128 launches to
+// four (index of 256 points: 0.91 -> 0.26 ms with the rest of the build).
 #include "radix_sort.hpp"
 
 namespace mhgp {
@@ -198,54 +198,46 @@ __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restr
   }
 }
 
-// Up to kSmallSort keys in one workgroup: a bitonic sort of (key, index) in
-// LDS, keys beyond n sorting last.
-__global__ void __launch_bounds__(kSmallBlock) rs_small(uint64_t *keys, uint32_t *vals, int n, int padded, int shift,
-                                                        uint64_t mask) {
-  __shared__ uint64_t k[kSmallSort];
-  __shared__ uint16_t at[kSmallSort];
-  for (int i = threadIdx.x; i < padded; i += kSmallBlock) {
-    k[i] = i < n ? (keys[i] >> shift) & mask : ~0ull;
-    at[i] = (uint16_t)i;
+// Up to kSmallSort keys: a key's place is the number of keys before it, counted
+// by all 16 waves of a workgroup for 64 keys (a lane each), every wave over its
+// share of the keys, which it reads with uniform addresses.  n^2 comparisons
+// spread over the chip cost less than the 91 barriers of one workgroup's
+// bitonic sort of 8 192 keys: the three sorts of a 256-point catalogue (256,
+// 256 and 4 790 keys) 126 -> 44 us.
+__global__ void __launch_bounds__(kSmallBlock) rs_rank(const uint64_t *__restrict__ keys, const uint32_t *__restrict__ vals,
+                                                       int n, int shift, uint64_t mask, uint64_t *__restrict__ kout,
+                                                       uint32_t *__restrict__ vout) {
+  constexpr int kWaves = kSmallBlock / 64;
+  __shared__ uint32_t part[kWaves][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int first = blockIdx.x * 64, i = first + lane;
+  const uint64_t key = i < n ? keys[i] : 0, mine = (key >> shift) & mask;
+  const int share = (n + kWaves - 1) / kWaves, j0 = wave * share, j1 = min(j0 + share, n);
+  // equal keys keep their order: those at smaller positions come before
+  uint32_t before = 0;
+  const int lo = min(max(first, j0), j1), hi = min(max(first + 64, j0), j1);
+  for (int j = j0; j < lo; ++j) before += ((keys[j] >> shift) & mask) <= mine;
+  for (int j = lo; j < hi; ++j) {
+    const uint64_t k = (keys[j] >> shift) & mask;
+    before += k < mine || (k == mine && j < i);
   }
+  for (int j = hi; j < j1; ++j) before += ((keys[j] >> shift) & mask) < mine;
+  part[wave][lane] = before;
   __syncthreads();
-  for (int size = 2; size <= padded; size <<= 1)
-    for (int d = size >> 1; d > 0; d >>= 1) {
-      for (int p = threadIdx.x; p < padded / 2; p += kSmallBlock) {
-        const int i = 2 * p - (p & (d - 1)), j = i + d;  // bit d of i clear
-        const bool up = (i & size) == 0;
-        const uint64_t a = k[i], b = k[j];
-        const uint16_t x = at[i], y = at[j];
-        const bool above = a > b || (a == b && x > y);
-        if (above == up) {
-          k[i] = b;
-          k[j] = a;
-          at[i] = y;
-          at[j] = x;
-        }
-      }
-      __syncthreads();
-    }
-  // gather through registers: sources are read before any is overwritten
-  uint64_t kv[kSmallSort / kSmallBlock];
-  uint32_t vv[kSmallSort / kSmallBlock];
+  if (wave != 0 || i >= n) return;
+  uint32_t place = 0;
 #pragma unroll
-  for (int r = 0; r < kSmallSort / kSmallBlock; ++r) {
-    const int i = threadIdx.x + r * kSmallBlock;
-    if (i < n) {
-      kv[r] = keys[at[i]];
-      vv[r] = vals[at[i]];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < kSmallSort / kSmallBlock; ++r) {
-    const int i = threadIdx.x + r * kSmallBlock;
-    if (i < n) {
-      keys[i] = kv[r];
-      vals[i] = vv[r];
-    }
-  }
+  for (int w = 0; w < kWaves; ++w) place += part[w][lane];
+  kout[place] = key;
+  vout[place] = vals[i];
+}
+
+__global__ void rs_copy(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin, int n, uint64_t *kout,
+                        uint32_t *vout) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  kout[i] = kin[i];
+  vout[i] = vin[i];
 }
 
 template <int kTile, bool DIRECT>
@@ -264,10 +256,12 @@ void RadixSorter::sort(uint64_t *keys, uint32_t *vals, int64_t n, int begin_bit,
                        hipStream_t stream) {
   if (n <= 1) return;
   if (n <= kSmallSort) {
-    int padded = 2;
-    while (padded < n) padded <<= 1;
     const uint64_t mask = end_bit - begin_bit >= 64 ? ~0ull : (1ull << (end_bit - begin_bit)) - 1ull;
-    hipLaunchKernelGGL(rs_small, dim3(1), dim3(kSmallBlock), 0, stream, keys, vals, (int)n, padded, begin_bit, mask);
+    tmp_keys.ensure(n);
+    tmp_vals.ensure(n);
+    hipLaunchKernelGGL(rs_rank, dim3(blocks_for(n, 64)), dim3(kSmallBlock), 0, stream, keys, vals, (int)n, begin_bit, mask,
+                       tmp_keys.p, tmp_vals.p);
+    hipLaunchKernelGGL(rs_copy, dim3(blocks_for(n, 256)), dim3(256), 0, stream, tmp_keys.p, tmp_vals.p, (int)n, keys, vals);
     MHGP_LAUNCH_CHECK();
     return;
   }
