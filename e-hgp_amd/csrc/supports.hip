@@ -2206,7 +2206,9 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   uint64_t event_cap = std::max<uint64_t>(1024, (uint64_t)n * (smax >= 11 ? 640 : 64 * smax));
   uint64_t fb_cap = std::max<uint64_t>(4096, (uint64_t)n / 4);
   uint64_t reg_cap = std::max<uint64_t>(1 << 20, (uint64_t)n * 64);
-  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n * 16);
+  // a longer list costs the enumeration again (lattices displaced by 1% of
+  // their spacing leave several sides a point)
+  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n * (c.capacity_bytes > 0 ? 1 : 16));
   uint64_t ctr[kCounters];
   int64_t widened = 0;
   // The record queues have a fixed capacity per launch; records past it are
