@@ -415,7 +415,7 @@ def main() -> None:
         # roofline is the VALU's FP32 (unpacked) / FP64 peak, with the HBM
         # figures beside it.
         "roofline": {
-            "kernel": "k_anchor_lds (critical-sphere catalogue, one workgroup per anchor)",
+            "kernel": "k_anchor_probe + k_anchor_region (critical-sphere catalogue)",
             "bound": "valu",
             "achieved": round(tflops, 4),
             "peak": VALU_PEAK / 1e12,

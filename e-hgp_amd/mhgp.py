@@ -424,8 +424,8 @@ class Server:
 
 
 def batch_run(clouds, k_max, group: int = 32, memory_cap_bytes: int = 0, device: int = 0):
-    """Runs many clouds through mhgp_batch_run (groups side by side, one
-    persistent anchor launch per group).  k_max: one value or one per cloud.
+    """Runs many clouds through mhgp_batch_run, which is switched off and
+    refuses (MHGP_E_UNSUPPORTED).  k_max: one value or one per cloud.
     Returns (results, towers, info): per cloud a RequestResult and its tower
     (dict as Context.tower without vertical maps, or None), and the batch's
     BatchInfo."""
