@@ -92,10 +92,18 @@ __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restr
   // the scanned bounds of its keys
   uint32_t in_before = 0, in_all = 0;
   if (DIRECT) {
-    for (int i = 0; i < tiles; ++i) {
-      const uint32_t c = counts[(size_t)i * kDigits + t];
-      in_before += i < (int)blockIdx.x ? c : 0u;
-      in_all += c;
+    // sixteen rows in flight: one at a time the loop was the pass (60 000 keys,
+    // 59 tiles: 17.9 -> 8.5 us; 200 000 keys, 49 tiles of 4 096: 22.3 -> 14.5 us)
+    for (int i0 = 0; i0 < tiles; i0 += 16) {
+      uint32_t c[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) c[k] = counts[(size_t)min(i0 + k, tiles - 1) * kDigits + t];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const uint32_t v = i0 + k < tiles ? c[k] : 0u;
+        in_before += i0 + k < (int)blockIdx.x ? v : 0u;
+        in_all += v;
+      }
     }
   } else {
     const uint32_t lo = t == 0 ? 0u : counts[(size_t)t * tiles - 1];
