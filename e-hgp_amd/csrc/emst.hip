@@ -116,7 +116,11 @@ __global__ void __launch_bounds__(64) k_top_labels(WaveTree T, Rounds R) {
 
 // Lightest external edge under kappa of every point whose last one is gone:
 // each lane keeps its own best over the groups, the wave combines them at the
-// end.  The component's best offer bounds the search from the start.
+// end.  The component's best offer bounds the search from the start: a result
+// counts within the offer's rounding window (limit).  The search itself sees
+// points up to the window of any result that counts, because a result may be
+// kept for later rounds, where that offer is gone and nothing else shows that
+// another point is as near.
 constexpr int kSearchBlock = 256;  // four waves, four points
 __global__ void __launch_bounds__(kSearchBlock) k_search(WaveTree T, Rounds R) {
   const uint32_t lane = threadIdx.x & 63u;
@@ -132,7 +136,7 @@ __global__ void __launch_bounds__(kSearchBlock) k_search(WaveTree T, Rounds R) {
   double bd = INFINITY;
   uint32_t bp = kInvalid, bv = kInvalid;
   bool bx = true, near_tie = false;
-  double bound = limit;
+  double bound = offer * (1.0 + 4.0 * kSlack) + 4.0 * kSlackAbs;  // >= limit * (1 + kSlack) + kSlackAbs
   float Tf = Q.bound(bound);
   auto group = [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);

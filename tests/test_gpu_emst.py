@@ -1,5 +1,7 @@
 """Exact Borůvka EMST on the GPU vs the oracle's complete-graph Kruskal."""
 
+from fractions import Fraction
+
 import numpy as np
 import pytest
 
@@ -52,6 +54,46 @@ def test_emst_rounds_at_their_edges(name):
         ctx.upload(pts)
         e = ctx.emst().astype(np.int64)
     assert np.array_equal(e, np.asarray(ref, dtype=np.int64).reshape(e.shape))
+
+
+def _sq(q):  # squared length, rounded as the device does
+    return (q[0] * q[0] + q[1] * q[1]) + q[2] * q[2]
+
+
+def _kept_result_cloud():
+    """Two points x, y whose FP64 distances to p (the origin) are one ulp
+    apart in the order opposite to the exact one, and a point a of p's
+    component whose own result, kept from the round before, lies just far
+    enough below both that the first is within its rounding window and the
+    second is not.  Clusters with doubling gaps let p, a and the others merge
+    at smaller distances round by round until then."""
+    x, y, w = [-0.8190404901453785, 6.425679486307635e-05, 0.5737357156160684], [-0.820664404928251, -0.0007032900117319003, -0.5714100452975243], 0.9999999999994997
+    assert _sq(y) == np.nextafter(_sq(x), 2.0) and sum(Fraction(c) ** 2 for c in y) < sum(Fraction(c) ** 2 for c in x)
+    assert w * w * (1.0 + 1e-12) + 1e-300 == _sq(x) and _sq(x) - w * w > 1e-12 * (w * w)
+    pts = [[0, 0, 0], [0, 0.1, 0], [0, 0.45, 0], [0, 0.55, 0]]
+    pts += [[0, -0.9 - o, 0] for o in (0, 0.1, 0.4, 0.5)]
+    pts += [[w + o, 0.55, 0] for o in (0, 0.1, 0.4, 0.5, 1.1, 1.2, 1.5, 1.6)]
+    turns = np.array([x, [-1.62, 0, x[2]], [-1.62, 0, y[2]], y])
+    leg = np.linalg.norm(np.diff(turns, axis=0), axis=1)
+    ends = np.concatenate([[0.0], np.cumsum(leg)])
+    gaps = np.array([0.1, 0.2, 0.1, 0.3, 0.1, 0.2, 0.1, 0.4, 0.1, 0.2, 0.1, 0.3, 0.1, 0.2, 0.1])
+    for s in np.cumsum(gaps)[:-1] * ends[-1] / gaps.sum():
+        k = min(int(np.searchsorted(ends, s, side="right")) - 1, 2)
+        pts.append(list(turns[k] + (turns[k + 1] - turns[k]) * (s - ends[k]) / leg[k]))
+    return np.array(pts + [x, y], dtype=float)
+
+
+def test_emst_near_ties_of_kept_results():
+    """A search ends at the rounding window of its component's best offer; a
+    near tie just beyond it still has to be known when the result is used in a
+    later round, where that offer is gone."""
+    pts = _kept_result_cloud()
+    print("emst: near tie beyond an offer's window", flush=True)
+    ref = oracle.emst(oracle.canonicalize(pts))
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        e = ctx.emst().astype(np.int64)
+    assert np.array_equal(e, ref)
 
 
 def test_emst_50k_lattice_weight():
