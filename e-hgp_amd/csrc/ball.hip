@@ -89,8 +89,9 @@ __global__ void __launch_bounds__(kBallBlock) k_closed_ball(BallParams B) {
     if (lane == 0) B.flags[q] = kHostQuery;
     return;
   }
+  // distances are taken from o, and the centre never leaves that frame: o + off
+  // rounds by an ulp of o, which far from the origin exceeds the margin below
   r2 = dot(off, off);
-  const double c[3] = {o.x + off.x, o.y + off.y, o.z + off.z};
   const double R2 = r2 * (1.0 + 1e-6) + 1e-300;  // every point beyond is certainly outside
   uint32_t nin = 0, nsh = (uint32_t)m;
   // the interior row keeps the cap smallest ids, so a truncated list does not
@@ -101,20 +102,17 @@ __global__ void __launch_bounds__(kBallBlock) k_closed_ball(BallParams B) {
   const bool in_lanes = B.cap <= 64;
   uint32_t list = kInvalid, rmax = kInvalid;
   const WaveTree &T = B.tree;
-  const WaveQuery Q(T, c[0], c[1], c[2]);
+  const WaveQuery Q(T, o.x, o.y, o.z, off.x, off.y, off.z);
   float Tf = Q.bound(R2);
   wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
-    const double dx = T.LX[at] - c[0], dy = T.LY[at] - c[1], dz = T.LZ[at] - c[2];
-    bool near = lp < T.n && !(dx * dx + dy * dy + dz * dz > R2);
+    const V3 p = sub({T.LX[at], T.LY[at], T.LZ[at]}, o), d = sub(p, off);
+    bool near = lp < T.n && !(dot(d, d) > R2);
     if (!__ballot(near)) return;
     const uint32_t id = T.leaf_id[at];
     for (int i = 0; i < m; ++i) near = near && sid[i] != id;
     int sd = 1;
-    if (near) {
-      const V3 p = sub({T.LX[at], T.LY[at], T.LZ[at]}, o);
-      sd = m == 2 ? ps.side(p) : (m == 3 ? ts.side(p) : tt.side(p));
-    }
+    if (near) sd = m == 2 ? ps.side(p) : (m == 3 ? ts.side(p) : tt.side(p));
     if (near && sd == 0) {
       const unsigned long long slot = atomicAdd(B.nund, 1ull);
       if (slot < B.und_cap) {

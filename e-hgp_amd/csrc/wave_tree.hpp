@@ -22,10 +22,13 @@ namespace mhgp {
 // coordinates (their rounding stays below 1e-7 of it).
 struct WaveQuery {
   float q[3], qmax;
-  __device__ WaveQuery(const WaveTree &T, double x, double y, double z) {
-    q[0] = (float)(x - T.centre[0]);
-    q[1] = (float)(y - T.centre[1]);
-    q[2] = (float)(z - T.centre[2]);
+  // (x, y, z) + (dx, dy, dz): a point near a cloud far from the origin is given
+  // by one of the cloud's own and an offset, whose sum would round away
+  __device__ WaveQuery(const WaveTree &T, double x, double y, double z, double dx = 0.0, double dy = 0.0,
+                       double dz = 0.0) {
+    q[0] = (float)((x - T.centre[0]) + dx);
+    q[1] = (float)((y - T.centre[1]) + dy);
+    q[2] = (float)((z - T.centre[2]) + dz);
     qmax = fmaxf(fmaxf(fabsf(q[0]), fabsf(q[1])), fabsf(q[2]));
   }
   // Squared FP32 bound for boxes that a ball of squared radius r2 can meet:

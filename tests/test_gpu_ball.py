@@ -109,3 +109,25 @@ def test_closed_ball_interior_lists_at_the_lane_capacity(cap):
     pts = workloads.uniform_cloud(400, seed=35)
     print(f"closed ball: uniform n=400, cap {cap}", flush=True)
     _check(pts, _random_supports(np.random.default_rng(2), 400, 40), cap=cap)
+
+
+@pytest.mark.parametrize("exponent", [0, 27, 30, 40])
+def test_closed_ball_far_from_the_origin(exponent):
+    """A grid of spacing 2^-7 at 2^exponent on every axis (exact in binary64):
+    the sphere's centre in absolute coordinates rounds by more than the radius
+    allows, so points on the sphere or just inside it must be found from
+    coordinates relative to the support."""
+    g = np.arange(5, dtype=np.float64) / 128.0
+    pts = np.stack(np.meshgrid(g, g, g, indexing="ij"), axis=-1).reshape(-1, 3) + (2.0 ** exponent if exponent else 0.0)
+    rng = np.random.default_rng(3)
+    sups = [[17, 43, 54]]  # (0, 3, 2), (1, 3, 3), (2, 0, 4) of the grid
+    while len(sups) < 240:
+        sup = [int(x) for x in rng.choice(len(pts), size=2 + len(sups) % 3, replace=False)]
+        a = (pts[sup[1:]] - pts[sup[0]]) * 128.0
+        if len(sup) == 3 and not np.any(np.cross(a[0], a[1]) != 0):
+            continue
+        if len(sup) == 4 and abs(np.linalg.det(a)) < 0.5:
+            continue
+        sups.append(sup)
+    print(f"closed ball: 5x5x5 grid at 2^{exponent}, {len(sups)} supports", flush=True)
+    _check(pts, sups, cap=20)
