@@ -11,12 +11,11 @@
 #include <vector>
 
 #include "../../include/mhgp.h"
+#include "budget.hpp"
 #include "pipeline.hpp"
 #include "tower_state.hpp"
 
 namespace mhgp {
-
-int64_t predict_bytes(int64_t n, int k_max);  // server.cpp
 
 namespace {
 

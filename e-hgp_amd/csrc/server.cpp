@@ -16,6 +16,7 @@
 #include <thread>
 #include <unordered_map>
 
+#include "budget.hpp"
 #include "pipeline.hpp"
 #include "supports.hpp"
 #include "tower_state.hpp"
@@ -39,13 +40,6 @@ struct Request {
 };
 
 }  // namespace
-
-// Predicted device bytes of one cloud: catalogue records dominate
-// (about 640 per point at K_max = 10, 72 B each) plus the LBVH and gathers.
-int64_t predict_bytes(int64_t n, int k_max) {
-  const int64_t per_point_records = k_max >= 10 ? 640 : 64 * (k_max + 1);
-  return n * (per_point_records * (int64_t)(sizeof(EventRec) + 16) + 1024) + (64ll << 20);
-}
 
 struct Server {
   int device = 0;

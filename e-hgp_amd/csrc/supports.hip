@@ -672,6 +672,7 @@ struct Rescan {
   uint32_t side;    // side | cin << 1
   float lo, hi;
 };
+static_assert(sizeof(Rescan) == kRescanBytes, "rescan layout");
 
 // Apexes of one side among the FP32 list its face's pass filled: bit j for
 // entry j.  rescan: a point left or missed the list with a lower bound within
@@ -1457,14 +1458,6 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
   anchor_faces<true, false, kBlock / 64, 11>(P, w, u, M, &sK, &sregion);
 }
 
-// Slab of one probed anchor (in doubles), for G gathered points:
-// [0, 3G) coordinates x, y, z relative to the anchor; [3G, 3G + kCells) cell
-// radii (float); [3G + kCells, 9G + kCells) masks, six words per point; then
-// PointIds.  The global-memory kernel adds its own arrays behind them.
-__host__ __device__ inline uint64_t slab_masks(uint64_t G) { return 3 * G + kCells; }
-__host__ __device__ inline uint64_t slab_ids(uint64_t G) { return 9 * G + kCells; }
-__host__ __device__ inline uint64_t probe_slab_doubles(uint64_t G) { return (slab_ids(G) + (G + 1) / 2 + 1) & ~1ull; }
-
 __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t M) {
   if (M > P.region_limit) {
     // budget stop: the anchor stays open, the catalogue is conditional
@@ -2203,12 +2196,9 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   MHGP_LAUNCH_CHECK();
   double bounds[6];
   copy_wait(bounds, c.bounds.p, sizeof(bounds), hipMemcpyDeviceToHost, s);
-  uint64_t event_cap = std::max<uint64_t>(1024, (uint64_t)n * (smax >= 11 ? 640 : 64 * smax));
-  uint64_t fb_cap = std::max<uint64_t>(4096, (uint64_t)n / 4);
-  uint64_t reg_cap = std::max<uint64_t>(1 << 20, (uint64_t)n * 64);
-  // a longer list costs the enumeration again (lattices displaced by 1% of
-  // their spacing leave several sides a point)
-  uint64_t rescan_cap = std::max<uint64_t>(1 << 14, (uint64_t)n * (c.capacity_bytes > 0 ? 1 : 16));
+  const CatalogueQueues queues = first_queues(n, smax);
+  uint64_t event_cap = queues.events, fb_cap = queues.fallbacks, reg_cap = queues.region_words;
+  uint64_t rescan_cap = c.capacity_bytes > 0 ? std::max<uint64_t>(1 << 14, (uint64_t)n) : queues.rescans;
   uint64_t ctr[kCounters];
   int64_t widened = 0;
   // The record queues have a fixed capacity per launch; records past it are
@@ -2306,7 +2296,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   // least 1 MiB), each chunk enumerated before the next one takes its slabs.
   auto probe_lds = [&](const uint32_t *anchors, uint32_t count, uint32_t g) {
     const uint64_t slab = probe_slab_doubles(g);
-    uint64_t budget = 2ull << 30;
+    uint64_t budget = kProbeSlabs;
     if (c.capacity_bytes > 0)
       budget = std::clamp<int64_t>((c.capacity_bytes - device_bytes(c)) / 4 + (int64_t)B.scratch.bytes(), 1 << 20, 1 << 30);
     const uint32_t most = (uint32_t)std::max<uint64_t>(1, budget / (slab * 8));

@@ -3,12 +3,11 @@
 
 #include <vector>
 
+#include "budget.hpp"
 #include "stages.hpp"
 
 namespace mhgp {
 
-constexpr int kCells = 384;      // 6 cube faces x 8 x 8 direction cells
-constexpr int kGatherCap = 600;  // gathered neighbours the probe holds in LDS
 constexpr uint32_t kRegionCapTiny = 96, kRegionCapLittle = 180;  // members that one and two waves hold in LDS
 constexpr int kRegionCap = 384;  // region members the smallest enumeration holds in LDS
 constexpr uint32_t kRegionLimitMax = 2048;  // largest candidate region any path enumerates
@@ -27,7 +26,7 @@ struct EventRec {
   float level_err;
   double level;
 };
-static_assert(sizeof(EventRec) == 72, "event layout");
+static_assert(sizeof(EventRec) == kRecordBytes, "event layout");
 
 // Work the device could not certify: the host settles it exactly.
 // kind 2: pair (u, v); 3: face (u, v, w) incl. its triangle and apexes;
