@@ -20,8 +20,17 @@ constexpr uint64_t slab_masks(uint64_t G) { return 3 * G + kCells; }
 constexpr uint64_t slab_ids(uint64_t G) { return 9 * G + kCells; }
 constexpr uint64_t probe_slab_doubles(uint64_t G) { return (slab_ids(G) + (G + 1) / 2 + 1) & ~1ull; }
 
-// Most memory that the slabs of one probe launch take.
+// Most memory that the slabs of one probe launch take, and the least that a
+// context with a device capacity keeps for them.
 constexpr int64_t kProbeSlabs = int64_t(2) << 30;
+constexpr int64_t probe_slabs_least(int64_t n) { return std::max<int64_t>(1 << 20, 64 * n); }
+
+// Bytes for a launch's slabs: those held and a quarter of what is left, within
+// [least, most].
+constexpr uint64_t probe_slab_budget(int64_t left, uint64_t held, int64_t least, int64_t most) {
+  const uint64_t b = (uint64_t)std::max<int64_t>(left, 0) / 4 + held;
+  return std::min<uint64_t>(std::max<uint64_t>(b, (uint64_t)least), (uint64_t)most);
+}
 
 // First capacities of the catalogue's queues (a catalogue that outgrows them
 // runs again with larger ones).
@@ -34,6 +43,17 @@ inline CatalogueQueues first_queues(int64_t n, int s_max) {
   // of their spacing leave several sides a point)
   return {std::max<uint64_t>(1024, m * (s_max >= 11 ? 640 : 64 * (uint64_t)s_max)), std::max<uint64_t>(4096, m / 4),
           std::max<uint64_t>(1 << 20, m * 64), std::max<uint64_t>(1 << 14, m * 16)};
+}
+// The same in a context with a device capacity: one rescan a point.  The queues give up what the slabs' least, the
+// rescans, the tables and the anchor lists and neighbour rows take: the
+// fallback regions the fixed part, the records 234 bytes a point (3.25 of at
+// least 128 records), so that a capacity for the whole queues holds it all.
+inline CatalogueQueues first_queues_bounded(int64_t n, int s_max) {
+  CatalogueQueues q = first_queues(n, s_max);
+  q.rescans = std::max<uint64_t>(1 << 14, (uint64_t)n);
+  q.region_words -= ((1 << 20) + (1 << 14) * kRescanBytes + 53248) / 4;
+  q.events -= (uint64_t)n * 13 / 4;
+  return q;
 }
 
 // Predicted device bytes of one request (upload, EMST, catalogue, tower on one

@@ -349,8 +349,9 @@ void supports_fetch(Context &c, uint32_t *ids, uint32_t *meta, uint32_t *interio
   hipStream_t s = c.stream;
   const int width = std::max(B.s_max - 1, 1);
   const size_t rec = 16 + 8 + 8 + 4 + 4 * (size_t)width;
-  const int64_t most = std::max<int64_t>(1, (int64_t)(B.scratch.bytes() / rec));
-  B.scratch.ensure(rec);
+  // (a context with a device capacity has given it back)
+  B.scratch.ensure(std::min<size_t>(n * rec, kExportPinned) / sizeof(double) + 1);
+  const int64_t most = (int64_t)(B.scratch.bytes() / rec);
   for (int64_t first = 0; first < n; first += most) {
     const int64_t m = std::min(most, n - first);
     char *d = reinterpret_cast<char *>(B.scratch.p);

@@ -2196,9 +2196,22 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   MHGP_LAUNCH_CHECK();
   double bounds[6];
   copy_wait(bounds, c.bounds.p, sizeof(bounds), hipMemcpyDeviceToHost, s);
-  const CatalogueQueues queues = first_queues(n, smax);
-  uint64_t event_cap = queues.events, fb_cap = queues.fallbacks, reg_cap = queues.region_words;
-  uint64_t rescan_cap = c.capacity_bytes > 0 ? std::max<uint64_t>(1 << 14, (uint64_t)n) : queues.rescans;
+  // under a capacity the slabs and rescans are given back when the call ends:
+  // what they took is the next stage's room
+  const bool bounded = c.capacity_bytes > 0;
+  auto give_back = [&] {
+    if (!bounded) return;
+    B.scratch.release();
+    B.rescans.release();
+  };
+  give_back();  // of a call that failed
+  CatalogueQueues cap = bounded ? first_queues_bounded(n, smax) : first_queues(n, smax);
+  // bytes that queues of these capacities take beyond those that are held
+  auto more = [&](const CatalogueQueues &q) {
+    auto grown = [](uint64_t want, uint64_t have, uint64_t bytes) { return want > have ? want * bytes - have * bytes : 0; };
+    return (int64_t)(grown(q.events, B.events.cap, sizeof(EventRec)) + grown(q.fallbacks, B.fallbacks.cap, sizeof(FallbackRec)) +
+                     grown(q.region_words, B.fb_region.cap, 4) + grown(q.rescans, B.rescans.cap / sizeof(Rescan), sizeof(Rescan)));
+  };
   uint64_t ctr[kCounters];
   int64_t widened = 0;
   // The record queues have a fixed capacity per launch; records past it are
@@ -2206,20 +2219,16 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   // again with queues sized from the counts (the widened gather radii are
   // kept), unless the device cannot hold them.
   for (int attempt = 0;; ++attempt) {
-  if (c.capacity_bytes > 0) {
+  if (bounded) {
     // the record queues are the catalogue's large, data-sized allocation
-    const int64_t more = (int64_t)(event_cap - std::min<uint64_t>(event_cap, B.events.cap)) * (int64_t)sizeof(EventRec) +
-                         (int64_t)(fb_cap - std::min<uint64_t>(fb_cap, B.fallbacks.cap)) * (int64_t)sizeof(FallbackRec) +
-                         (int64_t)(reg_cap - std::min<uint64_t>(reg_cap, B.fb_region.cap)) * 4 +
-                         (int64_t)(rescan_cap - std::min<uint64_t>(rescan_cap, B.rescans.cap / sizeof(Rescan))) * (int64_t)sizeof(Rescan);
-    if (device_bytes(c) + more > c.capacity_bytes)
-      throw CapacityError("the catalogue's record queues (" + std::to_string(event_cap) + " records) exceed the " +
+    if (device_bytes(c) + more(cap) > c.capacity_bytes)
+      throw CapacityError("the catalogue's record queues (" + std::to_string(cap.events) + " records) exceed the " +
                           "context's device capacity of " + std::to_string(c.capacity_bytes) + " bytes");
   }
-  B.events.ensure(event_cap);
-  B.fallbacks.ensure(fb_cap);
-  B.fb_region.ensure(reg_cap);
-  B.rescans.ensure(rescan_cap * sizeof(Rescan));
+  B.events.ensure(cap.events);
+  B.fallbacks.ensure(cap.fallbacks);
+  B.fb_region.ensure(cap.region_words);
+  B.rescans.ensure(cap.rescans * sizeof(Rescan));
   MHGP_HIP(hipMemsetAsync(B.counters.p, 0, kCounters * 8, s));
   widened = 0;
   Params P{};
@@ -2233,10 +2242,10 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   P.region = B.region.p;
   P.lists = B.lists.p;
   P.list_cap = (uint32_t)n;
-  P.events = B.events.p; P.event_cap = event_cap;
-  P.fallbacks = B.fallbacks.p; P.fallback_cap = fb_cap;
-  P.fb_region = B.fb_region.p; P.fb_region_cap = reg_cap;
-  P.rescans = reinterpret_cast<Rescan *>(B.rescans.p); P.rescan_cap = rescan_cap;
+  P.events = B.events.p; P.event_cap = cap.events;
+  P.fallbacks = B.fallbacks.p; P.fallback_cap = cap.fallbacks;
+  P.fb_region = B.fb_region.p; P.fb_region_cap = cap.region_words;
+  P.rescans = reinterpret_cast<Rescan *>(B.rescans.p); P.rescan_cap = cap.rescans;
   P.counters = (unsigned long long *)B.counters.p;
   P.count_flops = c.count_flops ? 1 : 0;
   P.region_limit = std::min<uint32_t>(c.region_limit, kBigRegionMax);
@@ -2291,16 +2300,21 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
     return std::max<uint64_t>(1ull << 30, std::min<uint64_t>(8ull << 30, free_b / 4));
   };
-  // Probes `count` anchors of the device list in chunks whose slabs fit the
-  // chunk budget (2 GiB; under a capacity a quarter of what it leaves, at
-  // least 1 MiB), each chunk enumerated before the next one takes its slabs.
+  // Probes `count` anchors of the device list in chunks whose slabs fit 2 GiB,
+  // each chunk enumerated before the next one takes its slabs.  Under a capacity
+  // slabs beyond those held grow into a quarter of what that leaves, at least
+  // probe_slabs_least.
   auto probe_lds = [&](const uint32_t *anchors, uint32_t count, uint32_t g) {
-    const uint64_t slab = probe_slab_doubles(g);
-    uint64_t budget = kProbeSlabs;
-    if (c.capacity_bytes > 0)
-      budget = std::clamp<int64_t>((c.capacity_bytes - device_bytes(c)) / 4 + (int64_t)B.scratch.bytes(), 1 << 20, 1 << 30);
-    const uint32_t most = (uint32_t)std::max<uint64_t>(1, budget / (slab * 8));
-    const uint32_t chunks = (count + most - 1) / most, per = (count + chunks - 1) / chunks;
+    const uint64_t slab = probe_slab_doubles(g), held = B.scratch.bytes();
+    uint32_t per = 0;
+    auto chunks_of = [&](uint64_t budget) {
+      const uint32_t most = (uint32_t)std::clamp<uint64_t>(budget / (slab * 8), 1, count);
+      const uint32_t chunks = (count + most - 1) / most;
+      per = (count + chunks - 1) / chunks;
+    };
+    chunks_of(kProbeSlabs);
+    if (bounded && per * slab * 8 > held)
+      chunks_of(probe_slab_budget(c.capacity_bytes - device_bytes(c), held, probe_slabs_least(n), kProbeSlabs / 2));
     B.scratch.ensure(slab * per);
     for (uint32_t a0 = 0; a0 < count; a0 += per) {
       Params Q = P;
@@ -2450,26 +2464,31 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   tm.mark("catalogue big anchors");
   read_counters();
   if (tm.on) std::fprintf(stderr, "[mhgp] sides left to the rescans, most in a launch: %llu\n", (unsigned long long)ctr[kRescanMost]);
-  if (ctr[0] <= event_cap && ctr[1] <= fb_cap && ctr[2] <= reg_cap && ctr[kRescanMost] <= rescan_cap) break;
+  if (ctr[0] <= cap.events && ctr[1] <= cap.fallbacks && ctr[2] <= cap.region_words && ctr[kRescanMost] <= cap.rescans) break;
   // a launch that ran out of rescans has also counted too few records
   if (attempt >= 3) throw CapacityError("catalogue record queues did not settle after regrowth");
-  const uint64_t ev2 = std::max(event_cap, ctr[0] + ctr[0] / 8), fb2 = std::max(fb_cap, ctr[1] + ctr[1] / 8),
-                 rg2 = std::max(reg_cap, ctr[2] + ctr[2] / 8);
-  rescan_cap = std::max(rescan_cap, ctr[kRescanMost] + ctr[kRescanMost] / 8);
+  auto needed = [&](int at) { return ctr[at] + ctr[at] / 8; };
+  const CatalogueQueues need{needed(0), needed(1), needed(2), needed(kRescanMost)};
+  cap = {std::max(cap.events, need.events), std::max(cap.fallbacks, need.fallbacks),
+         std::max(cap.region_words, need.region_words), std::max(cap.rescans, need.rescans)};
+  if (bounded && device_bytes(c) + more(cap) > c.capacity_bytes) {
+    // no room for the first capacities beside the grown ones: what was counted
+    cap = {std::max<uint64_t>(need.events, 1024), std::max<uint64_t>(need.fallbacks, 1024),
+           std::max<uint64_t>(need.region_words, 1024), std::max<uint64_t>(need.rescans, 1024)};
+    B.events.release();
+    B.fallbacks.release();
+    B.fb_region.release();
+    B.rescans.release();
+  }
   size_t free_b = 0, total_b = 0;
   MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
-  const uint64_t more = (ev2 - std::min<uint64_t>(ev2, B.events.cap)) * sizeof(EventRec) +
-                        (fb2 - std::min<uint64_t>(fb2, B.fallbacks.cap)) * sizeof(FallbackRec) +
-                        (rg2 - std::min<uint64_t>(rg2, B.fb_region.cap)) * 4 + rescan_cap * sizeof(Rescan);
-  if (more > free_b / 10 * 9)
+  if ((uint64_t)more(cap) > free_b / 10 * 9)
     throw CapacityError("the catalogue needs " + std::to_string(ctr[0]) + " record slots, more than the device can hold");
-  event_cap = ev2;
-  fb_cap = fb2;
-  reg_cap = rg2;
   // grown buffers start empty: release before the larger allocation
-  if (B.events.cap < event_cap) B.events.release();
-  if (B.fallbacks.cap < fb_cap) B.fallbacks.release();
-  if (B.fb_region.cap < reg_cap) B.fb_region.release();
+  if (B.events.cap < cap.events) B.events.release();
+  if (B.fallbacks.cap < cap.fallbacks) B.fallbacks.release();
+  if (B.fb_region.cap < cap.region_words) B.fb_region.release();
+  if (B.rescans.cap < cap.rescans * sizeof(Rescan)) B.rescans.release();
   }
   // records stay on the device; only the host's share of the work moves
   (void)events;
@@ -2478,6 +2497,7 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
   fb_region.resize(ctr[2]);
   if (ctr[1]) copy_wait(fbs.data(), B.fallbacks.p, ctr[1] * sizeof(FallbackRec), hipMemcpyDeviceToHost, s);
   if (ctr[2]) copy_wait(fb_region.data(), B.fb_region.p, ctr[2] * 4, hipMemcpyDeviceToHost, s);
+  give_back();
   tm.mark("catalogue download");
   info->candidate_count = (int64_t)ctr[3];
   info->anchors_widened = widened;

@@ -20,9 +20,11 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(PKG, "csrc"),
                     os.path.join(HERE, "native", "budget_check.cpp"), "-o", str(out)], check=True, capture_output=True)
     lib = ctypes.CDLL(str(out))
-    for f in (lib.budget_predict, lib.budget_catalogue):
+    for f in (lib.budget_predict, lib.budget_catalogue, lib.budget_queues, lib.budget_bounded):
         f.argtypes = [ctypes.c_int64, ctypes.c_int]
         f.restype = ctypes.c_int64
+    lib.budget_slabs.argtypes = [ctypes.c_int64, ctypes.c_uint64, ctypes.c_int64, ctypes.c_int64]
+    lib.budget_slabs.restype = ctypes.c_uint64
     return lib
 
 
@@ -32,6 +34,25 @@ def test_prediction_covers_the_first_allocations(lib, n):
         rows = n * (64 * 4 + 9)  # a tower's neighbour rows
         assert lib.budget_predict(n, k) >= lib.budget_catalogue(n, k) + rows
         assert lib.budget_predict(n, k) >= lib.budget_predict(n, max(k - 1, 1))
+
+
+@pytest.mark.parametrize("n", [2, 7, 64, 1000, 16384, 16385, 17117, 50000, 2000000])
+def test_bounded_queues_leave_room_for_slabs_and_rescans(lib, n):
+    """With rescans, the slabs' least, the tables (53 248 bytes) and the wider
+    rows and lists (138 bytes a point) the queues of a context with a device
+    capacity take no more than the plain queues."""
+    for k in range(1, 11):
+        assert lib.budget_bounded(n, k) + 53248 + 138 * n <= lib.budget_queues(n, k)
+
+
+def test_slabs_grow_into_a_quarter_of_what_is_left(lib):
+    mib = 1 << 20
+    assert lib.budget_slabs(400 * mib, 0, mib, 2048 * mib) == 100 * mib
+    assert lib.budget_slabs(400 * mib, 50 * mib, mib, 2048 * mib) == 150 * mib
+    assert lib.budget_slabs(0, 0, mib, 2048 * mib) == mib
+    assert lib.budget_slabs(-5, 0, mib, 2048 * mib) == mib
+    assert lib.budget_slabs(1 << 40, 0, mib, 2048 * mib) == 2048 * mib
+    assert lib.budget_slabs(0, 0, 4096 * mib, 2048 * mib) == 2048 * mib
 
 
 @pytest.mark.gpu
