@@ -44,7 +44,8 @@ inline CatalogueQueues first_queues(int64_t n, int s_max) {
   return {std::max<uint64_t>(1024, m * (s_max >= 11 ? 640 : 64 * (uint64_t)s_max)), std::max<uint64_t>(4096, m / 4),
           std::max<uint64_t>(1 << 20, m * 64), std::max<uint64_t>(1 << 14, m * 16)};
 }
-// The same in a context with a device capacity: one rescan a point.  The queues give up what the slabs' least, the
+// The same in a context with a device capacity: one rescan a point (more where
+// the capacity leaves room).  The queues give up what the slabs' least, the
 // rescans, the tables and the anchor lists and neighbour rows take: the
 // fallback regions the fixed part, the records 234 bytes a point (3.25 of at
 // least 128 records), so that a capacity for the whole queues holds it all.

@@ -2355,6 +2355,16 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     B.glist.ensure(tot + 1);
     launch_gather<true>(s, c, B, cnt);
     P.glist = B.glist.p;
+    if (bounded && iter == 0) {
+      // an eighth of what is left for rescans, up to an unbounded context's;
+      // the list is still empty
+      const uint64_t left = (uint64_t)std::max<int64_t>(0, c.capacity_bytes - device_bytes(c));
+      const uint64_t held = B.rescans.cap / sizeof(Rescan), full = first_queues(n, smax).rescans;
+      if (held < full && left / 8 >= sizeof(Rescan)) B.rescans.ensure(std::min<uint64_t>(full, held + left / 8 / sizeof(Rescan)) * sizeof(Rescan));
+      cap.rescans = std::max(cap.rescans, B.rescans.cap / sizeof(Rescan));
+      P.rescans = reinterpret_cast<Rescan *>(B.rescans.p);
+      P.rescan_cap = cap.rescans;
+    }
     tm.mark("catalogue gather");
     uint64_t before[kCounters];
     copy_wait(before, B.counters.p, sizeof before, hipMemcpyDeviceToHost, s);

@@ -58,3 +58,20 @@ def test_capacity_of_queues_and_workspaces_is_enough(kind, n, k, catalogue, towe
     for key in ("ids", "meta", "interior", "level", "level_class"):
         assert np.array_equal(got[key], ref[key]), key
 
+
+def test_rescans_of_a_nearly_regular_cloud_fit_at_once(capfd, monkeypatch):
+    """Lattices displaced by 1% of their spacing leave several sides a point to
+    the rescans: where the capacity has room for them the list does not start
+    at one a point, which would run the enumeration twice."""
+    n = 6000
+    pts = workloads.jittered_lattice(n, side=19, sigma=0.01, seed=5)
+    monkeypatch.setenv("MHGP_TIMING", "1")
+    print(f"capacity: nearly regular lattice n={n}", flush=True)
+    with mhgp.Context(0, capacity_bytes=4 << 30) as ctx:
+        ctx.upload(pts)
+        capfd.readouterr()
+        ctx.supports(10, fetch=False)
+    lines = [ln for ln in capfd.readouterr().err.splitlines() if "sides left to the rescans" in ln]
+    most = int(lines[-1].split()[-1])
+    assert most > max(1 << 14, n), "the cloud no longer leaves sides to the rescans"
+    assert len(lines) == 1  # one run of the enumeration
