@@ -2301,9 +2301,10 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
     return std::max<uint64_t>(1ull << 30, std::min<uint64_t>(8ull << 30, free_b / 4));
   };
   // Probes `count` anchors of the device list in chunks whose slabs fit 2 GiB,
-  // each chunk enumerated before the next one takes its slabs.  Under a capacity
-  // slabs beyond those held grow into a quarter of what that leaves, at least
-  // probe_slabs_least.
+  // each chunk enumerated before the next one takes its slabs.  Slabs beyond
+  // those held grow into at most a quarter of the device memory still free
+  // (other contexts on the device keep theirs), under a capacity a quarter of
+  // what that leaves; at least probe_slabs_least.
   auto probe_lds = [&](const uint32_t *anchors, uint32_t count, uint32_t g) {
     const uint64_t slab = probe_slab_doubles(g), held = B.scratch.bytes();
     uint32_t per = 0;
@@ -2313,8 +2314,12 @@ void supports_device(Context &c, int k_max, std::vector<EventRec> &events,
       per = (count + chunks - 1) / chunks;
     };
     chunks_of(kProbeSlabs);
-    if (bounded && per * slab * 8 > held)
-      chunks_of(probe_slab_budget(c.capacity_bytes - device_bytes(c), held, probe_slabs_least(n), kProbeSlabs / 2));
+    if (per * slab * 8 > held) {
+      size_t free_b = 0, total_b = 0;
+      if (!bounded) MHGP_HIP(hipMemGetInfo(&free_b, &total_b));
+      chunks_of(bounded ? probe_slab_budget(c.capacity_bytes - device_bytes(c), held, probe_slabs_least(n), kProbeSlabs / 2)
+                        : probe_slab_budget((int64_t)free_b, held, probe_slabs_least(n), kProbeSlabs));
+    }
     B.scratch.ensure(slab * per);
     for (uint32_t a0 = 0; a0 < count; a0 += per) {
       Params Q = P;
