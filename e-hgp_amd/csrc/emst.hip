@@ -12,9 +12,10 @@
 // search, one wave per point -> per-component minima -> hooking with 2-cycle
 // breaking -> roots.  A point's nearest external point stays its nearest
 // while it is external (the external set only shrinks), so a search is run
-// again only for points whose last result was absorbed, and not at all when
-// that result's distance, a lower bound ever after, exceeds what another point
-// of the component already offers.  FP64 distances that are not provably
+// again only for points whose last result was absorbed or tied (what tied with
+// it may have been absorbed), and not at all when that result's distance, a
+// lower bound ever after, exceeds what another point of the component already
+// offers.  FP64 distances that are not provably
 // ordered (near ties that are not both exact) are flagged and settled on the
 // host with exact integer arithmetic.
 #include <algorithm>
@@ -94,12 +95,13 @@ __global__ void __launch_bounds__(kLabelBlock) k_group_labels(WaveTree T, Rounds
     if (!valid) continue;
     const uint32_t b = R.best_p[p];
     if (b == kInvalid) continue;
-    if (R.label[b] == l) {
-      R.best_p[p] = kInvalid;  // absorbed; its distance stays a lower bound
-    } else {
+    const bool external = R.label[b] != l;
+    if (external) {
       const uint64_t d = dbits(R.best_d[p]);
       if (d < R.comp_d[l]) atomicMin((unsigned long long *)&R.comp_d[l], (unsigned long long)d);
     }
+    // absorbed, or tied in its round: searched again; its distance stays a lower bound
+    if (!external || (R.best_flag[p] & 1)) R.best_p[p] = kInvalid;
   }
   __syncthreads();
   if (wave == 0) {
@@ -347,7 +349,7 @@ void emst_host(Context &c, uint32_t *edges_out) {
   const Rounds R{B.label.p,  B.node_label.p, B.best_v.p,  B.best_d.p,  B.best_flag.p,  B.comp_d.p, B.comp_e.p,
                  B.comp_amb.p, B.comp_cw.p,    B.comp_ce.p, B.hook.p,    B.next_label.p, B.edges.p,  B.counters.p};
   hipLaunchKernelGGL(k_start, G, B256, 0, s, n, R);
-  int64_t components = n;
+  int64_t components = n, settled = 0;
   for (int round = 0; components > 1; ++round) {
     if (round > 64) throw std::runtime_error("Borůvka did not converge");
     hipLaunchKernelGGL(k_group_labels, dim3(W.c1), dim3(kLabelBlock), 0, s, W, R);
@@ -380,6 +382,7 @@ void emst_host(Context &c, uint32_t *edges_out) {
       const std::vector<double> &xyz = c.host->xyz;
       for (int64_t l = 0; l < n; ++l) {
         if (!amb[l]) continue;
+        settled++;
         uint64_t best = ~0ull;
         for (int64_t u = 0; u < n; ++u) {
           if (label[u] != (uint32_t)l) continue;
@@ -395,6 +398,7 @@ void emst_host(Context &c, uint32_t *edges_out) {
     }
   }
   StageTimer tm(s);
+  if (tm.on) std::fprintf(stderr, "[mhgp] emst components settled on the host: %lld\n", (long long)settled);
   // kappa order: FP64 squared lengths sorted on the device; runs of values
   // within rounding of their neighbours are ordered exactly on the host
   const int64_t m = n - 1;

@@ -96,6 +96,20 @@ def test_emst_near_ties_of_kept_results():
     assert np.array_equal(e, ref)
 
 
+def test_emst_ties_of_absorbed_points_are_not_settled_again(capfd, monkeypatch):
+    """The same cloud: only the two components of the last round hold a tie.
+    Others' results tied in an earlier round with a point that has been
+    absorbed since; the host (quadratic in the component) need not see them."""
+    monkeypatch.setenv("MHGP_TIMING", "1")
+    print("emst: ties of absorbed points", flush=True)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(_kept_result_cloud())
+        capfd.readouterr()
+        ctx.emst()
+    lines = [ln for ln in capfd.readouterr().err.splitlines() if "settled on the host" in ln]
+    assert [int(ln.split()[-1]) for ln in lines] == [2]
+
+
 def test_emst_50k_lattice_weight():
     from scipy.sparse import coo_matrix
     from scipy.sparse.csgraph import minimum_spanning_tree
