@@ -661,21 +661,22 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
     }
   };
   std::vector<std::exception_ptr> lane_error(lanes);
-  std::vector<std::thread> others;
+  Threads others;  // a lane that gets no thread leaves its orders to the others
   for (int l = 1; l < lanes; ++l)
-    others.emplace_back([&, l] {
-      try {
-        lane(*c.tower_lanes[l - 1]);
-      } catch (...) {
-        lane_error[l] = std::current_exception();
-      }
-    });
+    if (!others.start([&, l] {
+          try {
+            lane(*c.tower_lanes[l - 1]);
+          } catch (...) {
+            lane_error[l] = std::current_exception();
+          }
+        }))
+      break;
   try {
     lane(W0);
   } catch (...) {
     lane_error[0] = std::current_exception();
   }
-  for (auto &t : others) t.join();
+  others.join();
   for (auto &e : lane_error)
     if (e) {
       for (auto &t : workers)

@@ -3,11 +3,10 @@
 
 #include <cmath>
 #include <cstdint>
-#include <functional>
-#include <thread>
 #include <vector>
 
 #include "stages.hpp"
+#include "threads.hpp"
 
 namespace mhgp {
 
@@ -115,17 +114,15 @@ struct TowerState {
   // copied before its threads would have started.
   template <class F>
   void each_order(F f) const {
-    std::vector<std::thread> th;
+    Threads th;
     int64_t nb = 0, cb = 0, below = 0;
     const bool small = node_count < 1 << 15;
     for (const Forest &G : forests) {
-      if (small) f(G, nb, cb, below);
-      else th.emplace_back(f, std::cref(G), nb, cb, below);
+      if (small || !th.start([=, &G] { f(G, nb, cb, below); })) f(G, nb, cb, below);
       below = nb;
       nb += (int64_t)G.order.size();
       cb += (int64_t)G.children.size();
     }
-    for (auto &t : th) t.join();
   }
 };
 
