@@ -270,3 +270,23 @@ def test_reused_context_one_point_cloud_has_an_empty_catalogue():
         ctx.upload(np.array([[1.0, 2.0, 3.0]]))
         cat = ctx.supports(4)
         assert cat.info.event_count == 0 and len(cat.size) == 0
+
+
+@pytest.mark.parametrize("n,k", [(1100, 4), (2300, 3)])
+def test_wide_gathers_take_the_slab_mask_probe(n, k, monkeypatch, capfd):
+    """The clouds of the agreement test above do reach the probe they are
+    meant for: its launches are counted in the timing trace."""
+    monkeypatch.setenv("MHGP_TIMING", "1")
+    pts = workloads.gaussian_mixture(n, blobs=3, noise_fraction=0.15, box=10.0, snap_bits=None, seed=43)
+    print(f"wide gathers: which probes, mixture n={n} k={k}", flush=True)
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        capfd.readouterr()
+        ctx.supports(k, fetch=False)
+    err = capfd.readouterr().err
+    wider = [int(ln.split()[-1]) for ln in err.splitlines() if "wide anchors" in ln]
+    big = [int(ln.split("big anchors:")[1].split(",")[0]) for ln in err.splitlines() if "big anchors:" in ln]
+    print(f"wider {wider} big {big}", flush=True)
+    assert sum(wider) > 0
+    if n > 2048:
+        assert sum(big) > 0
