@@ -1,5 +1,7 @@
 """Canonical cloud, exact Morton LBVH snapshot and k-NN on the GPU vs the oracle."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -162,3 +164,28 @@ def test_snapshot_totals_of_equal_codes(runs):
             if child != 0xFFFFFFFFFFFFFFFF:
                 depth[int(child)] = depth[i] + 1
     assert counters[2] == depth.max()
+
+
+def test_a_run_that_needs_the_full_sort_is_not_built_twice():
+    """Half the points in one cell of the coarse key: in lexicographic source
+    order the coarse sort leaves them in order, shuffled they need the sort of
+    the full coordinates.  That sort costs a few tenths of a millisecond; the
+    leaves of equal codes (milliseconds here) must not be made for both."""
+    rng = np.random.default_rng(4)
+    pts = rng.uniform(size=(50_000, 3))
+    pts[:25_000] *= 1e-8
+    pts = pts[np.lexsort((pts[:, 2], pts[:, 1], pts[:, 0]))]
+    print("upload of 25 000 points in one cell, in order and shuffled", flush=True)
+    best = []
+    for cloud in (pts, pts[rng.permutation(len(pts))]):
+        with mhgp.Context(0) as ctx:
+            times = []
+            for _ in range(8):
+                start = time.perf_counter()
+                ctx.upload(cloud)
+                times.append(time.perf_counter() - start)
+            xyz, _ = ctx.canonical_points()
+        assert np.array_equal(xyz, pts)
+        best.append(min(times))
+    print(f"in order {best[0] * 1e3:.2f} ms, shuffled {best[1] * 1e3:.2f} ms", flush=True)
+    assert best[1] < 1.4 * best[0]
