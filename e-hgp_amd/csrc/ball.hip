@@ -102,9 +102,9 @@ __global__ void __launch_bounds__(kBallBlock) k_closed_ball(BallParams B) {
   const bool in_lanes = B.cap <= 64;
   uint32_t list = kInvalid, rmax = kInvalid;
   const WaveTree &T = B.tree;
-  const WaveQuery Q(T, o.x, o.y, o.z, off.x, off.y, off.z);
-  float Tf = Q.bound(R2);
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  const WaveOffsetQuery Q(o.x, o.y, o.z, off.x, off.y, off.z);
+  double most = wave_bound(R2);
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const V3 p = sub({T.LX[at], T.LY[at], T.LZ[at]}, o), d = sub(p, off);
     bool near = lp < T.n && !(dot(d, d) > R2);

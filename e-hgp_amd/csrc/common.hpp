@@ -100,15 +100,14 @@ static_assert(sizeof(WideNode) == 128, "wide node layout");
 
 // Box of a wave-tree group and the tree itself (wave_tree.hpp).
 struct alignas(16) GroupBox {
-  float lo[3], pad0, hi[3], pad1;
+  double lo[3], hi[3];
 };
-static_assert(sizeof(GroupBox) == 32, "group box layout");
+static_assert(sizeof(GroupBox) == 48, "group box layout");
 
 struct WaveTree {
   const GroupBox *l0, *l1, *l2;
   uint32_t c0, c1, c2;  // groups per level
   uint32_t n;           // leaves
-  double centre[3];
   const double *LX, *LY, *LZ;
   const uint32_t *leaf_id;
 };

@@ -62,8 +62,7 @@ struct Context {
   DevBuf<uint32_t> wit;       // 6 witnesses per internal node (lo xyz, hi xyz)
   DevBuf<uint64_t> snapshot;  // a fetched snapshot on its way out
   DevBuf<WideNode> wide;      // FP32 two-level copy of the internal nodes (ball and k-NN queries)
-  DevBuf<GroupBox> groups;    // wave tree: level 0, 1 and 2 boxes (wave_tree.hpp), relative to centre
-  double centre[3] = {0, 0, 0};
+  DevBuf<GroupBox> groups;    // wave tree: level 0, 1 and 2 boxes (wave_tree.hpp)
   DevBuf<uint8_t> group_exact;  // the groups' exact boxes with witnesses (lbvh.hip)
   RadixSorter sorter;
   Scanner scanner;

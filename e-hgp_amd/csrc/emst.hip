@@ -134,12 +134,12 @@ __global__ void __launch_bounds__(kSearchBlock) k_search(WaveTree T, Rounds R) {
   if (R.best_d[p] > limit) return;
   const uint32_t u = T.leaf_id[p];
   const double q[3] = {T.LX[p], T.LY[p], T.LZ[p]};
-  const WaveQuery Q(T, q[0], q[1], q[2]);
+  const WaveQuery Q(q[0], q[1], q[2]);
   double bd = INFINITY;
   uint32_t bp = kInvalid, bv = kInvalid;
   bool bx = true, near_tie = false;
   double bound = offer * (1.0 + 4.0 * kSlack) + 4.0 * kSlackAbs;  // >= limit * (1 + kSlack) + kSlackAbs
-  float Tf = Q.bound(bound);
+  double most = wave_bound(bound);
   auto group = [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const bool valid = lp < T.n && R.label[at] != lu;
@@ -164,13 +164,13 @@ __global__ void __launch_bounds__(kSearchBlock) k_search(WaveTree T, Rounds R) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o));
     bound = fmin(bound, m * (1.0 + kSlack) + kSlackAbs);
-    Tf = Q.bound(bound);
+    most = wave_bound(bound);
   };
   const uint32_t own = p >> 6;
   if (R.glabel[own] == kInvalid) group(own);
   const uint32_t *gl = R.glabel;
   wave_tree_visit(
-      T, Q, Tf,
+      T, Q, most,
       [&](int level, uint32_t i) { return gl[(level == 0 ? 0u : level == 1 ? T.c0 : T.c0 + T.c1) + i] != lu; },
       [&](uint32_t g) {
         if (g != own) group(g);

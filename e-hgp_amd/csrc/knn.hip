@@ -37,12 +37,12 @@ __global__ void __launch_bounds__(kKnnBlock) k_knn(WaveTree T, int k, uint32_t *
   const int kk = min(k + 1, (int)T.n - 1);  // slots that decide (k, plus one tie probe)
   const uint32_t self = T.leaf_id[p];
   const double q[3] = {T.LX[p], T.LY[p], T.LZ[p]};
-  const WaveQuery Q(T, q[0], q[1], q[2]);
+  const WaveQuery Q(q[0], q[1], q[2]);
   double bd = INFINITY;
   uint32_t bi = kInvalid;
   uint32_t bx = 0;         // 1: the distance is exact
   double cut = INFINITY;   // squared distance of the kk-th best so far
-  float Tf = INFINITY;
+  double most = INFINITY;
   auto group = [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const uint32_t id = T.leaf_id[at];
@@ -66,11 +66,11 @@ __global__ void __launch_bounds__(kKnnBlock) k_knn(WaveTree T, int k, uint32_t *
       cut = lane_f64(bd, kk - 1);
       cand &= __ballot(d <= cut);
     }
-    Tf = Q.bound(cut * (1.0 + kSlack) + kSlackAbs);
+    most = wave_bound(cut);
   };
   const uint32_t own = p >> 6;
   group(own);
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     if (g != own) group(g);
   });
   const double nd = __shfl_down(bd, 1u);
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(kPartBlock) k_knn_partition(PartParams P) {
     return x;
   };
   const double qq[3] = {P.q[3 * q], P.q[3 * q + 1], P.q[3 * q + 2]};
-  const WaveQuery Q(T, qq[0], qq[1], qq[2]);
+  const WaveQuery Q(qq[0], qq[1], qq[2]);
   const int k = P.k;
   auto distance = [&](uint32_t at) {
     const double dx = T.LX[at] - qq[0], dy = T.LY[at] - qq[1], dz = T.LZ[at] - qq[2];
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(kPartBlock) k_knn_partition(PartParams P) {
   };
   // pass 1: the FP64 k-th smallest squared distance over eligible points
   double bd = INFINITY, cut = INFINITY;
-  float Tf = INFINITY;
+  double most = INFINITY;
   auto group = [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const double d = distance(at);
@@ -161,11 +161,11 @@ __global__ void __launch_bounds__(kPartBlock) k_knn_partition(PartParams P) {
       cut = lane_f64(bd, k - 1);
       cand &= __ballot(d < cut);
     }
-    Tf = Q.bound(cut * (1.0 + kSlack) + kSlackAbs);
+    most = wave_bound(cut);
   };
   const uint32_t first = wave_near_group(T, Q);
   group(first);
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     if (g != first) group(g);
   });
   if (!(cut < INFINITY)) {
@@ -180,8 +180,8 @@ __global__ void __launch_bounds__(kPartBlock) k_knn_partition(PartParams P) {
   const double R = (rk * (1.0 + 1e-12) + 2.0 * P.slack[q]) * (1.0 + 1e-12) + 1e-300;
   const double R2 = R * R * (1.0 + 1e-12);
   uint32_t nc = 0;
-  Tf = Q.bound(R2 * (1.0 + kSlack) + kSlackAbs);
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  most = wave_bound(R2);
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     bool in = lp < T.n && !(distance(at) > R2);
     if (!__ballot(in)) return;

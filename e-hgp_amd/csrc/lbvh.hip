@@ -586,17 +586,15 @@ __global__ void k_wide_nodes(int64_t m, const Node *__restrict__ nodes, const do
   out[i] = w;
 }
 
-// Wave-tree boxes (wave_tree.hpp) of levels 0 and 1 from the exact group
-// boxes, in the unit 2^e, relative to the centre and rounded outward.
-__global__ void k_wave_boxes(int64_t count, const Box *__restrict__ in, int e, double cx, double cy, double cz,
-                             GroupBox *out) {
+// Wave-tree boxes (wave_tree.hpp) of levels 0 and 1 from the boxes with
+// witnesses, in the unit 2^e.
+__global__ void k_wave_boxes(int64_t count, const Box *__restrict__ in, int e, GroupBox *out) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= count) return;
-  const double c[3] = {cx, cy, cz};
-  GroupBox b{};
+  GroupBox b;
   for (int a = 0; a < 3; ++a) {
-    b.lo[a] = __double2float_rd(ldexp(in[g].v[a], e) - c[a]);
-    b.hi[a] = __double2float_ru(ldexp(in[g].v[3 + a], e) - c[a]);
+    b.lo[a] = ldexp(in[g].v[a], e);
+    b.hi[a] = ldexp(in[g].v[3 + a], e);
   }
   out[g] = b;
 }
@@ -604,7 +602,7 @@ __global__ void k_wave_boxes(int64_t count, const Box *__restrict__ in, int e, d
 // Level-2 boxes, one wave per group (clouds of more than 262 144 points).
 __global__ void __launch_bounds__(64) k_group_top(uint32_t c1, const GroupBox *__restrict__ l1, GroupBox *l2) {
   const uint32_t i = blockIdx.x * 64 + threadIdx.x;
-  float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
   if (i < c1)
     for (int a = 0; a < 3; ++a) {
       v[a] = l1[i].lo[a];
@@ -614,10 +612,10 @@ __global__ void __launch_bounds__(64) k_group_top(uint32_t c1, const GroupBox *_
   for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      v[a] = fminf(v[a], __shfl_xor(v[a], o));
-      v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o));
+      v[a] = fmin(v[a], __shfl_xor(v[a], o));
+      v[3 + a] = fmax(v[3 + a], __shfl_xor(v[3 + a], o));
     }
-  if (threadIdx.x == 0) l2[blockIdx.x] = GroupBox{{v[0], v[1], v[2]}, 0.f, {v[3], v[4], v[5]}, 0.f};
+  if (threadIdx.x == 0) l2[blockIdx.x] = GroupBox{{v[0], v[1], v[2]}, {v[3], v[4], v[5]}};
 }
 
 // Power-of-two change of unit (context.hpp, scale_exp): possible only when
@@ -768,10 +766,8 @@ void canonicalize_and_build(Context &c) {
                        c.LY.p, c.LZ.p, c.wide.p);
   const int64_t c0 = (n + 63) / 64, c1 = (c0 + 63) / 64, c2 = (c1 + 63) / 64;
   c.groups.ensure(c0 + c1 + c2);
-  for (int a = 0; a < 3; ++a) c.centre[a] = std::ldexp(0.5 * bounds[a] + 0.5 * bounds[3 + a], c.scale_exp);
   hipLaunchKernelGGL(k_wave_boxes, dim3(blocks_for(c0 + c1, 256)), dim3(256), 0, s, c0 + c1,
-                     reinterpret_cast<const Box *>(c.group_exact.p), c.scale_exp, c.centre[0], c.centre[1],
-                     c.centre[2], c.groups.p);
+                     reinterpret_cast<const Box *>(c.group_exact.p), c.scale_exp, c.groups.p);
   if (c2 > 1)
     hipLaunchKernelGGL(k_group_top, dim3(c2), dim3(64), 0, s, (uint32_t)c1, c.groups.p + c0, c.groups.p + c0 + c1);
   MHGP_LAUNCH_CHECK();
@@ -781,7 +777,7 @@ void canonicalize_and_build(Context &c) {
 WaveTree wave_tree(const Context &c) {
   const uint32_t n = (uint32_t)c.n, c0 = (n + 63) / 64, c1 = (c0 + 63) / 64, c2 = (c1 + 63) / 64;
   return {c.groups.p, c.groups.p + c0, c.groups.p + c0 + c1, c0, c1, c2, n,
-          {c.centre[0], c.centre[1], c.centre[2]}, c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p};
+          c.LX.p, c.LY.p, c.LZ.p, c.leaf_id.p};
 }
 
 void canonical_points(Context &c, double *xyz_out, uint32_t *source_index_out) {

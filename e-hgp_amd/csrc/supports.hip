@@ -1976,11 +1976,11 @@ __global__ void __launch_bounds__(kGatherBlock) k_gather(WaveTree T, const uint3
   const double q[3] = {T.LX[p], T.LY[p], T.LZ[p]};
   const double R = radius[u];
   const double R2 = R * R * (1.0 + 1e-9);
-  const WaveQuery Q(T, q[0], q[1], q[2]);
-  float Tf = Q.bound(R2);
+  const WaveQuery Q(q[0], q[1], q[2]);
+  double most = wave_bound(R2);
   const uint64_t base = EMIT ? goff[u] : 0;
   uint32_t cnt = 0;
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const double dx = T.LX[at] - q[0], dy = T.LY[at] - q[1], dz = T.LZ[at] - q[2];
     const bool hit = lp < T.n && lp != p && dx * dx + dy * dy + dz * dz <= R2;
@@ -2004,12 +2004,13 @@ __global__ void __launch_bounds__(kRadiusBlock) k_knn_radius(WaveTree T, int kq,
   if (p >= T.n) return;
   const double x = T.LX[p], y = T.LY[p], z = T.LZ[p];
   const float q[3] = {(float)x, (float)y, (float)z};
-  const WaveQuery Q(T, x, y, z);
+  const WaveQuery Q(x, y, z);
   // the differences are taken in the input's frame, whose FP32 rounding
   // (query half an ulp, box one ulp per axis) can bring a point nearer by up
   // to this much
   const float off = 3.5e-7f * fmaxf(fmaxf(fabsf(q[0]), fabsf(q[1])), fabsf(q[2]));
-  float best = INFINITY, cut = INFINITY, Tf = INFINITY;
+  float best = INFINITY, cut = INFINITY;
+  double most = INFINITY;
   auto group = [&](uint32_t g) {
     const uint32_t lp = g * 64 + lane, at = min(lp, T.n - 1);
     const double v[3] = {T.LX[at], T.LY[at], T.LZ[at]};
@@ -2033,11 +2034,11 @@ __global__ void __launch_bounds__(kRadiusBlock) k_knn_radius(WaveTree T, int kq,
       cand &= __ballot(d2 < cut);
     }
     const double r = sqrt((double)cut) * (1.0 + 1e-6) + (double)off;
-    Tf = cut > 0.f ? Q.bound(r * r) : -1.f;  // nothing enters below a zero distance
+    most = cut > 0.f ? wave_bound(r * r) : -1.0;  // nothing enters below a zero distance
   };
   const uint32_t own = p >> 6;
   group(own);
-  wave_tree_visit(T, Q, Tf, [&](uint32_t g) {
+  wave_tree_visit(T, Q, most, [&](uint32_t g) {
     if (g != own) group(g);
   });
   if (lane == 0) radius[T.leaf_id[p]] = (double)factor * (sqrt((double)cut) * (1.0 + 1e-6));

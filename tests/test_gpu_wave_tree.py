@@ -3,6 +3,8 @@ leaves, 64 groups, 262 144 leaves per top group): neighbour lists against the
 exact oracle, and against sorted FP64 distances where the oracle's full scan
 would be long."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,32 @@ def test_neighbour_lists_across_top_groups(offset):
         near = np.argsort(d, kind="stable")[: k + 1]
         # distances of a random cloud are distinct far beyond the rounding of the sums
         assert np.array_equal(ids[u], near[:k]), u
+
+
+def test_a_far_outlier_does_not_slow_the_others():
+    """One point a million times the cloud's extent away: the boxes still tell
+    the others apart.  (Where they cannot, each query looks at every point: 25
+    times as long at this size.  The outlier itself costs about a factor of two:
+    the others share a few Morton cells, so their groups are slabs.)"""
+    n, k = 200_000, 8
+    pts = workloads.uniform_cloud(n, seed=12)
+    far = pts.copy()
+    far[5] = [1.0e6, 0.0, 0.0]
+    print(f"wave tree: knn n={n} with a far outlier", flush=True)
+    best = []
+    for cloud in (pts, far):
+        with mhgp.Context(0) as ctx:
+            ctx.upload(cloud)
+            times = []
+            for _ in range(5):
+                start = time.perf_counter()
+                ids = ctx.knn(k)
+                times.append(time.perf_counter() - start)
+            xyz, _ = ctx.canonical_points()
+        best.append(min(times))
+    print(f"without {best[0] * 1e3:.2f} ms, with {best[1] * 1e3:.2f} ms", flush=True)
+    for u in np.random.default_rng(1).integers(0, n - 1, size=8):
+        d = ((xyz - xyz[u]) ** 2).sum(1)
+        d[u] = np.inf
+        assert np.array_equal(ids[u], np.argsort(d, kind="stable")[:k]), u
+    assert best[1] < 6.0 * best[0]
