@@ -21,6 +21,9 @@
 //               well-centred <=> N.(b x d), N.(d x a), N.(a x b) > 0 and
 //               2 V^2 - N.(b x d) - N.(d x a) - N.(a x b) > 0
 //               P = V (V pp - p.N),  r^2 = |N|^2 / (4 V^2)
+// What a level is made of is written as explicit fused chains, so that a
+// support's level is the same double from every kernel and on the host (left to
+// the compiler, one copy of a function contracts another product than the next).
 // (circumcentre in the affine hull and barycentric well-centring as in the
 // reference's exact/center.hpp:263-340 and exact/support.hpp:41-135).
 #pragma once
@@ -48,12 +51,15 @@ __host__ __device__ inline int cert_sign(double v, double vabs) {
 struct V3 {
   double x, y, z;
 };
-__host__ __device__ inline double dot(const V3 &a, const V3 &b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__host__ __device__ inline double dot(const V3 &a, const V3 &b) {
+  return __builtin_fma(a.z, b.z, __builtin_fma(a.x, b.x, a.y * b.y));
+}
 __host__ __device__ inline double adot(const V3 &a, const V3 &b) {
   return fabs(a.x * b.x) + fabs(a.y * b.y) + fabs(a.z * b.z);
 }
 __host__ __device__ inline V3 cross(const V3 &a, const V3 &b) {
-  return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+  return {__builtin_fma(a.y, b.z, -(a.z * b.y)), __builtin_fma(a.z, b.x, -(a.x * b.z)),
+          __builtin_fma(a.x, b.y, -(a.y * b.x))};
 }
 __host__ __device__ inline V3 across(const V3 &a, const V3 &b) {
   return {fabs(a.y * b.z) + fabs(a.z * b.y), fabs(a.z * b.x) + fabs(a.x * b.z),
@@ -86,7 +92,7 @@ struct TriSphere {
     bb = dot(b, b);
     ab = dot(a, b);
     abA = adot(a, b);
-    D = aa * bb - ab * ab;
+    D = __builtin_fma(-ab, ab, aa * bb);
     DA = aa * bb + abA * abA;
     al = bb * (aa - ab);
     alA = bb * (aa + abA);
@@ -138,12 +144,12 @@ struct TetSphere {
     d = vd;
     V3 bxd = cross(b, d), dxa = cross(d, a), axb = cross(a, b);
     V3 bxdA = across(b, d), dxaA = across(d, a), axbA = across(a, b);
-    V = dot(a, bxd);
+    V = __builtin_fma(a.z, bxd.z, __builtin_fma(a.y, bxd.y, a.x * bxd.x));
     VA = adot(vabs(a), bxdA);
     if (cert_sign(V, VA) == 0) return 0;
     double aa = dot(a, a), bb = dot(b, b), dd = dot(d, d);
-    N = {aa * bxd.x + bb * dxa.x + dd * axb.x, aa * bxd.y + bb * dxa.y + dd * axb.y,
-         aa * bxd.z + bb * dxa.z + dd * axb.z};
+    auto sum = [&](double x, double y, double z) { return __builtin_fma(dd, z, __builtin_fma(bb, y, aa * x)); };
+    N = {sum(bxd.x, dxa.x, axb.x), sum(bxd.y, dxa.y, axb.y), sum(bxd.z, dxa.z, axb.z)};
     NA = {aa * bxdA.x + bb * dxaA.x + dd * axbA.x, aa * bxdA.y + bb * dxaA.y + dd * axbA.y,
           aa * bxdA.z + bb * dxaA.z + dd * axbA.z};
     double nv = dot(N, bxd), nw = dot(N, dxa), nz = dot(N, axb);
