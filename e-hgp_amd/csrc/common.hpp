@@ -89,7 +89,7 @@ static_assert(sizeof(Node) == 64, "node layout");
 
 constexpr uint32_t kLeafBit = 0x80000000u;
 
-// LBVH internal node for FP32 ball queries, two levels collapsed into one
+// LBVH internal node for the descents' FP32 ball queries, two levels collapsed into one
 // 128-byte line: the node's grandchildren (or a child that is a leaf), their
 // boxes rounded outward, children as in Node::left/right (kInvalid: none).
 struct alignas(128) WideNode {

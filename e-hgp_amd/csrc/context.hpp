@@ -20,8 +20,9 @@ struct TowerWork;        // tower_gpu.hpp
 struct Context {
   int device = 0;
   int64_t capacity_bytes = 0;  // device memory bound of the context (0: none)
-  // device lanes of the tower (streams with their own workspaces); a server
-  // slot uses one, since the server already overlaps whole requests
+  // device lanes of the tower (streams with their own workspaces), more where
+  // its orders hold few records (tower.cpp); a server slot uses one, since the
+  // server already overlaps whole requests
   int tower_lane_count = 2;
   hipStream_t stream = nullptr;
   bool poisoned = false;
@@ -61,7 +62,7 @@ struct Context {
   DevBuf<uint32_t> parent_int, parent_leaf;
   DevBuf<uint32_t> wit;       // 6 witnesses per internal node (lo xyz, hi xyz)
   DevBuf<uint64_t> snapshot;  // a fetched snapshot on its way out
-  DevBuf<WideNode> wide;      // FP32 two-level copy of the internal nodes (ball and k-NN queries)
+  DevBuf<WideNode> wide;      // FP32 two-level copy of the internal nodes (the descents' slow steps)
   DevBuf<GroupBox> groups;    // wave tree: level 0, 1 and 2 boxes (wave_tree.hpp)
   DevBuf<uint8_t> group_exact;  // the groups' exact boxes with witnesses (lbvh.hip)
   RadixSorter sorter;

@@ -1,4 +1,5 @@
-// k nearest neighbours (k <= 32) of every data point by LBVH traversal.
+// k nearest neighbours (up to 63; the public call up to 32) of every data point
+// over the wave tree, and top-k partitions of rational points.
 //
 // Semantics follow the reference's exact top-k (morsehgp3d/src/cpu/spatial/
 // lbvh.cpp:1098-1198 lbvh_top_k): neighbours ordered by exact squared distance,
@@ -6,7 +7,7 @@
 // per query, queries taken in Morton order so that neighbouring waves read
 // the same groups.  Distances are FP64; a pair of candidates whose values
 // are within rounding of each other and not both exact is reported in
-// tie_flags so that the host can settle the order exactly.
+// `flags` so that the host can settle the order exactly.
 #include <algorithm>
 #include <cmath>
 

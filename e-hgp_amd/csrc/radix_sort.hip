@@ -211,7 +211,10 @@ __global__ void __launch_bounds__(kSortBlock) rs_scatter(const uint64_t *__restr
 // share of the keys, which it reads with uniform addresses.  n^2 comparisons
 // spread over the chip cost less than the 91 barriers of one workgroup's
 // bitonic sort of 8 192 keys: the three sorts of a 256-point catalogue (256,
-// 256 and 4 790 keys) 126 -> 44 us.
+// 256 and 4 790 keys) 126 -> 44 us.  Against the passes, by builds of uniform
+// clouds (two sorts each): 2 048 points 194 and 314 us, 4 096 227 and 330,
+// 8 192 271 and 339, 12 000 314 and 345, 16 384 356 and 347; the line leaves
+// what a chip shared with other streams costs the counting.
 __global__ void __launch_bounds__(kSmallBlock) rs_rank(const uint64_t *__restrict__ keys, const uint32_t *__restrict__ vals,
                                                        int n, int shift, uint64_t mask, uint64_t *__restrict__ kout,
                                                        uint32_t *__restrict__ vout) {

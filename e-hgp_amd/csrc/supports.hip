@@ -1490,7 +1490,9 @@ __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t 
 // 48 KB then remain, three workgroups a CU).  Such gathers took the
 // global-memory kernel, whose 256 lanes scan all points for 384 cells and whose
 // regions are not in increasing distance: 2 003-point mixture, 1 531 such
-// anchors, catalogue 29.8 -> 26.0 ms.
+// anchors, catalogue 29.8 -> 26.0 ms.  Up to 4 096 points (98 KB, one workgroup a
+// CU) it is no better: mixtures of 2 003, 3 000 and 4 000 points, K 10, 21.3,
+// 130.5 and 459 ms with 2 048, 25.1, 126.8 and 486 with 4 096.
 constexpr int kProbeBlock = kCells;
 template <int GCAP, bool SLAB>
 __global__ void __launch_bounds__(kProbeBlock) k_anchor_probe(Params P) {

@@ -536,9 +536,10 @@ void tower(Context &c, int k_max, mhgp_tower_info *info) {
   std::mutex mu;  // workers, the host descender
   // Vertical maps of the order pair (o -> o - 1) need both orders contracted:
   // whichever of the two contractions finishes last runs the pair, while the
-  // lanes go on with the orders below.  The element gathers share the first
-  // lane's scratch (sized here for every order, so that no buffer is freed
-  // while the lanes run) and take turns.
+  // lanes go on with the orders below.  The pairs share the first lane's
+  // scratch and take turns: the element gathers' is sized here for every order,
+  // that of the device targets (as large as the forests turn out) grows with
+  // the first towers of a context, each time waiting for the lanes' kernels.
   std::vector<char> contracted(K + 2, 0), pair_done(K + 2, 0);
   std::mutex vm_mu, vm_gather_mu;
   {

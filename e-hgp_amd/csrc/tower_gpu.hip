@@ -216,7 +216,6 @@ __device__ inline void load_label(const Saddles &D, uint32_t s, uint32_t (&L)[K 
 
 struct ArmParams {
   Saddles sad;
-  const uint32_t *sizes;       // inclusive scan of the arm counts
   int64_t saddles;
   MinimaTable table;
   const double *X, *Y, *Z;
@@ -1582,7 +1581,6 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
                      arm_saddle.p);
   ArmParams A{};
   A.sad = sad;
-  A.sizes = sizes.p;
   A.saddles = S;
   A.table = table;
   A.X = c.X.p; A.Y = c.Y.p; A.Z = c.Z.p;

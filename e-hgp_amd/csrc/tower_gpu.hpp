@@ -113,9 +113,12 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
 void tower_vm_gather(Context &c, const std::vector<uint32_t> &pos, std::vector<uint32_t> &out);
 // Vertical targets of an order pair on the device, from the two forests and
 // the elements by rank-index position (base, span: order o's minima); false
-// below kVerticalOnDevice nodes, where the host's sweep is faster than some
-// twenty launches and seven copies (one caller at a time, as the gather).
-// 500 000 nodes: 16 ms on the host, 1.3 here.
+// below kVerticalOnDevice nodes (one caller at a time, as the gather).  Up to
+// 18 000 nodes the host's sweep is faster than some twenty launches and seven
+// copies (0.1-0.6 ms against 0.1-0.5); between, which is faster depends on what
+// the lanes do beside it (24 000 nodes 0.7 ms on the host and 0.3 here, 36 000
+// 1.0 and 0.4, 34 000 beside a longer order 1.1 and 0.8, 50 000 0.6 and 0.7);
+// beyond, the device is (70 000 nodes 1.6 and 0.3, 500 000 16 and 1.3).
 struct Forest;
 constexpr int64_t kVerticalOnDevice = 1 << 16;
 bool tower_vm_targets(Context &c, const Forest &S, const Forest &T, uint32_t base, uint32_t span,
