@@ -386,11 +386,15 @@ struct SupSphere {
   }
 };
 
-// 1 / x from the hardware estimate (about 24 bits) and one Newton step.
+// 1 / x: the hardware's estimate, in FP64 (about 24 bits of it) with one Newton
+// step.
+__device__ inline float reciprocal(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline double reciprocal(double x) {
   const double r = __builtin_amdgcn_rcp(x);
   return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
 }
+__device__ inline float at_least_0(float x) { return fmaxf(x, 0.0f); }
+__device__ inline double at_least_0(double x) { return fmax(x, 0.0); }
 
 // Support of the smallest ball holding K points, by walking a centre: T are
 // points on the ball's boundary; the centre moves towards its projection onto
@@ -400,28 +404,29 @@ __device__ inline double reciprocal(double x) {
 // (K. Fischer, B. Gaertner, M. Kutz, Fast Smallest-Enclosing-Ball Computation in
 // High Dimensions, ESA 2003.)  Every lane does the same work per move, unlike
 // Welzl's nested restarts.  The result is a proposal, certified by the caller.
-// FP64: in FP32 the time is the same (50 000-point pipeline 98.0 and 98.8 ms,
-// its runs 2.7% apart), but nearly cospherical facets fail the certificate (a
-// 1 000-point lattice displaced by 1e-7 of its spacing: 4 645 of 25 496 steps).
+// T: float first, whose supports of nearly cospherical facets fail the
+// certificate (a 1 000-point lattice displaced by 1e-7 of its spacing: 4 645 of
+// 25 496 steps); those walk again in double.  In double at once k_descend takes
+// 225 instead of 168 VGPRs at order 10 and 1.3 times as long.
 // Returns the size of the support (positions in at[]), 0 when the walk does not
 // settle.
-template <int K>
-__device__ inline int walk_miniball(const double (&x)[K], const double (&y)[K], const double (&z)[K], int (&at)[4]) {
-  double cx = 0.0, cy = 0.0, cz = 0.0;
+template <int K, class T>
+__device__ inline int walk_miniball(const T (&x)[K], const T (&y)[K], const T (&z)[K], int (&at)[4]) {
+  T cx = 0, cy = 0, cz = 0;
 #pragma unroll
   for (int i = 0; i < K; ++i) {
     cx += x[i];
     cy += y[i];
     cz += z[i];
   }
-  cx *= 1.0 / K;
-  cy *= 1.0 / K;
-  cz *= 1.0 / K;
-  double far = -1.0;
-  double tx[4] = {}, ty[4] = {}, tz[4] = {};
+  cx *= (T)(1.0 / K);
+  cy *= (T)(1.0 / K);
+  cz *= (T)(1.0 / K);
+  T far = -1;
+  T tx[4] = {}, ty[4] = {}, tz[4] = {};
 #pragma unroll
   for (int i = 0; i < K; ++i) {
-    const double dx = x[i] - cx, dy = y[i] - cy, dz = z[i] - cz, d = dx * dx + dy * dy + dz * dz;
+    const T dx = x[i] - cx, dy = y[i] - cy, dz = z[i] - cz, d = dx * dx + dy * dy + dz * dz;
     const bool take = d > far;
     far = take ? d : far;
     at[0] = take ? i : at[0];
@@ -433,48 +438,48 @@ __device__ inline int walk_miniball(const double (&x)[K], const double (&y)[K], 
   uint32_t in = 1u << at[0];
 #pragma unroll 1
   for (int it = 0; it < 24; ++it) {
-    const double wx = cx - tx[0], wy = cy - ty[0], wz = cz - tz[0];
-    double la = 0.0, lb = 0.0, lc = 0.0;
-    const double ux = tx[1] - tx[0], uy = ty[1] - ty[0], uz = tz[1] - tz[0];
-    const double vx = tx[2] - tx[0], vy = ty[2] - ty[0], vz = tz[2] - tz[0];
-    double qx = tx[0], qy = ty[0], qz = tz[0];
+    const T wx = cx - tx[0], wy = cy - ty[0], wz = cz - tz[0];
+    T la = 0, lb = 0, lc = 0;
+    const T ux = tx[1] - tx[0], uy = ty[1] - ty[0], uz = tz[1] - tz[0];
+    const T vx = tx[2] - tx[0], vy = ty[2] - ty[0], vz = tz[2] - tz[0];
+    T qx = tx[0], qy = ty[0], qz = tz[0];
     if (m == 2) {
       la = (wx * ux + wy * uy + wz * uz) * reciprocal(ux * ux + uy * uy + uz * uz);
     } else if (m >= 3) {
       // solved with the normal of the first three points
-      const double nx = uy * vz - uz * vy, ny = uz * vx - ux * vz, nz = ux * vy - uy * vx;
+      const T nx = uy * vz - uz * vy, ny = uz * vx - ux * vz, nz = ux * vy - uy * vx;
       if (m == 3) {
-        const double in2 = reciprocal(nx * nx + ny * ny + nz * nz);
+        const T in2 = reciprocal(nx * nx + ny * ny + nz * nz);
         // w x v . n and u x w . n
         la = ((wy * vz - wz * vy) * nx + (wz * vx - wx * vz) * ny + (wx * vy - wy * vx) * nz) * in2;
         lb = ((uy * wz - uz * wy) * nx + (uz * wx - ux * wz) * ny + (ux * wy - uy * wx) * nz) * in2;
       } else {
-        const double ex = tx[3] - tx[0], ey = ty[3] - ty[0], ez = tz[3] - tz[0];
-        const double id = reciprocal(ex * nx + ey * ny + ez * nz);
+        const T ex = tx[3] - tx[0], ey = ty[3] - ty[0], ez = tz[3] - tz[0];
+        const T id = reciprocal(ex * nx + ey * ny + ez * nz);
         lc = (wx * nx + wy * ny + wz * nz) * id;
-        const double rx = wx - lc * ex, ry = wy - lc * ey, rz = wz - lc * ez;
-        const double in2 = reciprocal(nx * nx + ny * ny + nz * nz);
+        const T rx = wx - lc * ex, ry = wy - lc * ey, rz = wz - lc * ez;
+        const T in2 = reciprocal(nx * nx + ny * ny + nz * nz);
         la = ((ry * vz - rz * vy) * nx + (rz * vx - rx * vz) * ny + (rx * vy - ry * vx) * nz) * in2;
         lb = ((uy * rz - uz * ry) * nx + (uz * rx - ux * rz) * ny + (ux * ry - uy * rx) * nz) * in2;
       }
     }
-    double step = 1.0;
+    T step = 1;
     int hit = -1;
-    double hx = 0.0, hy = 0.0, hz = 0.0;
+    T hx = 0, hy = 0, hz = 0;
     if (m < 4) {
       qx += la * ux + lb * vx;
       qy += la * uy + lb * vy;
       qz += la * uz + lb * vz;
-      const double dx = qx - cx, dy = qy - cy, dz = qz - cz;
-      const double ww = wx * wx + wy * wy + wz * wz;
+      const T dx = qx - cx, dy = qy - cy, dz = qz - cz;
+      const T ww = wx * wx + wy * wy + wz * wz;
 #pragma unroll
       for (int i = 0; i < K; ++i) {
-        const double px = cx - x[i], py = cy - y[i], pz = cz - z[i];
+        const T px = cx - x[i], py = cy - y[i], pz = cz - z[i];
         // 2 d . (t0 - p), the rate at which p nears the boundary
-        const double rate = 2.0 * (dx * (px - wx) + dy * (py - wy) + dz * (pz - wz));
-        const double gap = ww - (px * px + py * py + pz * pz);
-        const double t = fmax(gap, 0.0) * reciprocal(rate);
-        const bool take = rate > 0.0 && t < step && !((in >> i) & 1u);
+        const T rate = 2 * (dx * (px - wx) + dy * (py - wy) + dz * (pz - wz));
+        const T gap = ww - (px * px + py * py + pz * pz);
+        const T t = at_least_0(gap) * reciprocal(rate);
+        const bool take = rate > 0 && t < step && !((in >> i) & 1u);
         step = take ? t : step;
         hit = take ? i : hit;
         hx = take ? x[i] : hx;
@@ -498,8 +503,8 @@ __device__ inline int walk_miniball(const double (&x)[K], const double (&y)[K], 
       m++;
       continue;
     }
-    const double l[4] = {1.0 - la - lb - lc, la, lb, lc};
-    double least = -1e-12;
+    const T l[4] = {1 - la - lb - lc, la, lb, lc};
+    T least = sizeof(T) == 4 ? (T)-1e-5 : (T)-1e-12;
     int out = -1;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -509,7 +514,7 @@ __device__ inline int walk_miniball(const double (&x)[K], const double (&y)[K], 
     }
     if (out < 0) return m;
     // the last of T takes the place of the one that leaves
-    double ex = tx[0], ey = ty[0], ez = tz[0];
+    T ex = tx[0], ey = ty[0], ez = tz[0];
     int ei = at[0], oi = at[0];
 #pragma unroll
     for (int q = 1; q < 4; ++q) {
@@ -541,8 +546,9 @@ struct DescentItems {
   uint32_t *F, *origin;
   uint64_t cap;
 };
-// counters of a round
-enum { D_OUT = 0, D_SLOW = 1, D_STEPS = 2 };
+// counters of a round: what still descends, what FP32 leaves open, the steps
+// taken, what FP64 leaves open
+enum { D_OUT = 0, D_OPEN = 1, D_STEPS = 2, D_SLOW = 3 };
 
 // One descent step of facet F (sorted ids): F := F - y + x, where x is the
 // least point strictly inside the facet's miniball and y its least support
@@ -552,21 +558,21 @@ enum { D_OUT = 0, D_SLOW = 1, D_STEPS = 2 };
 // that radius stays below the distance to its last entry (with margins far
 // above the FP64 rounding), and its walk ends at the first entry beyond it.
 // False: the certified filters or the list cannot decide the step.
-template <int K>
+template <int K, class T>
 __device__ inline bool descent_step(const ArmParams &A, uint32_t (&F)[K]) {
   int at[4] = {0, 0, 0, 0};
   int m;
   {
     const V3 o = P3(A.X, A.Y, A.Z, F[0]);
-    double x[K], y[K], z[K];
+    T x[K], y[K], z[K];
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const V3 p = sub(P3(A.X, A.Y, A.Z, F[i]), o);
-      x[i] = p.x;
-      y[i] = p.y;
-      z[i] = p.z;
+      x[i] = (T)p.x;
+      y[i] = (T)p.y;
+      z[i] = (T)p.z;
     }
-    m = walk_miniball<K>(x, y, z, at);
+    m = walk_miniball<K, T>(x, y, z, at);
   }
   if (m < 2) return false;
   uint32_t sid[4];
@@ -653,16 +659,18 @@ __device__ inline bool descent_step(const ArmParams &A, uint32_t (&F)[K]) {
 
 // One round of the descents: up to `steps` steps per item, each followed by
 // the lookup of the new facet; what still descends goes to `out`, what the
-// step leaves open to `slow`.  queue != nullptr: the first round, whose items
+// step leaves open to `slow`.  T = float, then double over what that left open
+// (one step).  queue != nullptr: the first round, whose items
 // are queued arms.  Bound by the gathers of the neighbours' coordinates and
 // the FP64 predicates; Welzl's miniball and a tree traversal per step, with
 // the facet in scratch memory, took 66 ms of the 50 000-point tower at 0.22
 // lane utilisation (order 10: 28 ms, 7 here).
 constexpr int kDescentBlock = 256;
-template <int K>
+template <int K, class T>
 __global__ void __launch_bounds__(kDescentBlock) k_descend(ArmParams A, const uint32_t *queue, DescentItems in,
                                                            uint32_t n_in, DescentItems out, DescentItems slow,
                                                            int steps, unsigned long long *counters) {
+  constexpr int kLeft = sizeof(T) == 4 ? D_OPEN : D_SLOW;
   const uint64_t i = (uint64_t)blockIdx.x * kDescentBlock + threadIdx.x;
   bool next = false, open = false;
   uint32_t F[K], origin = 0, done = 0;
@@ -681,7 +689,7 @@ __global__ void __launch_bounds__(kDescentBlock) k_descend(ArmParams A, const ui
     next = true;
 #pragma unroll 1
     for (int t = 0; next && t < steps; ++t) {
-      if (!descent_step<K>(A, F)) {
+      if (!descent_step<K, T>(A, F)) {
         next = false;
         open = true;
         break;
@@ -704,7 +712,7 @@ __global__ void __launch_bounds__(kDescentBlock) k_descend(ArmParams A, const ui
     out.origin[at] = origin;
   }
   (void)block_append<kDescentBlock / 64>(done, counters + D_STEPS);
-  const unsigned long long sl = block_append<kDescentBlock / 64>(open ? 1u : 0u, counters + D_SLOW);
+  const unsigned long long sl = block_append<kDescentBlock / 64>(open ? 1u : 0u, counters + kLeft);
   if (open) {
 #pragma unroll
     for (int q = 0; q < K; ++q) slow.F[q * slow.cap + sl] = F[q];
@@ -918,9 +926,10 @@ __device__ bool slow_step(const ArmParams &A, int k, uint32_t *F, uint32_t *stk,
 }
 
 template <int K>
-__global__ void __launch_bounds__(kSlowBlock) k_descend_slow(ArmParams A, DescentItems in, uint32_t n_in,
-                                                             DescentItems out, unsigned long long *counters) {
+__global__ void __launch_bounds__(kSlowBlock) k_descend_slow(ArmParams A, DescentItems in, DescentItems out,
+                                                             unsigned long long *counters) {
   __shared__ uint32_t stk[kSlowStack * kSlowBlock];
+  const uint64_t n_in = counters[D_SLOW];  // the launch has threads for more
   const int lane = threadIdx.x;
   const uint64_t i = (uint64_t)blockIdx.x * kSlowBlock + lane;
   bool next = false, stepped = false;
@@ -1620,7 +1629,7 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
   }
   uint64_t steps_total = 0, slow_total = 0;
   if (nq && k >= 2) {
-    DescentItems items[3];  // two rounds' items, and what the fast steps leave open
+    DescentItems items[3];  // two rounds' items, and what FP32 leaves open
     for (int q = 0; q < 3; ++q) {
       W.dF[q].ensure((size_t)k * nq);
       W.dO[q].ensure(nq);
@@ -1639,18 +1648,20 @@ void tower_order_device(Context &c, TowerWork &W, const TowerWork &R, int k, Tow
       const int steps = active <= 1u << 17 ? 8 : 1;
       hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, W.dcount.p, (int64_t)4, 0ull);
       with_order(k, [&](auto K) {
-        hipLaunchKernelGGL((k_descend<K.value>), dim3(blocks_for(active, kDescentBlock)), dim3(kDescentBlock), 0, s, A,
-                           round == 0 ? queue.p : nullptr, items[q ^ 1], active, items[q], items[2], steps, counters);
+        hipLaunchKernelGGL((k_descend<K.value, float>), dim3(blocks_for(active, kDescentBlock)), dim3(kDescentBlock), 0,
+                           s, A, round == 0 ? queue.p : nullptr, items[q ^ 1], active, items[q], items[2], steps, counters);
       });
-      copy_wait(got, W.dcount.p, 24, hipMemcpyDeviceToHost, s);
-      const uint32_t slow = (uint32_t)got[D_SLOW];
-      if (slow) {
+      copy_wait(got, W.dcount.p, sizeof got, hipMemcpyDeviceToHost, s);
+      if (const uint32_t open = (uint32_t)got[D_OPEN]) {
+        // the round's input is done: its list takes what FP64 leaves open too
         with_order(k, [&](auto K) {
-          hipLaunchKernelGGL((k_descend_slow<K.value>), dim3(blocks_for(slow, kSlowBlock)), dim3(kSlowBlock), 0, s, A,
-                             items[2], slow, items[q], counters);
+          hipLaunchKernelGGL((k_descend<K.value, double>), dim3(blocks_for(open, kDescentBlock)), dim3(kDescentBlock), 0, s,
+                             A, nullptr, items[2], open, items[q], items[q ^ 1], 1, counters);
+          hipLaunchKernelGGL((k_descend_slow<K.value>), dim3(blocks_for(open, kSlowBlock)), dim3(kSlowBlock), 0, s, A,
+                             items[q ^ 1], items[q], counters);
         });
-        copy_wait(got, W.dcount.p, 24, hipMemcpyDeviceToHost, s);
-        slow_total += slow;
+        copy_wait(got, W.dcount.p, sizeof got, hipMemcpyDeviceToHost, s);
+        slow_total += got[D_SLOW];
       }
       steps_total += got[D_STEPS];
       active = (uint32_t)got[D_OUT];
