@@ -28,6 +28,7 @@ struct ExactJob {
   // Exact classification of a support against a region (the region holds
   // every point of any relevant sphere through the anchor).
   void support(const int64_t *ids, int m, const uint32_t *region, uint32_t len) {
+    if (m > s_max) return;  // its closed rank is at least m
     ExactSupport S;
     predicates++;
     if (!S.analyze(ex, ids, m) || !S.well) return;

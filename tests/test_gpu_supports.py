@@ -290,3 +290,18 @@ def test_wide_gathers_take_the_slab_mask_probe(n, k, monkeypatch, capfd):
     assert sum(wider) > 0
     if n > 2048:
         assert sum(big) > 0
+
+
+@pytest.mark.parametrize("k", [1, 2])
+@pytest.mark.parametrize("name", ["grid", "tenths", "snapped"])
+def test_degenerate_clouds_keep_to_the_closed_rank(name, k):
+    """Clouds whose faces go to the host undecided, at K_max 1 and 2: the host
+    tries no support of more points than the closed rank allows."""
+    g = np.stack(np.meshgrid(np.arange(4), np.arange(4), np.arange(4), indexing="ij"), axis=-1).reshape(-1, 3)
+    if name == "grid":
+        pts = g.astype(float)[np.random.default_rng(1).permutation(64)[:50]]
+    elif name == "tenths":
+        pts = (g * 0.1)[np.random.default_rng(2).permutation(64)[:50]]
+    else:
+        pts = workloads.gaussian_mixture(70, blobs=3, noise_fraction=0.15, box=2.0, snap_bits=3, seed=117)
+    _compare(pts, k, f"{name}-k{k}")
