@@ -458,54 +458,75 @@ struct BehindList {
   }
 };
 
-// The same two lists in 32-bit fixed point, filled for both sides during a
-// face's pass without a branch: a point of the other side goes in as the
-// weakest value.  Keys are scaled so that the end of the face's pencil is
-// kLimit; a point whose key lies past it cannot be an apex.  An entry of the
-// sweep list is the key's upper bound, above SB bits of region slot, so that
-// one median of three per entry keeps bound and slot in order; its lower bound
-// is the entry less the face's widest interval.  All bounds err outwards: a
-// wider interval only admits more apex candidates, which are classified
-// exactly, or sends a side to k_rescan.
-__device__ inline uint32_t umed3(uint32_t a, uint32_t b, uint32_t c) { return max(min(a, b), min(max(a, b), c)); }
-template <int SB>
+// The same two lists in FP32, filled for both sides during a face's pass
+// without a branch: a point of the other side goes in as the weakest value.  An
+// entry of the sweep list is a double whose high word is the key's FP32 upper
+// bound (at least 0, so the word's order is the bound's, and no double that
+// begins with it is infinite or NaN) and whose low word is the region slot: one
+// minimum and one maximum per entry keep bound and slot in order.  A point whose
+// key lies past the end of the face's pencil cannot be an apex, so bounds end
+// there.  An entry's lower bound is the entry less the face's widest interval.
+// All bounds err outwards: a wider interval only admits more apex candidates,
+// which are classified exactly, or sends a side to k_rescan.  Against one word
+// an entry (22 to 24 bits of fixed point above the slot, a median of three
+// each) this costs nothing that the runs show (50 000 points K 10: 43.7 and
+// 43.9 ms; the 2 003-point mixture 27.5 and 27.6), and a face whose pencil has
+// no end keeps its keys apart.
+// Minimum and maximum are the bare instructions: on values that a loop carries
+// the compiler has fmin and fmax quiet a signalling NaN first, which no entry is
+// (the mixture 29.7 ms with them).
+__device__ inline double min_entry(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline double max_entry(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 struct SweepListF {
   static constexpr int kCap = 8;  // >= s_max - 3 for s_max <= 11
-  static constexpr float kLimit = (float)((1u << (32 - SB)) - 8u);
-  uint32_t hi[kCap];  // entries, ascending; kInvalid: empty
-  uint32_t evicted;   // smallest entry that left or missed the list
+  static constexpr int kNone = 0x7f900000;  // past every bound (infinity is 0x7f800000)
+  double hi[kCap];  // entries, ascending
+  double evicted;   // smallest entry that left or missed the list
+  __device__ static double none() { return __hiloint2double(kNone, 0); }
+  __device__ static bool used(double e) { return __double2hiint(e) != kNone; }
+  __device__ static float bound(double e) { return __int_as_float(__double2hiint(e)); }
+  __device__ static uint32_t slot(double e) { return (uint32_t)__double2loint(e); }
   __device__ void init() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) hi[j] = kInvalid;
-    evicted = kInvalid;
+    for (int j = 0; j < kCap; ++j) hi[j] = none();
+    evicted = none();
   }
-  __device__ void insert(uint32_t e) {
-    evicted = min(evicted, max(hi[kCap - 1], e));
+  __device__ void insert(double e) {
+    evicted = min_entry(evicted, max_entry(hi[kCap - 1], e));
 #pragma unroll
-    for (int j = kCap - 1; j > 0; --j) hi[j] = umed3(hi[j - 1], e, hi[j]);
-    hi[0] = min(hi[0], e);
+    for (int j = kCap - 1; j > 0; --j) hi[j] = max_entry(hi[j - 1], min_entry(hi[j], e));
+    hi[0] = min_entry(hi[0], e);
   }
-  __device__ uint32_t threshold(int need) const {
-    uint32_t r = kInvalid;
+  // upper bound of the need-th entry, infinite when there are fewer
+  __device__ float threshold(int need) const {
+    double r = none();
 #pragma unroll
     for (int j = 0; j < kCap; ++j) r = (j == need - 1) ? hi[j] : r;
-    return r >> SB;
+    return used(r) ? bound(r) : INFINITY;
   }
 };
 struct BehindListF {
   static constexpr int kCap = 4;
-  uint32_t v[kCap];
+  float v[kCap];
   __device__ void init() {
 #pragma unroll
-    for (int j = 0; j < kCap; ++j) v[j] = 0;
+    for (int j = 0; j < kCap; ++j) v[j] = 0.0f;
   }
-  __device__ void insert(uint32_t x) {
+  __device__ void insert(float x) {
     // descending: the median of the entry above, x and the entry
 #pragma unroll
-    for (int j = kCap - 1; j > 0; --j) v[j] = umed3(v[j - 1], x, v[j]);
-    v[0] = max(v[0], x);
+    for (int j = kCap - 1; j > 0; --j) v[j] = __builtin_amdgcn_fmed3f(v[j - 1], x, v[j]);
+    v[0] = fmaxf(v[0], x);
   }
-  __device__ int count_above(uint32_t x) const {
+  __device__ int count_above(float x) const {
     int c = 0;
 #pragma unroll
     for (int j = 0; j < kCap; ++j) c += v[j] > x;
@@ -677,22 +698,21 @@ static_assert(sizeof(Rescan) == kRescanBytes, "rescan layout");
 // Apexes of one side among the FP32 list its face's pass filled: bit j for
 // entry j.  rescan: a point left or missed the list with a lower bound within
 // the threshold, so the side takes its own passes instead.
-template <int SB>
-__device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF<SB> &top, const BehindListF &beh,
-                                     uint32_t widest, bool &rescan) {
+__device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF &top, const BehindListF &beh,
+                                     float widest, bool &rescan) {
   rescan = false;
   if (cin_side >= K) return 0;
-  const uint32_t thr = top.threshold(K - cin_side) + widest;
-  if (top.evicted != kInvalid && (top.evicted >> SB) <= thr) {
+  const float thr = (top.threshold(K - cin_side) + widest) * (1.0f + 1e-6f);  // past both roundings
+  if (SweepListF::used(top.evicted) && SweepListF::bound(top.evicted) <= thr) {
     rescan = true;
     return 0;
   }
   uint32_t cand = 0;
 #pragma unroll
-  for (int j = 0; j < SweepListF<SB>::kCap; ++j) {
+  for (int j = 0; j < SweepListF::kCap; ++j) {
     // inside points behind: counted while their key exceeds z's
-    const uint32_t h = top.hi[j] >> SB;
-    const bool ok = top.hi[j] != kInvalid && h <= thr && cin_side + beh.count_above(h) < K;
+    const float h = SweepListF::bound(top.hi[j]);
+    const bool ok = SweepListF::used(top.hi[j]) && h <= thr && cin_side + beh.count_above(h) < K;
     cand |= ok ? (1u << j) : 0u;
   }
   return cand;
@@ -708,7 +728,7 @@ __device__ inline uint32_t apex_mask(int cin_side, int K, const SweepListF<SB> &
 // The pass runs on the region's FP32 copies (FP64 only for the points whose FP32
 // signs are not certified) and sees the points that some sphere of the face's
 // pencil within [lo, hi] (face_interval; n oriented as v x w) can hold.
-template <bool QUEUED, int SB>
+template <bool QUEUED>
 __device__ __attribute__((always_inline)) inline void process_face(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t vi,
                              uint32_t wi, float lo, float hi, uint32_t *region_slot, WaveQueues *q) {
   // the sphere is built from its points in PointId order, so its FP64 level
@@ -740,7 +760,7 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
   // s_max - 3 <= 8)
   uint32_t tri_pk[kPacked] = {};
   uint32_t evals = 0;
-  SweepListF<SB> top0, top1;  // outside points ahead of side 0 / 1
+  SweepListF top0, top1;  // outside points ahead of side 0 / 1
   BehindListF beh0, beh1;  // inside points behind side 0 / 1
   top0.init();
   top1.init();
@@ -748,10 +768,8 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
   beh1.init();
   constexpr uint32_t kFlopPoint = kFlopFacePoint + kFlopSweepKey;
   uint32_t tests32 = 0, evals32 = 0;  // FP32 work
-  constexpr float kLimit = SweepListF<SB>::kLimit;
-  const double per_key = kLimit / pen.end;
-  const float scale = per_key < 1e37 ? (float)per_key : 0.0f;  // 0: all keys are equal
-  uint32_t widest = 0;                                          // widest key interval
+  const float end = pen.end > 1e-30 ? (float)(pen.end * (1.0 + 1e-6)) : INFINITY;  // no apex past it
+  float widest = 0.0f;                                                             // widest key interval
   const int tri_limit = tri ? smax - 2 : 0;  // inside points that exclude the triangle
   TriSphereF f32;
   f32.init(f);
@@ -791,22 +809,22 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
         key_bounds_f(tau, terr, hf, lf);
         outer = sp > 0;
         above = sh > 0;
+        if (!(lf <= hf)) hf = INFINITY, lf = 0.0f;  // overflow: unknown
+        lf = fmaxf(lf, 0.0f);                        // used of outside points, whose keys are positive
         if (!outer) hf = fminf(hf, 0.0f);  // a key interval that reaches past 0: weakest
       }
-      // fixed point, the multiplication's rounding and the truncation within 2
-      const uint32_t h = (uint32_t)fminf(fabsf(hf * scale), kLimit);
       // outside: ahead of side 0 when above, of side 1 otherwise
-      const float ls = lf * scale;
-      const bool ahead = outer && !(ls >= kLimit);
-      const uint32_t e = (h + 2u) << SB | gi, width = h + 4u - (uint32_t)__builtin_amdgcn_fmed3f(ls, 0.0f, kLimit);
-      widest = max(widest, ahead ? width : 0u);
-      top0.insert(ahead && above ? e : kInvalid);
-      top1.insert(ahead && !above ? e : kInvalid);
+      const bool ahead = outer && !(lf >= end);
+      hf = fminf(hf, end);
+      widest = fmaxf(widest, ahead ? hf - lf : 0.0f);
+      const int key = __float_as_int(hf);
+      top0.insert(__hiloint2double(ahead && above ? key : SweepListF::kNone, (int)gi));
+      top1.insert(__hiloint2double(ahead && !above ? key : SweepListF::kNone, (int)gi));
       // inside: behind side 1 when above, behind side 0 otherwise; -hf is a
       // lower bound of -tau - terr
-      const uint32_t x = outer ? 0u : max(h, 2u) - 2u;
-      beh0.insert(above ? 0u : x);
-      beh1.insert(above ? x : 0u);
+      const float x = outer ? 0.0f : -hf;
+      beh0.insert(above ? 0.0f : x);
+      beh1.insert(above ? x : 0.0f);
       if (outer) continue;
       push_packed(tri_pk, gi);
       total_in++;
@@ -838,18 +856,17 @@ __device__ __attribute__((always_inline)) inline void process_face(const Params 
   if (K <= 0) return;
   bool rescan[2];
   uint32_t cand = apex_mask(cin0, K, top0, beh0, widest, rescan[0]);
-  cand |= apex_mask(cin1, K, top1, beh1, widest, rescan[1]) << SweepListF<SB>::kCap;
+  cand |= apex_mask(cin1, K, top1, beh1, widest, rescan[1]) << SweepListF::kCap;
   // queued on the LDS paths, in place on the global-memory path
   while (cand) {
     const int j = __ffs(cand) - 1;
     cand &= cand - 1;
-    uint32_t ent = 0;  // selected by static index, the lists stay in registers
+    uint32_t zi = 0;  // selected by static index, the lists stay in registers
 #pragma unroll
-    for (int e = 0; e < SweepListF<SB>::kCap; ++e) {
-      ent = e == j ? top0.hi[e] : ent;
-      ent = e + SweepListF<SB>::kCap == j ? top1.hi[e] : ent;
+    for (int e = 0; e < SweepListF::kCap; ++e) {
+      zi = e == j ? SweepListF::slot(top0.hi[e]) : zi;
+      zi = e + SweepListF::kCap == j ? SweepListF::slot(top1.hi[e]) : zi;
     }
-    const uint32_t zi = ent & ((1u << SB) - 1u);
     if (w.gid[zi] <= wid) continue;
     if (QUEUED) {
       const uint32_t at = atomicAdd(q->ntet, 1u);
@@ -1092,7 +1109,7 @@ __device__ inline bool face_interval(const Params &P, const Work &w, uint32_t si
 // beyond one per kSplitFaces candidate faces have nothing to do (2 048: the
 // mixture's catalogue 3% slower; 512 below a wave's round).
 constexpr uint64_t kSplitFaces = 1024;
-template <bool BIG, bool SPLIT, int WAVES, int SB>
+template <bool BIG, bool SPLIT, int WAVES>
 __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_t M, uint32_t *sK_,
                              uint32_t *sregion_) {
   uint32_t &sK = *sK_;
@@ -1162,7 +1179,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       uint32_t si, sj;
       face_of(fidx, si, sj);
       float lo, hi, key;
-      if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false, SB>(P, w, u, M, si, sj, lo, hi, &sregion, q);
+      if (face_interval(P, w, si, sj, lo, hi, key)) process_face<false>(P, w, u, M, si, sj, lo, hi, &sregion, q);
     }
   } else {
     // Each wave lists the candidate faces that share a cell (q_pair), takes 64
@@ -1245,7 +1262,7 @@ __device__ void anchor_faces(const Params &P, const Work &w, uint32_t u, uint32_
       if ((uint32_t)lane < take) {
         const uint32_t fv = q_face[wave][nf + lane];
         const uint32_t si = fv & 1023u, sj = fv >> 10;
-        process_face<true, SB>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
+        process_face<true>(P, w, u, M, si, sj, q_lo[wave][nf + lane], q_hi[wave][nf + lane], &sregion, q);
       }
       wave_sync();
       // whole rounds of 64 tetrahedra (the top of the queue); the rest waits
@@ -1455,7 +1472,7 @@ __device__ void anchor_work(const Params &P, const Work &w, uint32_t u, uint32_t
     if (t == 0) probed(P, u, a, M);
     return;
   }
-  anchor_faces<true, false, kBlock / 64, 11>(P, w, u, M, &sK, &sregion);
+  anchor_faces<true, false, kBlock / 64>(P, w, u, M, &sK, &sregion);
 }
 
 __device__ inline void probed(const Params &P, uint32_t u, uint32_t a, uint32_t M) {
@@ -1828,7 +1845,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_anchor_region(Params P
   __syncthreads();
   Work w{gx, gy, gz, gid, rho, nullptr, rmask, kidx, nullptr, &cand, P.count_flops ? &flops : nullptr, f,
          P.count_flops ? &flops32 : nullptr, true, a, cell};
-  anchor_faces<false, true, WAVES, RCAP <= 256 ? 8 : RCAP <= 512 ? 9 : 10>(P, w, u, M, &sK, &sregion);
+  anchor_faces<false, true, WAVES>(P, w, u, M, &sK, &sregion);
 }
 
 // Sides of faces left by the enumeration of one launch, one per wave, in FP64

@@ -305,3 +305,26 @@ def test_degenerate_clouds_keep_to_the_closed_rank(name, k):
     else:
         pts = workloads.gaussian_mixture(70, blobs=3, noise_fraction=0.15, box=2.0, snap_bits=3, seed=117)
     _compare(pts, k, f"{name}-k{k}")
+
+
+@pytest.mark.parametrize("bend", [1e-4, 1e-5])
+def test_sides_of_nearly_collinear_faces_are_decided_by_their_lists(bend, capfd, monkeypatch):
+    """Three points nearly on a line have a pencil of spheres without an end;
+    the FP32 keys of the points ahead of such a face still tell its apexes
+    apart, so fewer than one such triple in twenty is left to the rescans."""
+    r = np.random.default_rng(1)
+    n, m, step = 600, 200, 0.05
+    pts = r.uniform(size=(n, 3))
+    along = r.normal(size=(m, 3))
+    along /= np.linalg.norm(along, axis=1)[:, None]
+    across = np.cross(along, r.normal(size=(m, 3)))
+    across /= np.linalg.norm(across, axis=1)[:, None]
+    pts = np.concatenate([pts, pts[:m] + step * along, pts[:m] + 2 * step * along + step * bend * across])
+    monkeypatch.setenv("MHGP_TIMING", "1")
+    with mhgp.Context(0) as ctx:
+        ctx.upload(pts)
+        capfd.readouterr()
+        info = ctx.supports(8, fetch=False)
+    lines = [ln for ln in capfd.readouterr().err.splitlines() if "sides left to the rescans" in ln]
+    assert info.status == 0 and lines
+    assert max(int(ln.split()[-1]) for ln in lines) < m // 20
